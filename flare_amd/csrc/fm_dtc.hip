@@ -370,8 +370,10 @@ __global__ void k_var_efs(int n_out, int dtc, const double *kself, const double 
   int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= n_out) return;
   double q = 0, v = 0;
-  for (int t = 0; t < nq; t++) q += Qp[(size_t)t * n_out + c];
-  for (int t = 0; t < nv; t++) v += Vp[(size_t)t * n_out + c];
+  for (int t = 0; t < nq; t += 2)
+    q += Qp[(size_t)t * n_out + c] + Qp[(size_t)(t + 1) * n_out + c];
+  for (int t = 0; t < nv; t += 2)
+    v += Vp[(size_t)t * n_out + c] + Vp[(size_t)(t + 1) * n_out + c];
   var[c] = dtc ? kself[c] - q + v : v;
 }
 
@@ -676,8 +678,8 @@ void predict_dense(fm_model m, fm_structure s, int kind, double *mean_efs, doubl
   if (dtc) self_kernel(m, s, ks);
   // |L_inv K_c|^2 per species block and |R_inv^T K_c|^2.
   int nq = 0;
-  for (int t = 0; t < m->nos; t++) nq += dtc ? gemm_row_tiles(FM_FORM_FP64, m->L_rows[t]) : 0;
-  int nv = gemm_row_tiles(FM_FORM_FP64, M);
+  for (int t = 0; t < m->nos; t++) nq += dtc ? gemm_row_tiles(m->L_rows[t]) : 0;
+  int nv = gemm_row_tiles(M);
   DevBuf Qp(pool, std::max<size_t>(1, (size_t)nq * n_out * sizeof(double)));
   DevBuf Vp(pool, std::max<size_t>(1, (size_t)nv * n_out * sizeof(double)));
   int qo = 0;
@@ -689,7 +691,7 @@ void predict_dense(fm_model m, fm_structure s, int kind, double *mean_efs, doubl
       eq.part_ld = n_out;
       gemm_f64(st, EP_SUMSQ, m->L_rows[t], (int)n_out, m->M_by_type[t], m->L[t].as<double>(),
                m->M_by_type[t], Kt.as<double>() + m->off[t], M, m->L_lower[t], eq);
-      qo += gemm_row_tiles(FM_FORM_FP64, m->L_rows[t]);
+      qo += gemm_row_tiles(m->L_rows[t]);
     }
   {
     EpArgs ev;

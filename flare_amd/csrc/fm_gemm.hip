@@ -1,29 +1,30 @@
-// Kernel contraction on the matrix cores. Every contraction of the path has
-// the form C = A . B^T with both operands contiguous along the reduction
-// index; a workgroup of 4 wavefronts (2 x 2) computes a tile, each wave
-// TM x TN MFMA tiles of 16 x 16, with a fused epilogue:
+// Contractions on the matrix cores. Every contraction of the path has the
+// form C = A . B^T with both operands contiguous along the reduction index
+// and a fused epilogue:
 //
-//   EpKernel  C = B_s . X_hat_s^T (atoms x sparse): S = C / |B_i|,
+//   EP_KERNEL C = B_s . X_hat_s^T (atoms x sparse): S = C / |B_i|,
 //             k = sigma^2 S^p, w = sigma^2 alpha_j p S^(p-1); writes w and
 //             (optionally) k atom-major and per-tile partial energies
 //             sum_j k alpha_j (normalized_dot_product.cpp:117-177 contracted
 //             with alpha as sparse_gp.cpp:664).
-//   EpStore   plain store: G = W . X_hat_s (the kernel-gradient contraction).
-//   EpSumSq   Q = L_s^-1 . K^T with per-tile column sums of Q^2, the local
+//   EP_STORE  plain store: G = W . X_hat_s (the kernel-gradient contraction).
+//   EP_SUMSQ  Q = L_s^-1 . K^T with per-tile column sums of Q^2, the local
 //             variance term |L_inv k|^2 (sparse_gp.cpp:121-131); A is lower
 //             triangular so each row tile stops at its last nonzero column.
 //
-// FP64 form: v_mfma_f64_16x16x4f64, 64 x 64 tiles, for all three. Chosen
-// form: EpKernel is exact on int8 MFMA (v_mfma_i32_32x32x32_i8) over five
-// power-of-two-scaled slices of each operand row, int32 accumulation per
-// slice-pair diagonal and an FP64 epilogue (k_gemm_i8); EpStore is
-// split-BF16 x3 on v_mfma_f32_16x16x32_bf16 (a = a_hi + a_lo, ab ~ a_hi b_hi
-// + a_hi b_lo + a_lo b_hi, FP32 accumulation), 128 x 128 tiles, on operands
-// split once where they are produced, the three products of a k-step run
-// over all 16 accumulators of a wave before the next, so consecutive MFMAs
-// are independent; EpSumSq stays FP64.
+// FP64 form: k_gemm_f64 for all three. Chosen form: EP_KERNEL is exact on
+// int8 MFMA (v_mfma_i32_32x32x32_i8) over five power-of-two-scaled slices of
+// each operand row, int32 accumulation per slice-pair diagonal and an FP64
+// epilogue (k_gemm_i8); EP_STORE is split-BF16 x3 on
+// v_mfma_f32_16x16x32_bf16 (a = a_hi + a_lo, ab ~ a_hi b_hi + a_hi b_lo +
+// a_lo b_hi, FP32 accumulation), on operands split once where they are
+// produced, the three products of a k-step run over all accumulators of a
+// wave before the next, so consecutive MFMAs are independent; EP_SUMSQ stays
+// FP64.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -95,103 +96,13 @@ __device__ __forceinline__ int tile_row(int lane, int i) {
   return sizeof(Acc) == 8 ? (lane >> 4) + 4 * i : 4 * (lane >> 4) + i;
 }
 
+// Kept out of line: inlined into every element of an unrolled epilogue, pow
+// makes the loops too large to unroll.
+__device__ __noinline__ double pow_general(double x, double p) { return pow(x, p); }
 __device__ __forceinline__ double fpow(double x, double p, int pi) {
   if (pi == 2) return x * x;
   if (pi == 1) return x;
-  return pow(x, p);
-}
-// Kept out of line: inlined into every element of the unrolled FP32
-// epilogue, powf makes the loop too large to unroll.
-__device__ __noinline__ float powf_general(float x, float p) { return powf(x, p); }
-__device__ __forceinline__ float fpow(float x, float p, int pi) {
-  if (pi == 2) return x * x;
-  if (pi == 1) return x;
-  return powf_general(x, p);
-}
-
-template <typename Acc, typename TW, int TM, int TN>
-__device__ __forceinline__ void ep_kernel(const EpArgs &e, const TileOut<Acc, TM, TN> &t, int row0, int col0,
-                          int M, int N, int lane, int wr, int wc, double *red) {
-  constexpr int BMc = 32 * TM;
-  // rows: atoms of this species block, cols: sparse environments.
-  int pi = e.power == 2.0 ? 2 : (e.power == 1.0 ? 1 : 0);
-  double rs[TM][4];
-#pragma unroll
-  for (int ti = 0; ti < TM; ti++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) rs[ti][i] = 0;
-#pragma unroll
-  for (int ti = 0; ti < TM; ti++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      int r = row0 + wr * 16 * TM + ti * 16 + tile_row<Acc>(lane, i);
-      if (r >= M) continue;
-      double nrm = e.row_norm[r];
-      bool empty = nrm < kEmptyThresh;
-      Acc ninv = empty ? Acc(0) : Acc(1.0 / nrm);
-#pragma unroll
-      for (int tj = 0; tj < TN; tj++) {
-        int c = col0 + wc * 16 * TN + tj * 16 + (lane & 15);
-        if (c >= N) continue;
-        Acc s = t.v[ti][tj][i] * ninv;
-        Acc a = (Acc)e.alpha[c];
-        Acc kv = empty ? Acc(0) : Acc(e.sig2) * fpow(s, (Acc)e.power, pi);
-        Acc pm1 = pi == 2 ? s : (pi == 1 ? Acc(1) : fpow(s, (Acc)(e.power - 1), 0));
-        Acc wv = empty ? Acc(0) : Acc(e.sig2) * a * (Acc)e.power * pm1;
-        if constexpr (sizeof(Acc) == 4) {  // split-BF16 form: w as BF16 pairs
-          float wf = (float)wv;
-          __bf16 h = (__bf16)wf;
-          reinterpret_cast<__bf16 *>(e.Wh)[(size_t)r * e.ldw + c] = h;
-          reinterpret_cast<__bf16 *>(e.Wl)[(size_t)r * e.ldw + c] = (__bf16)(wf - (float)h);
-        } else {
-          e.W_as<TW>()[(size_t)r * e.ldw + c] = (TW)wv;
-        }
-        if (e.K) e.K_as<Acc>()[(size_t)r * e.ldk + c] = kv;
-        rs[ti][i] += (double)(kv * a);
-      }
-    }
-  if constexpr (sizeof(Acc) == 4) {
-    // Padding columns [N, ldw) of the split output are zero: they are the
-    // reduction tail of the next contraction.
-#pragma unroll
-    for (int ti = 0; ti < TM; ti++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        int r = row0 + wr * 16 * TM + ti * 16 + tile_row<Acc>(lane, i);
-        if (r >= M) continue;
-#pragma unroll
-        for (int tj = 0; tj < TN; tj++) {
-          int c = col0 + wc * 16 * TN + tj * 16 + (lane & 15);
-          if (c >= N && c < e.ldw) {
-            reinterpret_cast<__bf16 *>(e.Wh)[(size_t)r * e.ldw + c] = (__bf16)0.0f;
-            reinterpret_cast<__bf16 *>(e.Wl)[(size_t)r * e.ldw + c] = (__bf16)0.0f;
-          }
-        }
-      }
-  }
-  // Sum over the 16 columns of each lane group, then over the two wave
-  // columns through LDS; one partial per (column tile, row).
-#pragma unroll
-  for (int ti = 0; ti < TM; ti++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      double v = rs[ti][i];
-#pragma unroll
-      for (int off = 8; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-      rs[ti][i] = v;
-    }
-  if ((lane & 15) == 0) {
-#pragma unroll
-    for (int ti = 0; ti < TM; ti++)
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-        red[wc * BMc + wr * 16 * TM + ti * 16 + tile_row<Acc>(lane, i)] = rs[ti][i];
-  }
-  __syncthreads();
-  for (int q = threadIdx.x; q < BMc; q += blockDim.x) {
-    int r = row0 + q;
-    if (r < M) e.part[(size_t)(col0 / (32 * TN)) * e.part_ld + r] = red[q] + red[BMc + q];
-  }
+  return pow_general(x, p);
 }
 
 template <typename Acc, typename TW, int TM, int TN>
@@ -211,156 +122,536 @@ __device__ __forceinline__ void ep_store(const EpArgs &e, const TileOut<Acc, TM,
     }
 }
 
-template <typename Acc, int TM, int TN>
-__device__ __forceinline__ void ep_sumsq(const EpArgs &e, const TileOut<Acc, TM, TN> &t, int row0, int col0,
-                         int M, int N, int lane, int wr, int wc, double *red) {
-  constexpr int BNc = 32 * TN;
-  // rows: L rows, cols: atoms. Column sums of squares over this row tile.
-  double cs[TN];
+// ---------------------------------------------------------------------------
+// FP64 contraction C = A B^T (rows of both K-contiguous) on
+// v_mfma_f64_16x16x4: k_gemm_f64 with fragments straight from global memory
+// and k_gemm_f64_lds with 128 x 128 tiles staged in LDS; f64_tile chooses.
+//
+// What bounds them: an FP64 16x16x4 MFMA holds its SIMD's vector ALU for 64
+// cycles, so a wave with 64 x 64 outputs needs 16 KB per 4096 cycles; smaller
+// wave tiles need more and are bound by their loads (12 TB/s from L2). The
+// kernel these two replace (64 x 64 to 128 x 128 tiles in LDS, two barriers
+// and transposed 8-byte LDS stores per 16 k, all accumulators moved between
+// register files in every iteration) ran the kernel contraction of 32,000 x
+// 1,000 x 2,100 at 48 TFLOP/s.
+//
+// The variance sigma^2 - |Q|^2 amplifies rounding (near the sparse set one ulp
+// of |Q|^2 is 1e-9 of it), so the kernel contraction and Q keep one order of
+// sums whatever the tile: 4 consecutive k per MFMA, ascending from k = 0, and
+// |Q|^2 over 32 rows of L at a time. The gradient contraction (EP_STORE) takes
+// its 16 k per step in an order that loads better, the same for any tile. So
+// the choice of tile changes no bit: batched, tiled and single evaluations
+// agree.
+// ---------------------------------------------------------------------------
+// Sum over the 16 lanes of a row on the VALU (no LDS round trips): partners
+// 1, 2, 7 and 15 lanes away by quad permutes and row mirrors.
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double x) {
+  long long v = __builtin_bit_cast(long long, x);
+  int lo = __builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
+  int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double row16_sum(double x) {
+  x += dpp_f64<0xb1>(x);   // quad_perm 1, 0, 3, 2
+  x += dpp_f64<0x4e>(x);   // quad_perm 2, 3, 0, 1
+  x += dpp_f64<0x141>(x);  // row_half_mirror
+  x += dpp_f64<0x140>(x);  // row_mirror
+  return x;
+}
+
+// Element j of lane group g (lanes 16 g .. 16 g + 15) becomes element g of
+// group j: a 4 x 4 transpose across the four lane groups.
+__device__ __forceinline__ void transpose_groups(double (&x)[4]) {
+  unsigned d[4][2];
 #pragma unroll
-  for (int tj = 0; tj < TN; tj++) {
-    cs[tj] = 0;
+  for (int j = 0; j < 4; j++) {
+    unsigned long long v = __builtin_bit_cast(unsigned long long, x[j]);
+    d[j][0] = (unsigned)v, d[j][1] = (unsigned)(v >> 32);
+  }
 #pragma unroll
-    for (int ti = 0; ti < TM; ti++)
+  for (int w = 0; w < 2; w++) {
+#pragma unroll
+    for (int j = 0; j < 2; j++) {  // groups 2, 3 of j against 0, 1 of j + 2
+      auto r = __builtin_amdgcn_permlane32_swap(d[j][w], d[j + 2][w], false, false);
+      d[j][w] = r[0], d[j + 2][w] = r[1];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j += 2) {  // groups 1, 3 of j against 0, 2 of j + 1
+      auto r = __builtin_amdgcn_permlane16_swap(d[j][w], d[j + 1][w], false, false);
+      d[j][w] = r[0], d[j + 1][w] = r[1];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+    x[j] = __builtin_bit_cast(double, (unsigned long long)d[j][1] << 32 | d[j][0]);
+}
+
+// 16 bytes at 8-byte alignment (rows of odd length).
+typedef double v2d __attribute__((ext_vector_type(2), aligned(8)));
+typedef double v2da __attribute__((ext_vector_type(2)));
+
+constexpr int kF64Groups = 8;
+struct F64Groups {
+  F64Gemm g[kF64Groups];
+  int first[kF64Groups + 1];  // first workgroup of each group
+  int ntx[kF64Groups], nty[kF64Groups];
+  int n;
+};
+
+// Workgroup -> group and tile. Triangular operands keep the hardware's round
+// robin over XCDs and take the longest rows first, so the last workgroups to
+// start are the shortest; else each XCD gets a contiguous run of tiles, four
+// row tiles at a time (their columns share its L2; 1 to 16 measured the same).
+__device__ __forceinline__ int f64_workgroup(const F64Groups &gs, int &tx, int &ty) {
+  constexpr int kRows = 4;
+  int id = blockIdx.x;
+  if (!gs.g[0].lower_tri) {
+    int per = gridDim.x / 8, rest = gridDim.x % 8, x = id % 8, l = id / 8;
+    id = x * per + min(x, rest) + l;
+  }
+  int gi = 0;
+  while (gi + 1 < gs.n && id >= gs.first[gi + 1]) gi++;
+  int local = id - gs.first[gi], ntx = gs.ntx[gi], nty = gs.nty[gi];
+  if (gs.g[gi].lower_tri) {
+    tx = local % ntx;
+    ty = nty - 1 - local / ntx;
+  } else {
+    int f = local / (kRows * ntx) * kRows, n_in = min(kRows, nty - f), r = local % (kRows * ntx);
+    tx = r / n_in;
+    ty = f + r % n_in;
+  }
+  return gi;
+}
+
+// EP_KERNEL for powers other than 1 and 2: two calls of pow per element, in
+// kernels of their own so that the common ones stay free of calls.
+constexpr int EP_KERNEL_POW = 3;
+
+// The last K % 4 values of k (zeros after them) of 16 rows of an operand.
+__device__ __forceinline__ double f64_tail(const double *row, int K, int q4) {
+  int k = (K & ~3) + q4;
+  return k < K ? row[k] : 0.0;
+}
+
+// One accumulator tile in VGPRs, here and not before (without the empty
+// statement the compiler copies all of them at once and spills).
+__device__ __forceinline__ v4d f64_tile_out(const v4d &acc) {
+  v4d t = acc;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
+// Epilogue of a wave's 16T x 16T tile at (row0, col0): lane l holds column
+// l % 16 of each 16 x 16 tile, rows l / 16 + 4 i. `red` (EP_SUMSQ at T = 1):
+// LDS through which the upper 16 rows of a 32-row half pass their sums on to
+// the lower ones (wave rows 0 and 1 of the workgroup).
+template <int EP, int T>
+__device__ __forceinline__ void f64_epilogue(const F64Gemm &g, const v4d (&acc)[T][T], int row0,
+                                             int col0, int wid, double *red) {
+  const EpArgs &e = g.e;
+  const int M = g.M, N = g.N;
+  int lane = threadIdx.x & 63, r16 = lane & 15, q4 = lane >> 4;
+  if constexpr (EP == EP_STORE) {
+#pragma unroll
+    for (int a = 0; a < T; a++)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        int r = row0 + wr * 16 * TM + ti * 16 + tile_row<Acc>(lane, i);
-        double v = r < M ? (double)t.v[ti][tj][i] : 0.0;
-        cs[tj] += v * v;
+        int r = row0 + 16 * a + q4 + 4 * i;
+        if (r >= M) continue;
+        double *w = e.W_as<double>() + (size_t)r * e.ldw;
+#pragma unroll
+        for (int b = 0; b < T; b++) {
+          int c = col0 + 16 * b + r16;
+          if (c < N) w[c] = acc[a][b][i];
+        }
+      }
+  } else if constexpr (EP == EP_KERNEL || EP == EP_KERNEL_POW) {
+    // Rows: atoms, columns: sparse environments. k = sigma^2 S^p and
+    // w = sigma^2 alpha p S^(p-1) per element, the energy summed over each
+    // 16 columns.
+    int pi = EP == EP_KERNEL_POW ? 0 : (e.power == 2.0 ? 2 : 1);
+    double alpha[T];
+#pragma unroll
+    for (int b = 0; b < T; b++) alpha[b] = e.alpha[min(col0 + 16 * b + r16, N - 1)];
+#pragma unroll
+    for (int a = 0; a < T; a++) {
+      double nrm[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) nrm[i] = e.row_norm[min(row0 + 16 * a + q4 + 4 * i, M - 1)];
+      v4d t[T];
+#pragma unroll
+      for (int b = 0; b < T; b++) t[b] = f64_tile_out(acc[a][b]);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        int r = row0 + 16 * a + q4 + 4 * i;
+        bool empty = nrm[i] < kEmptyThresh;
+        double ninv = empty ? 0.0 : 1.0 / nrm[i];
+        double *wr = e.W_as<double>() + (size_t)min(r, M - 1) * e.ldw;
+        double *kr = e.K_as<double>() + (size_t)min(r, M - 1) * e.ldk;
+#pragma unroll
+        for (int b = 0; b < T; b++) {
+          int c = col0 + 16 * b + r16;
+          bool in = r < M && c < N;
+          double s = t[b][i] * ninv;
+          double sp, pm1;
+          if constexpr (EP == EP_KERNEL_POW) {
+            sp = pow_general(s, e.power);
+            pm1 = pow_general(s, e.power - 1);
+          } else {
+            sp = pi == 2 ? s * s : s;
+            pm1 = pi == 2 ? s : 1.0;
+          }
+          double kv = empty ? 0.0 : e.sig2 * sp;
+          double wv = empty ? 0.0 : e.sig2 * alpha[b] * e.power * pm1;
+          if (in) wr[c] = wv;
+          if (in && e.K) kr[c] = kv;
+          double sum = row16_sum(c < N ? kv * alpha[b] : 0.0);
+          if (r16 == 0 && in) e.part[(size_t)(col0 / 16 + b) * e.part_ld + r] = sum;
+        }
+      }
+    }
+  } else {
+    // Rows: rows of L, columns: atoms. Sums of squares over each 32 rows, per
+    // lane in row order (rows past M are copies of the last one: left out),
+    // then over the four lane groups.
+    static_assert(T != 3, "a wave's rows must not straddle a 32-row half");
+#pragma unroll
+    for (int b = 0; b < T; b++)
+#pragma unroll
+      for (int a0 = 0; a0 < T; a0 += 2) {
+        double v = 0;
+        if constexpr (T == 1) {
+          if (wid >> 1) v = red[64 * (wid & 1) + lane];
+        }
+#pragma unroll
+        for (int a = a0; a < a0 + 2 && a < T; a++) {
+          v4d t = f64_tile_out(acc[a][b]);
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            double x = row0 + 16 * a + q4 + 4 * i < M ? t[i] : 0.0;
+            v += x * x;
+          }
+        }
+        if constexpr (T == 1) {
+          if (!(wid >> 1)) {
+            red[64 * (wid & 1) + lane] = v;
+            continue;
+          }
+        }
+        v += __shfl_xor(v, 16, 64);
+        v += __shfl_xor(v, 32, 64);
+        int half = (row0 + 16 * a0) / 32, c = col0 + 16 * b + r16;
+        if (q4 == 0 && c < N && half < (M + 63) / 64 * 2) e.part[(size_t)half * e.part_ld + c] = v;
       }
   }
-#pragma unroll
-  for (int tj = 0; tj < TN; tj++) {
-    double v = cs[tj];
-    v += __shfl_xor(v, 16, 64);
-    v += __shfl_xor(v, 32, 64);
-    cs[tj] = v;
-  }
-  if (lane < 16) {
-#pragma unroll
-    for (int tj = 0; tj < TN; tj++) red[wr * BNc + wc * 16 * TN + tj * 16 + lane] = cs[tj];
-  }
-  __syncthreads();
-  for (int q = threadIdx.x; q < BNc; q += blockDim.x) {
-    int c = col0 + q;
-    if (c < N) e.part[(size_t)(row0 / (32 * TM)) * e.part_ld + c] = red[q] + red[BNc + q];
-  }
 }
 
-template <int EP, typename Acc, typename TW, int TM, int TN>
-__device__ __forceinline__ void run_epilogue(const EpArgs &e, const TileOut<Acc, TM, TN> &t,
-                                             int row0, int col0, int M, int N, int lane, int wr,
-                                             int wc, double *red) {
-  if (EP == EP_KERNEL) ep_kernel<Acc, TW, TM, TN>(e, t, row0, col0, M, N, lane, wr, wc, red);
-  else if (EP == EP_STORE) ep_store<Acc, TW, TM, TN>(e, t, row0, col0, M, N, lane, wr, wc);
-  else ep_sumsq<Acc, TM, TN>(e, t, row0, col0, M, N, lane, wr, wc, red);
-}
-
-// ---------------------------------------------------------------------------
-// FP64 MFMA GEMM, (32 TM) x (32 TN) tiles; 4 waves (2 x 2), each TM x TN
-// MFMA tiles of 16 x 16. LDS holds k-major tiles so a fragment read (16 rows
-// at one k) is contiguous. Each thread loads 4 consecutive k of rows
-// tid / 4 + 64 j.
-// ---------------------------------------------------------------------------
-// Base shape: the partial arrays (gemm_col_tiles / gemm_row_tiles) follow it.
-constexpr int F64_TM = 2, F64_TN = 2, F64_BM = 32 * F64_TM, F64_BN = 32 * F64_TN;
-constexpr int BK64 = 16;
-constexpr int PAD64 = 1;  // row stride 65 or 129 doubles: the transposed stores spread over the banks
-
-// Four consecutive k of one row, widened to FP64: one or two 16-byte loads
-// when `vec` (the row start is 16-byte aligned and k + 4 <= kend), else
-// element by element with zeros past the row count or kend.
-template <typename T>
-__device__ __forceinline__ void load_row4(const T *P, long long ld, int r, int rows, int k,
-                                          int kend, bool vec, double (&o)[4]) {
-  const T *p = P + (size_t)(r < rows ? r : 0) * ld + k;
-  if (r < rows && vec && k + 4 <= kend) {
-    if constexpr (sizeof(T) == 4) {
-      float4 v = *reinterpret_cast<const float4 *>(p);
-      o[0] = v.x, o[1] = v.y, o[2] = v.z, o[3] = v.w;
-    } else {
-      double2 a = *reinterpret_cast<const double2 *>(p);
-      double2 b = *reinterpret_cast<const double2 *>(p + 2);
-      o[0] = a.x, o[1] = a.y, o[2] = b.x, o[3] = b.y;
-    }
-  } else {
-#pragma unroll
-    for (int q = 0; q < 4; q++) o[q] = (r < rows && k + q < kend) ? (double)p[q] : 0.0;
-  }
-}
-
-template <int EP, int TM, int TN, typename TB = double>
-__global__ __launch_bounds__(256) void k_gemm_f64(int M, int N, int K, const double *A, long long lda,
-                                                  const TB *B, long long ldb, int lower_tri,
-                                                  int vec, EpArgs e) {
-  constexpr int BM = 32 * TM, BN = 32 * TN, RA = BM / 64, RB = BN / 64;
-  static_assert(BM % 64 == 0 && BN % 64 == 0, "tiles are multiples of 64");
-  __shared__ double As[BK64][BM + PAD64];
-  __shared__ double Bs[BK64][BN + PAD64];
-  __shared__ double red[2 * (BM > BN ? BM : BN)];
-  int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  int wr = wid >> 1, wc = wid & 1;
-  // A lower-triangular A makes row tiles uneven (row tile r reads r + 1
-  // k-tiles): keep the hardware's round-robin spread of tiles there.
+// A wave owns 16T x 16T outputs and loads its own fragments: lane l takes row
+// l % 16 of each 16-row group and 4 of each 16 k, as two 16-byte loads. For
+// EP_STORE these are k0 + 2 (l / 16) + {0, 1} and the same 8 further on, so one
+// load covers 64 contiguous bytes of 16 rows, and MFMA j contracts the k set
+// of element j, whatever k that is. In plain order (ORD) they are 4
+// consecutive k, and a transpose over the four lane groups gives MFMA j its
+// k = 4 j + {0, 1, 2, 3} (8-byte loads in that order cost twice the load
+// instructions and twice the time). No LDS, no barriers: on small problems the
+// waves are independent and the chain of one is short. Fragments of the next
+// 16 U k are loaded into registers while the current ones feed the MFMAs, all
+// loads of a step together: the two halves of a 128-byte line then meet in L1.
+// A barrier that kept a workgroup's waves in step cost 35 % (their loads queue
+// at one moment). U is 2 at T = 1 only, where a step of 16 k is 256 cycles.
+template <int EP, int T, int U>
+__global__ __launch_bounds__(256) void k_gemm_f64(F64Groups gs) {
+  constexpr bool ORD = EP != EP_STORE;
+  constexpr int LK = ORD ? 4 : 2, HS = ORD ? 16 : 64;  // k per lane group, bytes between its loads
+  __shared__ double red[EP == EP_SUMSQ && T == 1 ? 128 : 1];
   int tx, ty;
-  if (lower_tri) {
-    tx = blockIdx.x;
-    ty = blockIdx.y;
-  } else {
-    xcd_tile(tx, ty);
+  const F64Gemm &g = gs.g[f64_workgroup(gs, tx, ty)];
+  const int M = g.M, N = g.N;
+  int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int r16 = lane & 15, q4 = lane >> 4;
+  int row0 = ty * 32 * T + (wid >> 1) * 16 * T, col0 = tx * 32 * T + (wid & 1) * 16 * T;
+  // EP_SUMSQ writes zeros for the rows up to the next 64, and at T = 1 its wave
+  // rows meet in the epilogue.
+  constexpr bool MEET = EP == EP_SUMSQ && T == 1;
+  if (EP != EP_SUMSQ && (row0 >= M || col0 >= N)) return;
+  // Wave-uniform bases that advance along k and fixed lane offsets: an FP64
+  // MFMA keeps its SIMD's vector ALU, so every vector instruction of the loop
+  // (address arithmetic, register copies) adds to it. Rows past the end read
+  // the last row (their outputs are not stored).
+  const char *pa = reinterpret_cast<const char *>(g.A), *pb = reinterpret_cast<const char *>(g.B);
+  size_t oa[T], ob[T];
+#pragma unroll
+  for (int t = 0; t < T; t++) {
+    oa[t] = (min(row0 + 16 * t + r16, M - 1) * (size_t)g.lda + LK * q4) * 8;
+    ob[t] = (min(col0 + 16 * t + r16, N - 1) * (size_t)g.ldb + LK * q4) * 8;
   }
-  int row0 = ty * BM, col0 = tx * BN;
-  int kend = K;
-  if (lower_tri) kend = min(K, row0 + BM);
-  v4d acc[TM][TN];
+  // k steps of KS end at the operands' last k (in plain order: its last
+  // multiple of 4, the rest follows the loop); the first steps are padded with
+  // zeros in front, to an even number of steps. Past the diagonal of a lower
+  // triangular A every term is zero.
+  constexpr int KS = 16 * U;
+  int Kall = g.lower_tri ? min(g.K, row0 + 16 * T) : g.K;
+  int K = ORD ? Kall & ~3 : Kall;
+  int pairs = max(1, (K + 2 * KS - 1) / (2 * KS));
+  int k0 = K - 2 * KS * pairs;  // the next step's first k (negative: padding)
+  double ta[T], tb[T];
+  if constexpr (ORD) {
+    if (Kall & 3) {
 #pragma unroll
-  for (int a = 0; a < TM; a++)
-#pragma unroll
-    for (int b = 0; b < TN; b++) acc[a][b] = v4d{0, 0, 0, 0};
-  int lr = tid >> 2, lk = (tid & 3) * 4;
-  double ra[RA][4], rb[RB][4];
-  auto gload = [&](int k0) {
-#pragma unroll
-    for (int j = 0; j < RA; j++)
-      load_row4(A, lda, row0 + lr + 64 * j, M, k0 + lk, kend, vec & 1, ra[j]);
-#pragma unroll
-    for (int j = 0; j < RB; j++)
-      load_row4(B, ldb, col0 + lr + 64 * j, N, k0 + lk, kend, vec & 2, rb[j]);
-  };
-  gload(0);
-  for (int k0 = 0; k0 < kend; k0 += BK64) {
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-#pragma unroll
-      for (int j = 0; j < RA; j++) As[lk + q][lr + 64 * j] = ra[j][q];
-#pragma unroll
-      for (int j = 0; j < RB; j++) Bs[lk + q][lr + 64 * j] = rb[j][q];
+      for (int t = 0; t < T; t++) {
+        ta[t] = f64_tail(reinterpret_cast<const double *>(pa + oa[t]) - LK * q4, Kall, q4);
+        tb[t] = f64_tail(reinterpret_cast<const double *>(pb + ob[t]) - LK * q4, Kall, q4);
+      }
     }
+  }
+  v4d acc[T][T];
+#pragma unroll
+  for (int a = 0; a < T; a++)
+#pragma unroll
+    for (int b = 0; b < T; b++) acc[a][b] = v4d{0, 0, 0, 0};
+  // Fragments of one step: KS k of every row tile, MFMA j of the four per 16 k
+  // taking element j.
+  struct Frag {
+    double a[U][T][4], b[U][T][4];
+  };
+  // A step inside the rows: [k0, k0 + KS).
+  auto load = [&](Frag &f) {
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int t = 0; t < T; t++) {
+        const char *xa = pa + oa[t] + 128 * u, *xb = pb + ob[t] + 128 * u;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          v2d va = *reinterpret_cast<const v2d *>(xa + HS * h);
+          v2d vb = *reinterpret_cast<const v2d *>(xb + HS * h);
+          f.a[u][t][2 * h] = va.x, f.a[u][t][2 * h + 1] = va.y;
+          f.b[u][t][2 * h] = vb.x, f.b[u][t][2 * h + 1] = vb.y;
+        }
+      }
+    k0 += KS;
+    pa += 8 * KS;
+    pb += 8 * KS;
+  };
+  // One of the first two steps: zeros for k < 0.
+  auto load_head = [&](Frag &f) {
+    if (k0 >= 0) return load(f);
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int t = 0; t < T; t++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          int k = k0 + 16 * u + (ORD ? j : 8 * (j >> 1) + (j & 1));
+          bool in = k + LK * q4 >= 0;
+          f.a[u][t][j] = in ? *reinterpret_cast<const double *>(pa + (ptrdiff_t)oa[t] + 8 * k) : 0.0;
+          f.b[u][t][j] = in ? *reinterpret_cast<const double *>(pb + (ptrdiff_t)ob[t] + 8 * k) : 0.0;
+        }
+    k0 += KS;
+    int adv = k0 > 0 ? 8 * k0 : 0;
+    pa += adv;
+    pb += adv;
+  };
+  auto mma = [&](Frag &f) {
+    if constexpr (ORD) {
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int t = 0; t < T; t++) {
+          transpose_groups(f.a[u][t]);
+          transpose_groups(f.b[u][t]);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int a = 0; a < T; a++)
+#pragma unroll
+          for (int b = 0; b < T; b++)
+            acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(f.a[u][a][j], f.b[u][b][j],
+                                                             acc[a][b], 0, 0, 0);
+  };
+  // Empty statements that take the accumulators in AGPRs: an epilogue that
+  // computes with them would otherwise make the compiler carry them in VGPRs
+  // from one iteration to the next and copy all of them there and back.
+  auto pin = [&] {
+#pragma unroll
+    for (int a = 0; a < T; a++)
+#pragma unroll
+      for (int b = 0; b < T; b++) asm volatile("" : "+a"(acc[a][b]));
+  };
+  Frag f0, f1;
+  load_head(f0);
+  load_head(f1);
+  // All of the first two steps, here: the loop then needs to wait for the
+  // older of its two loads only (vmcnt; 0x0f70 leaves the other counters).
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+  pin();
+#pragma unroll 1
+  for (int p = 1; p < pairs; p++) {
+    mma(f0);
+    __builtin_amdgcn_sched_barrier(0);
+    load(f0);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(f1);
+    __builtin_amdgcn_sched_barrier(0);
+    load(f1);
+    __builtin_amdgcn_sched_barrier(0);
+    pin();
+  }
+  mma(f0);
+  mma(f1);
+  if constexpr (ORD) {
+    if (Kall & 3) {
+#pragma unroll
+      for (int a = 0; a < T; a++)
+#pragma unroll
+        for (int b = 0; b < T; b++)
+          acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ta[a], tb[b], acc[a][b], 0, 0, 0);
+    }
+  }
+  pin();
+  if constexpr (MEET) {
+    if (!(wid >> 1)) f64_epilogue<EP, T>(g, acc, row0, col0, wid, red);
     __syncthreads();
-    if (k0 + BK64 < kend) gload(k0 + BK64);
+    if (wid >> 1) f64_epilogue<EP, T>(g, acc, row0, col0, wid, red);
+  } else {
+    f64_epilogue<EP, T>(g, acc, row0, col0, wid, red);
+  }
+}
+
+// 128 x 128 tiles in plain k order, four waves of 64 x 64: the next 16 k of
+// both operands are in flight to registers while the current ones, in LDS,
+// feed the MFMAs; two LDS buffers, one barrier per 16 k (4096 MFMA cycles), two
+// workgroups per CU. A row's 16 k are 8 chunks of 16 bytes, chunk c of row r at
+// place c ^ (r % 8), so that the 16-byte stores and the 8-byte fragment reads
+// (16 rows, 4 consecutive k) spread over all banks.
+template <int EP>
+__global__ __launch_bounds__(256, 2) void k_gemm_f64_lds(F64Groups gs) {
+  constexpr int T = 4, KS = 16, TILE = 128 * KS;
+  __shared__ __align__(16) double As[2 * TILE], Bs[2 * TILE];
+  int tx, ty;
+  const F64Gemm &g = gs.g[f64_workgroup(gs, tx, ty)];
+  const int M = g.M, N = g.N;
+  int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int r16 = lane & 15, q4 = lane >> 4;
+  int brow = ty * 128, bcol = tx * 128;
+  int row0 = brow + (wid >> 1) * 64, col0 = bcol + (wid & 1) * 64;
+  // Steps of 16 end at the last multiple of 4, with zeros in front of the first
+  // one; past the diagonal of a lower triangular A every term is zero.
+  int Kall = g.lower_tri ? min(g.K, brow + 128) : g.K;
+  int K = Kall & ~3;
+  int steps = (K + KS - 1) / KS;
+  int k0 = K - KS * steps;
+  // Load i of thread t: chunk t % 8 of row 32 i + t / 8.
+  const double *pa[4], *pb[4];
+  int tid = threadIdx.x, chunk = tid & 7;
 #pragma unroll
-    for (int kk = 0; kk < BK64; kk += 4) {
-      double af[TM], bf[TN];
+  for (int i = 0; i < 4; i++) {
+    int r = 32 * i + (tid >> 3);
+    pa[i] = g.A + (size_t)min(brow + r, M - 1) * g.lda + 2 * chunk + k0;
+    pb[i] = g.B + (size_t)min(bcol + r, N - 1) * g.ldb + 2 * chunk + k0;
+  }
+  int put = (tid >> 3) * KS + 2 * (chunk ^ ((tid >> 3) & 7));  // its place in a tile's 32 rows
+  v2d ra[4], rb[4];
+  auto load = [&] {
 #pragma unroll
-      for (int t = 0; t < TM; t++) af[t] = As[kk + (lane >> 4)][wr * 16 * TM + t * 16 + (lane & 15)];
+    for (int i = 0; i < 4; i++) {
+      ra[i] = *reinterpret_cast<const v2d *>(pa[i]);
+      rb[i] = *reinterpret_cast<const v2d *>(pb[i]);
+      pa[i] += KS;
+      pb[i] += KS;
+    }
+  };
+  auto store = [&](int buf) {
 #pragma unroll
-      for (int t = 0; t < TN; t++) bf[t] = Bs[kk + (lane >> 4)][wc * 16 * TN + t * 16 + (lane & 15)];
+    for (int i = 0; i < 4; i++) {
+      *reinterpret_cast<v2da *>(&As[buf * TILE + 32 * i * KS + put]) = ra[i];
+      *reinterpret_cast<v2da *>(&Bs[buf * TILE + 32 * i * KS + put]) = rb[i];
+    }
+  };
+  // The first step when it starts before k = 0.
+  auto load_head = [&] {
 #pragma unroll
-      for (int a = 0; a < TM; a++)
+    for (int i = 0; i < 4; i++) {
 #pragma unroll
-        for (int b = 0; b < TN; b++)
+      for (int e = 0; e < 2; e++) {
+        bool in = k0 + 2 * chunk + e >= 0;
+        ra[i][e] = in ? pa[i][e] : 0.0;
+        rb[i][e] = in ? pb[i][e] : 0.0;
+      }
+      pa[i] += KS;
+      pb[i] += KS;
+    }
+  };
+  v4d acc[T][T];
+#pragma unroll
+  for (int a = 0; a < T; a++)
+#pragma unroll
+    for (int b = 0; b < T; b++) acc[a][b] = v4d{0, 0, 0, 0};
+  auto pin = [&] {  // see k_gemm_f64
+#pragma unroll
+    for (int a = 0; a < T; a++)
+#pragma unroll
+      for (int b = 0; b < T; b++) asm volatile("" : "+a"(acc[a][b]));
+  };
+  // Lane offsets of MFMA j's fragments: k = 4 j + q4 of rows r16 of each 16.
+  int fo[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+    fo[j] = r16 * KS + 2 * ((2 * j + (q4 >> 1)) ^ (r16 & 7)) + (q4 & 1);
+  auto compute = [&](int buf) {
+    const double *as = As + buf * TILE + (wid >> 1) * 64 * KS;
+    const double *bs = Bs + buf * TILE + (wid & 1) * 64 * KS;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      double af[T], bf[T];
+#pragma unroll
+      for (int t = 0; t < T; t++) {
+        af[t] = as[t * 16 * KS + fo[j]];
+        bf[t] = bs[t * 16 * KS + fo[j]];
+      }
+#pragma unroll
+      for (int a = 0; a < T; a++)
+#pragma unroll
+        for (int b = 0; b < T; b++)
           acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[a], bf[b], acc[a][b], 0, 0, 0);
     }
+  };
+  if (steps > 0) {
+    if (k0 < 0) load_head();
+    else load();
+    store(0);
   }
-  TileOut<double, TM, TN> t;
+  if (steps > 1) load();
+  __syncthreads();
+  pin();
+#pragma unroll 1
+  for (int s = 0; s < steps; s++) {
+    compute(s & 1);
+    pin();
+    if (s + 1 < steps) store((s + 1) & 1);  // read by compute(s - 1) last
+    if (s + 2 < steps) load();
+    __syncthreads();
+  }
+  if (Kall & 3) {
+    double ta[T], tb[T];
 #pragma unroll
-  for (int a = 0; a < TM; a++)
+    for (int t = 0; t < T; t++) {
+      ta[t] = f64_tail(g.A + (size_t)min(row0 + 16 * t + r16, M - 1) * g.lda, Kall, q4);
+      tb[t] = f64_tail(g.B + (size_t)min(col0 + 16 * t + r16, N - 1) * g.ldb, Kall, q4);
+    }
 #pragma unroll
-    for (int b = 0; b < TN; b++)
+    for (int a = 0; a < T; a++)
 #pragma unroll
-      for (int i = 0; i < 4; i++) t.v[a][b][i] = acc[a][b][i];
-  run_epilogue<EP, double, double, TM, TN>(e, t, row0, col0, M, N, lane, wr, wc, red);
+      for (int b = 0; b < T; b++)
+        acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ta[a], tb[b], acc[a][b], 0, 0, 0);
+  }
+  pin();
+  f64_epilogue<EP, T>(g, acc, row0, col0, wid, nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -506,7 +797,7 @@ __global__ __launch_bounds__(256) void k_gemm_split(int M, int N, int Kpad, Spli
     for (int b = 0; b < TN; b++)
 #pragma unroll
       for (int i = 0; i < 4; i++) t.v[a][b][i] = acc[a][b][i];
-  run_epilogue<EP, float, float, TM, TN>(e, t, row0, col0, M, N, lane, wr, wc, red);
+  ep_store<float, float, TM, TN>(e, t, row0, col0, M, N, lane, wr, wc);
 }
 
 // ---------------------------------------------------------------------------
@@ -786,43 +1077,31 @@ __global__ __launch_bounds__(512) void k_gemm_i8(int M, int N, int nk, const int
 }
 
 int gemm_col_tiles(int form, int N) {
-  int bn = form == FM_FORM_FP64 ? F64_BN : kI8TileN;
+  int bn = form == FM_FORM_FP64 ? 16 : kI8TileN;
   return (N + bn - 1) / bn;
 }
 
-int gemm_row_tiles(int form, int M) {
-  int bm = form == FM_FORM_FP64 ? F64_BM : B16_BM;
-  return (M + bm - 1) / bm;
-}
+int gemm_row_tiles(int M) { return (M + 63) / 64 * 2; }
 
 // ---------------------------------------------------------------------------
-// Tile autotuner. The first contraction of a given shape (epilogue, M and N
-// rounded up to powers of two, K, device) times every admissible tile shape
-// (the faster of two launches after a warm-up one) on the caller's stream
-// and keeps the fastest for later calls. Admissible shapes never change results: the energy partials
-// of EP_KERNEL are per column tile and the |Q|^2 partials of EP_SUMSQ per
-// row tile, so EP_KERNEL only varies TM and EP_SUMSQ only TN; every output
-// element sums its k terms in the same order whatever the tile.
+// Tile autotuner of the split contraction. The first contraction of a given
+// shape (M and N rounded up to powers of two, K, device) times every tile
+// shape (the faster of two launches after a warm-up one) on the caller's
+// stream and keeps the fastest for later calls. Shapes never change results:
+// every output element sums its k terms in the same order whatever the tile.
 // ---------------------------------------------------------------------------
 namespace {
 
-struct TileShape {
-  int tm, tn, db;
-};
-constexpr TileShape kF64Shapes[] = {{2, 2, 0}, {4, 2, 0}, {2, 4, 0}, {4, 4, 0}};
-// 8 x 4 and 4 x 8: 64 x 128 / 128 x 64 per wavefront, a third fewer LDS
-// fragment reads per MFMA than 64 x 64.
-constexpr TileShape kSplitShapes[] = {{4, 4, 0}, {2, 4, 0}, {4, 2, 0}, {4, 4, 1},
-                                      {4, 2, 1}, {8, 4, 0}, {4, 8, 0}};
-
-bool admissible(int ep, TileShape t, TileShape base) {
-  if (ep == EP_KERNEL) return t.tn == base.tn;
-  if (ep == EP_SUMSQ) return t.tm == base.tm;
-  return true;
+// FLARE_MI_TILE_SHAPE=i pins shape i of each contraction's table (tests check
+// that every shape gives the same results); -1 without it or past the table.
+int pinned_shape(int n_shapes) {
+  const char *f = std::getenv("FLARE_MI_TILE_SHAPE");
+  int i = f ? std::atoi(f) : -1;
+  return i < n_shapes ? i : -1;
 }
 
 std::mutex g_tune_mu;
-std::map<std::tuple<int, int, int, int, int, int, int>, int> g_tune;
+std::map<std::tuple<int, int, int, int>, int> g_tune;
 
 int next_pow2(int x) {
   int p = 64;
@@ -830,23 +1109,17 @@ int next_pow2(int x) {
   return p;
 }
 
-// Returns the tuned shape index for `key`, timing `launch(i)` for each
-// admissible index when the key is new. `launch` enqueues one contraction.
+// Returns the tuned shape index, timing `launch(i)` for each of n_shapes when
+// the size class is new. `launch` enqueues one contraction.
 template <typename Launch>
-int tuned(int family, int ep, int M, int N, int K, hipStream_t st, const TileShape *shapes,
-          int n_shapes, Launch &&launch) {
-  // FLARE_MI_TILE_SHAPE=i pins shape i for every contraction that admits it
-  // (tests check that each shape gives the same results).
-  if (const char *f = std::getenv("FLARE_MI_TILE_SHAPE")) {
-    int i = std::atoi(f);
-    if (i >= 0 && i < n_shapes && admissible(ep, shapes[i], shapes[0])) return i;
-  }
+int tuned(int M, int N, int K, hipStream_t st, int n_shapes, Launch &&launch) {
+  int pin = pinned_shape(n_shapes);
+  if (pin >= 0) return pin;
   int dev = 0;
   FM_HIP(hipGetDevice(&dev));
-  // M and N up to powers of two: the atom count of a new batch (rows of the
-  // kernel and gradient contractions, columns of the variance one) reuses the
+  // M and N up to powers of two: the atom count of a new batch reuses the
   // choice for its size class instead of timing every shape again.
-  auto key = std::make_tuple(family, ep, next_pow2(M), next_pow2(N), K, dev, 0);
+  auto key = std::make_tuple(next_pow2(M), next_pow2(N), K, dev);
   {
     std::lock_guard<std::mutex> g(g_tune_mu);
     auto it = g_tune.find(key);
@@ -858,7 +1131,6 @@ int tuned(int family, int ep, int M, int N, int K, hipStream_t st, const TileSha
   int best = -1;
   float best_ms = 0;
   for (int i = 0; i < n_shapes; i++) {
-    if (!admissible(ep, shapes[i], shapes[0])) continue;
     launch(i);  // warm-up (code object load, caches)
     float ms = 0;
     for (int r = 0; r < 2; r++) {  // the faster of two timed launches
@@ -882,27 +1154,18 @@ int tuned(int family, int ep, int M, int N, int K, hipStream_t st, const TileSha
   return best;
 }
 
-template <int EP, int TM, int TN, typename TB>
-void f64_launch(hipStream_t st, int M, int N, int K, const double *A, long long lda,
-                const TB *B, long long ldb, int lower_tri, const EpArgs &e) {
-  dim3 grid((N + 32 * TN - 1) / (32 * TN), (M + 32 * TM - 1) / (32 * TM));
-  // 16-byte loads where every row start is 16-byte aligned.
-  auto aligned = [](const void *p, long long ld, size_t esz) {
-    return (uintptr_t)p % 16 == 0 && (ld * (long long)esz) % 16 == 0;
-  };
-  int vec = (aligned(A, lda, sizeof(double)) ? 1 : 0) | (aligned(B, ldb, sizeof(TB)) ? 2 : 0);
-  hipLaunchKernelGGL((k_gemm_f64<EP, TM, TN, TB>), grid, dim3(256), 0, st, M, N, K, A, lda, B,
-                     ldb, lower_tri, vec, e);
-}
-
-template <int EP, typename TB>
-void f64_shape(int i, hipStream_t st, int M, int N, int K, const double *A, long long lda,
-               const TB *B, long long ldb, int lower_tri, const EpArgs &e) {
-  switch (i) {
-    case 0: f64_launch<EP, 2, 2>(st, M, N, K, A, lda, B, ldb, lower_tri, e); break;
-    case 1: f64_launch<EP, 4, 2>(st, M, N, K, A, lda, B, ldb, lower_tri, e); break;
-    case 2: f64_launch<EP, 2, 4>(st, M, N, K, A, lda, B, ldb, lower_tri, e); break;
-    default: f64_launch<EP, 4, 4>(st, M, N, K, A, lda, B, ldb, lower_tri, e); break;
+template <int EP>
+void f64_launch(hipStream_t st, int T, int blocks, const F64Groups &gs) {
+  dim3 grid(blocks), block(256);
+  if (T == 1) {
+    hipLaunchKernelGGL((k_gemm_f64<EP, 1, 2>), grid, block, 0, st, gs);
+  } else if (T == 2) {
+    hipLaunchKernelGGL((k_gemm_f64<EP, 2, 1>), grid, block, 0, st, gs);
+  } else if constexpr (EP == EP_STORE) {
+    if (T == 3) hipLaunchKernelGGL((k_gemm_f64<EP, 3, 1>), grid, block, 0, st, gs);
+    else hipLaunchKernelGGL((k_gemm_f64<EP, 4, 1>), grid, block, 0, st, gs);
+  } else {
+    hipLaunchKernelGGL((k_gemm_f64_lds<EP>), grid, block, 0, st, gs);
   }
 }
 
@@ -978,16 +1241,79 @@ void gemm_i8_kernel(hipStream_t st, int M, int N, int Kq, const SliceOperand &A,
   FM_HIP(hipGetLastError());
 }
 
+// Wave tile of a launch, 16T x 16T: the least estimated time per 16 k, rounds
+// of waves over the SIMDs times the measured time of one wave's 16 k. That
+// time is nearly the same whether a wave has its SIMD to itself (three groups
+// of 170 x 167 x 1,500) or the chip is full (32,000 x 1,000 x 2,100):
+//   T = 4  2.1 us (full chip: 68 TFLOP/s for EP_STORE, 60 for EP_KERNEL
+//                  through LDS; the matrix cores' limit, where the kernel
+//                  before had 48)
+//   T = 3  1.25   (63, EP_STORE only)
+//   T = 2  0.72   (50, 47; bound by its loads)
+//   T = 1  0.35   (27, the same)
+// EP_KERNEL in us at T = 4, 2, 1: 2 x 2,000 x 500 x 2,100 takes 309, 193, 332;
+// 3 x 8,000 x 200 x 1,500 405, 411, 613; 2 x 512 x 200 x 4,080 574, 228, 117;
+// 3 x 170 x 167 x 1,500 218, 78, 35 (one species after the other on 64 x 64
+// workgroup tiles it had taken 309). EP_SUMSQ, 2 x 1,000 x 16,000, triangular:
+// 592, 677, 1229 (941 before).
+static int f64_tile(int ep, const std::vector<F64Gemm> &gs) {
+  constexpr double kTime[5] = {0, 0.35, 0.72, 1.25, 2.1};
+  int pin = pinned_shape(4);
+  if (pin >= 0 && !(pin == 1 && ep != EP_STORE)) return 4 - pin;
+  constexpr int kSimds = 1024;  // 256 CUs
+  int best = 0;
+  double best_cost = 0;
+  for (int T = 4; T >= 1; T--) {
+    if (T == 3 && ep != EP_STORE) continue;
+    int b = 16 * T;
+    double waves = 0;
+    for (const F64Gemm &g : gs)
+      waves += (double)((g.M + b - 1) / b) * ((g.N + b - 1) / b);
+    double rounds = std::ceil(waves / kSimds);
+    // Triangular rows take half the steps on average, the last ones all.
+    if (gs[0].lower_tri) rounds = 0.5 * rounds + 0.5;
+    if (best == 0 || rounds * kTime[T] < best_cost) {
+      best = T;
+      best_cost = rounds * kTime[T];
+    }
+  }
+  return best;
+}
+
+void gemm_f64_groups(hipStream_t st, int ep, const std::vector<F64Gemm> &all) {
+  std::vector<F64Gemm> live;
+  for (const F64Gemm &g : all)
+    if (g.M > 0 && g.N > 0) live.push_back(g);
+  if (live.empty()) return;
+  int T = f64_tile(ep, live);
+  for (size_t g0 = 0; g0 < live.size(); g0 += kF64Groups) {
+    F64Groups gs{};
+    gs.n = (int)std::min<size_t>(kF64Groups, live.size() - g0);
+    long long blocks = 0;
+    for (int k = 0; k < gs.n; k++) {
+      const F64Gemm &g = gs.g[k] = live[g0 + k];
+      FM_CHECK(g.lower_tri == live[g0].lower_tri, FM_ERR_INVALID,
+               "one launch takes triangular operands only or none");
+      gs.first[k] = (int)blocks;
+      gs.ntx[k] = (g.N + 32 * T - 1) / (32 * T);
+      int rows = ep == EP_SUMSQ ? (g.M + 63) / 64 * 64 : g.M;
+      gs.nty[k] = (rows + 32 * T - 1) / (32 * T);
+      blocks += (long long)gs.ntx[k] * gs.nty[k];
+      FM_CHECK(blocks < (1LL << 31), FM_ERR_CAPACITY, "contraction too large for one launch");
+    }
+    gs.first[gs.n] = (int)blocks;
+    bool p12 = live[g0].e.power == 2.0 || live[g0].e.power == 1.0;  // one model, one power
+    if (ep == EP_KERNEL && p12) f64_launch<EP_KERNEL>(st, T, (int)blocks, gs);
+    else if (ep == EP_KERNEL) f64_launch<EP_KERNEL_POW>(st, T, (int)blocks, gs);
+    else if (ep == EP_STORE) f64_launch<EP_STORE>(st, T, (int)blocks, gs);
+    else f64_launch<EP_SUMSQ>(st, T, (int)blocks, gs);
+    FM_HIP(hipGetLastError());
+  }
+}
+
 void gemm_f64(hipStream_t st, int ep, int M, int N, int K, const double *A, long long lda,
               const double *B, long long ldb, int lower_tri, const EpArgs &e) {
-  if (M <= 0 || N <= 0) return;
-  auto launch = [&](int i) {
-    if (ep == EP_KERNEL) f64_shape<EP_KERNEL>(i, st, M, N, K, A, lda, B, ldb, lower_tri, e);
-    else if (ep == EP_STORE) f64_shape<EP_STORE>(i, st, M, N, K, A, lda, B, ldb, lower_tri, e);
-    else f64_shape<EP_SUMSQ>(i, st, M, N, K, A, lda, B, ldb, lower_tri, e);
-    FM_HIP(hipGetLastError());
-  };
-  launch(tuned(0, ep, M, N, K, st, kF64Shapes, 4, launch));
+  gemm_f64_groups(st, ep, {F64Gemm{A, B, lda, ldb, M, N, K, lower_tri, e}});
 }
 
 void gemm_split(hipStream_t st, int ep, int np, int M, int N, int Kpad, const SplitOperand &A,
@@ -1012,7 +1338,7 @@ void gemm_split(hipStream_t st, int ep, int np, int M, int N, int Kpad, const Sp
     split_shape<EP_STORE>(i, st, M, N, Kpad, a, A.ld, b, B.ld, e);
     FM_HIP(hipGetLastError());
   };
-  launch(tuned(1, ep, M, N, Kpad, st, kSplitShapes, 7, launch));
+  launch(tuned(M, N, Kpad, st, 7, launch));
 }
 
 static uint16_t bf16_rne(float x) {

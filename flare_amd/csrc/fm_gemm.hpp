@@ -4,6 +4,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <vector>
 
 namespace fm {
 
@@ -24,7 +25,8 @@ struct EpArgs {
   void *W = nullptr;
   void *Wh = nullptr, *Wl = nullptr;
   long long ldw = 0;
-  // EP_KERNEL: energy partials [column tile][row]; EP_SUMSQ: [row tile][col].
+  // EP_KERNEL: energy partials [column tile][row]; EP_SUMSQ: [row tile][col]
+  // (16 columns, 32 rows of L in the FP64 contraction).
   double *part = nullptr;
   long long part_ld = 0;
   template <typename T>
@@ -37,12 +39,25 @@ struct EpArgs {
   }
 };
 
-// Number of column / row tiles a contraction of the given form uses (the
-// energy partials have one slot per column tile, the variance partials one
-// per row tile).
+// Number of column tiles a kernel contraction of the given form uses (one
+// energy partial each), and of the FP64 contraction's variance partials, one per
+// 32 rows, whose sum takes the two of each 64 rows together (always even).
 int gemm_col_tiles(int form, int N);
-int gemm_row_tiles(int form, int M);
+int gemm_row_tiles(int M);
 
+// One FP64 contraction C (M x N) = A B^T, rows of A (M x K) and B (N x K)
+// contiguous with leading dimensions lda and ldb, any alignment of 8 bytes.
+// lower_tri: A is lower triangular (zeros above the diagonal).
+struct F64Gemm {
+  const double *A = nullptr, *B = nullptr;
+  long long lda = 0, ldb = 0;
+  int M = 0, N = 0, K = 0, lower_tri = 0;
+  EpArgs e;
+};
+// Several contractions with one epilogue (a model's species) in one launch:
+// their workgroups share the chip, where one species at a time would leave it
+// part empty on small structures. All triangular or none.
+void gemm_f64_groups(hipStream_t st, int ep, const std::vector<F64Gemm> &groups);
 void gemm_f64(hipStream_t st, int ep, int M, int N, int K, const double *A, long long lda,
               const double *B, long long ldb, int lower_tri, const EpArgs &e);
 // Split-BF16 x3 contraction (EP_STORE: the gradient contraction G = W X_hat

@@ -28,7 +28,9 @@ __device__ __forceinline__ double row_variance(int r, const double *Qpart, int n
     double nd = nnr / (nrm * nrm);
     double ks = sig2 * (power == 2.0 ? nd * nd : pow(nd, power));
     double q = 0;
-    for (int t = 0; t < n_qtiles; t++) q += Qpart[(size_t)t * part_ld + r];
+#pragma unroll 8
+    for (int t = 0; t < n_qtiles; t += 2)
+      q += Qpart[(size_t)t * part_ld + r] + Qpart[(size_t)(t + 1) * part_ld + r];
     v = ks - q;
   }
   return v;
@@ -41,6 +43,7 @@ __global__ void k_species_final(int n_rows, int ro, const double *Epart, int n_e
   int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= n_rows) return;
   double e = 0;
+#pragma unroll 8
   for (int t = 0; t < n_etiles; t++) e += Epart[(size_t)t * part_ld + r];
   E_row[ro + r] = e;
   if (var_row)
@@ -342,7 +345,7 @@ static void predict_tiled(fm_model m, fm_structure s, int flags, int form, doubl
     Mmax = std::max(Mmax, Ms);
     eo[t + 1] = eo[t] + ns * (size_t)std::max(1, gemm_col_tiles(form, Ms));
     int Lr = want_var ? m->L_rows[t] : 0;
-    qo[t + 1] = qo[t] + ns * (size_t)gemm_row_tiles(FM_FORM_FP64, Lr);
+    qo[t + 1] = qo[t] + ns * (size_t)gemm_row_tiles(Lr);
   }
   // Whole-structure buffers.
   DevBuf Epart(pool, std::max<size_t>(1, eo[nos] * sizeof(double)));
@@ -375,7 +378,7 @@ static void predict_tiled(fm_model m, fm_structure s, int flags, int form, doubl
   for (int t = 0; t < nos; t++) {
     int ns = s->n_by_type[t], Ms = m->M_by_type[t], ro = s->type_off[t];
     int n_et = Ms == 0 ? 1 : gemm_col_tiles(form, Ms);
-    int n_qt = (want_var && Ms > 0) ? gemm_row_tiles(FM_FORM_FP64, m->L_rows[t]) : 0;
+    int n_qt = (want_var && Ms > 0) ? gemm_row_tiles(m->L_rows[t]) : 0;
     int Ts = species_tile_rows(ctx, T, Ms, form);
     for (int c0 = 0; c0 < ns; c0 += Ts) {
       int cnt = std::min(Ts, ns - c0), r0 = ro + c0;
@@ -498,13 +501,13 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
       ko(nos + 1, 0), kld(nos, 0);
   for (int t = 0; t < nos; t++) {
     size_t ns = s->n_by_type[t], Ms = m->M_by_type[t];
-    wo[t + 1] = wo[t] + ns * Ms;
-    kld[t] = (Ms + 15) / 16 * 16;  // rows of whole 128-byte lines
+    kld[t] = (Ms + 15) / 16 * 16;  // rows of whole 128-byte lines (w and k)
+    wo[t + 1] = wo[t] + ns * kld[t];
     ko[t + 1] = ko[t] + ns * kld[t];
     so[t + 1] = so[t] + ns * (size_t)split_ld((long long)Ms);
     eo[t + 1] = eo[t] + ns * (size_t)std::max(1, gemm_col_tiles(form, (int)Ms));
     int Lr = want_var ? m->L_rows[t] : 0;
-    qo[t + 1] = qo[t] + ns * (size_t)gemm_row_tiles(FM_FORM_FP64, Lr);
+    qo[t + 1] = qo[t] + ns * (size_t)gemm_row_tiles(Lr);
   }
   DevBuf W, Wh, Wl;
   if (f64) {
@@ -537,8 +540,10 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
   DevBuf out(pool, (size_t)n_out * sizeof(double));
   double sig2 = m->sigma * m->sigma;
 
-  // Kernel contraction S = B_s X_hat_s^T with the fused epilogue.
+  // Kernel contraction S = B_s X_hat_s^T with the fused epilogue (FP64: all
+  // species in one launch).
   ctx->mark_begin(ST_SGEMM);
+  std::vector<F64Gemm> f64_k, f64_g, f64_q;
   for (int t = 0; t < nos; t++) {
     int ns = s->n_by_type[t], Ms = m->M_by_type[t], ro = s->type_off[t];
     if (ns == 0) continue;
@@ -554,7 +559,7 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
     ek.alpha = m->alpha[t].as<double>();
     if (f64) {
       ek.W = W.as<double>() + wo[t];
-      ek.ldw = Ms;
+      ek.ldw = (long long)kld[t];
     } else {
       ek.Wh = Wh.as<uint16_t>() + so[t];
       ek.Wl = Wl.as<uint16_t>() + so[t];
@@ -567,9 +572,8 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
     ek.part = Epart.as<double>() + eo[t];
     ek.part_ld = ns;
     if (f64) {
-      KScope timer(ctx, KT_SGEMM);
-      gemm_f64(st, EP_KERNEL, ns, Ms, nd, s->B.as<double>() + (size_t)ro * nd, nd,
-               m->X[t].as<double>(), nd, 0, ek);
+      f64_k.push_back({s->B.as<double>() + (size_t)ro * nd, m->X[t].as<double>(), nd, nd, ns, Ms,
+                       nd, 0, ek});
     } else {
       SliceOperand A;
       if (s->has_q) {
@@ -584,6 +588,10 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
       kernel_contraction_i8(m, st, t, A, ns, nd, ek);
     }
     ctx->launches[ST_SGEMM]++;
+  }
+  if (!f64_k.empty()) {
+    KScope timer(ctx, KT_SGEMM);
+    gemm_f64_groups(st, EP_KERNEL, f64_k);
   }
   ctx->mark_end(ST_SGEMM);
 
@@ -600,11 +608,11 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
     EpArgs eg;
     eg.W = Grow;
     eg.ldw = nd;
-    KScope timer(ctx, KT_GGEMM);
-    if (f64)
-      gemm_f64(st, EP_STORE, ns, nd, Ms, W.as<double>() + wo[t], Ms, m->XT[t].as<double>(), Ms,
-               0, eg);
-    else {
+    if (f64) {
+      f64_g.push_back({W.as<double>() + wo[t], m->XT[t].as<double>(), (long long)kld[t], Ms, ns,
+                       nd, Ms, 0, eg});
+    } else {
+      KScope timer(ctx, KT_GGEMM);
       long long ldm = split_ld(Ms);
       SplitOperand A, Bx;
       A.piece[0] = Wh.as<uint16_t>() + so[t];
@@ -616,6 +624,10 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
       gemm_split(st, EP_STORE, 2, ns, nd, (int)ldm, A, Bx, eg);
     }
     ctx->launches[ST_GGEMM]++;
+  }
+  if (!f64_g.empty()) {
+    KScope timer(ctx, KT_GGEMM);
+    gemm_f64_groups(st, EP_STORE, f64_g);
   }
   ctx->mark_end(ST_GGEMM);
 
@@ -650,21 +662,27 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
     FM_HIP(hipEventRecord(ctx->ev_fork, st));
     FM_HIP(hipStreamWaitEvent(sd, ctx->ev_fork, 0));
     ctx->mark_begin(ST_VAR, sd);
+    std::vector<F64Gemm> full_q;  // species whose L block is not triangular
     for (int t = 0; t < nos; t++) {
       int ns = s->n_by_type[t], Ms = m->M_by_type[t];
       if (ns == 0 || Ms == 0 || m->L_rows[t] == 0) continue;
       EpArgs eq;
       eq.part = Qpart.as<double>() + qo[t];
       eq.part_ld = ns;
-      KScope timer(ctx, KT_VAR, sd);
-      gemm_f64(sd, EP_SUMSQ, m->L_rows[t], ns, Ms, m->L[t].as<double>(), Ms,
-               Kb.as<double>() + ko[t], (long long)kld[t], m->L_lower[t], eq);
+      std::vector<F64Gemm> &q = m->L_lower[t] ? f64_q : full_q;
+      q.push_back({m->L[t].as<double>(), Kb.as<double>() + ko[t], Ms, (long long)kld[t],
+                   m->L_rows[t], ns, Ms, m->L_lower[t], eq});
       ctx->launches[ST_VAR]++;
+    }
+    {
+      KScope timer(ctx, KT_VAR, sd);
+      gemm_f64_groups(sd, EP_SUMSQ, f64_q);
+      gemm_f64_groups(sd, EP_SUMSQ, full_q);
     }
     for (int t = 0; t < nos; t++) {
       int ns = s->n_by_type[t], Ms = m->M_by_type[t], ro = s->type_off[t];
       if (ns == 0) continue;
-      int n_qt = Ms > 0 ? gemm_row_tiles(FM_FORM_FP64, m->L_rows[t]) : 0;
+      int n_qt = Ms > 0 ? gemm_row_tiles(m->L_rows[t]) : 0;
       hipLaunchKernelGGL(k_var_final, dim3((ns + 255) / 256), dim3(256), 0, sd, ns, ro,
                          Qpart.as<double>() + qo[t], n_qt, (long long)ns, s->norm.as<double>(),
                          s->nn.as<double>(), sig2, m->power, var_row.as<double>());
