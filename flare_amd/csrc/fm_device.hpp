@@ -22,6 +22,23 @@ __device__ __forceinline__ T wave_sum(T v) {
   return v;
 }
 
+// Sum over the 16 lanes of a row on the VALU (no LDS round trips): partners
+// 1, 2, 7 and 15 lanes away by quad permutes and row mirrors.
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double x) {
+  long long v = __builtin_bit_cast(long long, x);
+  int lo = __builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
+  int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double row16_sum(double x) {
+  x += dpp_f64<0xb1>(x);   // quad_perm 1, 0, 3, 2
+  x += dpp_f64<0x4e>(x);   // quad_perm 2, 3, 0, 1
+  x += dpp_f64<0x141>(x);  // row_half_mirror
+  x += dpp_f64<0x140>(x);  // row_mirror
+  return x;
+}
+
 // Chebyshev values T_n(x) and dT_n/dr on x = (r - r1) / (rc - r1)
 // (radial.cpp:138-169), times the cutoff f_c(r) (cutoffs.cpp:44-73).
 // g[n] = T_n f_c, dg[n] = T_n' f_c + T_n f_c' (so grad g_n = dg[n] r_hat).

@@ -143,23 +143,6 @@ __device__ __forceinline__ void ep_store(const EpArgs &e, const TileOut<Acc, TM,
 // the choice of tile changes no bit: batched, tiled and single evaluations
 // agree.
 // ---------------------------------------------------------------------------
-// Sum over the 16 lanes of a row on the VALU (no LDS round trips): partners
-// 1, 2, 7 and 15 lanes away by quad permutes and row mirrors.
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double x) {
-  long long v = __builtin_bit_cast(long long, x);
-  int lo = __builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
-  int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), CTRL, 0xf, 0xf, true);
-  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
-}
-__device__ __forceinline__ double row16_sum(double x) {
-  x += dpp_f64<0xb1>(x);   // quad_perm 1, 0, 3, 2
-  x += dpp_f64<0x4e>(x);   // quad_perm 2, 3, 0, 1
-  x += dpp_f64<0x141>(x);  // row_half_mirror
-  x += dpp_f64<0x140>(x);  // row_mirror
-  return x;
-}
-
 // Element j of lane group g (lanes 16 g .. 16 g + 15) becomes element g of
 // group j: a 4 x 4 transpose across the four lane groups.
 __device__ __forceinline__ void transpose_groups(double (&x)[4]) {

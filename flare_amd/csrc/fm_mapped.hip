@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "fm_device.hpp"
+#include "fm_gather.hpp"
 #include "fm_gemm.hpp"
 #include "fm_internal.hpp"
 
@@ -119,46 +120,14 @@ __global__ void k_mapped_energy(int ns, int ro, int d, const double *B, const do
   if (lane == 0) E_row[row] = e;
 }
 
-// Forces (atom order), per-atom energies, and per-chunk virial partials;
-// one block per chunk of <= 256 atoms of one structure.
-__global__ void k_mapped_gather(const int *chunk_begin, const int *chunk_end, const int *bond_off,
-                                const int *in_off, const int *in_bond, const double *fbond,
-                                const int *row_of_atom, const double *E_row, const double *vir,
-                                double *F, double *Eatom, double *blk_part) {
-  __shared__ double sh[6][256];
-  int c = blockIdx.x;
-  int i = chunk_begin[c] + threadIdx.x;
-  double v[6] = {0, 0, 0, 0, 0, 0};
-  if (i < chunk_end[c]) {
-    double f[3] = {0, 0, 0};
-    for (int b = bond_off[i]; b < bond_off[i + 1]; b++)
-      for (int q = 0; q < 3; q++) f[q] += fbond[3 * (size_t)b + q];
-    for (int a = in_off[i]; a < in_off[i + 1]; a++) {
-      int b = in_bond[a];
-      for (int q = 0; q < 3; q++) f[q] -= fbond[3 * (size_t)b + q];
-    }
-    for (int q = 0; q < 3; q++) F[3 * (size_t)i + q] = f[q];
-    Eatom[i] = E_row[row_of_atom[i]];
-    for (int q = 0; q < 6; q++) v[q] = vir[6 * (size_t)i + q];
-  }
-  for (int q = 0; q < 6; q++) sh[q][threadIdx.x] = v[q];
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (threadIdx.x < st)
-      for (int q = 0; q < 6; q++) sh[q][threadIdx.x] += sh[q][threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x < 6) blk_part[(size_t)c * 6 + threadIdx.x] = sh[threadIdx.x][0];
-}
-
-__global__ void k_mapped_sum(int n_struct, const int *struct_chunk_off, const double *blk_part,
-                             double *vir) {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n_struct) return;
-  double acc[6] = {0, 0, 0, 0, 0, 0};
-  for (int c = struct_chunk_off[k]; c < struct_chunk_off[k + 1]; c++)
-    for (int q = 0; q < 6; q++) acc[q] += blk_part[(size_t)c * 6 + q];
-  for (int q = 0; q < 6; q++) vir[6 * (size_t)k + q] = acc[q];
+// Virial of each structure (one wave each) from its chunks' sums.
+__global__ __launch_bounds__(64) void k_mapped_sum(const int *struct_chunk_off, const double *part,
+                                                   double *vir) {
+  int k = blockIdx.x;
+  double acc[6];
+  structure_sums<6>(struct_chunk_off, part, k, acc);
+  if (threadIdx.x == 0)
+    for (int q = 0; q < 6; q++) vir[6 * (size_t)k + q] = acc[q];
 }
 
 __global__ void k_zero(double *x, long long n) {
@@ -230,11 +199,14 @@ static void mapped_run(fm_mapped mp, fm_structure s, const MappedBufs &b, double
   if (n > 0) {
     launch_adjoint(s, b.G, d, b.fbond, b.vir, mp->normalized ? 1 : 0, -1.0, 1e-8, nullptr, 0,
                    b.U);
-    hipLaunchKernelGGL(k_mapped_gather, dim3(s->n_chunks), dim3(256), 0, st,
-                       s->d_chunk_begin.as<int>(), s->d_chunk_end.as<int>(), s->bond_off.as<int>(),
-                       s->in_off.as<int>(), s->in_bond.as<int>(), b.fbond,
-                       s->row_of_atom.as<int>(), b.E_row, b.vir, b.F, b.Ea, b.blk);
-    hipLaunchKernelGGL(k_mapped_sum, dim3((s->n_struct + 63) / 64), dim3(64), 0, st, s->n_struct,
+    hipLaunchKernelGGL(k_forces<double>, dim3((n + kGatherAtoms - 1) / kGatherAtoms), dim3(256),
+                       0, st, n, (const int *)nullptr, (const int *)nullptr,
+                       (const long long *)nullptr, s->bond_off.as<int>(), s->in_off.as<int>(),
+                       s->in_bond.as<int>(), b.fbond, s->row_of_atom.as<int>(), b.E_row, b.F, b.Ea);
+    hipLaunchKernelGGL(k_chunk_sums<6>, dim3(s->n_chunks), dim3(256), 0, st,
+                       s->d_chunk_begin.as<int>(), s->d_chunk_end.as<int>(),
+                       (const int *)nullptr, (const double *)nullptr, b.vir, b.blk);
+    hipLaunchKernelGGL(k_mapped_sum, dim3(s->n_struct), dim3(64), 0, st,
                        s->d_struct_chunk_off.as<int>(), b.blk, b.vsum);
   }
   FM_HIP(hipGetLastError());

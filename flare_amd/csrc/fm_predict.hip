@@ -6,10 +6,13 @@
 // normalized_dot_product.cpp:117-214).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "fm_device.hpp"
+#include "fm_gather.hpp"
 #include "fm_gemm.hpp"
 #include "fm_internal.hpp"
 
@@ -51,66 +54,66 @@ __global__ void k_species_final(int n_rows, int ro, const double *Epart, int n_e
         row_variance(r, Qpart, n_qtiles, part_ld, norm[ro + r], nn[ro + r], sig2, power);
 }
 
-// The variance half alone (run on the side stream).
-__global__ void k_var_final(int n_rows, int ro, const double *Qpart, int n_qtiles,
-                            long long part_ld, const double *norm, const double *nn, double sig2,
+// Row sums of the untiled path for up to kFinalTypes species in one launch:
+// species u's rows are [ro[u], ro[u + 1]), its nt[u] partials of ld ro[u + 1] -
+// ro[u] at part[u].
+constexpr int kFinalTypes = 8;
+struct FinalArgs {
+  int types, ro[kFinalTypes + 1], nt[kFinalTypes];
+  const double *part[kFinalTypes];
+};
+
+// Local energies.
+__global__ void k_energy_final(FinalArgs a, double *E_row) {
+  int r = a.ro[0] + blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= a.ro[a.types]) return;
+  int u = 0;
+  while (r >= a.ro[u + 1]) u++;
+  long long ld = a.ro[u + 1] - a.ro[u];
+  const double *p = a.part[u] + (r - a.ro[u]);
+  double e = 0;
+#pragma unroll 8
+  for (int t = 0; t < a.nt[u]; t++) e += p[t * ld];
+  E_row[r] = e;
+}
+
+// Local variances.
+__global__ void k_var_final(FinalArgs a, const double *norm, const double *nn, double sig2,
                             double power, double *var_row) {
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n_rows) return;
-  var_row[ro + r] =
-      row_variance(r, Qpart, n_qtiles, part_ld, norm[ro + r], nn[ro + r], sig2, power);
+  int r = a.ro[0] + blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= a.ro[a.types]) return;
+  int u = 0;
+  while (r >= a.ro[u + 1]) u++;
+  var_row[r] = row_variance(r - a.ro[u], a.part[u], a.nt[u], a.ro[u + 1] - a.ro[u], norm[r],
+                            nn[r], sig2, power);
 }
 
-// Forces: F_i = sum_{bonds b of i} f_b - sum_{bonds b with neighbour i} f_b
-// (normalized_dot_product.cpp:197-199 after K^T alpha), each list in fixed
-// order, written at the atom's slot of its structure's mean_efs. One block
-// per chunk of <= 256 atoms of one structure; the block also reduces the
-// chunk's energies and virials.
-template <typename TF>
-__global__ void k_gather(const int *chunk_begin, const int *chunk_end, const int *atom_struct,
-                         const int *atom_off, const long long *mean_off, const int *bond_off,
-                         const int *in_off, const int *in_bond, const TF *fbond,
-                         const int *row_of_atom, const double *E_row, const double *vir,
-                         double *out, double *blk_part) {
-  __shared__ double sh[7][256];
-  int c = blockIdx.x;
-  int i = chunk_begin[c] + threadIdx.x;
-  double e = 0, v[6] = {0, 0, 0, 0, 0, 0};
-  if (i < chunk_end[c]) {
-    double f[3] = {0, 0, 0};
-    for (int b = bond_off[i]; b < bond_off[i + 1]; b++)
-      for (int q = 0; q < 3; q++) f[q] += (double)fbond[3 * (size_t)b + q];
-    for (int a = in_off[i]; a < in_off[i + 1]; a++) {
-      int b = in_bond[a];
-      for (int q = 0; q < 3; q++) f[q] -= (double)fbond[3 * (size_t)b + q];
+// Calls launch(args, rows) for the species of a structure, kFinalTypes at a
+// time; part(t) gives species t's partials and their count.
+template <typename Part, typename Launch>
+static void for_final_types(fm_structure s, Part &&part, Launch &&launch) {
+  for (int t0 = 0; t0 < s->nos; t0 += kFinalTypes) {
+    FinalArgs a{};
+    a.types = std::min(kFinalTypes, s->nos - t0);
+    for (int u = 0; u < a.types; u++) {
+      a.ro[u] = s->type_off[t0 + u];
+      part(t0 + u, a.part[u], a.nt[u]);
     }
-    int k = atom_struct[i];
-    double *F = out + mean_off[k] + 1 + 3 * (size_t)(i - atom_off[k]);
-    for (int q = 0; q < 3; q++) F[q] = f[q];
-    e = E_row[row_of_atom[i]];
-    for (int q = 0; q < 6; q++) v[q] = vir[6 * (size_t)i + q];
+    a.ro[a.types] = s->type_off[t0 + a.types];
+    if (a.ro[a.types] > a.ro[0]) launch(a, a.ro[a.types] - a.ro[0]);
   }
-  sh[0][threadIdx.x] = e;
-  for (int q = 0; q < 6; q++) sh[1 + q][threadIdx.x] = v[q];
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (threadIdx.x < st)
-      for (int q = 0; q < 7; q++) sh[q][threadIdx.x] += sh[q][threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x < 7) blk_part[(size_t)c * 7 + threadIdx.x] = sh[threadIdx.x][0];
+  FM_HIP(hipGetLastError());
 }
 
-// Per structure, the sum of its chunk partials in chunk order: energy and
-// stress -1/V sum_b f (x) r (normalized_dot_product.cpp:201-206).
-__global__ void k_final_sum(int n_struct, const int *struct_chunk_off, const double *blk_part,
-                            const double *vol_inv, const long long *mean_off,
-                            const int *atom_off, double *out) {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n_struct) return;
-  double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-  for (int c = struct_chunk_off[k]; c < struct_chunk_off[k + 1]; c++)
-    for (int q = 0; q < 7; q++) acc[q] += blk_part[(size_t)c * 7 + q];
+// Per structure (one wave each): energy and stress -1/V sum_b f (x) r
+// (normalized_dot_product.cpp:201-206).
+__global__ __launch_bounds__(64) void k_final_sum(const int *struct_chunk_off, const double *part,
+                                                  const double *vol_inv, const long long *mean_off,
+                                                  const int *atom_off, double *out) {
+  int k = blockIdx.x;
+  double acc[7];
+  structure_sums<7>(struct_chunk_off, part, k, acc);
+  if (threadIdx.x != 0) return;
   double *o = out + mean_off[k];
   int nk = atom_off[k + 1] - atom_off[k];
   o[0] = acc[0];
@@ -130,21 +133,21 @@ static void gather_forces(fm_structure s, bool f64, DevBuf &fbond, DevBuf &vir, 
   Pool *pool = &s->ctx->pool;
   DevBuf blk(pool, (size_t)s->n_chunks * 7 * sizeof(double));
   KScope timer(s->ctx, KT_GATHER);
-  if (f64)
-    hipLaunchKernelGGL(k_gather<double>, dim3(s->n_chunks), dim3(256), 0, st,
-                       s->d_chunk_begin.as<int>(), s->d_chunk_end.as<int>(),
-                       s->atom_struct.as<int>(), s->d_atom_off.as<int>(),
+  auto forces = [&](auto *f) {
+    using TF = std::remove_const_t<std::remove_pointer_t<decltype(f)>>;
+    hipLaunchKernelGGL(k_forces<TF>, dim3((s->n + kGatherAtoms - 1) / kGatherAtoms), dim3(256), 0,
+                       st, s->n, s->atom_struct.as<int>(), s->d_atom_off.as<int>(),
                        s->d_mean_off.as<long long>(), s->bond_off.as<int>(), s->in_off.as<int>(),
-                       s->in_bond.as<int>(), fbond.as<double>(), s->row_of_atom.as<int>(),
-                       E_row.as<double>(), vir.as<double>(), o, blk.as<double>());
-  else
-    hipLaunchKernelGGL(k_gather<float>, dim3(s->n_chunks), dim3(256), 0, st,
-                       s->d_chunk_begin.as<int>(), s->d_chunk_end.as<int>(),
-                       s->atom_struct.as<int>(), s->d_atom_off.as<int>(),
-                       s->d_mean_off.as<long long>(), s->bond_off.as<int>(), s->in_off.as<int>(),
-                       s->in_bond.as<int>(), fbond.as<float>(), s->row_of_atom.as<int>(),
-                       E_row.as<double>(), vir.as<double>(), o, blk.as<double>());
-  hipLaunchKernelGGL(k_final_sum, dim3((s->n_struct + 63) / 64), dim3(64), 0, st, s->n_struct,
+                       s->in_bond.as<int>(), (const TF *)f, s->row_of_atom.as<int>(),
+                       E_row.as<double>(), o, (double *)nullptr);
+  };
+  if (f64) forces(fbond.as<double>());
+  else forces(fbond.as<float>());
+  hipLaunchKernelGGL(k_chunk_sums<7>, dim3(s->n_chunks), dim3(256), 0, st,
+                     s->d_chunk_begin.as<int>(), s->d_chunk_end.as<int>(),
+                     s->row_of_atom.as<int>(), E_row.as<double>(), vir.as<double>(),
+                     blk.as<double>());
+  hipLaunchKernelGGL(k_final_sum, dim3(s->n_struct), dim3(64), 0, st,
                      s->d_struct_chunk_off.as<int>(), blk.as<double>(), s->d_vol_inv.as<double>(),
                      s->d_mean_off.as<long long>(), s->d_atom_off.as<int>(), o);
 }
@@ -547,11 +550,7 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
   for (int t = 0; t < nos; t++) {
     int ns = s->n_by_type[t], Ms = m->M_by_type[t], ro = s->type_off[t];
     if (ns == 0) continue;
-    if (Ms == 0) {
-      hipLaunchKernelGGL(k_fill, dim3((ns + 255) / 256), dim3(256), 0, st,
-                         Epart.as<double>() + eo[t], (long long)ns, 0.0);
-      continue;
-    }
+    if (Ms == 0) continue;
     EpArgs ek;
     ek.sig2 = sig2;
     ek.power = m->power;
@@ -632,16 +631,16 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
   ctx->mark_end(ST_GGEMM);
 
   // Local energies from the energy partials (main stream).
-  for (int t = 0; t < nos; t++) {
-    int ns = s->n_by_type[t], Ms = m->M_by_type[t], ro = s->type_off[t];
-    if (ns == 0) continue;
-    int n_et = Ms == 0 ? 1 : gemm_col_tiles(form, Ms);
-    hipLaunchKernelGGL(k_species_final, dim3((ns + 255) / 256), dim3(256), 0, st, ns, ro,
-                       Epart.as<double>() + eo[t], n_et, nullptr, 0, (long long)ns,
-                       s->norm.as<double>(), s->nn.as<double>(), sig2, m->power,
-                       E_row.as<double>(), nullptr);
-  }
-  FM_HIP(hipGetLastError());
+  for_final_types(
+      s,
+      [&](int t, const double *&p, int &nt) {
+        p = Epart.as<double>() + eo[t];
+        nt = m->M_by_type[t] == 0 ? 0 : gemm_col_tiles(form, m->M_by_type[t]);
+      },
+      [&](const FinalArgs &a, int rows) {
+        hipLaunchKernelGGL(k_energy_final, dim3((rows + 255) / 256), dim3(256), 0, st, a,
+                           E_row.as<double>());
+      });
 
   // Variance contraction Q = L_s^-1 K^T (FP64 in both forms) on the side
   // stream, after the kernel contraction that wrote k; it overlaps the
@@ -679,15 +678,17 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
       gemm_f64_groups(sd, EP_SUMSQ, f64_q);
       gemm_f64_groups(sd, EP_SUMSQ, full_q);
     }
-    for (int t = 0; t < nos; t++) {
-      int ns = s->n_by_type[t], Ms = m->M_by_type[t], ro = s->type_off[t];
-      if (ns == 0) continue;
-      int n_qt = Ms > 0 ? gemm_row_tiles(m->L_rows[t]) : 0;
-      hipLaunchKernelGGL(k_var_final, dim3((ns + 255) / 256), dim3(256), 0, sd, ns, ro,
-                         Qpart.as<double>() + qo[t], n_qt, (long long)ns, s->norm.as<double>(),
-                         s->nn.as<double>(), sig2, m->power, var_row.as<double>());
-    }
-    FM_HIP(hipGetLastError());
+    for_final_types(
+        s,
+        [&](int t, const double *&p, int &nt) {
+          p = Qpart.as<double>() + qo[t];
+          nt = m->M_by_type[t] > 0 ? gemm_row_tiles(m->L_rows[t]) : 0;
+        },
+        [&](const FinalArgs &a, int rows) {
+          hipLaunchKernelGGL(k_var_final, dim3((rows + 255) / 256), dim3(256), 0, sd, a,
+                             s->norm.as<double>(), s->nn.as<double>(), sig2, m->power,
+                             var_row.as<double>());
+        });
     ctx->mark_end(ST_VAR, sd);
     FM_HIP(hipEventRecord(ctx->ev_join, sd));
     join.active = true;
