@@ -133,17 +133,6 @@ void d2h(T *dst, const fm::DevBuf &src, size_t count, hipStream_t st) {
   if (dst && count) FM_HIP(hipMemcpyAsync(dst, src.as<T>(), count * sizeof(T), hipMemcpyDeviceToHost, st));
 }
 
-// flags[0]: bit 1 non-finite position, bit 2 negative species;
-// flags[1]: largest species.
-__global__ void k_check_positions(int n, const double *pos, const int *species, int *flags) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  for (int k = 0; k < 3; k++)
-    if (!isfinite(pos[3 * i + k])) atomicOr(&flags[0], 1);
-  if (species[i] < 0) atomicOr(&flags[0], 2);
-  atomicMax(&flags[1], species[i]);
-}
-
 }  // namespace
 
 namespace fm {
@@ -192,6 +181,17 @@ void fm_context_s::mark_end(int s, hipStream_t on) {
   (void)hipEventRecord(ev_end[s], on ? on : stream);
   recorded[s] = true;
 }
+char *fm_context_s::stage(size_t bytes) {
+  if (staging_bytes < bytes) {
+    size_t want = std::max<size_t>(2 * bytes, 64 << 10);
+    if (staging) FM_HIP(hipHostFree(staging));
+    staging = nullptr;
+    staging_bytes = 0;
+    FM_HIP(hipHostMalloc(reinterpret_cast<void **>(&staging), want, hipHostMallocDefault));
+    staging_bytes = want;
+  }
+  return staging;
+}
 void fm_context_s::kt_clear(int first, int last) {
   for (int k = first; k <= last; k++) kt[k].used = 0;
 }
@@ -222,14 +222,17 @@ int fm_context_create(int device, fm_context *out) {
     FM_CHECK(out, FM_ERR_INVALID, "null output handle");
     FM_HIP(hipSetDevice(device));
     fm::scratch_setup(device);
+    fm::descriptor_setup();
     auto *c = new fm_context_s();
     c->device = device;
     FM_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     FM_HIP(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
     FM_HIP(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
     FM_HIP(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
+    FM_HIP(hipEventCreateWithFlags(&c->ev_sizes, hipEventDisableTiming));
     FM_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->pinned),
                          fm_context_s::kPinnedWords * sizeof(int), hipHostMallocDefault));
+    FM_HIP(hipHostGetDevicePointer(reinterpret_cast<void **>(&c->pinned_dev), c->pinned, 0));
     for (int s = 0; s < fm::ST_COUNT; s++) {
       FM_HIP(hipEventCreate(&c->ev_begin[s]));
       FM_HIP(hipEventCreate(&c->ev_end[s]));
@@ -251,6 +254,8 @@ static void context_delete(fm_context ctx) {
     hipStream_t st = ctx->stream, side = ctx->side;
     (void)hipStreamSynchronize(side);
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
+    if (ctx->staging) (void)hipHostFree(ctx->staging);
+    (void)hipEventDestroy(ctx->ev_sizes);
     (void)hipEventDestroy(ctx->ev_fork);
     (void)hipEventDestroy(ctx->ev_join);
     delete ctx;
@@ -292,6 +297,9 @@ int fm_context_stream(fm_context ctx, void **stream) {
   return guarded([&] { *stream = (void *)ctx->stream; });
 }
 
+// Host species and positions up to this many bytes join the pinned upload.
+constexpr size_t kStageAtoms = 256 << 10;
+
 static int structure_create(fm_context ctx, int n_struct, const double *cells,
                             const int32_t *n_atoms, const int32_t *species,
                             const double *positions, double cutoff, bool device_ptrs,
@@ -319,15 +327,18 @@ static int structure_create(fm_context ctx, int n_struct, const double *cells,
       s->cellargs.resize(n_struct);
       s->volumes.resize(n_struct);
       s->sweep_cutoffs.resize(n_struct);
-      std::vector<int> ast(n);
       std::vector<double> vol_inv(n_struct);
+      std::vector<int> bin_off(n_struct + 1, 0);
       for (int k = 0; k < n_struct; k++) {
-        make_cellargs(cells + 9 * (size_t)k, cutoff, s->cellargs[k], s->volumes[k],
-                      s->sweep_cutoffs[k]);
+        fm::CellArgs &ca = s->cellargs[k];
+        make_cellargs(cells + 9 * (size_t)k, cutoff, ca, s->volumes[k], s->sweep_cutoffs[k]);
         vol_inv[k] = 1.0 / s->volumes[k];
         s->atom_off[k + 1] = s->atom_off[k] + n_atoms[k];
-        for (int i = s->atom_off[k]; i < s->atom_off[k + 1]; i++) ast[i] = k;
+        long long nb = (long long)ca.nb[0] * ca.nb[1] * ca.nb[2];
+        FM_CHECK(n == 0 || bin_off[k] + nb < (1LL << 30), FM_ERR_CAPACITY, "cell list too large");
+        bin_off[k + 1] = n == 0 ? 0 : bin_off[k] + (int)nb;
       }
+      s->n_bins = bin_off[n_struct];
       const fm::CellArgs &c0 = s->cellargs[0];
       for (int i = 0; i < 9; i++) {
         s->cell[i] = c0.cell[i];
@@ -339,14 +350,6 @@ static int structure_create(fm_context ctx, int n_struct, const double *cells,
       s->single_sweep_cutoff = s->sweep_cutoffs[0];
       s->cutoff = cutoff;
       s->sweep = c0.sweep;
-      auto up = [&](fm::DevBuf &buf, const void *src, size_t bytes) {
-        buf.alloc(pool, std::max<size_t>(1, bytes));
-        if (bytes) FM_HIP(hipMemcpyAsync(buf.as<void>(), src, bytes, hipMemcpyHostToDevice, st));
-      };
-      up(s->d_cellargs, s->cellargs.data(), s->cellargs.size() * sizeof(fm::CellArgs));
-      up(s->atom_struct, ast.data(), ast.size() * sizeof(int));
-      up(s->d_atom_off, s->atom_off.data(), s->atom_off.size() * sizeof(int));
-      up(s->d_vol_inv, vol_inv.data(), vol_inv.size() * sizeof(double));
       // mean_efs offsets and reduction chunks per structure.
       s->mean_off.assign(n_struct + 1, 0);
       std::vector<int> cb, ce, sco(n_struct + 1, 0);
@@ -360,31 +363,57 @@ static int structure_create(fm_context ctx, int n_struct, const double *cells,
       }
       s->n_chunks = (int)cb.size();
       std::vector<long long> mo(s->mean_off.begin(), s->mean_off.end());
-      up(s->d_mean_off, mo.data(), mo.size() * sizeof(long long));
-      up(s->d_chunk_begin, cb.data(), cb.size() * sizeof(int));
-      up(s->d_chunk_end, ce.data(), ce.size() * sizeof(int));
-      up(s->d_struct_chunk_off, sco.data(), sco.size() * sizeof(int));
-      s->species.alloc(pool, std::max<size_t>(1, (size_t)n * sizeof(int)));
-      s->positions.alloc(pool, std::max<size_t>(1, 3 * (size_t)n * sizeof(double)));
-      hipMemcpyKind kind = device_ptrs ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-      if (n > 0) {
-        FM_HIP(hipMemcpyAsync(s->species.as<int>(), species, (size_t)n * sizeof(int), kind, st));
-        FM_HIP(hipMemcpyAsync(s->positions.as<double>(), positions, 3 * (size_t)n * sizeof(double),
-                              kind, st));
-        // The position / species flags are read back with the neighbour
-        // build's size readback (one synchronisation); the neighbour kernels
-        // only bin (clamped) and copy species, so bad input cannot take
-        // them out of bounds before it is reported.
-        fm::DevBuf flags(pool, 2 * sizeof(int));
-        FM_HIP(hipMemsetAsync(flags.as<int>(), 0, 2 * sizeof(int), st));
-        hipLaunchKernelGGL(k_check_positions, dim3((n + 255) / 256), dim3(256), 0, st, n,
-                           s->positions.as<double>(), s->species.as<int>(), flags.as<int>());
-        FM_HIP(hipMemcpyAsync(ctx->pinned, flags.as<int>(), 2 * sizeof(int),
-                              hipMemcpyDeviceToHost, st));
+      // All host arrays in one upload from pinned memory (each a copy of its
+      // own from pageable memory cost 5 us of launch and 3 us of GPU), small
+      // species and positions among them.
+      size_t n_pos = 3 * (size_t)n * sizeof(double), n_sp = (size_t)n * sizeof(int);
+      bool staged = !device_ptrs && n_pos + n_sp <= kStageAtoms;
+      struct Part {
+        fm::DevBuf *buf;
+        const void *src;
+        size_t bytes;
+      };
+      std::vector<Part> parts = {
+          {&s->d_cellargs, s->cellargs.data(), s->cellargs.size() * sizeof(fm::CellArgs)},
+          {&s->d_atom_off, s->atom_off.data(), s->atom_off.size() * sizeof(int)},
+          {&s->d_bin_off, bin_off.data(), bin_off.size() * sizeof(int)},
+          {&s->d_vol_inv, vol_inv.data(), vol_inv.size() * sizeof(double)},
+          {&s->d_mean_off, mo.data(), mo.size() * sizeof(long long)},
+          {&s->d_chunk_begin, cb.data(), cb.size() * sizeof(int)},
+          {&s->d_chunk_end, ce.data(), ce.size() * sizeof(int)},
+          {&s->d_struct_chunk_off, sco.data(), sco.size() * sizeof(int)}};
+      if (staged) {
+        parts.push_back({&s->species, species, n_sp});
+        parts.push_back({&s->positions, positions, n_pos});
+      }
+      size_t total = 0;
+      for (const Part &p : parts) total += (p.bytes + 15) / 16 * 16;
+      char *stage = ctx->stage(total);
+      s->meta.alloc(pool, std::max<size_t>(1, total));
+      size_t at = 0;
+      for (const Part &p : parts) {
+        if (p.bytes) std::memcpy(stage + at, p.src, p.bytes);
+        p.buf->view(s->meta, at, p.bytes);
+        at += (p.bytes + 15) / 16 * 16;
+      }
+      FM_HIP(hipMemcpyAsync(s->meta.as<void>(), stage, total, hipMemcpyHostToDevice, st));
+      s->atom_struct.alloc(pool, std::max<size_t>(1, n_sp));
+      if (!staged) {
+        s->species.alloc(pool, std::max<size_t>(1, n_sp));
+        s->positions.alloc(pool, std::max<size_t>(1, n_pos));
+        if (n > 0 && !device_ptrs) {
+          FM_HIP(hipMemcpyAsync(s->species.as<int>(), species, n_sp, hipMemcpyHostToDevice, st));
+          FM_HIP(hipMemcpyAsync(s->positions.as<double>(), positions, n_pos,
+                                hipMemcpyHostToDevice, st));
+        }
       }
       ctx->mark_begin(fm::ST_NEIGH);
       if (n > 0) {
-        fm::build_neighbors(s);  // synchronises: ctx->pinned[0, 2) is valid after
+        // The position / species checks come back with the size readback (one
+        // synchronisation); the neighbour kernels only bin (clamped) and copy
+        // species, so bad input cannot take them out of bounds before it is
+        // reported.
+        fm::build_neighbors(s, device_ptrs ? species : nullptr, device_ptrs ? positions : nullptr);
         int hf0 = ctx->pinned[0], hf1 = ctx->pinned[1];
         FM_CHECK(!(hf0 & 1), FM_ERR_INVALID, "positions contain NaN or Inf");
         FM_CHECK(!(hf0 & 2), FM_ERR_INVALID, "species must be non-negative");
@@ -392,6 +421,7 @@ static int structure_create(fm_context ctx, int n_struct, const double *cells,
       } else {
         s->cumulative.alloc(pool, sizeof(int));
         FM_HIP(hipMemsetAsync(s->cumulative.as<int>(), 0, sizeof(int), st));
+        FM_HIP(hipStreamSynchronize(st));  // the staging buffer is free again
       }
       ctx->mark_end(fm::ST_NEIGH);
     } catch (...) {
@@ -516,20 +546,12 @@ static void compute_descriptor(fm_structure s, const fm_b2_settings *st_in, int 
       // Species must lie in [0, n_species) for this descriptor.
       FM_CHECK(s->max_species < s->nos, FM_ERR_INVALID, "species outside [0, n_species)");
     }
-    std::vector<int> pairs;
-    for (int a = 0; a < nr; a++)
-      for (int b = a; b < nr; b++) {
-        pairs.push_back(a);
-        pairs.push_back(b);
-      }
-    s->pair_table.alloc(pool, pairs.size() * sizeof(int));
-    FM_HIP(hipMemcpyAsync(s->pair_table.as<int>(), pairs.data(), pairs.size() * sizeof(int),
-                          hipMemcpyHostToDevice, stream));
     ctx->mark_begin(fm::ST_DESC);
     ctx->kt_clear(fm::KT_DESC, fm::KT_DESC);
     if (s->n > 0) fm::build_bonds(s);
     else {
       s->n_by_type.assign(s->nos, 0);
+      s->nb_by_type.assign(s->nos, 0);
       s->type_off.assign(s->nos + 1, 0);
       s->n_bonds = 0;
     }
@@ -552,12 +574,12 @@ static void compute_descriptor(fm_structure s, const fm_b2_settings *st_in, int 
     s->nn.alloc(pool, std::max<size_t>(1, (size_t)s->n * sizeof(double)));
     if (s->n > 0) {
       fm::launch_b2(s, kind == 2);
+      fm::bonds_ready(s);  // sizes of the bond build, while the descriptors run
       if (kind == 3 && s->row_tile == 0) fm::launch_b3(s);
     }
     ctx->mark_end(fm::ST_DESC);
     // Per-structure species-sorted position of every row (batches only).
     fm::build_var_pos(s);
-    s->nb_by_type.clear();  // filled on first export (nb_by_type_of)
     s->has_dervs = false;    // dense derivatives are rebuilt on demand
     s->DB.release();
     s->has_b2 = true;
@@ -572,26 +594,10 @@ int fm_structure_compute_b3(fm_structure s, const fm_b2_settings *st_in, int for
   return guarded([&] { compute_descriptor(s, st_in, form, 3); });
 }
 
-// Neighbour counts by species (b2.cpp:106-112), computed on first use.
-static void nb_by_type_of(fm_structure s) {
-  if (!s->nb_by_type.empty()) return;
-  s->nb_by_type.assign(s->nos, 0);
-  if (s->n == 0) return;
-  hipStream_t st = s->ctx->stream;
-  std::vector<int> bo(s->n + 1), sp(s->n);
-  FM_HIP(hipMemcpyAsync(bo.data(), s->bond_off.as<int>(), (s->n + 1) * sizeof(int),
-                        hipMemcpyDeviceToHost, st));
-  FM_HIP(hipMemcpyAsync(sp.data(), s->species.as<int>(), s->n * sizeof(int),
-                        hipMemcpyDeviceToHost, st));
-  FM_HIP(hipStreamSynchronize(st));
-  for (int i = 0; i < s->n; i++) s->nb_by_type[sp[i]] += bo[i + 1] - bo[i];
-}
-
 int fm_structure_b2_sizes(fm_structure s, int *n_descriptors, int32_t *n_clusters_by_type,
                           int32_t *n_neighbors_by_type) {
   return guarded([&] {
     FM_CHECK(s && s->has_b2, FM_ERR_STATE, "descriptors have not been computed");
-    nb_by_type_of(s);
     if (n_descriptors) *n_descriptors = s->nd;
     for (int t = 0; t < s->nos; t++) {
       if (n_clusters_by_type) n_clusters_by_type[t] = s->n_by_type[t];

@@ -36,7 +36,6 @@ struct B2Args {
   double r1;
   const int *species, *bond_off, *bond_q, *nspec, *row_of_atom;
   const double *rel, *cutoffs;
-  const int2 *pairs;  // n1, n2 of each radial pair in B2 order
 };
 
 __constant__ double c_knorm[kMaxH];
@@ -937,7 +936,6 @@ static B2Args make_args(fm_structure s) {
   a.row_of_atom = s->row_of_atom.as<int>();
   a.rel = s->rel.as<double>();
   a.cutoffs = s->d_cutoffs.as<double>();
-  a.pairs = s->pair_table.as<int2>();
   return a;
 }
 
@@ -953,21 +951,13 @@ void knorm_values(int lmax, double *out) {
     }
 }
 
-// The whole table (l <= 10) is written every time: entries do not depend on
-// the descriptor's lmax, so uploads from several streams write equal values.
-static void upload_knorm(hipStream_t st, int) {
-  static thread_local double host[kMaxH];
-  knorm_values(kMaxL, host);
-  FM_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_knorm), host, sizeof(host), 0, hipMemcpyHostToDevice,
-                                st));
-}
-
-static void upload_rcp(hipStream_t st) {
-  static thread_local double host[kMaxL + 2];
-  host[0] = 0;
-  for (int k = 1; k < kMaxL + 2; k++) host[k] = 1.0 / k;
-  FM_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_rcp), host, sizeof(host), 0, hipMemcpyHostToDevice,
-                                st));
+// The constant tables of the current device, l <= kMaxL.
+void descriptor_setup() {
+  double kn[kMaxH], rcp[kMaxL + 2] = {0};
+  knorm_values(kMaxL, kn);
+  for (int k = 1; k < kMaxL + 2; k++) rcp[k] = 1.0 / k;
+  FM_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_knorm), kn, sizeof(kn), 0, hipMemcpyHostToDevice));
+  FM_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_rcp), rcp, sizeof(rcp), 0, hipMemcpyHostToDevice));
 }
 
 void launch_b2(fm_structure s, bool want_b2) {
@@ -975,8 +965,6 @@ void launch_b2(fm_structure s, bool want_b2) {
   hipStream_t st = ctx->stream;
   FM_CHECK(s->N <= kMaxN, FM_ERR_INVALID, "n_max above 16 is not supported");
   FM_CHECK(s->lmax <= kMaxL, FM_ERR_INVALID, "l_max above 10 is not supported");
-  upload_knorm(st, s->lmax);
-  upload_rcp(st);
   B2Args a = make_args(s);
   // The chosen form's B2 rows are computed in FP64 (mixed: FP32 row and c
   // for the adjoint, int8 slices of the FP64 row for the kernel
@@ -1023,29 +1011,18 @@ void launch_b2(fm_structure s, bool want_b2) {
   s->C.alloc(&ctx->pool, std::max<size_t>(1, (size_t)s->n * a.nrad * a.H * esz));
   MixedOut mo{};
   if (mixed) {
-    // Each species' rows start a row tile of the slices.
+    // Each species' rows start a row tile of the slices (q_shift, from the
+    // row build); at most a tile less one of padding per species.
     s->ldq = i8_ld(a.nd);
-    s->q_tile_row.assign(s->nos, 0);
-    std::vector<int> &shift = s->q_shift_host;  // kept with the structure for the async copy
-    shift.assign(s->nos, 0);
-    long long qrows = 0;
-    for (int t = 0; t < s->nos; t++) {
-      s->q_tile_row[t] = qrows;
-      shift[t] = (int)(qrows - s->type_off[t]);
-      qrows += (s->n_by_type[t] + kI8TileA - 1) / kI8TileA * kI8TileA;
-    }
+    long long qrows = s->n + (long long)s->nos * (kI8TileA - 1);
     FM_CHECK(qrows < (1LL << 31), FM_ERR_CAPACITY, "too many descriptor rows for the slices");
     s->Bq.alloc(&ctx->pool, std::max<size_t>(1, i8_tiled_bytes(qrows, kI8TileA, s->ldq)));
     s->Bq_scale.alloc(&ctx->pool, std::max<size_t>(1, (size_t)s->n * sizeof(double)));
-    s->q_shift.alloc(&ctx->pool, (size_t)s->nos * sizeof(int));
-    FM_HIP(hipMemcpyAsync(s->q_shift.as<int>(), shift.data(), shift.size() * sizeof(int),
-                          hipMemcpyHostToDevice, st));
     mo = MixedOut{s->B.as<float>(), s->C.as<float>(), s->Bq.as<int8_t>(),
                   s->Bq_scale.as<double>(), s->ldq / kI8Pad, s->q_shift.as<int>()};
   } else {
     s->Bq.release();
     s->Bq_scale.release();
-    s->q_shift.release();
   }
   s->has_q = mixed;
   if (nblk == 0) return;
@@ -1103,8 +1080,6 @@ void launch_adjoint(fm_structure s, const void *G, int64_t g_ld, void *fbond,
   hipStream_t st = ctx->stream;
   B2Args a = make_args(s);
   FM_CHECK(a.lmax + 1 < kMaxL + 2, FM_ERR_INVALID, "l_max above 10 is not supported");
-  upload_knorm(st, s->lmax);
-  upload_rcp(st);
   bool f64 = s->form == FM_FORM_FP64;
   size_t esz = f64 ? sizeof(double) : sizeof(float);
   size_t nc = (size_t)a.nrad * a.H;
@@ -1162,8 +1137,6 @@ void launch_bond_forces(fm_structure s, const void *U, void *fbond, double *viri
   if (n_list == 0) return;
   hipStream_t st = s->ctx->stream;
   B2Args a = make_args(s);
-  upload_knorm(st, s->lmax);
-  upload_rcp(st);
   bool f64 = s->form == FM_FORM_FP64;
   size_t esz = f64 ? sizeof(double) : sizeof(float);
   AdjArgs aa{1, empty_norm, empty_nn, nullptr, 0};

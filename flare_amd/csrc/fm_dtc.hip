@@ -436,6 +436,15 @@ void compute_dervs(fm_structure s) {
   s->DB.alloc(pool, std::max<size_t>(1, nb * 3 * nd * sizeof(double)));
   s->fdots.alloc(pool, std::max<size_t>(1, nb * 3 * sizeof(double)));
   upload_knorm_d(st, s->lmax);
+  // n1, n2 of each radial pair in B2 order.
+  std::vector<int> pairs;
+  for (int a = 0; a < nrad; a++)
+    for (int b = a; b < nrad; b++) {
+      pairs.push_back(a);
+      pairs.push_back(b);
+    }
+  DevBuf pair_table;
+  up(pair_table, pairs.data(), pairs.size() * sizeof(int));
   size_t lds = ((size_t)nrad * H + (size_t)s->N * H * 3) * sizeof(double);
   FM_CHECK(lds <= 160 * 1024, FM_ERR_CAPACITY, "derivative workspace exceeds LDS");
   if (n > 0)
@@ -443,7 +452,7 @@ void compute_dervs(fm_structure s) {
                        nd, s->cutkind, s->r1, s->species.as<int>(), s->bond_off.as<int>(),
                        s->bond_q.as<int>(), s->nspecies.as<int>(), s->rel.as<double>(),
                        s->d_cutoffs.as<double>(), s->row_of_atom.as<int>(), s->sb_off.as<int>(),
-                       s->pair_table.as<int2>(), s->B.as<double>(), s->DB.as<double>(),
+                       pair_table.as<int2>(), s->B.as<double>(), s->DB.as<double>(),
                        s->fdots.as<double>());
   FM_HIP(hipGetLastError());
   FM_HIP(hipStreamSynchronize(st));

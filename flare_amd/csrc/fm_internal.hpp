@@ -85,6 +85,14 @@ class DevBuf {
     if (p_ && pool_) pool_->put(p_, cls_);
     p_ = nullptr;
   }
+  // A range of another buffer, which stays its owner (and must outlive this).
+  void view(const DevBuf &owner, size_t offset, size_t bytes) {
+    release();
+    pool_ = nullptr;
+    p_ = owner.as<char>() + offset;
+    bytes_ = bytes;
+    cls_ = 0;
+  }
   template <typename T>
   T *as() const {
     return reinterpret_cast<T *>(p_);
@@ -130,16 +138,23 @@ struct fm_context_s {
   int device = 0;
   hipStream_t stream = nullptr;
   fm::Pool pool;
-  // Pinned host words for small device-to-host readbacks (sizes, flags), so
-  // several can be queued and waited for with one stream synchronisation.
-  // Calls on one context are sequential (they share its stream).
-  static constexpr int kPinnedWords = 64;
-  int *pinned = nullptr;
+  // Pinned host words that kernels write sizes and flags to directly (pinned_dev
+  // is their device address), read after the stream synchronisation of the
+  // call. Calls on one context are sequential (they share its stream).
+  static constexpr int kPinnedWords = 256;
+  int *pinned = nullptr, *pinned_dev = nullptr;
+  // Pinned staging for a structure's small host arrays (one upload per
+  // structure). Reused by the next structure: each build waits for its stream
+  // after the upload.
+  char *staging = nullptr;
+  size_t staging_bytes = 0;
+  char *stage(size_t bytes);
   // Second stream (default priority) for work that overlaps the main one:
   // the variance contraction runs there while the gradient contraction and
   // the adjoint run on `stream`. fork / join order them with events.
   hipStream_t side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  hipEvent_t ev_sizes = nullptr;  // after the sizes of a bond build are written
   // Row tile for B3 descriptors computed on this context (0: automatic).
   int64_t row_tile = 0;
   hipEvent_t ev_begin[fm::ST_COUNT], ev_end[fm::ST_COUNT];
@@ -195,6 +210,7 @@ struct fm_structure_s {
   std::vector<int> atom_off;
   std::vector<fm::CellArgs> cellargs;
   std::vector<double> volumes, sweep_cutoffs;
+  fm::DevBuf meta;  // owner of the host arrays uploaded together (views below)
   fm::DevBuf d_cellargs, atom_struct, d_bin_off, d_atom_off, d_mean_off, d_vol_inv;
   // Output offsets of each structure in mean_efs (1 + 3 N_k + 6 per structure)
   // and the reduction chunks (<= 256 atoms, never crossing a structure).
@@ -209,6 +225,7 @@ struct fm_structure_s {
   double volume = 0, single_sweep_cutoff = 0, cutoff = 0;
   int sweep = 0;
   int64_t n_nb = 0;
+  int n_bins = 0;  // cell-list bins of all structures
   fm::DevBuf species, positions, wrapped, count, cumulative, sidx, nspecies, rel;
   // Descriptor state (B2, or B3 built from the same bond coefficients)
   bool has_b2 = false;
@@ -221,7 +238,7 @@ struct fm_structure_s {
   int64_t n_bonds = 0;
   std::vector<int> n_by_type, nb_by_type, type_off;
   fm::DevBuf d_cutoffs, bond_off, bond_q, in_off, in_bond, row_of_atom,
-      atom_of_row, pair_table, B, norm, nn;
+      atom_of_row, B, norm, nn;
   // Density coefficients c (atom-major, n x nrad H, descriptor precision),
   // kept for the adjoint.
   fm::DevBuf C;
@@ -234,7 +251,6 @@ struct fm_structure_s {
   // type_off[t] on the device).
   fm::DevBuf Bq, Bq_scale, q_shift;
   std::vector<long long> q_tile_row;
-  std::vector<int> q_shift_host;
   long long ldq = 0;
   bool has_q = false;
   // Dense descriptor derivatives (FP64, single structure): bonds in the
@@ -301,9 +317,16 @@ void mapped_compute_noalloc(fm_mapped mp, fm_structure s, double *atom_energy, d
 void scratch_setup(int device);
 void mapped_upload(fm_mapped mp, const double *beta);
 void mapped_parse(const std::string &path, fm_mapped mp, std::vector<double> &beta);
-// Launchers (fm_neighbors.hip)
-void build_neighbors(fm_structure s);
+// Launchers (fm_neighbors.hip). build_neighbors takes the caller's device
+// species and positions (null: the structure's own are filled already), checks
+// them and synchronises: ctx->pinned[0] holds their flags (bit 1 non-finite
+// position, bit 2 negative species), [1] the largest species.
+void build_neighbors(fm_structure s, const int *species_dev, const double *positions_dev);
+// Queues the bond lists and species rows; bonds_ready waits for their sizes
+// (n_bonds, n_by_type, type_off, nb_by_type) without waiting for kernels queued
+// in between.
 void build_bonds(fm_structure s);
+void bonds_ready(fm_structure s);
 // fm_descriptors.hip (want_b2 = false computes and keeps only c)
 void launch_b2(fm_structure s, bool want_b2 = true);
 // Device var_pos of a batch (after build_bonds); releases it for one structure.
@@ -349,6 +372,11 @@ void self_kernel_struc(fm_model m, fm_structure s, double *kself_out);
 void predict_dense(fm_model m, fm_structure s, int kind, double *mean_efs, double *var_efs);
 // fm_descriptors.hip: normalisation constants of the real spherical harmonics
 void knorm_values(int lmax, double *out);
-// scans (fm_neighbors.hip)
-int scan_exclusive(fm_context ctx, const int *in, int *out, int n, bool want_total);
+// Constant tables of the current device (called when a context is created).
+void descriptor_setup();
+// out[0..n] = exclusive scan of in[0..n), out[n] the total (fm_neighbors.hip);
+// with `host` (device address of pinned words) the total goes to host[0] too and
+// the device word `extra`, if given, to host[1].
+void scan_exclusive(fm_context ctx, const int *in, int *out, int n, int *host = nullptr,
+                    const int *extra = nullptr);
 }  // namespace fm

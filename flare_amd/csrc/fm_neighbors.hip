@@ -15,6 +15,7 @@
 #include <cmath>
 
 #include "fm_device.hpp"
+#include "fm_gemm.hpp"
 #include "fm_internal.hpp"
 
 namespace fm {
@@ -51,60 +52,74 @@ __device__ __forceinline__ int block_excl_scan(int v, int *sh, int &total) {
   return base + x - v;
 }
 
-__global__ void k_scan_block_sums(const int *in, int n, int *bsum) {
+// One block: each thread scans kScanItems consecutive values.
+constexpr int kScanItems = 8;
+__global__ __launch_bounds__(kScanBlock) void k_scan_one(const int *in, int n, int *out,
+                                                         int *host, const int *extra) {
   __shared__ int sh[16];
-  int i = blockIdx.x * kScanBlock + threadIdx.x;
-  int v = i < n ? in[i] : 0;
-  int tot;
-  block_excl_scan(v, sh, tot);
+  int i0 = threadIdx.x * kScanItems, v[kScanItems], sum = 0, tot;
+#pragma unroll
+  for (int e = 0; e < kScanItems; e++) {
+    v[e] = i0 + e < n ? in[i0 + e] : 0;
+    sum += v[e];
+  }
+  int x = block_excl_scan(sum, sh, tot);
+#pragma unroll
+  for (int e = 0; e < kScanItems; e++) {
+    if (i0 + e < n) out[i0 + e] = x;
+    x += v[e];
+  }
+  if (threadIdx.x == 0) {
+    out[n] = tot;
+    if (host) host[0] = tot;
+    if (host && extra) host[1] = *extra;
+  }
+}
+
+__global__ __launch_bounds__(kScanBlock) void k_scan_block_sums(const int *in, int n, int *bsum) {
+  __shared__ int sh[16];
+  int i = blockIdx.x * kScanBlock + threadIdx.x, tot;
+  block_excl_scan(i < n ? in[i] : 0, sh, tot);
   if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
 }
 
-__global__ void k_scan_sums(int *bsum, int nb) {
+// Every block sums the totals of the blocks before it, then scans its own.
+__global__ __launch_bounds__(kScanBlock) void k_scan_apply(const int *in, int n, const int *bsum,
+                                                           int *out, int *host,
+                                                           const int *extra) {
   __shared__ int sh[16];
-  int carry = 0;
-  for (int b0 = 0; b0 < nb; b0 += kScanBlock) {
-    int i = b0 + threadIdx.x;
-    int v = i < nb ? bsum[i] : 0;
-    int tot;
-    int e = block_excl_scan(v, sh, tot);
-    if (i < nb) bsum[i] = carry + e;
-    carry += tot;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) bsum[nb] = carry;
-}
-
-__global__ void k_scan_apply(const int *in, int n, const int *bsum, int *out) {
-  __shared__ int sh[16];
+  int before = 0, base, tot;
+  for (int b = threadIdx.x; b < blockIdx.x; b += kScanBlock) before += bsum[b];
+  block_excl_scan(before, sh, base);  // base: the sum over all threads
   int i = blockIdx.x * kScanBlock + threadIdx.x;
   int v = i < n ? in[i] : 0;
-  int tot;
   int e = block_excl_scan(v, sh, tot);
-  if (i < n) out[i] = bsum[blockIdx.x] + e;
-  if (i == n - 1) out[n] = bsum[blockIdx.x] + e + v;
+  if (i < n) out[i] = base + e;
+  if (i == n - 1) {
+    out[n] = base + e + v;
+    if (host) host[0] = base + e + v;
+    if (host && extra) host[1] = *extra;
+  }
 }
 
-// out[0..n] = exclusive scan of in[0..n); out[n] = total. With want_total
-// it returns the total (synchronising the context stream), otherwise 0.
-int scan_exclusive(fm_context ctx, const int *in, int *out, int n, bool want_total) {
-  if (n == 0) {
-    FM_HIP(hipMemsetAsync(out, 0, sizeof(int), ctx->stream));
-    return 0;
+// One launch up to 8,192 values (a block of 1,024 threads, 4 us), else two (the
+// launch that scanned the block totals in between is gone: every block of the
+// second sums those before it, at most a few loads per thread).
+void scan_exclusive(fm_context ctx, const int *in, int *out, int n, int *host,
+                    const int *extra) {
+  hipStream_t st = ctx->stream;
+  if (n <= kScanBlock * kScanItems) {
+    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(kScanBlock), 0, st, in, n, out, host,
+                       extra);
+  } else {
+    int nb = (n + kScanBlock - 1) / kScanBlock;
+    DevBuf bsum(&ctx->pool, nb * sizeof(int));
+    hipLaunchKernelGGL(k_scan_block_sums, dim3(nb), dim3(kScanBlock), 0, st, in, n,
+                       bsum.as<int>());
+    hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(kScanBlock), 0, st, in, n, bsum.as<int>(),
+                       out, host, extra);
   }
-  int nb = (n + kScanBlock - 1) / kScanBlock;
-  DevBuf bsum(&ctx->pool, (nb + 1) * sizeof(int));
-  hipLaunchKernelGGL(k_scan_block_sums, dim3(nb), dim3(kScanBlock), 0, ctx->stream, in, n,
-                     bsum.as<int>());
-  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanBlock), 0, ctx->stream, bsum.as<int>(), nb);
-  hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(kScanBlock), 0, ctx->stream, in, n,
-                     bsum.as<int>(), out);
   FM_HIP(hipGetLastError());
-  if (!want_total) return 0;
-  int total = 0;
-  FM_HIP(hipMemcpyAsync(&total, out + n, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-  FM_HIP(hipStreamSynchronize(ctx->stream));
-  return total;
 }
 
 // ---------------------------------------------------------------------------
@@ -116,42 +131,87 @@ __device__ __forceinline__ void row3(const double *a, const double *B, double *o
   for (int k = 0; k < 3; k++) o[k] = (a[0] * B[k] + a[1] * B[3 + k]) + a[2] * B[6 + k];
 }
 
-// structure.cpp:120-133 per atom, plus the global bin of the wrapped position.
-__global__ void k_wrap(int n, const double *pos, const CellArgs *cas, const int *atom_struct,
-                       const int *bin_off, double *wrapped, int *bin) {
+// Zeros at the start of a build: the neighbour flags and maximum, the bin
+// counts.
+struct SetupWords {
+  int flags, max_species, max_count;
+};
+
+// Per atom: the structure it belongs to, its own copy of the caller's species
+// and position (where those are in device memory), their checks (flags: bit 1
+// non-finite position, bit 2 negative species), the wrapped position
+// (structure.cpp:120-133), its bin and the bin's count.
+__global__ __launch_bounds__(256) void k_setup(int n, int n_struct, const double *src_pos,
+                                               const int *src_species, double *pos, int *species,
+                                               const CellArgs *cas, const int *atom_off,
+                                               const int *bin_off, int *atom_struct,
+                                               double *wrapped, int *bin, int *bcount,
+                                               SetupWords *words) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const CellArgs &ca = cas[atom_struct[i]];
-  double p[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
-  double r1[3], fr[3], w1[3], w[3];
-  row3(p, ca.ct, r1);
-  row3(r1, ca.cdi, fr);
-  for (int k = 0; k < 3; k++) fr[k] = fr[k] - floor(fr[k]);
-  row3(fr, ca.cd, w1);
-  row3(w1, ca.cti, w);
-  for (int k = 0; k < 3; k++) wrapped[3 * i + k] = w[k];
-  // Bin from the fractional coordinates of the wrapped position.
-  row3(w, ca.ct, r1);
-  row3(r1, ca.cdi, fr);
-  int q[3];
-  for (int k = 0; k < 3; k++) {
-    int b = (int)floor(fr[k] * ca.nb[k]);
-    q[k] = min(max(b, 0), ca.nb[k] - 1);
+  bool live = i < n;
+  int sp = live ? src_species[i] : -1;
+  int bad = 0;
+  if (live) {
+    int k = 0;  // the structure with atom_off[k] <= i < atom_off[k + 1]
+    if (n_struct > 1) {
+      int lo = 0, hi = n_struct;
+      while (hi - lo > 1) {
+        int mid = (lo + hi) >> 1;
+        if (atom_off[mid] <= i) lo = mid;
+        else hi = mid;
+      }
+      k = lo;
+    }
+    atom_struct[i] = k;
+    const CellArgs &ca = cas[k];
+    double p[3] = {src_pos[3 * i], src_pos[3 * i + 1], src_pos[3 * i + 2]};
+    if (pos != src_pos) {
+      for (int q = 0; q < 3; q++) pos[3 * i + q] = p[q];
+      species[i] = sp;
+    }
+    for (int q = 0; q < 3; q++)
+      if (!isfinite(p[q])) bad |= 1;
+    if (sp < 0) bad |= 2;
+    double r1[3], fr[3], w1[3], w[3];
+    row3(p, ca.ct, r1);
+    row3(r1, ca.cdi, fr);
+    for (int q = 0; q < 3; q++) fr[q] = fr[q] - floor(fr[q]);
+    row3(fr, ca.cd, w1);
+    row3(w1, ca.cti, w);
+    for (int q = 0; q < 3; q++) wrapped[3 * i + q] = w[q];
+    // Bin from the fractional coordinates of the wrapped position.
+    row3(w, ca.ct, r1);
+    row3(r1, ca.cdi, fr);
+    int q3[3];
+    for (int q = 0; q < 3; q++) {
+      int b = (int)floor(fr[q] * ca.nb[q]);
+      q3[q] = min(max(b, 0), ca.nb[q] - 1);
+    }
+    int b = bin_off[k] + (q3[0] * ca.nb[1] + q3[1]) * ca.nb[2] + q3[2];
+    bin[i] = b;
+    atomicAdd(&bcount[b], 1);
   }
-  bin[i] = bin_off[atom_struct[i]] + (q[0] * ca.nb[1] + q[1]) * ca.nb[2] + q[2];
+  // One atomic per wave for the largest species.
+  int mx = sp;
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) mx = max(mx, __shfl_xor(mx, off, 64));
+  if ((threadIdx.x & 63) == 0 && mx > 0) atomicMax(&words->max_species, mx);
+  if (bad) atomicOr(&words->flags, bad);
 }
 
-__global__ void k_bin_count(int n, const int *bin, int *bcount) {
+// Places each atom in its bin (any order within a bin: neighbours are sorted
+// later), counting bcount down. Thread 0 passes the checks on to the host.
+__global__ __launch_bounds__(256) void k_bin_fill(int n, const int *bin, const int *bstart,
+                                                  int *bcount, int *order,
+                                                  const SetupWords *words, int *host_words) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) atomicAdd(&bcount[bin[i]], 1);
-}
-
-__global__ void k_bin_fill(int n, const int *bin, const int *bstart, int *cursor, int *order) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) {
+    host_words[0] = words->flags;
+    host_words[1] = words->max_species;
+  }
   if (i < n) {
     int b = bin[i];
-    int slot = atomicAdd(&cursor[b], 1);
-    order[bstart[b] + slot] = i;
+    order[bstart[b] + atomicAdd(&bcount[b], -1) - 1] = i;
   }
 }
 
@@ -453,23 +513,12 @@ __global__ void k_neighbors_big(int n, const double *wrapped, const int *bin_of,
   }
 }
 
-void build_neighbors(fm_structure s) {
+void build_neighbors(fm_structure s, const int *species_dev, const double *positions_dev) {
   fm_context ctx = s->ctx;
   hipStream_t st = ctx->stream;
   int n = s->n;
   Pool *pool = &ctx->pool;
-  // Global bin offsets of the structures of the batch.
-  std::vector<int> bin_off(s->n_struct + 1, 0);
-  for (int k = 0; k < s->n_struct; k++) {
-    const CellArgs &ca = s->cellargs[k];
-    long long nb = (long long)ca.nb[0] * ca.nb[1] * ca.nb[2];
-    FM_CHECK(bin_off[k] + nb < (1LL << 30), FM_ERR_CAPACITY, "cell list too large");
-    bin_off[k + 1] = bin_off[k] + (int)nb;
-  }
-  int ncell = bin_off[s->n_struct];
-  s->d_bin_off.alloc(pool, bin_off.size() * sizeof(int));
-  FM_HIP(hipMemcpyAsync(s->d_bin_off.as<int>(), bin_off.data(), bin_off.size() * sizeof(int),
-                        hipMemcpyHostToDevice, st));
+  int ncell = s->n_bins;
   const CellArgs *cas = s->d_cellargs.as<CellArgs>();
   const int *ast = s->atom_struct.as<int>();
   const int *boffp = s->d_bin_off.as<int>();
@@ -477,21 +526,23 @@ void build_neighbors(fm_structure s) {
   s->count.alloc(pool, (size_t)n * sizeof(int));
   s->cumulative.alloc(pool, ((size_t)n + 1) * sizeof(int));
   DevBuf bin(pool, (size_t)n * sizeof(int));
-  DevBuf bcount(pool, (size_t)ncell * sizeof(int));
+  DevBuf zeros(pool, sizeof(SetupWords) + (size_t)ncell * sizeof(int));
   DevBuf bstart(pool, ((size_t)ncell + 1) * sizeof(int));
-  DevBuf cursor(pool, (size_t)ncell * sizeof(int));
   DevBuf order(pool, (size_t)n * sizeof(int));
-  DevBuf maxc(pool, sizeof(int));
+  SetupWords *words = zeros.as<SetupWords>();
+  int *bcount = reinterpret_cast<int *>(words + 1), *maxc = &words->max_count;
+  int *hw = ctx->pinned_dev;
   int tpb = 256, nblk = (n + tpb - 1) / tpb;
-  hipLaunchKernelGGL(k_wrap, dim3(nblk), dim3(tpb), 0, st, n, s->positions.as<double>(), cas, ast,
-                     boffp, s->wrapped.as<double>(), bin.as<int>());
-  FM_HIP(hipMemsetAsync(bcount.as<int>(), 0, (size_t)ncell * sizeof(int), st));
-  FM_HIP(hipMemsetAsync(cursor.as<int>(), 0, (size_t)ncell * sizeof(int), st));
-  FM_HIP(hipMemsetAsync(maxc.as<int>(), 0, sizeof(int), st));
-  hipLaunchKernelGGL(k_bin_count, dim3(nblk), dim3(tpb), 0, st, n, bin.as<int>(), bcount.as<int>());
-  scan_exclusive(ctx, bcount.as<int>(), bstart.as<int>(), ncell, false);
+  FM_HIP(hipMemsetAsync(zeros.as<void>(), 0, sizeof(SetupWords) + (size_t)ncell * sizeof(int), st));
+  hipLaunchKernelGGL(k_setup, dim3(nblk), dim3(tpb), 0, st, n, s->n_struct,
+                     positions_dev ? positions_dev : s->positions.as<double>(),
+                     species_dev ? species_dev : s->species.as<int>(), s->positions.as<double>(),
+                     s->species.as<int>(), cas, s->d_atom_off.as<int>(), boffp,
+                     s->atom_struct.as<int>(), s->wrapped.as<double>(), bin.as<int>(), bcount,
+                     words);
+  scan_exclusive(ctx, bcount, bstart.as<int>(), ncell);
   hipLaunchKernelGGL(k_bin_fill, dim3(nblk), dim3(tpb), 0, st, n, bin.as<int>(), bstart.as<int>(),
-                     cursor.as<int>(), order.as<int>());
+                     bcount, order.as<int>(), words, hw);
   int wblk = (n + kNbrWaves - 1) / kNbrWaves;
   // One pass over the candidates that also parks each atom's sorted keys
   // (kNbrCapSmall per atom, while that area stays within 16 GB); else a
@@ -503,24 +554,19 @@ void build_neighbors(fm_structure s) {
     hipLaunchKernelGGL((k_neighbors<true, kNbrCapSmall>), dim3(wblk), dim3(64 * kNbrWaves), 0, st,
                        n, s->wrapped.as<double>(), bin.as<int>(), bstart.as<int>(),
                        order.as<int>(), s->species.as<int>(), cas, ast, boffp,
-                       s->count.as<int>(), nullptr, nullptr, nullptr, nullptr, maxc.as<int>(),
+                       s->count.as<int>(), nullptr, nullptr, nullptr, nullptr, maxc,
                        slots.as<long long>());
   } else {
     hipLaunchKernelGGL(k_neighbors<false>, dim3(wblk), dim3(64 * kNbrWaves), 0, st, n,
                        s->wrapped.as<double>(), bin.as<int>(), bstart.as<int>(), order.as<int>(),
                        s->species.as<int>(), cas, ast, boffp, s->count.as<int>(), nullptr,
-                       nullptr, nullptr, nullptr, maxc.as<int>());
+                       nullptr, nullptr, nullptr, maxc);
   }
   FM_HIP(hipGetLastError());
-  scan_exclusive(ctx, s->count.as<int>(), s->cumulative.as<int>(), n, false);
-  // Total and largest count in pinned words [2, 4), one synchronisation
-  // (which also completes any readback queued before, e.g. words [0, 2)).
-  int *hw = ctx->pinned;
-  FM_HIP(hipMemcpyAsync(hw + 2, s->cumulative.as<int>() + n, sizeof(int), hipMemcpyDeviceToHost,
-                        st));
-  FM_HIP(hipMemcpyAsync(hw + 3, maxc.as<int>(), sizeof(int), hipMemcpyDeviceToHost, st));
+  // Total and largest count to pinned words 2 and 3, then one synchronisation.
+  scan_exclusive(ctx, s->count.as<int>(), s->cumulative.as<int>(), n, hw + 2, maxc);
   FM_HIP(hipStreamSynchronize(st));
-  int total = hw[2], max_count = hw[3];
+  int total = ctx->pinned[2], max_count = ctx->pinned[3];
   s->n_nb = total;
   s->sidx.alloc(pool, std::max<size_t>(1, (size_t)total * sizeof(int)));
   s->nspecies.alloc(pool, std::max<size_t>(1, (size_t)total * sizeof(int)));
@@ -563,7 +609,8 @@ void build_neighbors(fm_structure s) {
 // ballot gives each kept entry its place.
 __global__ __launch_bounds__(256) void k_bond_count(int n, const int *species, const int *cum,
                                                     const int *nspec, const double *rel,
-                                                    const double *cutoffs, int nos, int *bcount) {
+                                                    const double *cutoffs, int nos, int *bcount,
+                                                    int *in_count) {
   int lane = threadIdx.x & 63;
   int i = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (i >= n) return;
@@ -573,16 +620,21 @@ __global__ __launch_bounds__(256) void k_bond_count(int n, const int *species, c
     bool keep = q < cum[i + 1] && rel[4 * (size_t)q] <= cutoffs[si * nos + nspec[q]];
     c += __popcll(__ballot(keep));
   }
-  if (lane == 0) bcount[i] = c;
+  if (lane == 0) {
+    bcount[i] = c;
+    in_count[i] = 0;
+  }
 }
 
 __global__ __launch_bounds__(256) void k_bond_fill(int n, const int *species, const int *cum,
                                                    const int *nspec, const double *rel,
                                                    const double *cutoffs, int nos,
                                                    const int *boff, const int *sidx, int *bond_q,
-                                                   int *in_count) {
+                                                   int *in_count, const int *bonds_by_type,
+                                                   int *host_by_type) {
   int lane = threadIdx.x & 63;
   int i = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (blockIdx.x == 0 && threadIdx.x < nos) host_by_type[threadIdx.x] = bonds_by_type[threadIdx.x];
   if (i >= n) return;
   int si = species[i], o = boff[i];
   unsigned long long below = (1ull << lane) - 1ull;
@@ -598,13 +650,15 @@ __global__ __launch_bounds__(256) void k_bond_fill(int n, const int *species, co
   }
 }
 
-__global__ void k_in_fill(int nbonds, const int *bond_q, const int *sidx, const int *in_off,
-                          int *cursor, int *in_bond) {
+// Incoming bonds of each atom in any order, counting in_count down (the launch
+// covers all neighbours; the bonds are the first bond_off[n] of them).
+__global__ __launch_bounds__(256) void k_in_fill(int n, const int *bond_off, const int *bond_q,
+                                                 const int *sidx, const int *in_off,
+                                                 int *in_count, int *in_bond) {
   int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nbonds) return;
+  if (b >= bond_off[n]) return;
   int j = sidx[bond_q[b]];
-  int slot = atomicAdd(&cursor[j], 1);
-  in_bond[in_off[j] + slot] = b;
+  in_bond[in_off[j] + atomicAdd(&in_count[j], -1) - 1] = b;
 }
 
 // Incoming bonds of atom j in ascending bond order (so the force gather sums
@@ -625,85 +679,184 @@ __global__ __launch_bounds__(256) void k_in_rank(int n, const int *in_off, const
   }
 }
 
-__global__ void k_species_flag(int n, const int *species, int t, int *flag) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) flag[i] = species[i] == t ? 1 : 0;
+// Species-sorted rows (b2.cpp:148-176; atom order kept within a species).
+constexpr int kRowBlock = 1024;
+
+// Atoms of each species per block of 1,024, species-major.
+__global__ __launch_bounds__(kRowBlock) void k_species_count(int n, const int *species, int nos,
+                                                             int *hist) {
+  extern __shared__ int cnt[];
+  for (int t = threadIdx.x; t < nos; t += kRowBlock) cnt[t] = 0;
+  __syncthreads();
+  int i = blockIdx.x * kRowBlock + threadIdx.x;
+  int sp = i < n ? species[i] : -1;
+  for (int t = 0; t < nos; t++) {
+    unsigned long long m = __ballot(sp == t);
+    if ((threadIdx.x & 63) == 0 && m) atomicAdd(&cnt[t], (int)__popcll(m));
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < nos; t += kRowBlock) hist[(size_t)t * gridDim.x + blockIdx.x] = cnt[t];
 }
 
-__global__ void k_species_rows(int n, const int *species, int t, const int *rank, int off,
-                               int *row_of_atom, int *atom_of_row) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && species[i] == t) {
-    int r = off + rank[i];
+// Cutoffs passed by value for up to four species.
+struct CutoffArgs {
+  double c[16];
+};
+
+// Row of each atom: the rows of the lower species and of the blocks before
+// (`off`, the scan of the counts above; with one block from the block itself),
+// then the atom's rank in its block. Block 0 also writes the species' atom
+// counts to the host, the slice-row shift of each species (its rows start a
+// tile of `tile` slice rows), zeros for the bond counts by species, and the
+// cutoffs when they come by value.
+__global__ __launch_bounds__(kRowBlock) void k_species_rows(int n, const int *species, int nos,
+                                                            const int *off, int *row_of_atom,
+                                                            int *atom_of_row, int *host_by_type,
+                                                            int tile, int *shift,
+                                                            int *bonds_by_type, CutoffArgs cut,
+                                                            int n_cut, double *cutoffs) {
+  extern __shared__ int wc[];  // [16 waves][nos], then the species' first rows [nos + 1]
+  int *first = wc + 16 * nos;
+  int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nb = gridDim.x;
+  int i = blockIdx.x * kRowBlock + threadIdx.x;
+  int sp = i < n ? species[i] : -1;
+  int rank = 0;
+  for (int t = 0; t < nos; t++) {
+    unsigned long long m = __ballot(sp == t);
+    if (sp == t) rank = __popcll(m & ((1ull << lane) - 1ull));
+    if (lane == 0) wc[w * nos + t] = __popcll(m);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int o = 0;
+    for (int t = 0; t <= nos; t++) {
+      first[t] = nb > 1 ? off[(size_t)t * nb] : o;  // off[nos nb] = n
+      if (nb == 1 && t < nos)
+        for (int v = 0; v < 16; v++) o += wc[v * nos + t];
+    }
+  }
+  __syncthreads();
+  if (sp >= 0) {
+    int r = (nb > 1 ? off[(size_t)sp * nb + blockIdx.x] : first[sp]) + rank;
+    for (int v = 0; v < w; v++) r += wc[v * nos + sp];
     row_of_atom[i] = r;
     atom_of_row[r] = i;
   }
+  if (blockIdx.x == 0) {
+    for (int t = threadIdx.x; t < nos; t += kRowBlock) {
+      host_by_type[t] = first[t + 1] - first[t];
+      bonds_by_type[t] = 0;
+    }
+    if (threadIdx.x < n_cut) cutoffs[threadIdx.x] = cut.c[threadIdx.x];
+    if (threadIdx.x == 0) {
+      int rows = 0;
+      for (int t = 0; t < nos; t++) {
+        shift[t] = rows - first[t];
+        rows += (first[t + 1] - first[t] + tile - 1) / tile * tile;
+      }
+    }
+  }
 }
+
+// Bonds by the species of their centre (b2.cpp:106-112), summed per block.
+__global__ __launch_bounds__(256) void k_bonds_by_type(int n, const int *species,
+                                                       const int *bcount, int nos,
+                                                       int *bonds_by_type) {
+  extern __shared__ int cnt[];
+  for (int t = threadIdx.x; t < nos; t += blockDim.x) cnt[t] = 0;
+  __syncthreads();
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    atomicAdd(&cnt[species[i]], bcount[i]);
+  __syncthreads();
+  for (int t = threadIdx.x; t < nos; t += blockDim.x)
+    if (cnt[t]) atomicAdd(&bonds_by_type[t], cnt[t]);
+}
+
+// Pinned words of a bond build: the bond total, then atoms and bonds by species.
+constexpr int kWordBonds = 4, kWordTypes = 8;
 
 void build_bonds(fm_structure s) {
   fm_context ctx = s->ctx;
   hipStream_t st = ctx->stream;
   Pool *pool = &ctx->pool;
-  int n = s->n, tpb = 256, nblk = (n + tpb - 1) / tpb;
-  FM_CHECK(s->nos + 1 <= fm_context_s::kPinnedWords, FM_ERR_INVALID, "too many species");
-  s->d_cutoffs.alloc(pool, s->cutoffs.size() * sizeof(double));
-  FM_HIP(hipMemcpyAsync(s->d_cutoffs.as<double>(), s->cutoffs.data(),
-                        s->cutoffs.size() * sizeof(double), hipMemcpyHostToDevice, st));
-  // Species-sorted rows: one scan of species flags per species.
+  int n = s->n, nos = s->nos, tpb = 256;
+  FM_CHECK(nos < 64, FM_ERR_INVALID, "too many species");
+  int *hw = ctx->pinned_dev;
+  int *host_types = hw + kWordTypes, *host_bonds = hw + kWordTypes + nos;
+  int nc = nos * nos;
+  s->d_cutoffs.alloc(pool, nc * sizeof(double));
+  CutoffArgs cut{};
+  bool by_value = nc <= 16;
+  if (by_value)
+    std::copy(s->cutoffs.begin(), s->cutoffs.end(), cut.c);
+  else
+    FM_HIP(hipMemcpyAsync(s->d_cutoffs.as<double>(), s->cutoffs.data(), nc * sizeof(double),
+                          hipMemcpyHostToDevice, st));
+  // Species-sorted rows: one launch up to 1,024 atoms, else three.
   s->row_of_atom.alloc(pool, (size_t)n * sizeof(int));
   s->atom_of_row.alloc(pool, (size_t)n * sizeof(int));
-  DevBuf flag(pool, (size_t)n * sizeof(int));
-  DevBuf rank(pool, (size_t)s->nos * ((size_t)n + 1) * sizeof(int));
-  for (int t = 0; t < s->nos; t++) {
-    hipLaunchKernelGGL(k_species_flag, dim3(nblk), dim3(tpb), 0, st, n, s->species.as<int>(), t,
-                       flag.as<int>());
-    scan_exclusive(ctx, flag.as<int>(), rank.as<int>() + (size_t)t * (n + 1), n, false);
+  s->q_shift.alloc(pool, nos * sizeof(int));
+  DevBuf by_type(pool, nos * sizeof(int));
+  int nb = (n + kRowBlock - 1) / kRowBlock;
+  DevBuf hist, off;
+  if (nb > 1) {
+    hist.alloc(pool, (size_t)nos * nb * sizeof(int));
+    off.alloc(pool, ((size_t)nos * nb + 1) * sizeof(int));
+    hipLaunchKernelGGL(k_species_count, dim3(nb), dim3(kRowBlock), nos * sizeof(int), st, n,
+                       s->species.as<int>(), nos, hist.as<int>());
+    scan_exclusive(ctx, hist.as<int>(), off.as<int>(), nos * nb);
   }
-  DevBuf bcount(pool, (size_t)n * sizeof(int));
+  hipLaunchKernelGGL(k_species_rows, dim3(nb), dim3(kRowBlock), (17 * nos + 1) * sizeof(int), st,
+                     n, s->species.as<int>(), nos, off.as<int>(), s->row_of_atom.as<int>(),
+                     s->atom_of_row.as<int>(), host_types, kI8TileA, s->q_shift.as<int>(),
+                     by_type.as<int>(), cut, by_value ? nc : 0, s->d_cutoffs.as<double>());
+  DevBuf bcount(pool, (size_t)n * sizeof(int)), in_count(pool, (size_t)n * sizeof(int));
   s->bond_off.alloc(pool, ((size_t)n + 1) * sizeof(int));
   hipLaunchKernelGGL(k_bond_count, dim3((n + 3) / 4), dim3(256), 0, st, n, s->species.as<int>(),
                      s->cumulative.as<int>(), s->nspecies.as<int>(), s->rel.as<double>(),
-                     s->d_cutoffs.as<double>(), s->nos, bcount.as<int>());
-  scan_exclusive(ctx, bcount.as<int>(), s->bond_off.as<int>(), n, false);
-  // Bond total and per-species atom counts: one readback, one synchronisation.
-  int *hw = ctx->pinned;
-  FM_HIP(hipMemcpyAsync(hw, s->bond_off.as<int>() + n, sizeof(int), hipMemcpyDeviceToHost, st));
-  for (int t = 0; t < s->nos; t++)
-    FM_HIP(hipMemcpyAsync(hw + 1 + t, rank.as<int>() + (size_t)t * (n + 1) + n, sizeof(int),
-                          hipMemcpyDeviceToHost, st));
-  FM_HIP(hipStreamSynchronize(st));
-  int nbonds = hw[0];
-  s->n_bonds = nbonds;
-  s->n_by_type.assign(s->nos, 0);
-  s->type_off.assign(s->nos + 1, 0);
-  for (int t = 0; t < s->nos; t++) {
-    s->n_by_type[t] = hw[1 + t];
-    s->type_off[t + 1] = s->type_off[t] + hw[1 + t];
-    hipLaunchKernelGGL(k_species_rows, dim3(nblk), dim3(tpb), 0, st, n, s->species.as<int>(), t,
-                       rank.as<int>() + (size_t)t * (n + 1), s->type_off[t],
-                       s->row_of_atom.as<int>(), s->atom_of_row.as<int>());
-  }
-  s->bond_q.alloc(pool, (size_t)nbonds * sizeof(int));
-  DevBuf in_count(pool, (size_t)n * sizeof(int));
-  FM_HIP(hipMemsetAsync(in_count.as<int>(), 0, (size_t)n * sizeof(int), st));
+                     s->d_cutoffs.as<double>(), nos, bcount.as<int>(), in_count.as<int>());
+  hipLaunchKernelGGL(k_bonds_by_type, dim3(std::min(64, (n + 255) / 256)), dim3(256),
+                     nos * sizeof(int), st, n, s->species.as<int>(), bcount.as<int>(), nos,
+                     by_type.as<int>());
+  scan_exclusive(ctx, bcount.as<int>(), s->bond_off.as<int>(), n, hw + kWordBonds);
+  // Bond arrays hold every neighbour, so nothing waits for the bond total.
+  size_t cap = std::max<size_t>(1, (size_t)s->n_nb);
+  s->bond_q.alloc(pool, cap * sizeof(int));
   hipLaunchKernelGGL(k_bond_fill, dim3((n + 3) / 4), dim3(256), 0, st, n, s->species.as<int>(),
                      s->cumulative.as<int>(), s->nspecies.as<int>(), s->rel.as<double>(),
-                     s->d_cutoffs.as<double>(), s->nos, s->bond_off.as<int>(), s->sidx.as<int>(),
-                     s->bond_q.as<int>(), in_count.as<int>());
+                     s->d_cutoffs.as<double>(), nos, s->bond_off.as<int>(), s->sidx.as<int>(),
+                     s->bond_q.as<int>(), in_count.as<int>(), by_type.as<int>(), host_bonds);
+  FM_HIP(hipEventRecord(ctx->ev_sizes, st));
   s->in_off.alloc(pool, ((size_t)n + 1) * sizeof(int));
-  scan_exclusive(ctx, in_count.as<int>(), s->in_off.as<int>(), n, false);
-  s->in_bond.alloc(pool, (size_t)nbonds * sizeof(int));
-  DevBuf cursor(pool, (size_t)n * sizeof(int));
-  DevBuf unordered(pool, (size_t)nbonds * sizeof(int));
-  FM_HIP(hipMemsetAsync(cursor.as<int>(), 0, (size_t)n * sizeof(int), st));
-  if (nbonds > 0) {
-    hipLaunchKernelGGL(k_in_fill, dim3((nbonds + tpb - 1) / tpb), dim3(tpb), 0, st, nbonds,
-                       s->bond_q.as<int>(), s->sidx.as<int>(), s->in_off.as<int>(),
-                       cursor.as<int>(), unordered.as<int>());
+  scan_exclusive(ctx, in_count.as<int>(), s->in_off.as<int>(), n);
+  s->in_bond.alloc(pool, cap * sizeof(int));
+  DevBuf unordered(pool, cap * sizeof(int));
+  if (s->n_nb > 0) {
+    hipLaunchKernelGGL(k_in_fill, dim3((unsigned)((s->n_nb + tpb - 1) / tpb)), dim3(tpb), 0, st, n,
+                       s->bond_off.as<int>(), s->bond_q.as<int>(), s->sidx.as<int>(),
+                       s->in_off.as<int>(), in_count.as<int>(), unordered.as<int>());
     hipLaunchKernelGGL(k_in_rank, dim3((n + 3) / 4), dim3(256), 0, st, n, s->in_off.as<int>(),
                        unordered.as<int>(), s->in_bond.as<int>());
   }
   FM_HIP(hipGetLastError());
+}
+
+void bonds_ready(fm_structure s) {
+  fm_context ctx = s->ctx;
+  FM_HIP(hipEventSynchronize(ctx->ev_sizes));
+  const int *hw = ctx->pinned;
+  int nos = s->nos;
+  s->n_bonds = hw[kWordBonds];
+  s->n_by_type.assign(hw + kWordTypes, hw + kWordTypes + nos);
+  s->nb_by_type.assign(hw + kWordTypes + nos, hw + kWordTypes + 2 * nos);
+  s->type_off.assign(nos + 1, 0);
+  s->q_tile_row.assign(nos, 0);
+  long long rows = 0;
+  for (int t = 0; t < nos; t++) {
+    s->type_off[t + 1] = s->type_off[t] + s->n_by_type[t];
+    s->q_tile_row[t] = rows;
+    rows += (s->n_by_type[t] + kI8TileA - 1) / kI8TileA * kI8TileA;
+  }
 }
 
 }  // namespace fm

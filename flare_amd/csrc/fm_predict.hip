@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <type_traits>
 #include <vector>
 
@@ -206,7 +207,7 @@ void build_var_pos(fm_structure s) {
   FM_HIP(hipMemsetAsync(cnt.as<int>(), 0, (size_t)m * sizeof(int), st));
   hipLaunchKernelGGL(k_struct_species_count, dim3((n + 255) / 256), dim3(256), 0, st, n,
                      s->species.as<int>(), s->atom_struct.as<int>(), ns, s->nos, cnt.as<int>());
-  scan_exclusive(ctx, cnt.as<int>(), ex.as<int>(), m, false);
+  scan_exclusive(ctx, cnt.as<int>(), ex.as<int>(), m);
   s->var_pos.alloc(&ctx->pool, (size_t)n * sizeof(int));
   hipLaunchKernelGGL(k_var_pos, dim3((n + 255) / 256), dim3(256), 0, st, n,
                      s->atom_of_row.as<int>(), s->species.as<int>(), s->atom_struct.as<int>(),
@@ -216,41 +217,62 @@ void build_var_pos(fm_structure s) {
 }
 
 // Results to the caller's host buffers (any may be null); returns after the
-// copies have finished.
+// copies have finished. Results of up to kStageOut bytes go through the
+// context's pinned memory (a copy to pageable memory waits for itself, 15 us
+// each).
+constexpr size_t kStageOut = 256 << 10;
+
 static void read_outputs(fm_structure s, const double *o, size_t n_out, const double *var_row,
                          const double *E_row, double *mean_efs, double *local_var,
                          double *local_energy) {
   hipStream_t st = s->ctx->stream;
   Pool *pool = &s->ctx->pool;
-  int n = s->n;
+  size_t n = s->n;
   DevBuf vperm, eperm;
-  if (mean_efs)
-    FM_HIP(hipMemcpyAsync(mean_efs, o, (size_t)n_out * sizeof(double), hipMemcpyDeviceToHost, st));
+  struct Part {
+    double *dst;
+    const double *src;
+    size_t count;
+  } parts[3] = {{mean_efs, o, n_out}, {nullptr, nullptr, 0}, {nullptr, nullptr, 0}};
   if (local_var && var_row && n > 0) {
     // Species-sorted rows of the batch to each structure's species-sorted
     // order (compute_cluster_uncertainties order).
     const double *src = var_row;
     if (s->n_struct > 1) {
-      vperm.alloc(pool, (size_t)n * sizeof(double));
-      hipLaunchKernelGGL(k_scatter_rows, dim3((n + 255) / 256), dim3(256), 0, st, n,
+      vperm.alloc(pool, n * sizeof(double));
+      hipLaunchKernelGGL(k_scatter_rows, dim3((n + 255) / 256), dim3(256), 0, st, (int)n,
                          s->var_pos.as<int>(), var_row, vperm.as<double>());
       src = vperm.as<double>();
     }
-    FM_HIP(hipMemcpyAsync(local_var, src, (size_t)n * sizeof(double), hipMemcpyDeviceToHost,
-                          st));
+    parts[1] = {local_var, src, n};
   }
   if (local_energy && n > 0) {
     // E_row is in species-sorted order; local energies are in atom order.
-    eperm.alloc(pool, (size_t)n * sizeof(double));
-    hipLaunchKernelGGL(k_scatter_rows, dim3((n + 255) / 256), dim3(256), 0, st, n,
+    eperm.alloc(pool, n * sizeof(double));
+    hipLaunchKernelGGL(k_scatter_rows, dim3((n + 255) / 256), dim3(256), 0, st, (int)n,
                        s->atom_of_row.as<int>(), E_row, eperm.as<double>());
-    FM_HIP(hipMemcpyAsync(local_energy, eperm.as<double>(), (size_t)n * sizeof(double),
-                          hipMemcpyDeviceToHost, st));
+    parts[2] = {local_energy, eperm.as<double>(), n};
   }
   FM_HIP(hipGetLastError());
+  size_t total = 0;
+  for (const Part &p : parts)
+    if (p.dst) total += p.count * sizeof(double);
+  char *stage = total <= kStageOut ? s->ctx->stage(total) : nullptr;
+  char *at = stage;
+  for (const Part &p : parts) {
+    if (!p.dst) continue;
+    FM_HIP(hipMemcpyAsync(stage ? (void *)at : (void *)p.dst, p.src, p.count * sizeof(double),
+                          hipMemcpyDeviceToHost, st));
+    if (stage) at += p.count * sizeof(double);
+  }
   FM_HIP(hipStreamSynchronize(st));
+  at = stage;
+  for (const Part &p : parts) {
+    if (!p.dst || !stage) continue;
+    std::memcpy(p.dst, at, p.count * sizeof(double));
+    at += p.count * sizeof(double);
+  }
 }
-
 
 // Rows per tile of one species in the chosen form: at most T and, when T
 // allows, a whole number of rounds of the kernel contraction's 128 x 64
@@ -462,13 +484,12 @@ static void predict_tiled(fm_model m, fm_structure s, int flags, int form, doubl
   ctx->mark_end(ST_SGEMM);
   ctx->mark_begin(ST_ADJ);
   double *o = out.as<double>();
-  FM_HIP(hipMemsetAsync(o, 0, (size_t)n_out * sizeof(double), st));
+  if (n == 0) FM_HIP(hipMemsetAsync(o, 0, (size_t)n_out * sizeof(double), st));
   if (n > 0) gather_forces(s, f64, fbond, vir, E_row, o);
   FM_HIP(hipGetLastError());
   ctx->mark_end(ST_ADJ);
   read_outputs(s, o, n_out, want_var ? var_row.as<double>() : nullptr, E_row.as<double>(),
                mean_efs, local_var, local_energy);
-  FM_HIP(hipStreamSynchronize(st));
 }
 
 void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
@@ -699,7 +720,7 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
   DevBuf fbond(pool, std::max<size_t>(1, (size_t)3 * s->n_bonds * esz));
   DevBuf vir(pool, std::max<size_t>(1, (size_t)6 * n * sizeof(double)));
   double *o = out.as<double>();
-  FM_HIP(hipMemsetAsync(o, 0, (size_t)n_out * sizeof(double), st));
+  if (n == 0) FM_HIP(hipMemsetAsync(o, 0, (size_t)n_out * sizeof(double), st));
   if (n > 0) {
     // FP64: G . B from the local energies (G . B = p |B| E, exact to
     // rounding). Split form: from the G and B rows, since G carries the
@@ -719,7 +740,6 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
 
   read_outputs(s, o, n_out, want_var ? var_row.as<double>() : nullptr, E_row.as<double>(),
                mean_efs, local_var, local_energy);
-  FM_HIP(hipStreamSynchronize(st));
 }
 
 }  // namespace fm
