@@ -2,8 +2,8 @@
 // and its adjoint (the arithmetic of lammps_descriptor.cpp:250-315 and
 // pair_flare.cpp:141-174, driven by dE/dB from the kernel contraction).
 //
-// Descriptor (k_b2): an atom's bonds are taken in chunks of 32; lanes write
-// the radial values g_n and all harmonics Y_lm of the chunk into LDS tables
+// Descriptor (k_b2): an atom's bonds are taken in chunks of 32 or 64; lanes
+// write the radial values g_n and all harmonics Y_lm of the chunk into LDS tables
 // grouped by neighbour species, and the density coefficients accumulate as
 // c_t += G_t^T Y_t on the matrix cores (16x16x4, FP32 or FP64) over that
 // species' rows only. The power spectrum B_l = C_l C_l^T is a second MFMA
@@ -28,8 +28,6 @@
 namespace fm {
 
 constexpr int kAtomsPerBlock = 4;
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 struct B2Args {
   int n, nos, N, lmax, H, nrad, nd, cutkind;
@@ -118,19 +116,25 @@ __device__ __forceinline__ void ylm_step(YlmState<T, kGrad> &y, int mm, int l, T
   }
 }
 
-template <typename T, bool kGrad, int LC = -1, typename F>
-__device__ __forceinline__ void ylm_sweep(int L, T ux, T uy, T uz, F &&f) {
+// `mine(m)` (wave-uniform) tells which m this wave takes.
+struct AllM {
+  __device__ __forceinline__ bool operator()(int) const { return true; }
+};
+template <typename T, bool kGrad, int LC = -1, typename F, typename Mine = AllM>
+__device__ __forceinline__ void ylm_sweep(int L, T ux, T uy, T uz, F &&f, Mine mine = Mine()) {
   YlmState<T, kGrad> y;
   if constexpr (LC >= 0) {
 #pragma unroll
     for (int mm = 0; mm <= LC; mm++) {
       ylm_m_begin<T, kGrad>(y, mm, ux, uy);
+      if (!mine(mm)) continue;
 #pragma unroll
       for (int l = mm; l <= LC; l++) ylm_step<T, kGrad>(y, mm, l, uz, f);
     }
   } else {
     for (int mm = 0; mm <= L; mm++) {
       ylm_m_begin<T, kGrad>(y, mm, ux, uy);
+      if (!mine(mm)) continue;
       for (int l = mm; l <= L; l++) ylm_step<T, kGrad>(y, mm, l, uz, f);
     }
   }
@@ -163,35 +167,53 @@ __device__ __forceinline__ int mfma_row(int lane, int q) {
   return sizeof(T) == 8 ? (lane >> 4) + 4 * q : 4 * (lane >> 4) + q;
 }
 
-// Bonds per table chunk of the descriptor kernel, CH (a template parameter):
-// lanes [0, CH) write the tables, so a 32-bond chunk leaves half the wave
-// idle in the harmonic sweep and a 64-bond chunk doubles the tables' LDS
-// (fewer atoms resident per CU). launch_b2 picks 64 where that costs at
-// most a third more LDS per atom, else 32.
+// 16-byte vectors in global memory at the alignment of their elements.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+
+__host__ __device__ inline int pad2(int n) { return (n + 1) & ~1; }
 
 // Workspace (elements of T) of one atom of the descriptor kernel: c, then the
-// bond tables of one chunk (Y ch x H, g ch x N).
-__host__ __device__ inline size_t b2_work(int nc, int H, int N, int ch) {
-  return (size_t)nc + (size_t)ch * ((size_t)H + (size_t)N);
+// bond tables of one chunk of ch bonds (Y ch x H, g ch x N) and later the row
+// of nd values (0 without B2) over them; even, so that every atom's row is
+// 16-byte aligned.
+__host__ __device__ inline size_t b2_work(int nc, int H, int N, int ch, int nd) {
+  size_t tab = (size_t)ch * ((size_t)H + (size_t)N), row = (size_t)nd;
+  return (size_t)pad2(nc) + ((tab > row ? tab : row) + 1) / 2 * 2;
+}
+
+// Ordering of LDS accesses among the W waves of an atom.
+template <int W>
+__device__ __forceinline__ void atom_sync() {
+  if constexpr (W > 1) {
+    __syncthreads();
+  } else {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
 }
 
 // c[(t N + n) H + lm] of atom i for all neighbour species t into LDS
-// (b2.cpp:367-395). For each chunk of up to CH bonds, lane k takes
-// bond k and writes its radial basis g_n and every Y_lm to LDS tables, the
+// (b2.cpp:367-395). For each chunk of up to ch bonds, lane k takes
+// bond k and writes its radial basis g_n and its Y_lm to LDS tables, the
 // rows grouped by neighbour species (list order kept within a species); then,
 // per species t and 16 harmonics, c_t += G_t^T Y_t on the matrix cores over
-// that species' rows only (A = g_n of the bonds, B = their Y_lm).
-template <typename T, int LC, int CH>
-__device__ void accumulate_c(const B2Args &a, int i, int lane, T *c, T *tab) {
+// that species' rows only (A = g_n of the bonds, B = their Y_lm). Of W waves
+// per atom, wave w takes the harmonics with m mod 2 W in {w, 2 W - 1 - w}
+// (wave 0 the radial basis too) and every W-th (t, 16 harmonics) tile; each value is the
+// same whoever computes it.
+template <typename T, int LC, int W>
+__device__ void accumulate_c(const B2Args &a, int i, int lane, int w, int ch, T *c, T *tab) {
   int si = a.species[i];
   int b0 = a.bond_off[i], b1 = a.bond_off[i + 1];
   int nc = a.nrad * a.H, H = a.H, N = a.N;
-  T *Yt = tab, *gt = tab + CH * (size_t)H;
-  for (int k = lane; k < nc; k += 64) c[k] = 0;
+  T *Yt = tab, *gt = tab + ch * (size_t)H;
+  for (int k = 64 * w + lane; k < nc; k += 64 * W) c[k] = 0;
   int r16 = lane & 15, k4 = lane >> 4;
   unsigned long long below = (1ull << lane) - 1ull;
-  for (int bb = b0; bb < b1; bb += CH) {
-    int nk = min(CH, b1 - bb);
+  for (int bb = b0; bb < b1; bb += ch) {
+    int nk = min(ch, b1 - bb);
     int q = 0, sj = -1;
     if (lane < nk) {
       q = a.bond_q[bb + lane];
@@ -205,29 +227,30 @@ __device__ void accumulate_c(const B2Args &a, int i, int lane, T *c, T *tab) {
       if (sj == t) pos = off + __popcll(m & below);
       off += __popcll(m);
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    atom_sync<W>();
     if (lane < nk) {
       const double *rp = a.rel + 4 * (size_t)q;
-      T g[kMaxN], dg[kMaxN];
-      radial_basis<T>((T)rp[0], (T)a.cutoffs[si * a.nos + sj], (T)a.r1, N, a.cutkind, g, dg);
+      if (w == 0) {
+        T g[kMaxN], dg[kMaxN];
+        radial_basis<T>((T)rp[0], (T)a.cutoffs[si * a.nos + sj], (T)a.r1, N, a.cutkind, g, dg);
 #pragma unroll
-      for (int nn = 0; nn < kMaxN; nn++)
-        if (nn < N) gt[pos * N + nn] = g[nn];
+        for (int nn = 0; nn < kMaxN; nn++)
+          if (nn < N) gt[pos * N + nn] = g[nn];
+      }
       T rinv = T(1) / (T)rp[0];
       T *yrow = Yt + (size_t)pos * H;
-      ylm_sweep<T, false, LC>(a.lmax, (T)rp[1] * rinv, (T)rp[2] * rinv, (T)rp[3] * rinv,
-                          [&](int lm, T Y, T, T, T) { yrow[lm] = Y; });
+      ylm_sweep<T, false, LC>(
+          a.lmax, (T)rp[1] * rinv, (T)rp[2] * rinv, (T)rp[3] * rinv,
+          [&](int lm, T Y, T, T, T) { yrow[lm] = Y; },
+          [&](int m) { m &= 2 * W - 1; return W == 1 || m == w || m == 2 * W - 1 - w; });
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    int r0 = 0;
+    atom_sync<W>();
+    int r0 = 0, tile = 0;
     for (int t = 0; t < a.nos; t++) {
       int r1 = r0 + __popcll(__ballot(sj == t));  // rows [r0, r1) are species t
       if (r1 > r0) {
         for (int ct = 0; ct < H; ct += 16) {
+          if (W > 1 && tile++ % W != w) continue;
           int lm = ct + r16;
           typename MfmaAcc<T>::type acc;
 #pragma unroll
@@ -238,15 +261,17 @@ __device__ void accumulate_c(const B2Args &a, int i, int lane, T *c, T *tab) {
           // Four k-steps per iteration: the loads (clamped in bounds, then
           // zeroed outside the species' rows) all issue before the MFMAs.
           int rc = r16 < N ? r16 : N - 1, lc = lm < H ? lm : H - 1;
+          int rn = r16 < N ? r1 : 0, rh = lm < H ? r1 : 0;
           for (int k0 = r0; k0 < r1; k0 += 16) {
             T av[4], bv[4];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
               int b = k0 + 4 * u + k4;
-              int bc = b < CH ? b : CH - 1;
-              T x = gt[bc * N + rc], y = Yt[bc * H + lc];
-              av[u] = (b < r1 && r16 < N) ? x : T(0);
-              bv[u] = (b < r1 && lm < H) ? y : T(0);
+              int bc = min(b, ch - 1);
+              T x = gt[bc * N + rc];
+              T y = Yt[bc * H + lc];
+              av[u] = b < rn ? x : T(0);
+              bv[u] = b < rh ? y : T(0);
             }
 #pragma unroll
             for (int u = 0; u < 4; u++)
@@ -262,26 +287,13 @@ __device__ void accumulate_c(const B2Args &a, int i, int lane, T *c, T *tab) {
       r0 = r1;
     }
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  atom_sync<W>();
 }
 
-// B2 (b2.cpp:209-231) per atom: B[k] = sum_m c[n1, lm] c[n2, lm], written at
-// the atom's species-sorted row, with |B| and B.B. The FP32 form also writes
-// each row as two BF16 pieces (b0 = bf16(B), b1 = bf16(B - b0)) with leading
-// dimension ldp and zero padding, the operand of the kernel contraction. The
-// coefficients c also go to HBM (Cg) for the adjoint.
-struct SplitOut {
-  __bf16 *p[2];
-};
-
-// The chosen form's outputs of the FP64 descriptor pass (k_b2 with MIXED
-// set; 1 stages the FP64 row in LDS and slices it after B_l, 2 slices each
-// value as it is formed and stages only the slices):
-// the B row and c in FP32 (for the adjoint) and the FP64 row as kI8Slices
-// int8 slices with a power-of-two scale (the kernel contraction's operand,
-// see k_slice_rows in fm_gemm.hip for the slicing).
+// The chosen form's outputs of the FP64 descriptor pass (k_b2 with MIXED): the
+// B row and c in FP32 (for the adjoint) and the FP64 row as kI8Slices int8
+// slices with a power-of-two scale (the kernel contraction's operand, see
+// k_slice_rows in fm_gemm.hip for the slicing).
 struct MixedOut {
   float *B, *C;
   int8_t *q;  // tiled slice layout, kI8TileA rows per tile
@@ -290,183 +302,268 @@ struct MixedOut {
   const int *shift;    // per species: slice row = species-sorted row + shift
 };
 
-template <typename T, int LC, int CH, int MIXED = 0>
-__global__ __launch_bounds__(64 * kAtomsPerBlock) void k_b2(B2Args a, T *B, double *norm,
-                                                              double *nn, SplitOut Bs, int ldp,
-                                                              T *Cg, int want_b2, int work,
-                                                              MixedOut mo) {
+// The slices of four consecutive values r (|r| < 1), packed four to a word.
+// Adding 1.5 2^(52 - s) rounds r to a multiple of 2^-s (to nearest, ties to
+// even) and leaves that multiple in the low bits of the sum; every difference
+// is exact.
+__device__ __forceinline__ void slice4(double (&r)[4], unsigned (&packed)[kI8Slices]) {
+#pragma unroll
+  for (int p = 0; p < kI8Slices; p++) {
+    const double magic = 6755399441055744.0 / (double)(1ll << (6 + 7 * p));
+    unsigned d[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      double u = r[j] + magic;
+      d[j] = (unsigned)__builtin_bit_cast(unsigned long long, u);
+      r[j] -= u - magic;
+    }
+    unsigned lo = __builtin_amdgcn_perm(d[1], d[0], 0x0c0c0400u);
+    unsigned hi = __builtin_amdgcn_perm(d[3], d[2], 0x0c0c0400u);
+    packed[p] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+  }
+}
+
+// B2 (b2.cpp:209-231) per atom: B[k] = sum_m c[n1, lm] c[n2, lm], written at
+// the atom's species-sorted row, with |B| and B.B; the coefficients c go to
+// HBM (Cg) for the adjoint. T = float is the bond pass of B3: c alone.
+//
+// What bounds it: vector instructions (five wave instructions in six cycles on
+// the 512-structure batch, where slicing each value on its own where the MFMA
+// tile leaves it was more than half of them). So the FP64 row is staged in LDS
+// (over the bond tables, no longer needed) and sliced four consecutive values
+// at a time, and the indices of a tile's values are formed once for all l. The
+// row is the largest part of an atom's LDS; where that leaves a CU few atoms,
+// W = 2 or 4 waves share one and split every phase. B.B keeps its order of
+// sums (the variances depend on its last bit): wave 0 takes it from the staged
+// row where the waves split the tiles. A row too long for LDS (stage = 0, one
+// wave, more than 32 radial functions) is written from the tiles.
+template <typename T, int LC, bool MIXED, int W>
+__global__ __launch_bounds__(256) void k_b2(B2Args a, T *B, double *norm, double *nn, T *Cg,
+                                            int want_b2, int work, int ch, int stage,
+                                            MixedOut mo) {
   extern __shared__ __align__(16) unsigned char smem[];
-  int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  int i = blockIdx.x * (blockDim.x >> 6) + w;
+  int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int w = wave % W, slot = wave / W;
+  int i = blockIdx.x * (blockDim.x / (64 * W)) + slot;  // W > 1: one atom per block
   if (i >= a.n) return;
+  constexpr int NT = 64 * W;
+  int tid = 64 * w + lane;  // thread of this atom
   int nc = a.nrad * a.H, H = a.H, nr = a.nrad;
-  T *c = reinterpret_cast<T *>(smem) + (size_t)w * work;  // work: elements per atom
-  T *tab = c + nc;
-  accumulate_c<T, LC, CH>(a, i, lane, c, tab);
+  T *c = reinterpret_cast<T *>(smem) + (size_t)slot * work;  // work: elements per atom
+  T *tab = c + pad2(nc);
+  accumulate_c<T, LC, W>(a, i, lane, w, ch, c, tab);
   if constexpr (MIXED) {
-    for (int k = lane; k < nc; k += 64) mo.C[(size_t)i * nc + k] = (float)c[k];
+    for (int k = tid; k < nc; k += NT) mo.C[(size_t)i * nc + k] = (float)c[k];
   } else {
-    for (int k = lane; k < nc; k += 64) Cg[(size_t)i * nc + k] = c[k];
+    for (int k = tid; k < nc; k += NT) Cg[(size_t)i * nc + k] = c[k];
   }
-  if (!want_b2) return;
-  // B_l = C_l C_l^T on the matrix cores (C_l[n][m] = c[n, l^2 + m]); the
-  // upper triangle n2 >= n1 belongs at p(n1, n2) (L + 1) + l of the row. FP64
-  // and MIXED 2's FP32 row store each element there directly (the L2 merges
-  // a row's scattered stores; staging would cost occupancy); FP32 and MIXED 1
-  // stage the row in LDS (over the bond tables, no longer needed) and write
-  // it with coalesced stores.
-  int L1 = a.lmax + 1;
-  int r16 = lane & 15, k4 = lane >> 4;
-  int row = a.row_of_atom[i];
-  T *Brow = B + (size_t)row * a.nd;
-  T *bst = tab;
-  T s2 = 0;
-  // MIXED 2: the row's power-of-two scale comes before the row itself: |B|'s
-  // largest element is a diagonal one, max_{n,l} sum_m c[n, lm]^2 (Cauchy-
-  // Schwarz within each l), so the values are sliced as they are formed and
-  // only the int8 slices (rows of Kq bytes, zero past nd) are staged in LDS
-  // over the bond tables; the FP32 row goes straight to HBM.
-  double q_inv = 0;
-  long long Kq = 0;
-  int8_t *qst = reinterpret_cast<int8_t *>(tab);
-  if constexpr (MIXED) Kq = mo.nk * kI8Pad;
-  if constexpr (MIXED == 2) {
-    double mx = 0;
-    for (int q = lane; q < nr * L1; q += 64) {
-      int n = q / L1, l = q % L1;
-      const T *cn = c + n * H + l * l;
-      double sq = 0;
-      for (int m = 0; m < 2 * l + 1; m++) sq += (double)cn[m] * (double)cn[m];
-      mx = fmax(mx, sq);
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
-    int E = 0;
-    if (mx > 0) frexp(mx, &E);  // mx = m 2^E, m in [0.5, 1)
-    q_inv = ldexp(1.0, -E);
-    if (lane == 0) mo.scale[row] = ldexp(1.0, E);
-    for (int q = a.nd + lane; q < Kq; q += 64)
-#pragma unroll
-      for (int p = 0; p < kI8Slices; p++) qst[p * Kq + q] = 0;
-  }
-  for (int l = 0; l <= a.lmax; l++) {
-    int nm = 2 * l + 1, lm0 = l * l;
-    for (int rt = 0; rt < nr; rt += 16) {
-      for (int cc = rt; cc < nr; cc += 16) {
-        typename MfmaAcc<T>::type acc = {};
-        int n1a = rt + r16, n2b = cc + r16;
-        const T *ca = c + (n1a < nr ? n1a : nr - 1) * H + lm0;
-        const T *cb = c + (n2b < nr ? n2b : nr - 1) * H + lm0;
-        for (int k0 = 0; k0 < nm; k0 += 8) {
-          T av[2], bv[2];
-#pragma unroll
-          for (int u = 0; u < 2; u++) {
-            int m = k0 + 4 * u + k4, mc = m < nm ? m : nm - 1;
-            T x = ca[mc], y = cb[mc];
-            av[u] = (n1a < nr && m < nm) ? x : T(0);
-            bv[u] = (n2b < nr && m < nm) ? y : T(0);
-          }
-#pragma unroll
-          for (int u = 0; u < 2; u++)
-            if (k0 + 4 * u < nm) acc = mfma_4(av[u], bv[u], acc);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          int n1 = rt + mfma_row<T>(lane, q), n2 = n2b;
-          if (n1 < nr && n2 < nr && n2 >= n1) {
-            int k = (n1 * nr - (n1 * (n1 - 1)) / 2 + (n2 - n1)) * L1 + l;
-            T v = acc[q];
-            if constexpr (MIXED == 2) {
-              mo.B[(size_t)row * a.nd + k] = (float)v;
-              double r = (double)v * q_inv;
-#pragma unroll
-              for (int p = 0; p < kI8Slices; p++) {
-                double sl = rint(ldexp(r, 6 + 7 * p));
-                r -= ldexp(sl, -(6 + 7 * p));
-                qst[p * Kq + k] = (int8_t)(int)sl;
-              }
-            } else if constexpr (sizeof(T) == 4 || MIXED == 1) {
-              bst[k] = v;
-            } else {
-              Brow[k] = v;
-            }
-            s2 += v * v;
-          }
-        }
+  if constexpr (sizeof(T) == 8) {
+    if (!want_b2) return;
+    // B_l = C_l C_l^T on the matrix cores (C_l[n][m] = c[n, l^2 + m]); the
+    // upper triangle n2 >= n1 belongs at p(n1, n2) (L + 1) + l of the row.
+    int L1 = a.lmax + 1;
+    int r16 = lane & 15, k4 = lane >> 4;
+    int row = a.row_of_atom[i];
+    T *bst = tab;
+    T s2 = 0;
+    // One 16 x 16 tile of B_l (operand elements past 2 l + 1, which are the
+    // next c values or lie in the tables, replaced by zero).
+    auto tile_of = [&](int l, int rt, int cc) {
+      int nm = 2 * l + 1, lm0 = l * l;
+      typename MfmaAcc<T>::type acc = {};
+      const T *ca = c + min(rt + r16, nr - 1) * H + lm0 + k4;
+      const T *cb = c + min(cc + r16, nr - 1) * H + lm0 + k4;
+#pragma unroll 2
+      for (int k0 = 0; k0 < nm; k0 += 4) {
+        T x = ca[k0], y = cb[k0];
+        bool in = k0 + k4 < nm;
+        acc = mfma_4(in ? x : T(0), in ? y : T(0), acc);
       }
-    }
-  }
-  if constexpr (sizeof(T) == 4) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    for (int k = lane; k < a.nd; k += 64) Brow[k] = bst[k];
-    // Pieces: 8 consecutive values per lane, one 16-byte store per piece
-    // (ldp is a multiple of 32; the padding past nd is zero).
-    for (int k8 = lane; k8 < ldp / 8; k8 += 64) {
-      bf16x8 h0, h1;
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        int k = 8 * k8 + e;
-        float r = k < a.nd ? (float)bst[k] : 0.0f;
-        __bf16 h = (__bf16)r;
-        h0[e] = h;
-        h1[e] = (__bf16)(r - (float)h);
-      }
-      *reinterpret_cast<bf16x8 *>(Bs.p[0] + (size_t)row * ldp + 8 * k8) = h0;
-      *reinterpret_cast<bf16x8 *>(Bs.p[1] + (size_t)row * ldp + 8 * k8) = h1;
-    }
-  }
-  if constexpr (MIXED) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    long long qrow = row + mo.shift[a.species[i]];
-    if constexpr (MIXED == 1) {
-      float *B32 = mo.B + (size_t)row * a.nd;
+      return acc;
+    };
+    // Place of this lane's value q of tile (rt, cc) for l = 0, or -1.
+    auto place = [&](int rt, int cc, int q) {
+      int n1 = rt + mfma_row<T>(lane, q), n2 = cc + r16;
+      return n1 < nr && n2 < nr && n2 >= n1 ? (n1 * nr - (n1 * (n1 - 1)) / 2 + (n2 - n1)) * L1
+                                            : -1;
+    };
+    // The row's power-of-two scale 2^E from its largest element, which is a
+    // diagonal one (Cauchy-Schwarz within each l); every wave finds it.
+    auto exponent = [&](auto diagonal) {
       double mx = 0;
-      for (int k = lane; k < a.nd; k += 64) {
-        B32[k] = (float)bst[k];
-        mx = fmax(mx, fabs((double)bst[k]));
+      for (int q = lane; q < nr * L1; q += 64) {
+        int n = q / L1;
+        mx = fmax(mx, diagonal(n, q - n * L1));
       }
 #pragma unroll
       for (int off = 32; off >= 1; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
       int E = 0;
       if (mx > 0) frexp(mx, &E);  // mx = m 2^E, m in [0.5, 1)
+      return E;
+    };
+    if (nr <= 32) {
+      // Up to three tiles: (0, 0), (0, 16), (16, 16), their places kept.
+      int at[3][4];
+#pragma unroll
+      for (int u = 0; u < 3; u++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) at[u][q] = place(u == 2 ? 16 : 0, u ? 16 : 0, q);
+      int nt = nr > 16 ? 3 : 1, tile = 0;
+      for (int l = 0; l <= a.lmax; l++) {
+#pragma unroll
+        for (int u = 0; u < 3; u++) {
+          if (u >= nt) continue;
+          if (W > 1 && tile++ % W != w) continue;
+          auto acc = tile_of(l, u == 2 ? 16 : 0, u ? 16 : 0);
+#pragma unroll
+          for (int q = 0; q < 4; q++)
+            if (at[u][q] >= 0) {
+              T v = acc[q];
+              bst[at[u][q] + l] = v;
+              if (W == 1) s2 += v * v;
+            }
+        }
+      }
+      if constexpr (W > 1) {
+        atom_sync<W>();
+        if (w == 0)
+          for (int l = 0; l <= a.lmax; l++)
+#pragma unroll
+            for (int u = 0; u < 3; u++) {
+              if (u >= nt) continue;
+#pragma unroll
+              for (int q = 0; q < 4; q++)
+                if (at[u][q] >= 0) {
+                  T v = bst[at[u][q] + l];
+                  s2 += v * v;
+                }
+            }
+      }
+    } else if (W == 1 && !stage) {
+      double inv = 0;
+      int8_t *qp = nullptr;
+      if constexpr (MIXED) {
+        int E = exponent([&](int n, int l) {
+          const T *cn = c + n * H + l * l;
+          double sq = 0;
+          for (int m = 0; m < 2 * l + 1; m++) sq += (double)cn[m] * (double)cn[m];
+          return sq;
+        });
+        inv = ldexp(1.0, -E);
+        if (lane == 0) mo.scale[row] = ldexp(1.0, E);
+        qp = mo.q + i8_tile_offset(kI8TileA, mo.nk, row + mo.shift[a.species[i]], 0, 0);
+      }
+      auto slices = [&](int k, double r) {
+        double rr[4] = {r, 0, 0, 0};
+        unsigned packed[kI8Slices];
+        slice4(rr, packed);
+        int8_t *dst = qp + (size_t)(k >> 6) * (kI8Slices * kI8TileA * kI8Pad) + (k & (kI8Pad - 1));
+        for (int p = 0; p < kI8Slices; p++) dst[p * (kI8TileA * kI8Pad)] = (int8_t)packed[p];
+      };
+      for (int l = 0; l <= a.lmax; l++)
+        for (int rt = 0; rt < nr; rt += 16)
+          for (int cc = rt; cc < nr; cc += 16) {
+            auto acc = tile_of(l, rt, cc);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+              int k = place(rt, cc, q) + l;
+              if (k < l) continue;
+              T v = acc[q];
+              s2 += v * v;
+              if constexpr (MIXED) {
+                mo.B[(size_t)row * a.nd + k] = (float)v;
+                slices(k, (double)v * inv);
+              } else {
+                B[(size_t)row * a.nd + k] = v;
+              }
+            }
+          }
+      if constexpr (MIXED)
+        for (int k = a.nd + lane; k < (int)(mo.nk * kI8Pad); k += 64) slices(k, 0.0);
+    } else {
+      int tile = 0;
+      for (int l = 0; l <= a.lmax; l++)
+        for (int rt = 0; rt < nr; rt += 16)
+          for (int cc = rt; cc < nr; cc += 16) {
+            if (W > 1 && tile++ % W != w) continue;
+            auto acc = tile_of(l, rt, cc);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+              int k = place(rt, cc, q);
+              if (k >= 0) {
+                T v = acc[q];
+                bst[k + l] = v;
+                if (W == 1) s2 += v * v;
+              }
+            }
+          }
+      if constexpr (W > 1) {
+        atom_sync<W>();
+        if (w == 0)
+          for (int l = 0; l <= a.lmax; l++)
+            for (int rt = 0; rt < nr; rt += 16)
+              for (int cc = rt; cc < nr; cc += 16)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                  int k = place(rt, cc, q);
+                  if (k >= 0) {
+                    T v = bst[k + l];
+                    s2 += v * v;
+                  }
+                }
+      }
+    }
+    if constexpr (W == 1) atom_sync<W>();
+    if (!stage) {
+    } else if constexpr (MIXED) {
+      int E = exponent([&](int n, int l) {
+        return (double)bst[(n * nr - (n * (n - 1)) / 2) * L1 + l];
+      });
       double inv = ldexp(1.0, -E);
-      if (lane == 0) mo.scale[row] = ldexp(1.0, E);
-      for (int k0 = 4 * lane; k0 < Kq; k0 += 256) {
-        int packed[kI8Slices];
+      if (tid == 0) mo.scale[row] = ldexp(1.0, E);
+      long long qrow = row + mo.shift[a.species[i]];
+      int Kq = (int)(mo.nk * kI8Pad);
+      float *B32 = mo.B + (size_t)row * a.nd;
+      int8_t *qp = mo.q + i8_tile_offset(kI8TileA, mo.nk, qrow, 0, 0);
+      for (int k0 = 4 * tid; k0 < Kq; k0 += 4 * NT) {
+        double r[4];
+        if (k0 + 4 <= a.nd) {
+          double2 x = *reinterpret_cast<const double2 *>(&bst[k0]);
+          double2 y = *reinterpret_cast<const double2 *>(&bst[k0 + 2]);
+          r[0] = x.x, r[1] = x.y, r[2] = y.x, r[3] = y.y;
+          f4u v = {(float)r[0], (float)r[1], (float)r[2], (float)r[3]};
+          *reinterpret_cast<f4u *>(B32 + k0) = v;
+        } else {
 #pragma unroll
-        for (int p = 0; p < kI8Slices; p++) packed[p] = 0;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          int k = k0 + j;
-          double r = k < a.nd ? (double)bst[k] * inv : 0.0;
-#pragma unroll
-          for (int p = 0; p < kI8Slices; p++) {
-            double v = rint(ldexp(r, 6 + 7 * p));
-            r -= ldexp(v, -(6 + 7 * p));
-            packed[p] |= ((int)v & 0xff) << (8 * j);
+          for (int j = 0; j < 4; j++) {
+            r[j] = k0 + j < a.nd ? bst[k0 + j] : 0.0;
+            if (k0 + j < a.nd) B32[k0 + j] = (float)r[j];
           }
         }
 #pragma unroll
-        for (int p = 0; p < kI8Slices; p++)
-          *reinterpret_cast<int *>(mo.q + i8_tile_offset(kI8TileA, mo.nk, qrow, k0, p)) =
-              packed[p];
-      }
-    } else {
-      for (int k0 = 4 * lane; k0 < Kq; k0 += 256)
+        for (int j = 0; j < 4; j++) r[j] *= inv;
+        unsigned packed[kI8Slices];
+        slice4(r, packed);
+        // k0's step of the row tile (kI8Slices blocks of kI8TileA rows), then
+        // its place in the row.
+        int8_t *dst = qp + (size_t)(k0 >> 6) * (kI8Slices * kI8TileA * kI8Pad) + (k0 & (kI8Pad - 1));
 #pragma unroll
         for (int p = 0; p < kI8Slices; p++)
-          *reinterpret_cast<int *>(mo.q + i8_tile_offset(kI8TileA, mo.nk, qrow, k0, p)) =
-              *reinterpret_cast<const int *>(&qst[p * Kq + k0]);
+          *reinterpret_cast<unsigned *>(dst + p * (kI8TileA * kI8Pad)) = packed[p];
+      }
+    } else {
+      T *Brow = B + (size_t)row * a.nd;
+      for (int k = 2 * tid; k + 1 < a.nd; k += 2 * NT)
+        *reinterpret_cast<d2u *>(Brow + k) = *reinterpret_cast<const d2u *>(&bst[k]);
+      if ((a.nd & 1) && tid == 0) Brow[a.nd - 1] = bst[a.nd - 1];
     }
-  }
-  s2 = wave_sum(s2);
-  if (lane == 0) {
-    norm[row] = (double)sqrt(s2);
-    nn[row] = (double)s2;
+    if (w == 0) {
+      s2 = wave_sum(s2);
+      if (lane == 0) {
+        norm[row] = (double)sqrt(s2);
+        nn[row] = (double)s2;
+      }
+    }
   }
 }
 
@@ -972,40 +1069,31 @@ void launch_b2(fm_structure s, bool want_b2) {
   bool mixed = want_b2 && s->form != FM_FORM_FP64;
   size_t esz = s->form == FM_FORM_FP64 ? sizeof(double) : sizeof(float);
   size_t csz = s->form == FM_FORM_FP64 || mixed ? sizeof(double) : sizeof(float);
-  // FP32 and mixed mode 1 stage the B row after c (over the bond tables);
-  // mixed mode 2 stages only the row's int8 slices (kI8Slices x Kq bytes).
-  auto work_of = [&](int ch, int mode) {
-    size_t w = b2_work(a.nrad * a.H, a.H, a.N, ch);
-    if (want_b2 && s->form != FM_FORM_FP64 && mode != 2)
-      w = std::max(w, (size_t)a.nrad * a.H + (size_t)a.nd);
-    if (mode == 2)
-      w = std::max(w, (size_t)a.nrad * a.H +
-                          ((size_t)kI8Slices * (size_t)i8_ld(a.nd) + csz - 1) / csz);
-    return w;
+  // 64-bond chunks fill all lanes of the bond basis and take half the passes;
+  // they cost LDS only where the row is shorter than their tables, and are
+  // used where four atoms still fit a CU (times with 64 and with 32 are within
+  // 5 %: 6.75 and 6.77 ms for 262144 atoms of three species, 0.62 and 0.60 ms
+  // for 32000 of two).
+  // Waves per atom: the fewest that give the CU 16 waves (its registers hold
+  // no more). One, two and four waves: 8.7, 8.0 and 6.8 ms (262144 atoms, three
+  // species, l_max 6, four atoms per CU), 0.78, 0.74 and 0.61 ms (32000 atoms, two
+  // species, four per CU), 2.43, 2.35 and 3.19 ms (512 structures, l_max 4,
+  // eight per CU: four waves only add instructions).
+  int row = a.nd;
+  auto work_of = [&](int ch) {
+    return b2_work(a.nrad * a.H, a.H, a.N, ch, want_b2 ? row : 0);
   };
-  // 64-bond chunks take half the chunk passes of 32-bond ones; they are used
-  // when they cost at most a third more LDS and keep as many atoms resident
-  // per CU (a staged row makes the two sizes close in LDS, where only the
-  // residency tells them apart).
-  auto chunk_of = [&](int mode) {
-    bool wide = 3 * work_of(64, mode) <= 4 * work_of(32, mode) &&
-                resident_atoms(work_of(64, mode) * csz) >= resident_atoms(work_of(32, mode) * csz);
-    return wide ? 64 : 32;
-  };
-  // Mixed mode 2 (slices formed with the values, FP32 row stored directly)
-  // spends more ALU per element than mode 1 (FP64 row staged, sliced after)
-  // and pays off only where its smaller LDS footprint keeps more atoms
-  // resident per CU.
-  int mode = 0;
-  if (mixed) {
-    size_t w1 = work_of(chunk_of(1), 1), w2 = work_of(chunk_of(2), 2);
-    mode = resident_atoms(w2 * csz) > resident_atoms(w1 * csz) ? 2 : 1;
-  }
-  int chunk = chunk_of(mode);
-  bool wide = chunk == 64;
-  size_t work = work_of(chunk, mode);
+  bool stage = work_of(32) * csz <= (size_t)160 * 1024;
+  if (!stage && a.nrad > 32) row = 0;
+  size_t res = resident_atoms(work_of(64) * csz);
+  int chunk = res >= 4 ? 64 : 32;
+  if (chunk == 32) res = resident_atoms(work_of(32) * csz);
+  size_t work = work_of(chunk);
   size_t per = work * csz;
-  int apb = atoms_per_block(per);
+  int W = csz == 4 || !stage ? 1 : res >= 16 ? 1 : res >= 8 ? 2 : 4;
+  int apb = W > 1 ? 1 : atoms_per_block(per);
+  FM_CHECK(per <= (size_t)160 * 1024, FM_ERR_CAPACITY,
+           "per-atom descriptor workspace exceeds LDS");
   size_t lds = apb * per;
   int nblk = (s->n + apb - 1) / apb;
   s->C.alloc(&ctx->pool, std::max<size_t>(1, (size_t)s->n * a.nrad * a.H * esz));
@@ -1026,49 +1114,35 @@ void launch_b2(fm_structure s, bool want_b2) {
   }
   s->has_q = mixed;
   if (nblk == 0) return;
-  // No BF16 copies of the rows: the chosen form's kernel contraction slices
-  // the FP32 rows itself.
-  SplitOut none{{nullptr, nullptr}};
   // The unrolled sweep (compile-time l_max) is faster for the FP64 kernel;
   // for FP32 its extra registers cost more occupancy than it saves at
   // l_max 6.
-  auto go = [&](auto ch) {
-    constexpr int CH = decltype(ch)::value;
-    if (s->form == FM_FORM_FP64)
-      with_lmax(a.lmax, [&](auto lc) {
-        constexpr int LC = decltype(lc)::value;
-        hipLaunchKernelGGL((k_b2<double, LC, CH>), dim3(nblk), dim3(64 * apb), lds, st, a,
-                           s->B.as<double>(), s->norm.as<double>(), s->nn.as<double>(), none, 0,
-                           s->C.as<double>(), (int)want_b2, (int)work, mo);
-      });
-    else if (mode == 1)
-      with_lmax(a.lmax, [&](auto lc) {
-        constexpr int LC = decltype(lc)::value;
-        hipLaunchKernelGGL((k_b2<double, LC, CH, 1>), dim3(nblk), dim3(64 * apb), lds, st,
-                           a, (double *)nullptr, s->norm.as<double>(), s->nn.as<double>(), none,
-                           0, (double *)nullptr, (int)want_b2, (int)work, mo);
-      });
-    else if (mode == 2)
-      with_lmax(a.lmax, [&](auto lc) {
-        constexpr int LC = decltype(lc)::value;
-        hipLaunchKernelGGL((k_b2<double, LC, CH, 2>), dim3(nblk), dim3(64 * apb), lds, st,
-                           a, (double *)nullptr, s->norm.as<double>(), s->nn.as<double>(), none,
-                           0, (double *)nullptr, (int)want_b2, (int)work, mo);
-      });
-    else
-      with_lmax(a.lmax <= 4 ? a.lmax : -1, [&](auto lc) {
-        constexpr int LC = decltype(lc)::value;
-        hipLaunchKernelGGL((k_b2<float, LC, CH>), dim3(nblk), dim3(64 * apb), lds, st, a,
-                           s->B.as<float>(), s->norm.as<double>(), s->nn.as<double>(), none, 0,
-                           s->C.as<float>(), (int)want_b2, (int)work, mo);
-      });
+  auto go = [&](auto waves) {
+    constexpr int NW = decltype(waves)::value;
+    dim3 grid(nblk), block(64 * NW * apb);
+    with_lmax(a.lmax, [&](auto lc) {
+      constexpr int LC = decltype(lc)::value;
+      if (mixed)
+        hipLaunchKernelGGL((k_b2<double, LC, true, NW>), grid, block, lds, st, a,
+                           (double *)nullptr, s->norm.as<double>(), s->nn.as<double>(),
+                           (double *)nullptr, 1, (int)work, chunk, (int)stage, mo);
+      else
+        hipLaunchKernelGGL((k_b2<double, LC, false, NW>), grid, block, lds, st, a,
+                           s->B.as<double>(), s->norm.as<double>(), s->nn.as<double>(),
+                           s->C.as<double>(), (int)want_b2, (int)work, chunk, (int)stage, mo);
+    });
   };
   {
     KScope timer(ctx, KT_DESC);
-    if (wide)
-      go(std::integral_constant<int, 64>{});
-    else
-      go(std::integral_constant<int, 32>{});
+    if (csz == 4)
+      with_lmax(a.lmax <= 4 ? a.lmax : -1, [&](auto lc) {
+        hipLaunchKernelGGL((k_b2<float, decltype(lc)::value, false, 1>), dim3(nblk),
+                           dim3(64 * apb), lds, st, a, (float *)nullptr, s->norm.as<double>(),
+                           s->nn.as<double>(), s->C.as<float>(), 0, (int)work, chunk, 1, mo);
+      });
+    else if (W == 4) go(std::integral_constant<int, 4>{});
+    else if (W == 2) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, 1>{});
   }
   FM_HIP(hipGetLastError());
 }
