@@ -1074,11 +1074,11 @@ void launch_b2(fm_structure s, bool want_b2) {
   // used where four atoms still fit a CU (times with 64 and with 32 are within
   // 5 %: 6.75 and 6.77 ms for 262144 atoms of three species, 0.62 and 0.60 ms
   // for 32000 of two).
-  // Waves per atom: the fewest that give the CU 16 waves (its registers hold
-  // no more). One, two and four waves: 8.7, 8.0 and 6.8 ms (262144 atoms, three
+  // Waves per atom: the fewest that give the CU 12 waves (its registers hold
+  // 16). One, two and four waves: 8.7, 8.0 and 6.8 ms (262144 atoms, three
   // species, l_max 6, four atoms per CU), 0.78, 0.74 and 0.61 ms (32000 atoms, two
   // species, four per CU), 2.43, 2.35 and 3.19 ms (512 structures, l_max 4,
-  // eight per CU: four waves only add instructions).
+  // seven per CU: four waves only add instructions).
   int row = a.nd;
   auto work_of = [&](int ch) {
     return b2_work(a.nrad * a.H, a.H, a.N, ch, want_b2 ? row : 0);
@@ -1090,7 +1090,7 @@ void launch_b2(fm_structure s, bool want_b2) {
   if (chunk == 32) res = resident_atoms(work_of(32) * csz);
   size_t work = work_of(chunk);
   size_t per = work * csz;
-  int W = csz == 4 || !stage ? 1 : res >= 16 ? 1 : res >= 8 ? 2 : 4;
+  int W = csz == 4 || !stage ? 1 : res >= 12 ? 1 : res >= 6 ? 2 : 4;
   int apb = W > 1 ? 1 : atoms_per_block(per);
   FM_CHECK(per <= (size_t)160 * 1024, FM_ERR_CAPACITY,
            "per-atom descriptor workspace exceeds LDS");
