@@ -13,7 +13,7 @@
 //             triangular so each row tile stops at its last nonzero column.
 //
 // FP64 form: k_gemm_f64 for all three. Chosen form: EP_KERNEL is exact on
-// int8 MFMA (v_mfma_i32_32x32x32_i8) over five power-of-two-scaled slices of
+// int8 MFMA (v_mfma_i32_16x16x64_i8) over five power-of-two-scaled slices of
 // each operand row, int32 accumulation per slice-pair diagonal and an FP64
 // epilogue (k_gemm_i8); EP_STORE is split-BF16 x3 on
 // v_mfma_f32_16x16x32_bf16 (a = a_hi + a_lo, ab ~ a_hi b_hi + a_hi b_lo +
@@ -76,19 +76,6 @@ __device__ __forceinline__ void xcd_tile(int &tx, int &ty, bool rows_fastest = f
     tx = id % ntx;
     ty = id / ntx;
   }
-}
-
-// As xcd_tile, with the logical tiles of each XCD's run taken in groups of
-// G row tiles, row index fastest within a group: the workgroups an XCD holds
-// at once then cover G row tiles by (resident / G) column tiles instead of
-// (resident / columns) row tiles by every column tile, so fewer A and B tile
-// bytes share that XCD's L2 per k step.
-__device__ __forceinline__ void xcd_tile_grouped(int &tx, int &ty, int G) {
-  int ntx = gridDim.x, nty = gridDim.y;
-  int id = xcd_id();
-  int gw = G * ntx, first = id / gw * G, gs = min(G, nty - first), r = id % gw;
-  tx = r / gs;
-  ty = first + r % gs;
 }
 
 template <typename Acc>
@@ -798,7 +785,6 @@ __global__ __launch_bounds__(256) void k_gemm_split(int M, int N, int Kpad, Spli
 // accuracy, where FP32 accumulation of BF16 pieces carries about 16 bits.
 // ---------------------------------------------------------------------------
 typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
 
 // One wave per row: the row maximum, its power-of-two scale and the slices
 // of 4 consecutive values per lane (zeros past nd up to Kq), stored in the
@@ -846,187 +832,254 @@ constexpr int kI8Flush = 65536;
 
 // 16-byte chunk position of k chunk c (0..3) in row r of an LDS slice block
 // (rows of 64 bytes, no padding): an XOR swizzle that keeps the fragment
-// reads (32 rows at one chunk) and the contiguous stores free of bank
-// conflicts for 8- and 16-lane phases.
-__device__ __forceinline__ int i8_chunk(int r, int c) { return c ^ (((r >> 1) ^ (r >> 3)) & 3); }
+// reads (16 rows at four chunks) free of bank conflicts (a third of the LDS
+// cycles were conflicts with r / 2 xor r / 8 in its place).
+__device__ __forceinline__ int i8_chunk(int r, int c) { return c ^ (-(r >> 2) & 3); }
 
-// 128 x 64 tiles (kI8TileA x kI8TileN), 8 waves (4 x 2), each 32 x 32 of
-// v_mfma_i32_32x32x32_i8 (lane l: operand row l % 32, bytes k = 16 (l / 32)
-// .. + 15; result column l % 32, rows 8 (j / 4) + 4 (l / 32) + j % 4); two
-// waves per SIMD, so one wave's loads, LDS traffic and barrier waits overlap
-// the other's MFMAs. One k step (64) of the workgroup's row tile and column
-// tile is one contiguous run of each operand (the tiled slice layout), loaded
-// with 16-byte vectors into registers one step ahead and stored to one of two
-// LDS buffers after the step before it computes: one barrier per k step. The slice
-// products run in rounds (round r: slice r of A against each slice of B it
-// pairs with), so consecutive MFMAs accumulate into different diagonals.
+// 128 x 32 RA tiles, 8 waves, each 16 RA x 32 of v_mfma_i32_16x16x64_i8 (lane
+// l: operand row l % 16, bytes k = 16 (l / 16) .. + 15; result column l % 16,
+// rows 4 (l / 16) + i).
+//
+// What bounds it: power. With operands in registers the card reaches 4.3
+// POP/s on such data with this instruction (3.4 with 32 x 32 x 32, 4.9 on
+// zeros), at a lower clock; every byte moved takes from that. So the tiles are as
+// large as the registers allow and are copied to LDS directly. 87,381 x 1,365 x
+// 3,264: 2.5 POP/s (70 % of the cycles have an MFMA in flight at 1.8 GHz; 1.8
+// before, with 32 x 32 x 32 on 128 x 64 tiles that passed through registers,
+// and all waves reading LDS or multiplying at the same time).
+//
+// One k step (64) of a row tile and of a column tile is one contiguous run of
+// either operand (the tiled slice layout), copied straight to one of two LDS
+// buffers a step ahead. The 15 slice products of a pair of 16-row blocks run
+// in rounds (round r: slice r of A against each slice of B it pairs with), so
+// consecutive MFMAs accumulate into different diagonals; between them the
+// fragments that the next pair of blocks needs are read (the pairs are walked
+// in a serpentine, so that is one block of 5 fragments at a time).
 // Epilogue as EpKernel, in FP64 from the exact sums: S, k (FP64), w as BF16
-// pairs, energy partials per column tile; k and w are staged in LDS and
+// pairs, energy partials per kI8TileN columns; k, then w, are staged in LDS and
 // stored as whole rows of the tile.
-template <bool LONG>
-__global__ __launch_bounds__(512) void k_gemm_i8(int M, int N, int nk, const int8_t *Ag,
-                                                 const double *sa, const int8_t *Bg,
-                                                 const double *sb, EpArgs e) {
-  constexpr int S = kI8Slices, BM = kI8TileA, BN = kI8TileN, NT = 512;
-  constexpr int A_SL = BM * kI8Pad, B_SL = BN * kI8Pad;  // bytes of one slice block
+typedef __attribute__((address_space(1))) const void gvoid;
+typedef __attribute__((address_space(3))) void lvoid;
+
+// One launch's contractions. Every XCD takes a contiguous run of the tiles,
+// kI8Group row tiles at a time, row index fastest: the workgroups that it holds
+// at once cover kI8Group row tiles by 32 / kI8Group column tiles, which share
+// its L2.
+constexpr int kI8Groups = 8;
+struct I8Groups {
+  I8Gemm g[kI8Groups];
+  int first[kI8Groups], n;
+};
+
+template <bool LONG, int RA>
+__global__ __launch_bounds__(512) void k_gemm_i8(I8Groups gs) {
+  constexpr int S = kI8Slices, BM = kI8TileA, BN = 32 * RA, NT = 512, WC = RA;  // wave columns
+  constexpr int A_SL = BM * kI8Pad, B_SL = BN * kI8Pad;  // bytes of one slice block in LDS
   constexpr int A_ST = S * A_SL, B_ST = S * B_SL;        // bytes of one k step
-  constexpr int NA = A_ST / (16 * NT);                   // 16-byte loads per thread (A)
-  constexpr int NB = (B_ST + 16 * NT - 1) / (16 * NT);   // (B; the last by some threads)
-  static_assert(A_ST % (16 * NT) == 0 && B_ST % (16 * NT / 2) == 0, "load split");
-  static_assert(BM * BN * (8 + 2 + 2) <= 2 * (A_ST + B_ST), "epilogue staging fits");
-  __shared__ __align__(16) int8_t smem[2 * (A_ST + B_ST)];
-  __shared__ double red[2 * BM];
-  int8_t *As = smem, *Bs = smem + 2 * A_ST;  // [2][A_ST], [2][B_ST]
-  int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  int wr = wid >> 1, wc = wid & 1;
-  int tx, ty;
-  xcd_tile_grouped(tx, ty, kI8Group);
+  constexpr int G_SL = kI8TileN * kI8Pad, G_ST = S * G_SL;  // of B in memory
+  constexpr int NB = (B_ST / 1024 + 7) / 8;  // 1 KB pieces of B per wave (A: S)
+  static_assert(BM == 128 && kI8TileN == 64 && kI8Pad == 64 && (RA == 2 || RA == 4), "tiling");
+  static_assert(BM * BN * 4 + 8 * BM * WC <= A_ST + B_ST, "epilogue staging fits");
+  __shared__ __align__(16) int8_t buf0[A_ST + B_ST], buf1[A_ST + B_ST];
+  int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int wr = wid / WC, wc = wid % WC;
+  int id = xcd_id(), gi = 0;
+  while (gi + 1 < gs.n && id >= gs.first[gi + 1]) gi++;
+  const I8Gemm &g = gs.g[gi];
+  const int M = g.M, N = g.N, nk = g.nk;
+  const EpArgs &e = g.e;
+  id -= gs.first[gi];
+  int ntx = (N + BN - 1) / BN, nty = (M + BM - 1) / BM, first = id / (kI8Group * ntx) * kI8Group;
+  int n_in = min(kI8Group, nty - first), tx = id % (kI8Group * ntx) / n_in;
+  int ty = first + id % (kI8Group * ntx) % n_in;
   int row0 = ty * BM, col0 = tx * BN;
-  const int8_t *Ab = Ag + (size_t)ty * nk * A_ST + 16 * tid;
-  const int8_t *Bb = Bg + (size_t)tx * nk * B_ST + 16 * tid;
-  v16i acc[S];
+  v4i acc[S][RA][2];
   // With LONG (Kq > kI8Flush) the int32 sums of the slice products
   // (p + q = d) are folded into one FP64 sum every kI8Flush k, before they
   // could overflow; otherwise once, after the loop.
-  constexpr int SJ = LONG ? 16 : 1;
+  constexpr int NV = 8 * RA, SJ = LONG ? NV : 1;  // values per lane
   double sacc[SJ];
   auto clear = [&]() {
 #pragma unroll
-    for (int d = 0; d < S; d++) acc[d] = v16i{};
+    for (int d = 0; d < S; d++)
+#pragma unroll
+      for (int q = 0; q < 2 * RA; q++) acc[d][q >> 1][q & 1] = v4i{};
   };
   auto diag_sum = [&](int j) {
     double sum = 0;
 #pragma unroll
-    for (int d = S - 1; d >= 0; d--) sum += ldexp((double)acc[d][j], -(12 + 7 * d));
+    for (int d = S - 1; d >= 0; d--)
+      sum += ldexp((double)acc[d][j >> 3][(j >> 2) & 1][j & 3], -(12 + 7 * d));
     return sum;
   };
-  auto fold = [&]() {
+  auto flush = [&](int ks) {
     if constexpr (LONG) {
+      if (ks > 0 && (ks % (kI8Flush / kI8Pad) == 0 || ks == nk)) {
 #pragma unroll
-      for (int j = 0; j < 16; j++) sacc[j] += diag_sum(j);
+        for (int j = 0; j < NV; j++) sacc[j] += diag_sum(j);
+        clear();
+      }
     }
   };
 #pragma unroll
   for (int j = 0; j < SJ; j++) sacc[j] = 0;
   clear();
-  v4i ra0[NA], rb0[NB];
-  auto gload = [&](auto &ra, auto &rb, int ks) {
-#pragma unroll
-    for (int j = 0; j < NA; j++)
-      ra[j] = *reinterpret_cast<const v4i *>(Ab + (size_t)ks * A_ST + 16 * NT * j);
-#pragma unroll
-    for (int j = 0; j < NB; j++)
-      if (16 * NT * j + 16 * tid < B_ST)
-        rb[j] = *reinterpret_cast<const v4i *>(Bb + (size_t)ks * B_ST + 16 * NT * j);
+  // Copies of a step's 1 KB pieces (16 rows of a slice): wave w takes piece w
+  // of each slice of A and of B (with 64 columns, which have 4 pieces a slice,
+  // piece w % 4 of slices w / 4, w / 4 + 2 and the last one). A lane's 16 bytes
+  // land at 16 lane; it fetches the chunk that belongs there. A column tile
+  // past the last 64 columns repeats them.
+  unsigned vsrc = (lane >> 2) * 64 + 16 * i8_chunk(lane >> 2, lane & 3);
+  int wb = wid % (B_SL / 1024), pb = wid / (B_SL / 1024);
+  int tb = min(tx * (BN / kI8TileN) + (wb >> 2), (N - 1) / kI8TileN);
+  const int8_t *Aw = g.A + (size_t)ty * nk * A_ST + wid * 1024;
+  const int8_t *Bw = g.B + (size_t)tb * nk * G_ST + (wb & 3) * 1024;
+  auto copy = [&](int8_t *dst, int ks, int i) {
+    if (i >= S + NB) return;
+    int p = i < S ? i : RA == 4 ? i - S : min(2 * (i - S) + pb, S - 1);
+    const int8_t *src = i < S ? Aw + ((size_t)ks * A_ST + p * A_SL)
+                              : Bw + ((size_t)ks * G_ST + p * G_SL);
+    asm volatile("" : "+s"(src));  // a scalar base: one vector register addresses all pieces
+    dst += i < S ? p * A_SL + wid * 1024 : A_ST + p * B_SL + wb * 1024;
+    __builtin_amdgcn_global_load_lds((gvoid *)(src + vsrc), (lvoid *)dst, 16, 0, 0);
   };
-  // Thread tid's 16 bytes at offset 16 tid + 16 NT j of a step: slice block,
-  // row (of 64 bytes) and k chunk; stored at the swizzled chunk.
-  auto lstore = [&](const auto &ra, const auto &rb, int buf) {
-#pragma unroll
-    for (int j = 0; j < NA; j++) {
-      int o = 16 * tid + 16 * NT * j, p = o / A_SL, w = o % A_SL, r = w >> 6;
-      *reinterpret_cast<v4i *>(
-          &As[buf * A_ST + p * A_SL + r * 64 + 16 * i8_chunk(r, (w >> 4) & 3)]) = ra[j];
-    }
-#pragma unroll
-    for (int j = 0; j < NB; j++) {
-      int o = 16 * tid + 16 * NT * j, p = o / B_SL, w = o % B_SL, r = w >> 6;
-      if (o < B_ST)
-        *reinterpret_cast<v4i *>(
-            &Bs[buf * B_ST + p * B_SL + r * 64 + 16 * i8_chunk(r, (w >> 4) & 3)]) = rb[j];
-    }
+  // Fragments: all slices of 16 rows of A and of 32 of B for a whole step.
+  v4i fa[S], fb[2][S];
+  int r16 = lane & 15, k16 = lane >> 4;
+  int frag = r16 * 64 + 16 * i8_chunk(r16, k16);
+  int oa = wr * 16 * RA * 64 + frag, ob = A_ST + wc * 32 * 64 + frag;
+  auto read_a = [&](const int8_t *src, int r, int p) {
+    fa[p] = *reinterpret_cast<const v4i *>(&src[p * A_SL + r * 1024 + oa]);
   };
-  auto compute = [&](int buf) {
-    int ra_ = wr * 32 + (lane & 31), rb_ = wc * 32 + (lane & 31);
-#pragma unroll
-    for (int kk = 0; kk < kI8Pad; kk += 32) {
-      int c = (kk >> 4) + (lane >> 5);
-      v4i af[S], bf[S];
-#pragma unroll
-      for (int p = 0; p < S; p++) {
-        af[p] = *reinterpret_cast<const v4i *>(
-            &As[buf * A_ST + p * A_SL + ra_ * 64 + 16 * i8_chunk(ra_, c)]);
-        bf[p] = *reinterpret_cast<const v4i *>(
-            &Bs[buf * B_ST + p * B_SL + rb_ * 64 + 16 * i8_chunk(rb_, c)]);
-      }
-#pragma unroll
-      for (int rd = 0; rd < S; rd++)
-#pragma unroll
-        for (int d = S - 1; d >= rd; d--)
-          acc[d] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[rd], bf[d - rd], acc[d], 0, 0, 0);
-    }
+  auto read_b = [&](const int8_t *src, int h, int p) {
+    fb[h][p] = *reinterpret_cast<const v4i *>(&src[p * B_SL + h * 1024 + ob]);
   };
-  auto flush = [&](int ks) {
-    if constexpr (LONG) {
-      if (ks > 0 && (ks * kI8Pad) % kI8Flush == 0) {
-        fold();
-        clear();
+  // The 15 slice products of blocks (r, h); other(i) issues copies and reads
+  // between them, after(rd) follows the last use of slice rd of A.
+  auto products = [&](int r, int h, auto other, auto after) {
+    int i = 0;
+#pragma unroll
+    for (int rd = 0; rd < S; rd++) {
+#pragma unroll
+      for (int d = S - 1; d >= rd; d--) {
+        acc[d][r][h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[rd], fb[h][d - rd],
+                                                             acc[d][r][h], 0, 0, 0);
+        other(i++);
+        if (d == rd) after(rd);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
   };
-  // Before step ks: LDS buffer ks % 2 holds step ks, the registers step ks + 1
-  // (issued after the previous step's barrier; the other wave on each SIMD
-  // computes while they land).
-  gload(ra0, rb0, 0);
-  lstore(ra0, rb0, 0);
-  if (nk > 1) gload(ra0, rb0, 1);
-  __syncthreads();
-#pragma unroll 1
-  for (int ks = 0; ks < nk; ks++) {
-    flush(ks);
-    compute(ks & 1);
-    if (ks + 1 < nk) lstore(ra0, rb0, (ks + 1) & 1);  // last read in step ks - 1
+  // Step ks, its column block h first: all pairs of blocks but the last, during
+  // which the next step's first fragments are read. dst receives step `next`.
+  auto body = [&](const int8_t *__restrict__ src, int8_t *__restrict__ dst, int next, int h) {
+#pragma unroll
+    for (int d = 0; d < S; d++)
+#pragma unroll
+      for (int q = 0; q < 2 * RA; q++) asm volatile("" : "+v"(acc[d][q >> 1][q & 1]));
+#pragma unroll
+    for (int r = 0; r < RA; r++) {
+      products(
+          r, (r & 1) ? h ^ 1 : h,
+          [&](int i) {
+            if (r == 0 && i % 3 == 0) read_b(src, h ^ 1, i / 3);
+            if (r == 0 && i % 3 == 1) copy(dst, next, i / 3);
+          },
+          [](int) {});
+      if (r < RA - 1)
+        products(
+            r, (r & 1) ? h : h ^ 1,
+            [&](int i) {
+              if (r == 0 && i % 3 == 1) copy(dst, next, 5 + i / 3);
+            },
+            [&](int rd) { read_a(src, r + 1, rd); });
+    }
+  };
+  auto tail = [&](const int8_t *src, int h) {
+    products(
+        RA - 1, h, [&](int i) { if (i % 3 == 1) read_b(src, h ^ 1, i / 3); },
+        [&](int rd) { read_a(src, 0, rd); });
+  };
+  auto landed = [&]() {
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // this wave's copies
     __syncthreads();
-    if (ks + 2 < nk) gload(ra0, rb0, ks + 2);
-  }
-  fold();
-  // Epilogue: values in FP64 per element, staged in LDS (over the operand
-  // buffers, free after the loop's last barrier) as k (BM x BN FP64) and the
-  // two BF16 pieces of w (BM x BN each).
-  double *Kst = reinterpret_cast<double *>(smem);
-  uint16_t *Hst = reinterpret_cast<uint16_t *>(smem + BM * BN * 8);
-  uint16_t *Lst = Hst + BM * BN;
-  int pi = e.power == 2.0 ? 2 : (e.power == 1.0 ? 1 : 0);
-  int cc = wc * 32 + (lane & 31), c = col0 + cc;
-  bool cin = c < N;
-  double a_c = cin ? e.alpha[c] : 0.0, s_c = cin ? sb[c] : 0.0;
-  double rsum[16];
+  };
 #pragma unroll
-  for (int j = 0; j < 16; j++) {
-    int rr = wr * 32 + 8 * (j / 4) + 4 * (lane >> 5) + (j & 3);
+  for (int i = 0; i < S + NB; i++) copy(buf0, 0, i);
+  landed();
+#pragma unroll
+  for (int p = 0; p < S; p++) {
+    read_a(buf0, 0, p);
+    read_b(buf0, 0, p);
+  }
+  int ks = 0;
+#pragma unroll 1
+  for (; ks + 2 <= nk; ks += 2) {
+    flush(ks);
+    body(buf0, buf1, ks + 1, 0);
+    landed();
+    tail(buf1, 0);
+    flush(ks + 1);
+    body(buf1, buf0, min(ks + 2, nk - 1), 1);
+    landed();
+    tail(buf0, 1);
+  }
+  if (ks < nk) {
+    flush(ks);
+    body(buf0, buf1, ks, 0);
+    tail(buf0, 0);
+  }
+  flush(nk);
+  landed();
+  // Epilogue: values in FP64 per element. k is staged in LDS over the operand
+  // buffers, w after it.
+  constexpr int HN = BN / 2;  // columns staged in each buffer
+  double *Kst = reinterpret_cast<double *>(wc < WC / 2 ? buf0 : buf1);
+  double *red = reinterpret_cast<double *>(buf0 + BM * HN * 8);  // [WC][BM]
+  uint16_t *Hst = reinterpret_cast<uint16_t *>(buf0), *Lst = reinterpret_cast<uint16_t *>(buf1);
+  int pi = e.power == 2.0 ? 2 : (e.power == 1.0 ? 1 : 0);
+  // Value j of a lane: row block j / 8, column block (j / 4) % 2, row j % 4.
+  bool cin[2];
+  double a_c[2], s_c[2], rsum[NV / 2];
+  float wf[NV];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    int c = col0 + wc * 32 + 16 * h + r16;
+    cin[h] = c < N;
+    a_c[h] = cin[h] ? e.alpha[c] : 0.0;
+    s_c[h] = cin[h] ? g.sb[c] : 0.0;
+  }
+#pragma unroll
+  for (int j = 0; j < NV; j++) {
+    int h = (j >> 2) & 1, cc = wc * 32 + 16 * h + r16;
+    int rr = wr * 16 * RA + 16 * (j >> 3) + 4 * k16 + (j & 3);
     int r = row0 + rr;
     double kv = 0.0;
-    float wf = 0.0f;
-    if (r < M && cin) {
+    wf[j] = 0.0f;
+    if (r < M && cin[h]) {
       double sum;
       if constexpr (LONG) sum = sacc[j];
       else sum = 0.0 + diag_sum(j);
       double nrm = e.row_norm[r];
       bool empty = nrm < kEmptyThresh;
-      double s = empty ? 0.0 : sum * sa[r] * s_c / nrm;
+      double s = empty ? 0.0 : sum * g.sa[r] * s_c[h] / nrm;
       kv = empty ? 0.0 : e.sig2 * fpow(s, e.power, pi);
       double pm1 = pi == 2 ? s : (pi == 1 ? 1.0 : fpow(s, e.power - 1, 0));
-      wf = (float)(empty ? 0.0 : e.sig2 * a_c * e.power * pm1);
+      wf[j] = (float)(empty ? 0.0 : e.sig2 * a_c[h] * e.power * pm1);
     }
-    __bf16 h = (__bf16)wf, l = (__bf16)(wf - (float)h);
-    Kst[rr * BN + cc] = kv;
-    Hst[rr * BN + cc] = __builtin_bit_cast(uint16_t, h);
-    Lst[rr * BN + cc] = __builtin_bit_cast(uint16_t, l);
-    rsum[j] = kv * a_c;
+    Kst[rr * HN + cc % HN] = kv;
+    int i = 4 * (j >> 3) + (j & 3);
+    if (h == 0) rsum[i] = kv * a_c[0];
+    else rsum[i] += kv * a_c[1];
   }
-  // Row sums over the 32 columns of each half-wave, then over the two wave
-  // columns through LDS: one energy partial per (column tile, row).
+  // Row sums over the wave's 32 columns, then over each two wave columns
+  // through LDS: one energy partial per (kI8TileN columns, row).
 #pragma unroll
-  for (int j = 0; j < 16; j++) {
-    double v = rsum[j];
+  for (int i = 0; i < NV / 2; i++) {
+    double v = rsum[i];
 #pragma unroll
-    for (int off = 16; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    rsum[j] = v;
-  }
-  if ((lane & 31) == 0) {
-#pragma unroll
-    for (int j = 0; j < 16; j++)
-      red[wc * BM + wr * 32 + 8 * (j / 4) + 4 * (lane >> 5) + (j & 3)] = rsum[j];
+    for (int off = 8; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+    if (r16 == 0) red[wc * BM + wr * 16 * RA + 16 * (i >> 2) + 4 * k16 + (i & 3)] = v;
   }
   __syncthreads();
   // k: rows of the tile as 16-byte pairs of columns (ldk even, 16-byte base).
@@ -1036,12 +1089,30 @@ __global__ __launch_bounds__(512) void k_gemm_i8(int M, int N, int nk, const int
       int rr = q / (BN / 2), c2 = 2 * (q % (BN / 2)), r = row0 + rr, cg = col0 + c2;
       if (r >= M || cg >= N) continue;
       double *dst = K + (size_t)r * e.ldk + cg;
+      const double *src =
+          reinterpret_cast<const double *>(c2 < HN ? buf0 : buf1) + rr * HN + c2 % HN;
       if (cg + 1 < N)
-        *reinterpret_cast<double2 *>(dst) = *reinterpret_cast<const double2 *>(&Kst[rr * BN + c2]);
+        *reinterpret_cast<double2 *>(dst) = *reinterpret_cast<const double2 *>(src);
       else
-        dst[0] = Kst[rr * BN + c2];
+        dst[0] = src[0];
     }
   }
+  for (int q = tid; q < BM * (BN / kI8TileN); q += NT) {
+    int r = row0 + q % BM, t = q / BM, ct = col0 / kI8TileN + t;
+    if (r < M && ct * kI8TileN < N)
+      e.part[(size_t)ct * e.part_ld + r] =
+          red[2 * t * BM + q % BM] + red[(2 * t + 1) * BM + q % BM];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NV; j++) {
+    int rr = wr * 16 * RA + 16 * (j >> 3) + 4 * k16 + (j & 3);
+    int cc = wc * 32 + 16 * ((j >> 2) & 1) + r16;
+    __bf16 hi = (__bf16)wf[j], lo = (__bf16)(wf[j] - (float)hi);
+    Hst[rr * BN + cc] = __builtin_bit_cast(uint16_t, hi);
+    Lst[rr * BN + cc] = __builtin_bit_cast(uint16_t, lo);
+  }
+  __syncthreads();
   // w pieces: 8 columns per 16-byte store; the padding columns [N, ldw) are
   // zero (the reduction tail of the gradient contraction), none past ldw
   // (a multiple of 32) is written.
@@ -1052,10 +1123,6 @@ __global__ __launch_bounds__(512) void k_gemm_i8(int M, int N, int nk, const int
         *reinterpret_cast<const v4i *>(&Hst[rr * BN + c8]);
     *reinterpret_cast<v4i *>(reinterpret_cast<uint16_t *>(e.Wl) + (size_t)r * e.ldw + cg) =
         *reinterpret_cast<const v4i *>(&Lst[rr * BN + c8]);
-  }
-  for (int q = tid; q < BM; q += NT) {
-    int r = row0 + q;
-    if (r < M) e.part[(size_t)(col0 / BN) * e.part_ld + r] = red[q] + red[BM + q];
   }
 }
 
@@ -1174,17 +1241,6 @@ void split_shape(int i, hipStream_t st, int M, int N, int Kpad, const SplitPtrs 
   }
 }
 
-// The integer contraction runs 128 x 64 tiles (kI8TileA x kI8TileN): the
-// column tile is fixed at 64 (the energy partials are per column tile).
-void i8_launch(hipStream_t st, int M, int N, int nk, const int8_t *a, const double *sa,
-               const int8_t *b, const double *sb, const EpArgs &e) {
-  dim3 grid((N + kI8TileN - 1) / kI8TileN, (M + kI8TileA - 1) / kI8TileA);
-  if ((long long)nk * kI8Pad > kI8Flush)
-    hipLaunchKernelGGL((k_gemm_i8<true>), grid, dim3(512), 0, st, M, N, nk, a, sa, b, sb, e);
-  else
-    hipLaunchKernelGGL((k_gemm_i8<false>), grid, dim3(512), 0, st, M, N, nk, a, sa, b, sb, e);
-}
-
 }  // namespace
 
 void slice_rows(hipStream_t st, const float *X, long long ldx, int n, int nd, int8_t *Q,
@@ -1205,23 +1261,47 @@ void slice_rows(hipStream_t st, const double *X, long long ldx, int n, int nd, i
   FM_HIP(hipGetLastError());
 }
 
-void gemm_i8_kernel(hipStream_t st, int M, int N, int Kq, const SliceOperand &A,
-                    const SliceOperand &B, const EpArgs &e) {
-  if (M <= 0 || N <= 0) return;
-  FM_CHECK(Kq > 0 && Kq % kI8Pad == 0 && A.Kq == Kq && B.Kq == Kq, FM_ERR_INVALID,
-           "sliced operands must share a reduction length padded to 64");
-  FM_CHECK(A.tr == kI8TileA && B.tr == kI8TileN, FM_ERR_INVALID,
-           "sliced operands must be tiled by 128 (rows) and 64 (columns)");
-  FM_CHECK(A.q && B.q && A.scale && B.scale &&
-               ((uintptr_t)A.q | (uintptr_t)B.q) % 16 == 0,
-           FM_ERR_INVALID, "sliced operands must be 16-byte aligned");
-  FM_CHECK(e.Wh && e.Wl && e.alpha && e.row_norm && e.part, FM_ERR_INVALID,
-           "integer contraction: missing epilogue outputs");
-  FM_CHECK(e.ldw % 32 == 0 && e.ldw >= N && ((uintptr_t)e.Wh | (uintptr_t)e.Wl) % 16 == 0 &&
-               (!e.K || (e.ldk % 2 == 0 && e.ldk >= N && (uintptr_t)e.K % 16 == 0)),
-           FM_ERR_INVALID, "integer contraction: k and w must be 16-byte aligned rows");
-  i8_launch(st, M, N, Kq / kI8Pad, A.q, A.scale, B.q, B.scale, e);
-  FM_HIP(hipGetLastError());
+// Columns of the integer contraction's tiles, 32 RA: 128 (RA = 4) moves less
+// data per product and is the faster one where the tiles fill the GPU (one
+// workgroup per CU: two LDS buffers of a step take 160 KB), 64 (RA = 2) where they
+// are few. A round of tiles over the 256 CUs takes 1.75 times as long at 128
+// columns (us per launch with 64 and with 128: 46 and 78 for 3,000 x 130 x 2,112,
+// one round each; 489 and 421 for 16,000 x 1,000 x 2,112, eight and four).
+// Reductions long enough for the LONG form have it at 64 columns.
+void gemm_i8_groups(hipStream_t st, const std::vector<I8Gemm> &all) {
+  for (size_t g0 = 0; g0 < all.size(); g0 += kI8Groups) {
+    I8Groups gs{};
+    gs.n = (int)std::min<size_t>(kI8Groups, all.size() - g0);
+    long long b2 = 0, b4 = 0, nk = 0;
+    for (int k = 0; k < gs.n; k++) {
+      const I8Gemm &g = gs.g[k] = all[g0 + k];
+      const EpArgs &e = g.e;
+      FM_CHECK(g.M > 0 && g.N > 0 && g.nk > 0, FM_ERR_INVALID, "empty integer contraction");
+      FM_CHECK(g.A && g.B && g.sa && g.sb && ((uintptr_t)g.A | (uintptr_t)g.B) % 16 == 0,
+               FM_ERR_INVALID, "sliced operands must be 16-byte aligned");
+      FM_CHECK(e.Wh && e.Wl && e.alpha && e.row_norm && e.part, FM_ERR_INVALID,
+               "integer contraction: missing epilogue outputs");
+      FM_CHECK(e.ldw % 32 == 0 && e.ldw >= g.N && ((uintptr_t)e.Wh | (uintptr_t)e.Wl) % 16 == 0 &&
+                   (!e.K || (e.ldk % 2 == 0 && e.ldk >= g.N && (uintptr_t)e.K % 16 == 0)),
+               FM_ERR_INVALID, "integer contraction: k and w must be 16-byte aligned rows");
+      long long rows = (g.M + kI8TileA - 1) / kI8TileA;
+      b2 += rows * ((g.N + 63) / 64);
+      b4 += rows * ((g.N + 127) / 128);
+      nk = std::max<long long>(nk, g.nk);
+      FM_CHECK(b2 < (1LL << 31), FM_ERR_CAPACITY, "contraction too large for one launch");
+    }
+    bool is_long = nk * kI8Pad > kI8Flush;
+    int RA = !is_long && 7 * ((b4 + 255) / 256) <= 4 * ((b2 + 255) / 256) ? 4 : 2;
+    for (int k = 0, first = 0; k < gs.n; k++) {
+      gs.first[k] = first;
+      first += (gs.g[k].M + kI8TileA - 1) / kI8TileA * ((gs.g[k].N + 32 * RA - 1) / (32 * RA));
+    }
+    dim3 grid(RA == 4 ? b4 : b2), block(512);
+    if (is_long) hipLaunchKernelGGL((k_gemm_i8<true, 2>), grid, block, 0, st, gs);
+    else if (RA == 2) hipLaunchKernelGGL((k_gemm_i8<false, 2>), grid, block, 0, st, gs);
+    else hipLaunchKernelGGL((k_gemm_i8<false, 4>), grid, block, 0, st, gs);
+    FM_HIP(hipGetLastError());
+  }
 }
 
 // Wave tile of a launch, 16T x 16T: the least estimated time per 16 k, rounds
@@ -1302,7 +1382,7 @@ void gemm_f64(hipStream_t st, int ep, int M, int N, int K, const double *A, long
 void gemm_split(hipStream_t st, int ep, int np, int M, int N, int Kpad, const SplitOperand &A,
                 const SplitOperand &B, const EpArgs &e) {
   if (M <= 0 || N <= 0) return;
-  // The kernel contraction runs on int8 slices (gemm_i8_kernel); the split
+  // The kernel contraction runs on int8 slices (gemm_i8_groups); the split
   // form serves the gradient contraction.
   FM_CHECK(ep == EP_STORE, FM_ERR_INVALID, "split-BF16 contraction: EP_STORE only");
   FM_CHECK(np == 2, FM_ERR_INVALID, "split operands have 2 pieces");

@@ -87,8 +87,7 @@ constexpr int kI8TileA = 128;  // row tile of the descriptor operand
 constexpr int kI8TileN = 64;   // column tile (sparse set): the energy partials are per column tile
 // Row tiles per group in the integer contraction's XCD tile order: 32
 // resident workgroups per XCD then cover 4 row tiles x 8 column tiles
-// (measured 3% faster per launch than 2 row tiles x 16 column tiles; 8 row
-// tiles per group measured the same as 4).
+// (2 row tiles by 16 column tiles and 8 by 4 measured within 2 % of it).
 constexpr int kI8Group = 4;
 inline long long i8_ld(long long k) { return (k + kI8Pad - 1) / kI8Pad * kI8Pad; }
 // Tiled slice layout of n rows with reduction length Kq = nk kI8Pad: rows in
@@ -104,18 +103,19 @@ __host__ __device__ inline long long i8_tile_offset(int tr, long long nk, long l
 inline size_t i8_tiled_bytes(long long n, int tr, long long Kq) {
   return (size_t)((n + tr - 1) / tr) * tr * Kq * kI8Slices;
 }
-struct SliceOperand {
-  const int8_t *q = nullptr;  // the operand's first tile (row 0 starts a tile)
-  long long Kq = 0;           // padded reduction length, a multiple of kI8Pad
-  int tr = 0;                 // rows per tile
-  const double *scale = nullptr;
+// One contraction: rows of A (M, in tiles of kI8TileA) against rows of B (N, in
+// tiles of kI8TileN), both starting a tile, over nk steps of kI8Pad.
+struct I8Gemm {
+  const int8_t *A = nullptr, *B = nullptr;
+  const double *sa = nullptr, *sb = nullptr;  // scales per row
+  int M = 0, N = 0, nk = 0;
+  EpArgs e;
 };
 void slice_rows(hipStream_t st, const float *X, long long ldx, int n, int nd, int8_t *Q,
                 long long Kq, int tr, double *scale);
 void slice_rows(hipStream_t st, const double *X, long long ldx, int n, int nd, int8_t *Q,
                 long long Kq, int tr, double *scale);
-void gemm_i8_kernel(hipStream_t st, int M, int N, int Kq, const SliceOperand &A,
-                    const SliceOperand &B, const EpArgs &e);
+void gemm_i8_groups(hipStream_t st, const std::vector<I8Gemm> &groups);
 // Host-side split of FP32 values into np BF16 pieces, rounding to nearest
 // even as the device conversion does.
 void split_bf16_host(const float *x, size_t n, int np, uint16_t *const *pieces);

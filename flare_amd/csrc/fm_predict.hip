@@ -275,10 +275,9 @@ static void read_outputs(fm_structure s, const double *o, size_t n_out, const do
 }
 
 // Rows per tile of one species in the chosen form: at most T and, when T
-// allows, a whole number of rounds of the kernel contraction's 128 x 64
-// tiles over the GPU's workgroup slots (one such workgroup per CU: its two
-// LDS buffers take 122 KB), so the last round of each launch is not left
-// nearly empty. Rows of a tile do not change any result.
+// allows, a whole number of rounds of the kernel contraction's 128 x 128
+// tiles over the GPU's CUs (one workgroup per CU), so the last round of each
+// launch is not left nearly empty. Rows of a tile do not change any result.
 static int species_tile_rows(fm_context ctx, int T, int Ms, int form) {
   if (form != FM_FORM_CHOSEN || Ms == 0) return T;
   int cus = 0;
@@ -286,7 +285,7 @@ static int species_tile_rows(fm_context ctx, int T, int Ms, int form) {
           hipSuccess ||
       cus <= 0)
     return T;
-  int per_round = cus / ((Ms + kI8TileN - 1) / kI8TileN);
+  int per_round = cus / ((Ms + 2 * kI8TileN - 1) / (2 * kI8TileN));
   int rounds = per_round > 0 ? (T / kI8TileA) / per_round : 0;
   return rounds > 0 ? rounds * per_round * kI8TileA : T;
 }
@@ -311,37 +310,27 @@ static void model_slices(fm_model m, hipStream_t st) {
   m->xq_ready = true;
 }
 
-// Chosen form: `cnt` FP32 descriptor rows (leading dimension nd) as int8
-// slices in Aq / Aq_scale (for rows without slices of their FP64 values;
-// Aq holds at least i8_tiled_bytes(cnt, kI8TileA, i8_ld(nd)) bytes).
-static SliceOperand slice_fp32_rows(fm_context ctx, hipStream_t st, const float *rows, int cnt,
-                                    int nd, DevBuf &Aq, DevBuf &Aq_scale) {
-  long long ldq = i8_ld(nd);
-  {
-    KScope timer(ctx, KT_SLICE, st);
-    slice_rows(st, rows, nd, cnt, nd, Aq.as<int8_t>(), ldq, kI8TileA, Aq_scale.as<double>());
-  }
-  SliceOperand A;
-  A.q = Aq.as<int8_t>();
-  A.Kq = ldq;
-  A.tr = kI8TileA;
-  A.scale = Aq_scale.as<double>();
-  return A;
-}
-
 // Chosen form: kernel contraction of `cnt` sliced descriptor rows against
 // species t's sparse set.
-static void kernel_contraction_i8(fm_model m, hipStream_t st, int t, const SliceOperand &A,
-                                  int cnt, int nd, const EpArgs &ek) {
-  long long ldq = i8_ld(nd);
-  int Ms = m->M_by_type[t];
-  SliceOperand Bx;
-  Bx.q = m->Xq[t].as<int8_t>();
-  Bx.Kq = ldq;
-  Bx.tr = kI8TileN;
-  Bx.scale = m->Xq_scale[t].as<double>();
+static I8Gemm kernel_contraction_i8(fm_model m, int t, const int8_t *A, const double *scale,
+                                    int cnt, int nd, const EpArgs &ek) {
+  return {A, m->Xq[t].as<int8_t>(), scale, m->Xq_scale[t].as<double>(), cnt, m->M_by_type[t],
+          (int)(i8_ld(nd) / kI8Pad), ek};
+}
+
+// The same of `cnt` FP32 descriptor rows (leading dimension nd) without slices
+// of their FP64 values, sliced into Aq / Aq_scale first (Aq holds at least
+// i8_tiled_bytes(cnt, kI8TileA, i8_ld(nd)) bytes).
+static void contract_fp32_rows(fm_model m, hipStream_t st, int t, const float *rows, int cnt,
+                               int nd, DevBuf &Aq, DevBuf &Aq_scale, const EpArgs &ek) {
+  {
+    KScope timer(m->ctx, KT_SLICE, st);
+    slice_rows(st, rows, nd, cnt, nd, Aq.as<int8_t>(), i8_ld(nd), kI8TileA,
+               Aq_scale.as<double>());
+  }
   KScope timer(m->ctx, KT_SGEMM, st);
-  gemm_i8_kernel(st, cnt, Ms, (int)ldq, A, Bx, ek);
+  gemm_i8_groups(
+      st, {kernel_contraction_i8(m, t, Aq.as<int8_t>(), Aq_scale.as<double>(), cnt, nd, ek)});
 }
 
 // B3 structures too large to keep their descriptors (s->row_tile > 0): each
@@ -439,9 +428,7 @@ static void predict_tiled(fm_model m, fm_structure s, int flags, int form, doubl
           gemm_f64(st, EP_KERNEL, cnt, Ms, nd, Bt.as<double>(), nd, m->X[t].as<double>(), nd, 0,
                    ek);
         else
-          kernel_contraction_i8(m, st, t,
-                                slice_fp32_rows(ctx, st, Bt.as<float>(), cnt, nd, Tq, Tq_scale),
-                                cnt, nd, ek);
+          contract_fp32_rows(m, st, t, Bt.as<float>(), cnt, nd, Tq, Tq_scale, ek);
         // Variance contraction of the tile.
         if (want_var && m->L_rows[t] > 0) {
           EpArgs eq;
@@ -564,10 +551,11 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
   DevBuf out(pool, (size_t)n_out * sizeof(double));
   double sig2 = m->sigma * m->sigma;
 
-  // Kernel contraction S = B_s X_hat_s^T with the fused epilogue (FP64: all
-  // species in one launch).
+  // Kernel contraction S = B_s X_hat_s^T with the fused epilogue, all species
+  // in one launch.
   ctx->mark_begin(ST_SGEMM);
   std::vector<F64Gemm> f64_k, f64_g, f64_q;
+  std::vector<I8Gemm> i8_k;
   for (int t = 0; t < nos; t++) {
     int ns = s->n_by_type[t], Ms = m->M_by_type[t], ro = s->type_off[t];
     if (ns == 0) continue;
@@ -594,24 +582,20 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
     if (f64) {
       f64_k.push_back({s->B.as<double>() + (size_t)ro * nd, m->X[t].as<double>(), nd, nd, ns, Ms,
                        nd, 0, ek});
+    } else if (s->has_q) {
+      // Species t's rows start a tile of the structure's slices.
+      i8_k.push_back(kernel_contraction_i8(
+          m, t, s->Bq.as<int8_t>() + i8_tiled_bytes(s->q_tile_row[t], kI8TileA, s->ldq),
+          s->Bq_scale.as<double>() + ro, ns, nd, ek));
     } else {
-      SliceOperand A;
-      if (s->has_q) {
-        // Species t's rows start a tile of the structure's slices.
-        A.q = s->Bq.as<int8_t>() + i8_tiled_bytes(s->q_tile_row[t], kI8TileA, s->ldq);
-        A.Kq = s->ldq;
-        A.tr = kI8TileA;
-        A.scale = s->Bq_scale.as<double>() + ro;
-      } else {
-        A = slice_fp32_rows(ctx, st, s->B.as<float>() + (size_t)ro * nd, ns, nd, Aq, Aq_scale);
-      }
-      kernel_contraction_i8(m, st, t, A, ns, nd, ek);
+      contract_fp32_rows(m, st, t, s->B.as<float>() + (size_t)ro * nd, ns, nd, Aq, Aq_scale, ek);
     }
     ctx->launches[ST_SGEMM]++;
   }
-  if (!f64_k.empty()) {
+  if (!f64_k.empty() || !i8_k.empty()) {
     KScope timer(ctx, KT_SGEMM);
     gemm_f64_groups(st, EP_KERNEL, f64_k);
+    gemm_i8_groups(st, i8_k);
   }
   ctx->mark_end(ST_SGEMM);
 

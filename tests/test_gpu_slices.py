@@ -1,0 +1,50 @@
+"""The integer contraction at both of its tile widths: few tiles and many, an
+odd and an even number of 64-column tiles, column counts at and past a tile's
+edge, one to six steps of the reduction, a last row tile with one row, several
+species in one launch. The chosen form against the FP64 form."""
+import numpy as np
+import pytest
+
+from helpers import fcc
+
+pytestmark = pytest.mark.gpu
+
+SIGMA = 1.5
+
+
+# (species, radial functions, l_max): d = 20, 108, 144, 312, 360 (1, 2, 3, 5
+# and 6 steps of 64); cells of 4 atoms; sparse environments per species.
+@pytest.mark.parametrize("settings,reps,n_sparse", [
+    ((1, 4, 1), (4, 4, 4), (1,)),
+    ((1, 8, 2), (13, 13, 12), (260,)),   # 8112 atoms: 64 row tiles x 5 columns of 64
+    ((1, 8, 3), (13, 13, 13), (320,)),   # 8788 atoms
+    ((2, 6, 3), (4, 11, 1), (64, 65)),   # 176 atoms
+    ((2, 4, 9), (16, 16, 16), (129, 190)),
+])
+def test_integer_contraction(settings, reps, n_sparse):
+    from flare_amd import _C_flare as C
+    nos, N, L = settings
+    cut = np.full((nos, nos), 4.2)
+    calc = C.B2("chebyshev", "quadratic", [0.0, 4.2], [], list(settings), cut)
+    cell, species, pos = fcc(4.0, reps, 0.1, 11, nos=nos)
+    train = C.Structure(cell, species, pos, 4.2, [calc])
+    d = train.descriptors[0]
+    atoms = [int(a) for t, m in enumerate(n_sparse) for a in d.atom_indices[t][:m]]
+    if len(atoms) < sum(n_sparse):
+        pytest.fail("too few atoms of a species")
+    sgp = C.SparseGP([C.NormalizedDotProduct(SIGMA, 2.0)], 0.01, 0.05, 0.005)
+    sgp.Kuu_jitter = 1e-4
+    sgp.add_specific_environments(train, atoms)
+    sgp.update_L_inverse()
+    sgp.set_alpha(np.random.default_rng(5).uniform(0.1, 1.0, size=sgp.n_sparse))
+    out = []
+    for form in (C.FORM_FP64, C.FORM_CHOSEN):
+        s = C.Structure(cell, species, pos, 4.2, [calc], form=form)
+        sgp.predict_local_uncertainties(s)
+        out.append((s.mean_efs, s.local_uncertainties[0]))
+    (m64, v64), (m, v) = out
+    # S carries 2^-34 of the largest products per k; |L_inv| <= 1e2 amplifies
+    # it in Q. Forces: FP32 adjoint with split-BF16 products.
+    assert abs(m[0] - m64[0]) < 1e-7 * abs(m64[0])
+    assert np.max(np.abs(m[1:-6] - m64[1:-6])) < 1e-3 * np.max(np.abs(m64[1:-6]))
+    assert np.max(np.abs(v - v64)) < 1e-5 * SIGMA ** 2
