@@ -869,10 +869,6 @@ void b3_order_model(fm_model m, fm_structure s) {
     if (Ms == 0) continue;
     permute_cols<double>(st, m->X[sp], pool, Ms, nd, nd, t.n_tri, t.n_ls, 1);
     permute_rows<double>(st, m->XT[sp], pool, nd, Ms, t.n_tri, t.n_ls, 1);
-    permute_cols<uint16_t>(st, m->Xs0[sp], pool, Ms, split_ld(nd), nd, t.n_tri, t.n_ls, 1);
-    permute_cols<uint16_t>(st, m->Xs1[sp], pool, Ms, split_ld(nd), nd, t.n_tri, t.n_ls, 1);
-    permute_rows<uint16_t>(st, m->XTs0[sp], pool, nd, split_ld(Ms), t.n_tri, t.n_ls, 1);
-    permute_rows<uint16_t>(st, m->XTs1[sp], pool, nd, split_ld(Ms), t.n_tri, t.n_ls, 1);
   }
   FM_HIP(hipStreamSynchronize(st));
   m->b3_ntri = t.n_tri;

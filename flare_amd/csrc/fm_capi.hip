@@ -713,8 +713,6 @@ int fm_model_create(fm_context ctx, const fm_model_desc *d, fm_model *out) {
     for (int t = 0; t < m->nos; t++) {
       int Ms = m->M_by_type[t], c0 = m->off[t];
       std::vector<double> X((size_t)Ms * nd, 0.0), XT((size_t)nd * Ms, 0.0), a(Ms, 0.0);
-      size_t ldd = fm::split_ld(nd), ldm = fm::split_ld(Ms);
-      std::vector<float> X32((size_t)Ms * ldd, 0.0f), XT32((size_t)nd * ldm, 0.0f);
       for (int j = 0; j < Ms; j++) {
         double nrm = d->sparse_norms[c0 + j];
         // Empty sparse environments contribute nothing
@@ -727,35 +725,16 @@ int fm_model_create(fm_context ctx, const fm_model_desc *d, fm_model *out) {
         }
         a[j] = d->alpha[c0 + j];
       }
-      for (int j = 0; j < Ms; j++)
-        for (int k = 0; k < nd; k++) X32[j * ldd + k] = (float)X[(size_t)j * nd + k];
-      for (int k = 0; k < nd; k++)
-        for (int j = 0; j < Ms; j++) XT32[k * ldm + j] = (float)XT[(size_t)k * Ms + j];
-      std::vector<uint16_t> xs[2], xts[2];
-      for (auto &v : xs) v.resize(X32.size());
-      for (auto &v : xts) v.resize(XT32.size());
-      uint16_t *xsp[2] = {xs[0].data(), xs[1].data()};
-      uint16_t *xtsp[2] = {xts[0].data(), xts[1].data()};
-      fm::split_bf16_host(X32.data(), X32.size(), 2, xsp);
-      fm::split_bf16_host(XT32.data(), XT32.size(), 2, xtsp);
       auto up = [&](fm::DevBuf &buf, const void *src, size_t bytes) {
         buf.alloc(pool, std::max<size_t>(1, bytes));
         if (bytes) FM_HIP(hipMemcpyAsync(buf.as<void>(), src, bytes, hipMemcpyHostToDevice, st));
       };
       m->X.emplace_back();
       m->XT.emplace_back();
-      m->Xs0.emplace_back();
-      m->Xs1.emplace_back();
-      m->XTs0.emplace_back();
-      m->XTs1.emplace_back();
       m->alpha.emplace_back();
       m->L.emplace_back();
       up(m->X.back(), X.data(), X.size() * sizeof(double));
       up(m->XT.back(), XT.data(), XT.size() * sizeof(double));
-      up(m->Xs0.back(), xs[0].data(), xs[0].size() * sizeof(uint16_t));
-      up(m->Xs1.back(), xs[1].data(), xs[1].size() * sizeof(uint16_t));
-      up(m->XTs0.back(), xts[0].data(), xts[0].size() * sizeof(uint16_t));
-      up(m->XTs1.back(), xts[1].data(), xts[1].size() * sizeof(uint16_t));
       up(m->alpha.back(), a.data(), a.size() * sizeof(double));
       int rows = 0, lower = 1;
       if (m->has_L && Ms > 0) {

@@ -27,9 +27,6 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
-#include <map>
-#include <mutex>
-#include <tuple>
 
 #include "fm_device.hpp"
 #include "fm_gemm.hpp"
@@ -41,21 +38,9 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
-// ---------------------------------------------------------------------------
-// Epilogues. Lane l holds column l % 16 of each 16 x 16 output tile; the
-// row of its value i (i < 4) is 4 (l / 16) + i for the FP32-output MFMAs and
-// l / 16 + 4 i for v_mfma_f64_16x16x4f64.
-// ---------------------------------------------------------------------------
-template <typename Acc, int TM, int TN>
-struct TileOut {
-  Acc v[TM][TN][4];
-};
-
-// Output tile of this workgroup. Workgroups are dealt to the 8 XCDs round
-// robin (id % 8); the dispatch id is remapped so each XCD gets a contiguous
-// run of logical tiles. With column index fastest (the default) the
-// workgroups sharing a row tile of A share that XCD's L2; with row index
-// fastest those sharing a column tile of B do.
+// Workgroups are dealt to the 8 XCDs round robin (id % 8); the id is remapped so
+// that each XCD gets a contiguous run of logical ones, whose operands share its
+// L2.
 __device__ __forceinline__ int xcd_id() {
   constexpr int kXcd = 8;
   int ntx = gridDim.x, nty = gridDim.y, nblk = ntx * nty;
@@ -66,23 +51,6 @@ __device__ __forceinline__ int xcd_id() {
   return xcd < tall ? xcd * per + local : tall * per + (xcd - tall) * (per - 1) + local;
 }
 
-__device__ __forceinline__ void xcd_tile(int &tx, int &ty, bool rows_fastest = false) {
-  int ntx = gridDim.x, nty = gridDim.y;
-  int id = xcd_id();
-  if (rows_fastest) {
-    ty = id % nty;
-    tx = id / nty;
-  } else {
-    tx = id % ntx;
-    ty = id / ntx;
-  }
-}
-
-template <typename Acc>
-__device__ __forceinline__ int tile_row(int lane, int i) {
-  return sizeof(Acc) == 8 ? (lane >> 4) + 4 * i : 4 * (lane >> 4) + i;
-}
-
 // Kept out of line: inlined into every element of an unrolled epilogue, pow
 // makes the loops too large to unroll.
 __device__ __noinline__ double pow_general(double x, double p) { return pow(x, p); }
@@ -90,23 +58,6 @@ __device__ __forceinline__ double fpow(double x, double p, int pi) {
   if (pi == 2) return x * x;
   if (pi == 1) return x;
   return pow_general(x, p);
-}
-
-template <typename Acc, typename TW, int TM, int TN>
-__device__ __forceinline__ void ep_store(const EpArgs &e, const TileOut<Acc, TM, TN> &t, int row0, int col0,
-                         int M, int N, int lane, int wr, int wc) {
-#pragma unroll
-  for (int ti = 0; ti < TM; ti++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      int r = row0 + wr * 16 * TM + ti * 16 + tile_row<Acc>(lane, i);
-      if (r >= M) continue;
-#pragma unroll
-      for (int tj = 0; tj < TN; tj++) {
-        int c = col0 + wc * 16 * TN + tj * 16 + (lane & 15);
-        if (c < N) e.W_as<TW>()[(size_t)r * e.ldw + c] = (TW)t.v[ti][tj][i];
-      }
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -625,149 +576,210 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f64_lds(F64Groups gs) {
 }
 
 // ---------------------------------------------------------------------------
-// Split-BF16 x3 GEMM (chosen form), (32 TM) x (32 TN) tiles, on operands stored as
-// two BF16 pieces of FP32 values (x = x_0 + x_1, split once where the operand
-// is produced: the sparse set at model upload, descriptors in the descriptor
-// kernel, w in the kernel-contraction epilogue). The products x_1 y_0,
-// x_0 y_1 and x_0 y_0 are summed in that order (smallest first). Threads copy
-// 16-byte vectors of consecutive k into k-contiguous LDS rows (SplitLoader);
-// lane l then reads 8 consecutive k at row l % 16, k offset 8 (l / 16).
+// Shared by the two contractions of the chosen form, whose operands are laid
+// out in pieces that a wave copies straight to LDS (1 KB: 16 rows of 64 bytes).
 // ---------------------------------------------------------------------------
-// Base shape of the split contraction (partials follow it).
-constexpr int B16_TM = 4, B16_TN = 4, B16_BM = 32 * B16_TM, B16_BN = 32 * B16_TN;
-constexpr int BK16 = 32;
-constexpr int PADB = 8;
-constexpr int LDK = BK16 + PADB;
-static_assert(BK16 == kSplitPad, "k-step equals the operand padding");
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) const void gvoid;
+typedef __attribute__((address_space(3))) void lvoid;
 
-struct SplitPtrs {
-  const __bf16 *p[3];
+// 16-byte chunk position of k chunk c (0..3) in row r of an LDS slice block
+// (rows of 64 bytes, no padding): an XOR swizzle that keeps the fragment
+// reads (16 rows at four chunks) free of bank conflicts (a third of the LDS
+// cycles were conflicts with r / 2 xor r / 8 in its place).
+__device__ __forceinline__ int i8_chunk(int r, int c) { return c ^ (-(r >> 2) & 3); }
+
+// This lane's 16 bytes of a piece: they land at 16 lane, so it fetches the chunk
+// that belongs there.
+__device__ __forceinline__ unsigned piece_lane(int lane) {
+  return (lane >> 2) * 64 + 16 * i8_chunk(lane >> 2, lane & 3);
+}
+// Wave-uniform base `src`, kept in scalar registers so that one vector register
+// addresses every piece.
+__device__ __forceinline__ void copy_piece(const void *src, unsigned vsrc, void *dst) {
+  asm volatile("" : "+s"(src));
+  __builtin_amdgcn_global_load_lds((gvoid *)((const char *)src + vsrc), (lvoid *)dst, 16, 0, 0);
+}
+// Waits for this wave's copies, then for the other waves.
+__device__ __forceinline__ void copies_landed() {
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+  __syncthreads();
+}
+
+// This workgroup's tile of a launch over several contractions (first tiles
+// `first`): every XCD takes a contiguous run of the tiles, kI8Group row tiles at
+// a time, row index fastest: the workgroups that it holds at once cover
+// kI8Group row tiles by a few column tiles, which share its L2.
+template <typename Groups>
+__device__ __forceinline__ int group_tile(const Groups &gs, int bm, int bn, int &tx, int &ty) {
+  int id = xcd_id(), gi = 0;
+  while (gi + 1 < gs.n && id >= gs.first[gi + 1]) gi++;
+  id -= gs.first[gi];
+  int ntx = (gs.g[gi].N + bn - 1) / bn, nty = (gs.g[gi].M + bm - 1) / bm;
+  int f = id / (kI8Group * ntx) * kI8Group, n_in = min(kI8Group, nty - f);
+  tx = id % (kI8Group * ntx) / n_in;
+  ty = f + id % (kI8Group * ntx) % n_in;
+  return gi;
+}
+
+// ---------------------------------------------------------------------------
+// Split-BF16 x3 GEMM (chosen form) on operands stored as two BF16 pieces of FP32
+// values (x = x_0 + x_1, split once where the operand is produced: the sparse
+// set on first use, w in the kernel contraction's epilogue), in the tiled split
+// layout. The products x_1 y_0, x_0 y_1 and x_0 y_0 of 32 k are summed in that
+// order (smallest first), then those of the next 32.
+// ---------------------------------------------------------------------------
+
+// X (n rows of K FP64 values) as BF16 pieces of their FP32 values, zeros in the
+// padding. One thread per 8 k of a row.
+__global__ __launch_bounds__(256) void k_split_rows(const double *X, long long ldx, int n, int K,
+                                                    long long nk, uint16_t *hi, uint16_t *lo) {
+  long long i = blockIdx.x * 256ll + threadIdx.x;  // chunk of the layout
+  long long blocks = (n + kSplitRows - 1) / kSplitRows * nk;
+  if (i >= blocks * 64) return;
+  long long row = i / 64 / nk * kSplitRows + (i & 63) / 4, k0 = i / 64 % nk * kSplitPad + (i & 3) * 8;
+  v8bf h, l;
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    float x = row < n && k0 + j < K ? (float)X[row * ldx + k0 + j] : 0.0f;
+    h[j] = (__bf16)x;
+    l[j] = (__bf16)(x - (float)h[j]);
+  }
+  *reinterpret_cast<v8bf *>(hi + 8 * i) = h;
+  *reinterpret_cast<v8bf *>(lo + 8 * i) = l;
+}
+
+constexpr int kSplitGroups = 8;
+struct SplitGroups {
+  SplitGemm g[kSplitGroups];
+  int first[kSplitGroups], n;
 };
 
-// Loader of one operand's rows [row0, row0 + BR) x 32 k, NP pieces: with
-// TPR = 256 / BR threads per row, thread tid takes row tid / TPR and
-// 32 / TPR consecutive k (one or two 16-byte vectors). Rows past `rows` read
-// row 0 (in bounds) and load zeros.
-template <int NP, int BR>
-struct SplitLoader {
-  static constexpr int TPR = 256 / BR, VPT = 4 / TPR;
-  int lr, lk;
-  bool valid;
-  size_t off;
-  v8bf r[NP][VPT];
-  __device__ __forceinline__ SplitLoader(int tid, int row0, int rows, long long ld) {
-    lr = tid / TPR;
-    lk = (tid % TPR) * 8 * VPT;
-    valid = row0 + lr < rows;
-    off = (size_t)(valid ? row0 + lr : 0) * ld + lk;
-  }
-  __device__ __forceinline__ void load(const SplitPtrs &g, int k0) {
-    const v8bf zero = {};
-    int q = k0 / 8;
-#pragma unroll
-    for (int pc = 0; pc < NP; pc++) {
-      const v8bf *p = reinterpret_cast<const v8bf *>(g.p[pc] + off);
-#pragma unroll
-      for (int v = 0; v < VPT; v++) r[pc][v] = valid ? p[q + v] : zero;
-    }
-  }
-  __device__ __forceinline__ void store(__bf16 (*lds)[BR * LDK]) const {
-#pragma unroll
-    for (int pc = 0; pc < NP; pc++)
-#pragma unroll
-      for (int v = 0; v < VPT; v++)
-        *reinterpret_cast<v8bf *>(&lds[pc][lr * LDK + lk + 8 * v]) = r[pc][v];
-  }
-};
-
-// With DB the LDS tiles are double-buffered: the next k-step's tile is
-// stored while the current one feeds the MFMAs, one barrier per k-step (the
-// products and their order are the same, so results are too). It pays on
-// long k (one workgroup of 82 KB per CU, against three single-buffered).
-template <int EP, int NP, int TM, int TN, bool DB>
-__global__ __launch_bounds__(256) void k_gemm_split(int M, int N, int Kpad, SplitPtrs Ag,
-                                                    long long lda, SplitPtrs Bg, long long ldb,
-                                                    EpArgs e) {
-  constexpr int BM = 32 * TM, BN = 32 * TN, NB = DB ? 2 : 1;
-  __shared__ __align__(16) __bf16 As[NB][NP][BM * LDK];
-  __shared__ __align__(16) __bf16 Bs[NB][NP][BN * LDK];
-  __shared__ double red[2 * (BM > BN ? BM : BN)];
-  int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  int wr = wid >> 1, wc = wid & 1;
-  int tx, ty;
-  xcd_tile(tx, ty);
+// Tiles of 16 RA WR x 16 RB WC, WR x WC waves of RA x RB blocks of
+// v_mfma_f32_16x16x32_bf16. One step of 32 k of either operand is copied to one of
+// two LDS buffers a step ahead; between the products the fragments of the next
+// row block, and in a step's last one those of the next step, are read.
+//
+// Bound by power like the integer contraction, so by the bytes moved per
+// product. Three groups of 87,381 x 3,255 x 1,365: 5.4 ms, 1.29 PFLOP/s of
+// products (8.0 ms before, from row-major operands through registers with all
+// waves reading LDS or multiplying at the same time, on tiles of which the first
+// call of a shape timed seven).
+template <int RA, int RB, int WR, int WC>
+__global__ __launch_bounds__(64 * WR * WC, 2) void k_gemm_split(SplitGroups gs) {
+  constexpr int NW = WR * WC, BM = 16 * RA * WR, BN = 16 * RB * WC;
+  constexpr int A_PC = BM * 64, B_PC = BN * 64;  // bytes of one piece of a step
+  constexpr int A_ST = 2 * A_PC, B_ST = 2 * B_PC;
+  constexpr int NA = A_ST / 1024 / NW, NB = B_ST / 1024 / NW;  // copies per wave
+  static_assert(NA % 2 == 0 && NB % 2 == 0 && NA + NB <= 3 * RB && 2 * RB + 2 <= 3 * RB, "split");
+  __shared__ __align__(16) int8_t buf0[A_ST + B_ST], buf1[A_ST + B_ST];
+  int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int wr = wid / WC, wc = wid % WC, tx, ty;
+  const SplitGemm &g = gs.g[group_tile(gs, BM, BN, tx, ty)];
+  const int M = g.M, N = g.N, nk = g.nk;
   int row0 = ty * BM, col0 = tx * BN;
-  v4f acc[TM][TN];
+  v4f acc[RA][RB];
 #pragma unroll
-  for (int a = 0; a < TM; a++)
+  for (int a = 0; a < RA; a++)
 #pragma unroll
-    for (int b = 0; b < TN; b++) acc[a][b] = v4f{0, 0, 0, 0};
-  SplitLoader<NP, BM> la(tid, row0, M, lda);
-  SplitLoader<NP, BN> lb(tid, col0, N, ldb);
-  la.load(Ag, 0);
-  lb.load(Bg, 0);
-  if (DB) {
-    la.store(As[0]);
-    lb.store(Bs[0]);
-    __syncthreads();
+    for (int b = 0; b < RB; b++) acc[a][b] = v4f{0, 0, 0, 0};
+  // Wave w copies both pieces of the blocks w NA / 2 .. of A and w NB / 2 .. of
+  // B (past the last block of an operand that one again).
+  unsigned vsrc = piece_lane(lane);
+  const char *src0[NA + NB];
+#pragma unroll
+  for (int i = 0; i < NA + NB; i++) {
+    int j = i < NA ? i : i - NA, blk = wid * ((i < NA ? NA : NB) / 2) + (j >> 1);
+    int at = min((i < NA ? row0 : col0) / 16 + blk, ((i < NA ? M : N) + 15) / 16 - 1);
+    src0[i] = reinterpret_cast<const char *>((i < NA ? g.A : g.B)[j & 1]) + (size_t)at * nk * 1024;
   }
-  int cur = 0;
-  for (int k0 = 0; k0 < Kpad; k0 += BK16) {
-    if (!DB) {
-      __syncthreads();
-      la.store(As[0]);
-      lb.store(Bs[0]);
-      __syncthreads();
-    }
-    bool more = k0 + BK16 < Kpad;
-    if (more) {
-      la.load(Ag, k0 + BK16);
-      lb.load(Bg, k0 + BK16);
-    }
-    v8bf af[NP][TM], bf[NP][TN];
-    int kk = 8 * (lane >> 4);
+  auto copy = [&](int8_t *dst, int ks, int i) {
+    if (i >= NA + NB) return;
+    int j = i < NA ? i : i - NA, blk = wid * ((i < NA ? NA : NB) / 2) + (j >> 1);
+    copy_piece(src0[i] + (size_t)ks * 1024, vsrc,
+               dst + (i < NA ? 0 : A_ST) + (j & 1) * (i < NA ? A_PC : B_PC) + blk * 1024);
+  };
+  v8bf fa[2][2], fb[2][RB][2];  // A of two blocks in turn, B of two steps in turn
+  int r16 = lane & 15, frag = r16 * 64 + 16 * i8_chunk(r16, lane >> 4);
+  int oa = wr * RA * 1024 + frag, ob = A_ST + wc * RB * 1024 + frag;
+  auto read_a = [&](const int8_t *src, int r, int pc) {
+    fa[r & 1][pc] = *reinterpret_cast<const v8bf *>(&src[pc * A_PC + r * 1024 + oa]);
+  };
+  auto read_b = [&](const int8_t *src, int set, int i) {
+    fb[set][i >> 1][i & 1] =
+        *reinterpret_cast<const v8bf *>(&src[(i & 1) * B_PC + (i >> 1) * 1024 + ob]);
+  };
+  // The products of row block r; other(i) issues reads and copies between them.
+  auto products = [&](int r, int set, auto other) {
 #pragma unroll
-    for (int pc = 0; pc < NP; pc++) {
+    for (int p = 0; p < 3; p++)
 #pragma unroll
-      for (int t = 0; t < TM; t++) {
-        int ar = wr * 16 * TM + t * 16 + (lane & 15);
-        af[pc][t] = *reinterpret_cast<const v8bf *>(&As[cur][pc][ar * LDK + kk]);
+      for (int h = 0; h < RB; h++) {
+        acc[r][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            fa[r & 1][p == 0 ? 1 : 0], fb[set][h][p == 1 ? 1 : 0], acc[r][h], 0, 0, 0);
+        other(p * RB + h);
+        __builtin_amdgcn_sched_barrier(0);
       }
+  };
+  auto body = [&](const int8_t *__restrict__ src, int set) {
 #pragma unroll
-      for (int t = 0; t < TN; t++) {
-        int br = wc * 16 * TN + t * 16 + (lane & 15);
-        bf[pc][t] = *reinterpret_cast<const v8bf *>(&Bs[cur][pc][br * LDK + kk]);
-      }
-    }
-    // Products of piece orders i + j <= NP - 1, smallest terms first.
-    auto prod = [&](const v8bf (&x)[TM], const v8bf (&y)[TN]) {
+    for (int a = 0; a < RA; a++)
 #pragma unroll
-      for (int a = 0; a < TM; a++)
+      for (int b = 0; b < RB; b++) asm volatile("" : "+v"(acc[a][b]));
 #pragma unroll
-        for (int b = 0; b < TN; b++)
-          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[a], y[b], acc[a][b], 0, 0, 0);
-    };
-    static_assert(NP == 2, "two pieces: products lo.hi, hi.lo, hi.hi");
-    prod(af[1], bf[0]);
-    prod(af[0], bf[1]);
-    prod(af[0], bf[0]);
-    if (DB) {
-      if (more) {
-        la.store(As[cur ^ 1]);
-        lb.store(Bs[cur ^ 1]);
-      }
-      __syncthreads();
-      cur ^= 1;
-    }
+    for (int r = 0; r < RA - 1; r++)
+      products(r, set, [&](int i) {
+        if (i < 2) read_a(src, r + 1, 1 - i);
+      });
+  };
+  // The step's last row block: after the barrier, so the next step is in
+  // `next` and this one's buffer takes step ks.
+  auto tail = [&](const int8_t *__restrict__ next, int8_t *__restrict__ dst, int ks, int set) {
+    products(RA - 1, set, [&](int i) {
+      if (i == 0) read_a(next, 0, 1);
+      else if (i == 1) read_a(next, 0, 0);
+      else if (i < 2 + 2 * RB) read_b(next, set ^ 1, i - 2);
+      copy(dst, ks, i);
+    });
+  };
+#pragma unroll
+  for (int i = 0; i < NA + NB; i++) copy(buf0, 0, i);
+#pragma unroll
+  for (int i = 0; i < NA + NB; i++) copy(buf1, min(1, nk - 1), i);
+  copies_landed();
+#pragma unroll
+  for (int pc = 0; pc < 2; pc++) read_a(buf0, 0, pc);
+#pragma unroll
+  for (int i = 0; i < 2 * RB; i++) read_b(buf0, 0, i);
+  int ks = 0;
+#pragma unroll 1
+  for (; ks + 2 <= nk; ks += 2) {
+    body(buf0, 0);
+    copies_landed();
+    tail(buf1, buf0, min(ks + 2, nk - 1), 0);
+    body(buf1, 1);
+    copies_landed();
+    tail(buf0, buf1, min(ks + 3, nk - 1), 1);
   }
-  TileOut<float, TM, TN> t;
+  if (ks < nk) {
+    body(buf0, 0);
+    products(RA - 1, 0, [](int) {});
+  }
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // no copy outlives the workgroup
+  float *W = g.e.W_as<float>();
 #pragma unroll
-  for (int a = 0; a < TM; a++)
+  for (int a = 0; a < RA; a++)
 #pragma unroll
-    for (int b = 0; b < TN; b++)
+    for (int i = 0; i < 4; i++) {
+      int r = row0 + (wr * RA + a) * 16 + 4 * (lane >> 4) + i;
+      if (r >= M) continue;
+      float *out = W + (size_t)r * g.e.ldw;
 #pragma unroll
-      for (int i = 0; i < 4; i++) t.v[a][b][i] = acc[a][b][i];
-  ep_store<float, float, TM, TN>(e, t, row0, col0, M, N, lane, wr, wc);
+      for (int b = 0; b < RB; b++) {
+        int c = col0 + (wc * RB + b) * 16 + r16;
+        if (c < N) out[c] = acc[a][b][i];
+      }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -784,8 +796,6 @@ __global__ __launch_bounds__(256) void k_gemm_split(int M, int N, int Kpad, Spli
 // k = sigma^2 S^p that the local variance amplifies by L_inv carry FP64-like
 // accuracy, where FP32 accumulation of BF16 pieces carries about 16 bits.
 // ---------------------------------------------------------------------------
-typedef int v4i __attribute__((ext_vector_type(4)));
-
 // One wave per row: the row maximum, its power-of-two scale and the slices
 // of 4 consecutive values per lane (zeros past nd up to Kq), stored in the
 // tiled slice layout (tr rows per tile).
@@ -830,12 +840,6 @@ __global__ __launch_bounds__(256) void k_slice_rows(const T *X, long long ldx, i
 // 64^2 = 4096: 65536 k keep it below 2^31 (5 x 4096 x 65536 = 1.3e9).
 constexpr int kI8Flush = 65536;
 
-// 16-byte chunk position of k chunk c (0..3) in row r of an LDS slice block
-// (rows of 64 bytes, no padding): an XOR swizzle that keeps the fragment
-// reads (16 rows at four chunks) free of bank conflicts (a third of the LDS
-// cycles were conflicts with r / 2 xor r / 8 in its place).
-__device__ __forceinline__ int i8_chunk(int r, int c) { return c ^ (-(r >> 2) & 3); }
-
 // 128 x 32 RA tiles, 8 waves, each 16 RA x 32 of v_mfma_i32_16x16x64_i8 (lane
 // l: operand row l % 16, bytes k = 16 (l / 16) .. + 15; result column l % 16,
 // rows 4 (l / 16) + i).
@@ -858,13 +862,6 @@ __device__ __forceinline__ int i8_chunk(int r, int c) { return c ^ (-(r >> 2) & 
 // Epilogue as EpKernel, in FP64 from the exact sums: S, k (FP64), w as BF16
 // pairs, energy partials per kI8TileN columns; k, then w, are staged in LDS and
 // stored as whole rows of the tile.
-typedef __attribute__((address_space(1))) const void gvoid;
-typedef __attribute__((address_space(3))) void lvoid;
-
-// One launch's contractions. Every XCD takes a contiguous run of the tiles,
-// kI8Group row tiles at a time, row index fastest: the workgroups that it holds
-// at once cover kI8Group row tiles by 32 / kI8Group column tiles, which share
-// its L2.
 constexpr int kI8Groups = 8;
 struct I8Groups {
   I8Gemm g[kI8Groups];
@@ -879,19 +876,15 @@ __global__ __launch_bounds__(512) void k_gemm_i8(I8Groups gs) {
   constexpr int G_SL = kI8TileN * kI8Pad, G_ST = S * G_SL;  // of B in memory
   constexpr int NB = (B_ST / 1024 + 7) / 8;  // 1 KB pieces of B per wave (A: S)
   static_assert(BM == 128 && kI8TileN == 64 && kI8Pad == 64 && (RA == 2 || RA == 4), "tiling");
-  static_assert(BM * BN * 4 + 8 * BM * WC <= A_ST + B_ST, "epilogue staging fits");
+  static_assert(BM * BN * 4 + 8 * BM * WC <= A_ST + B_ST && BM * (BN + 8) * 2 <= A_ST + B_ST,
+                "epilogue staging fits");
   __shared__ __align__(16) int8_t buf0[A_ST + B_ST], buf1[A_ST + B_ST];
   int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   int wr = wid / WC, wc = wid % WC;
-  int id = xcd_id(), gi = 0;
-  while (gi + 1 < gs.n && id >= gs.first[gi + 1]) gi++;
-  const I8Gemm &g = gs.g[gi];
+  int tx, ty;
+  const I8Gemm &g = gs.g[group_tile(gs, BM, BN, tx, ty)];
   const int M = g.M, N = g.N, nk = g.nk;
   const EpArgs &e = g.e;
-  id -= gs.first[gi];
-  int ntx = (N + BN - 1) / BN, nty = (M + BM - 1) / BM, first = id / (kI8Group * ntx) * kI8Group;
-  int n_in = min(kI8Group, nty - first), tx = id % (kI8Group * ntx) / n_in;
-  int ty = first + id % (kI8Group * ntx) % n_in;
   int row0 = ty * BM, col0 = tx * BN;
   v4i acc[S][RA][2];
   // With LONG (Kq > kI8Flush) the int32 sums of the slice products
@@ -926,10 +919,9 @@ __global__ __launch_bounds__(512) void k_gemm_i8(I8Groups gs) {
   clear();
   // Copies of a step's 1 KB pieces (16 rows of a slice): wave w takes piece w
   // of each slice of A and of B (with 64 columns, which have 4 pieces a slice,
-  // piece w % 4 of slices w / 4, w / 4 + 2 and the last one). A lane's 16 bytes
-  // land at 16 lane; it fetches the chunk that belongs there. A column tile
+  // piece w % 4 of slices w / 4, w / 4 + 2 and the last one). A column tile
   // past the last 64 columns repeats them.
-  unsigned vsrc = (lane >> 2) * 64 + 16 * i8_chunk(lane >> 2, lane & 3);
+  unsigned vsrc = piece_lane(lane);
   int wb = wid % (B_SL / 1024), pb = wid / (B_SL / 1024);
   int tb = min(tx * (BN / kI8TileN) + (wb >> 2), (N - 1) / kI8TileN);
   const int8_t *Aw = g.A + (size_t)ty * nk * A_ST + wid * 1024;
@@ -939,9 +931,8 @@ __global__ __launch_bounds__(512) void k_gemm_i8(I8Groups gs) {
     int p = i < S ? i : RA == 4 ? i - S : min(2 * (i - S) + pb, S - 1);
     const int8_t *src = i < S ? Aw + ((size_t)ks * A_ST + p * A_SL)
                               : Bw + ((size_t)ks * G_ST + p * G_SL);
-    asm volatile("" : "+s"(src));  // a scalar base: one vector register addresses all pieces
     dst += i < S ? p * A_SL + wid * 1024 : A_ST + p * B_SL + wb * 1024;
-    __builtin_amdgcn_global_load_lds((gvoid *)(src + vsrc), (lvoid *)dst, 16, 0, 0);
+    copy_piece(src, vsrc, dst);
   };
   // Fragments: all slices of 16 rows of A and of 32 of B for a whole step.
   v4i fa[S], fb[2][S];
@@ -1000,13 +991,9 @@ __global__ __launch_bounds__(512) void k_gemm_i8(I8Groups gs) {
         RA - 1, h, [&](int i) { if (i % 3 == 1) read_b(src, h ^ 1, i / 3); },
         [&](int rd) { read_a(src, 0, rd); });
   };
-  auto landed = [&]() {
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // this wave's copies
-    __syncthreads();
-  };
 #pragma unroll
   for (int i = 0; i < S + NB; i++) copy(buf0, 0, i);
-  landed();
+  copies_landed();
 #pragma unroll
   for (int p = 0; p < S; p++) {
     read_a(buf0, 0, p);
@@ -1017,11 +1004,11 @@ __global__ __launch_bounds__(512) void k_gemm_i8(I8Groups gs) {
   for (; ks + 2 <= nk; ks += 2) {
     flush(ks);
     body(buf0, buf1, ks + 1, 0);
-    landed();
+    copies_landed();
     tail(buf1, 0);
     flush(ks + 1);
     body(buf1, buf0, min(ks + 2, nk - 1), 1);
-    landed();
+    copies_landed();
     tail(buf0, 1);
   }
   if (ks < nk) {
@@ -1030,10 +1017,10 @@ __global__ __launch_bounds__(512) void k_gemm_i8(I8Groups gs) {
     tail(buf0, 0);
   }
   flush(nk);
-  landed();
+  copies_landed();
   // Epilogue: values in FP64 per element. k is staged in LDS over the operand
   // buffers, w after it.
-  constexpr int HN = BN / 2;  // columns staged in each buffer
+  constexpr int HN = BN / 2, WLD = BN + 8;  // k: columns in each buffer; w: padded rows
   double *Kst = reinterpret_cast<double *>(wc < WC / 2 ? buf0 : buf1);
   double *red = reinterpret_cast<double *>(buf0 + BM * HN * 8);  // [WC][BM]
   uint16_t *Hst = reinterpret_cast<uint16_t *>(buf0), *Lst = reinterpret_cast<uint16_t *>(buf1);
@@ -1109,20 +1096,22 @@ __global__ __launch_bounds__(512) void k_gemm_i8(I8Groups gs) {
     int rr = wr * 16 * RA + 16 * (j >> 3) + 4 * k16 + (j & 3);
     int cc = wc * 32 + 16 * ((j >> 2) & 1) + r16;
     __bf16 hi = (__bf16)wf[j], lo = (__bf16)(wf[j] - (float)hi);
-    Hst[rr * BN + cc] = __builtin_bit_cast(uint16_t, hi);
-    Lst[rr * BN + cc] = __builtin_bit_cast(uint16_t, lo);
+    Hst[rr * WLD + cc] = __builtin_bit_cast(uint16_t, hi);
+    Lst[rr * WLD + cc] = __builtin_bit_cast(uint16_t, lo);
   }
   __syncthreads();
-  // w pieces: 8 columns per 16-byte store; the padding columns [N, ldw) are
-  // zero (the reduction tail of the gradient contraction), none past ldw
-  // (a multiple of 32) is written.
+  // w pieces in the tiled split layout, 8 columns per 16-byte store; the padding
+  // columns [N, ldw) are zero (the reduction tail of the gradient contraction),
+  // none past ldw (a multiple of 32) is written.
   for (int q = tid; q < BM * (BN / 8); q += NT) {
-    int rr = q / (BN / 8), c8 = 8 * (q % (BN / 8)), r = row0 + rr, cg = col0 + c8;
+    int blk = q >> 6, rr = blk / (BN / 32) * 16 + ((q >> 2) & 15);
+    int c8 = blk % (BN / 32) * 32 + 8 * (q & 3), r = row0 + rr, cg = col0 + c8;
     if (r >= M || cg >= e.ldw) continue;
-    *reinterpret_cast<v4i *>(reinterpret_cast<uint16_t *>(e.Wh) + (size_t)r * e.ldw + cg) =
-        *reinterpret_cast<const v4i *>(&Hst[rr * BN + c8]);
-    *reinterpret_cast<v4i *>(reinterpret_cast<uint16_t *>(e.Wl) + (size_t)r * e.ldw + cg) =
-        *reinterpret_cast<const v4i *>(&Lst[rr * BN + c8]);
+    size_t o = split_offset(r, cg, e.ldw / kSplitPad);
+    *reinterpret_cast<v4i *>(reinterpret_cast<uint16_t *>(e.Wh) + o) =
+        *reinterpret_cast<const v4i *>(&Hst[rr * WLD + c8]);
+    *reinterpret_cast<v4i *>(reinterpret_cast<uint16_t *>(e.Wl) + o) =
+        *reinterpret_cast<const v4i *>(&Lst[rr * WLD + c8]);
   }
 }
 
@@ -1133,13 +1122,6 @@ int gemm_col_tiles(int form, int N) {
 
 int gemm_row_tiles(int M) { return (M + 63) / 64 * 2; }
 
-// ---------------------------------------------------------------------------
-// Tile autotuner of the split contraction. The first contraction of a given
-// shape (M and N rounded up to powers of two, K, device) times every tile
-// shape (the faster of two launches after a warm-up one) on the caller's
-// stream and keeps the fastest for later calls. Shapes never change results:
-// every output element sums its k terms in the same order whatever the tile.
-// ---------------------------------------------------------------------------
 namespace {
 
 // FLARE_MI_TILE_SHAPE=i pins shape i of each contraction's table (tests check
@@ -1148,60 +1130,6 @@ int pinned_shape(int n_shapes) {
   const char *f = std::getenv("FLARE_MI_TILE_SHAPE");
   int i = f ? std::atoi(f) : -1;
   return i < n_shapes ? i : -1;
-}
-
-std::mutex g_tune_mu;
-std::map<std::tuple<int, int, int, int>, int> g_tune;
-
-int next_pow2(int x) {
-  int p = 64;
-  while (p < x) p <<= 1;
-  return p;
-}
-
-// Returns the tuned shape index, timing `launch(i)` for each of n_shapes when
-// the size class is new. `launch` enqueues one contraction.
-template <typename Launch>
-int tuned(int M, int N, int K, hipStream_t st, int n_shapes, Launch &&launch) {
-  int pin = pinned_shape(n_shapes);
-  if (pin >= 0) return pin;
-  int dev = 0;
-  FM_HIP(hipGetDevice(&dev));
-  // M and N up to powers of two: the atom count of a new batch reuses the
-  // choice for its size class instead of timing every shape again.
-  auto key = std::make_tuple(next_pow2(M), next_pow2(N), K, dev);
-  {
-    std::lock_guard<std::mutex> g(g_tune_mu);
-    auto it = g_tune.find(key);
-    if (it != g_tune.end()) return it->second;
-  }
-  hipEvent_t e0, e1;
-  FM_HIP(hipEventCreate(&e0));
-  FM_HIP(hipEventCreate(&e1));
-  int best = -1;
-  float best_ms = 0;
-  for (int i = 0; i < n_shapes; i++) {
-    launch(i);  // warm-up (code object load, caches)
-    float ms = 0;
-    for (int r = 0; r < 2; r++) {  // the faster of two timed launches
-      FM_HIP(hipEventRecord(e0, st));
-      launch(i);
-      FM_HIP(hipEventRecord(e1, st));
-      FM_HIP(hipEventSynchronize(e1));
-      float t = 0;
-      FM_HIP(hipEventElapsedTime(&t, e0, e1));
-      ms = r == 0 ? t : std::min(ms, t);
-    }
-    if (best < 0 || ms < best_ms) {
-      best = i;
-      best_ms = ms;
-    }
-  }
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  std::lock_guard<std::mutex> g(g_tune_mu);
-  g_tune[key] = best;
-  return best;
 }
 
 template <int EP>
@@ -1216,28 +1144,6 @@ void f64_launch(hipStream_t st, int T, int blocks, const F64Groups &gs) {
     else hipLaunchKernelGGL((k_gemm_f64<EP, 4, 1>), grid, block, 0, st, gs);
   } else {
     hipLaunchKernelGGL((k_gemm_f64_lds<EP>), grid, block, 0, st, gs);
-  }
-}
-
-template <int EP, int TM, int TN, bool DB>
-void split_launch(hipStream_t st, int M, int N, int Kpad, const SplitPtrs &a, long long lda,
-                  const SplitPtrs &b, long long ldb, const EpArgs &e) {
-  dim3 grid((N + 32 * TN - 1) / (32 * TN), (M + 32 * TM - 1) / (32 * TM));
-  hipLaunchKernelGGL((k_gemm_split<EP, 2, TM, TN, DB>), grid, dim3(256), 0, st, M, N, Kpad, a,
-                     lda, b, ldb, e);
-}
-
-template <int EP>
-void split_shape(int i, hipStream_t st, int M, int N, int Kpad, const SplitPtrs &a,
-                 long long lda, const SplitPtrs &b, long long ldb, const EpArgs &e) {
-  switch (i) {
-    case 0: split_launch<EP, 4, 4, false>(st, M, N, Kpad, a, lda, b, ldb, e); break;
-    case 1: split_launch<EP, 2, 4, false>(st, M, N, Kpad, a, lda, b, ldb, e); break;
-    case 2: split_launch<EP, 4, 2, false>(st, M, N, Kpad, a, lda, b, ldb, e); break;
-    case 3: split_launch<EP, 4, 4, true>(st, M, N, Kpad, a, lda, b, ldb, e); break;
-    case 4: split_launch<EP, 4, 2, true>(st, M, N, Kpad, a, lda, b, ldb, e); break;
-    case 5: split_launch<EP, 8, 4, false>(st, M, N, Kpad, a, lda, b, ldb, e); break;
-    default: split_launch<EP, 4, 8, false>(st, M, N, Kpad, a, lda, b, ldb, e); break;
   }
 }
 
@@ -1379,49 +1285,50 @@ void gemm_f64(hipStream_t st, int ep, int M, int N, int K, const double *A, long
   gemm_f64_groups(st, ep, {F64Gemm{A, B, lda, ldb, M, N, K, lower_tri, e}});
 }
 
-void gemm_split(hipStream_t st, int ep, int np, int M, int N, int Kpad, const SplitOperand &A,
-                const SplitOperand &B, const EpArgs &e) {
-  if (M <= 0 || N <= 0) return;
-  // The kernel contraction runs on int8 slices (gemm_i8_groups); the split
-  // form serves the gradient contraction.
-  FM_CHECK(ep == EP_STORE, FM_ERR_INVALID, "split-BF16 contraction: EP_STORE only");
-  FM_CHECK(np == 2, FM_ERR_INVALID, "split operands have 2 pieces");
-  FM_CHECK(Kpad % kSplitPad == 0 && A.ld % kSplitPad == 0 && B.ld % kSplitPad == 0 &&
-               Kpad <= A.ld && Kpad <= B.ld,
-           FM_ERR_INVALID, "split operands must be padded to the k-step");
-  SplitPtrs a{}, b{};
-  for (int pc = 0; pc < np; pc++) {
-    FM_CHECK(A.piece[pc] && B.piece[pc], FM_ERR_INVALID, "missing split operand piece");
-    FM_CHECK(((uintptr_t)A.piece[pc] | (uintptr_t)B.piece[pc]) % 16 == 0, FM_ERR_INVALID,
-             "split operands must be 16-byte aligned");
-    a.p[pc] = reinterpret_cast<const __bf16 *>(A.piece[pc]);
-    b.p[pc] = reinterpret_cast<const __bf16 *>(B.piece[pc]);
-  }
-  auto launch = [&](int i) {
-    split_shape<EP_STORE>(i, st, M, N, Kpad, a, A.ld, b, B.ld, e);
-    FM_HIP(hipGetLastError());
-  };
-  launch(tuned(M, N, Kpad, st, 7, launch));
+void split_rows(hipStream_t st, const double *X, long long ldx, int n, int K, uint16_t *hi,
+                uint16_t *lo) {
+  if (n <= 0 || K <= 0) return;
+  long long nk = split_ld(K) / kSplitPad, chunks = (long long)(n + 15) / 16 * nk * 64;
+  hipLaunchKernelGGL(k_split_rows, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, X,
+                     ldx, n, K, nk, hi, lo);
+  FM_HIP(hipGetLastError());
 }
 
-static uint16_t bf16_rne(float x) {
-  uint32_t u;
-  std::memcpy(&u, &x, 4);
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
-}
-
-void split_bf16_host(const float *x, size_t n, int np, uint16_t *const *pieces) {
-  for (size_t k = 0; k < n; k++) {
-    float r = x[k];
-    for (int pc = 0; pc < np; pc++) {
-      uint16_t h = bf16_rne(r);
-      uint32_t hb = (uint32_t)h << 16;
-      float hf;
-      std::memcpy(&hf, &hb, 4);
-      pieces[pc][k] = h;
-      r = r - hf;
+// Tiles of 256 x 256 (one workgroup per CU) move half the data of 128 x 128 ones
+// (two per CU), but leave more of the last round and of ragged edges empty. A
+// round of large ones takes 1.92 times as long as one of small ones (us with
+// small and with large: 330 in 9 rounds and 359 in 5 for two groups of 16,000 x
+// 2,100 x 1,000; 1039 in 24 and 999 in 12 for three of 43,000 x 1,500 x 500; 5670
+// in 105 and 5405 in 53 for three of 87,381 x 3,255 x 1,365).
+void gemm_split_groups(hipStream_t st, const std::vector<SplitGemm> &all) {
+  for (size_t g0 = 0; g0 < all.size(); g0 += kSplitGroups) {
+    SplitGroups gs{};
+    gs.n = (int)std::min<size_t>(kSplitGroups, all.size() - g0);
+    auto tiles = [&](int k, int bm, int bn) {
+      return (long long)((gs.g[k].M + bm - 1) / bm) * ((gs.g[k].N + bn - 1) / bn);
+    };
+    long long small = 0, large = 0;
+    for (int k = 0; k < gs.n; k++) {
+      const SplitGemm &g = gs.g[k] = all[g0 + k];
+      FM_CHECK(g.M > 0 && g.N > 0 && g.nk > 0 && g.e.W, FM_ERR_INVALID, "empty split contraction");
+      for (int pc = 0; pc < 2; pc++)
+        FM_CHECK(g.A[pc] && g.B[pc] && ((uintptr_t)g.A[pc] | (uintptr_t)g.B[pc]) % 16 == 0,
+                 FM_ERR_INVALID, "split operands must be 16-byte aligned");
+      small += tiles(k, 128, 128);
+      large += tiles(k, 256, 256);
+      FM_CHECK(small < (1LL << 31), FM_ERR_CAPACITY, "contraction too large for one launch");
     }
+    bool big = 25 * ((large + 255) / 256) <= 13 * ((small + 511) / 512);
+    int t = big ? 256 : 128;
+    for (int k = 0, first = 0; k < gs.n; k++) {
+      gs.first[k] = first;
+      first += (int)tiles(k, t, t);
+    }
+    if (big)
+      hipLaunchKernelGGL((k_gemm_split<8, 4, 2, 4>), dim3(large), dim3(512), 0, st, gs);
+    else
+      hipLaunchKernelGGL((k_gemm_split<4, 4, 2, 2>), dim3(small), dim3(256), 0, st, gs);
+    FM_HIP(hipGetLastError());
   }
 }
 

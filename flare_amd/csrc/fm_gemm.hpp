@@ -20,8 +20,8 @@ struct EpArgs {
   long long ldk = 0;
   // EP_KERNEL writes w, EP_STORE writes C, into W (rows x ldw). In the int8
   // contraction EP_KERNEL instead writes w as the BF16 pair (hi, lo) of its
-  // FP32 value into Wh / Wl (rows x ldw), zero in the padding columns
-  // [N, ldw), the operand of the split-BF16 gradient contraction.
+  // FP32 value into Wh / Wl (tiled split layout, ldw columns), zero in the
+  // padding columns [N, ldw), the operand of the split-BF16 gradient contraction.
   void *W = nullptr;
   void *Wh = nullptr, *Wl = nullptr;
   long long ldw = 0;
@@ -64,18 +64,28 @@ void gemm_f64(hipStream_t st, int ep, int M, int N, int K, const double *A, long
 // of the chosen form) on operands stored as two BF16 pieces of FP32
 // values, x = x_0 + x_1 with x_0 = bf16(x), x_1 = bf16(x - x_0); it sums
 // x_1 y_0 + x_0 y_1 + x_0 y_0 (3 MFMAs per product, about 16 significant
-// bits; FP32 accumulation). Rows of A and B are K-contiguous with leading
-// dimensions that are multiples of kSplitPad, padded with zeros up to Kpad (a
-// multiple of kSplitPad), and 16-byte aligned. np must be 2 (the number of
-// pieces each operand carries).
-constexpr int kSplitPad = 32;
+// bits; FP32 accumulation). Tiled split layout of a piece of n rows: blocks of
+// kSplitRows rows x kSplitPad k (row, then k: 1 KB), the blocks of a row block
+// one after the other along k; zeros in the padding of k, rows past n in the
+// last block are never part of a kept result.
+constexpr int kSplitPad = 32, kSplitRows = 16;
 inline long long split_ld(long long k) { return (k + kSplitPad - 1) / kSplitPad * kSplitPad; }
-struct SplitOperand {
-  const uint16_t *piece[3] = {nullptr, nullptr, nullptr};
-  long long ld = 0;
+inline size_t split_elems(long long n, long long k) {
+  return (size_t)((n + kSplitRows - 1) / kSplitRows * kSplitRows * split_ld(k));
+}
+__host__ __device__ inline size_t split_offset(long long row, long long k, long long nk) {
+  return (size_t)((row / kSplitRows * nk + k / kSplitPad) * (kSplitRows * kSplitPad) +
+                  row % kSplitRows * kSplitPad + k % kSplitPad);
+}
+struct SplitGemm {
+  const uint16_t *A[2] = {nullptr, nullptr}, *B[2] = {nullptr, nullptr};
+  int M = 0, N = 0, nk = 0;  // nk steps of kSplitPad
+  EpArgs e;                  // W, ldw
 };
-void gemm_split(hipStream_t st, int ep, int np, int M, int N, int Kpad, const SplitOperand &A,
-                const SplitOperand &B, const EpArgs &e);
+void gemm_split_groups(hipStream_t st, const std::vector<SplitGemm> &groups);
+// The pieces of n FP64 rows of K values.
+void split_rows(hipStream_t st, const double *X, long long ldx, int n, int K, uint16_t *hi,
+                uint16_t *lo);
 // Exact-integer kernel contraction (the chosen form's S = B X_hat^T with the
 // EP_KERNEL epilogue, k in FP64 and w as BF16 pairs): both operands as
 // kI8Slices int8 slices of their rows with a power-of-two scale per row, in
@@ -116,8 +126,5 @@ void slice_rows(hipStream_t st, const float *X, long long ldx, int n, int nd, in
 void slice_rows(hipStream_t st, const double *X, long long ldx, int n, int nd, int8_t *Q,
                 long long Kq, int tr, double *scale);
 void gemm_i8_groups(hipStream_t st, const std::vector<I8Gemm> &groups);
-// Host-side split of FP32 values into np BF16 pieces, rounding to nearest
-// even as the device conversion does.
-void split_bf16_host(const float *x, size_t n, int np, uint16_t *const *pieces);
 
 }  // namespace fm

@@ -270,16 +270,15 @@ struct fm_model_s {
   bool has_L = false;
   std::vector<int> L_rows;   // rows of the L_inv column block of each species
   std::vector<int> L_lower;  // 1 when that block is lower triangular
-  // Per species: X-hat (M_s x d) and X-hat^T (d x M_s) in FP64 and as two
-  // BF16 pieces of their FP32 values (Xs: M_s x split_ld(d), for the kernel
-  // contraction; XTs: d x split_ld(M_s), for the gradient contraction; zero
-  // padded), alpha (zero for empty sparse environments) and the L_inv block
-  // (L_rows x M_s, starting at the species' first row).
-  std::vector<fm::DevBuf> X, XT, Xs0, Xs1, XTs0, XTs1, alpha, L;
+  // Per species: X-hat (M_s x d) and X-hat^T (d x M_s), alpha (zero for empty
+  // sparse environments) and the L_inv block (L_rows x M_s, starting at the
+  // species' first row).
+  std::vector<fm::DevBuf> X, XT, alpha, L;
   // Chosen form: X-hat rows as int8 slices with their power-of-two scales
-  // (the kernel contraction's operand), made from X on first use and again
-  // after the B3 reordering of X.
-  std::vector<fm::DevBuf> Xq, Xq_scale;
+  // (the kernel contraction's operand) and X-hat^T as two BF16 pieces (the
+  // gradient contraction's), made from X and XT on first use and again after
+  // the B3 reordering.
+  std::vector<fm::DevBuf> Xq, Xq_scale, XTs0, XTs1;
   bool xq_ready = false;
   std::vector<double> host_alpha;
   // Non-zero once the sparse set has been permuted to the device order of

@@ -291,7 +291,8 @@ static int species_tile_rows(fm_context ctx, int T, int Ms, int form) {
 }
 
 // The model's sparse rows as int8 slices for the chosen form's kernel
-// contraction, made on the context stream from the FP64 rows on first use.
+// contraction and their transpose as BF16 pieces for its gradient contraction,
+// made on the context stream from the FP64 rows on first use.
 static void model_slices(fm_model m, hipStream_t st) {
   if (m->xq_ready) return;
   int nd = m->nd;
@@ -299,6 +300,8 @@ static void model_slices(fm_model m, hipStream_t st) {
   Pool *pool = &m->ctx->pool;
   m->Xq.resize(m->nos);
   m->Xq_scale.resize(m->nos);
+  m->XTs0.resize(m->nos);
+  m->XTs1.resize(m->nos);
   for (int t = 0; t < m->nos; t++) {
     int Ms = m->M_by_type[t];
     if (Ms == 0) continue;
@@ -306,6 +309,10 @@ static void model_slices(fm_model m, hipStream_t st) {
     m->Xq_scale[t].alloc(pool, (size_t)Ms * sizeof(double));
     slice_rows(st, m->X[t].as<double>(), nd, Ms, nd, m->Xq[t].as<int8_t>(), ldq, kI8TileN,
                m->Xq_scale[t].as<double>());
+    for (DevBuf *b : {&m->XTs0[t], &m->XTs1[t]})
+      b->alloc(pool, split_elems(nd, Ms) * sizeof(uint16_t));
+    split_rows(st, m->XT[t].as<double>(), Ms, nd, Ms, m->XTs0[t].as<uint16_t>(),
+               m->XTs1[t].as<uint16_t>());
   }
   m->xq_ready = true;
 }
@@ -318,7 +325,19 @@ static I8Gemm kernel_contraction_i8(fm_model m, int t, const int8_t *A, const do
           (int)(i8_ld(nd) / kI8Pad), ek};
 }
 
-// The same of `cnt` FP32 descriptor rows (leading dimension nd) without slices
+// Chosen form: gradient contraction of `cnt` rows of w (pieces Wh, Wl) with
+// species t's sparse set.
+static SplitGemm gradient_contraction(fm_model m, int t, const uint16_t *Wh, const uint16_t *Wl,
+                                      int cnt, int nd, const EpArgs &eg) {
+  return {{Wh, Wl},
+          {m->XTs0[t].as<uint16_t>(), m->XTs1[t].as<uint16_t>()},
+          cnt,
+          nd,
+          (int)(split_ld(m->M_by_type[t]) / kSplitPad),
+          eg};
+}
+
+// The kernel contraction of `cnt` FP32 descriptor rows (leading dimension nd) without slices
 // of their FP64 values, sliced into Aq / Aq_scale first (Aq holds at least
 // i8_tiled_bytes(cnt, kI8TileA, i8_ld(nd)) bytes).
 static void contract_fp32_rows(fm_model m, hipStream_t st, int t, const float *rows, int cnt,
@@ -372,7 +391,6 @@ static void predict_tiled(fm_model m, fm_structure s, int flags, int form, doubl
   DevBuf fbond(pool, std::max<size_t>(1, (size_t)3 * s->n_bonds * esz));
   DevBuf vir(pool, std::max<size_t>(1, (size_t)6 * n * sizeof(double)));
   // Tile buffers. k is FP64 in both forms (rows padded to 128 bytes).
-  long long ldm = split_ld(std::max(Mmax, 1));
   size_t kld = ((size_t)Mmax + 15) / 16 * 16;  // rows of whole 128-byte lines
   DevBuf Bt(pool, std::max<size_t>(1, (size_t)T * nd * esz));
   DevBuf Gt(pool, std::max<size_t>(1, (size_t)T * nd * esz));
@@ -383,8 +401,9 @@ static void predict_tiled(fm_model m, fm_structure s, int flags, int form, doubl
     model_slices(m, st);
     Tq.alloc(pool, std::max<size_t>(1, i8_tiled_bytes(T, kI8TileA, i8_ld(nd))));
     Tq_scale.alloc(pool, std::max<size_t>(1, (size_t)T * sizeof(double)));
-    Wh.alloc(pool, std::max<size_t>(1, (size_t)T * ldm * sizeof(uint16_t)));
-    Wl.alloc(pool, std::max<size_t>(1, (size_t)T * ldm * sizeof(uint16_t)));
+    size_t w = split_elems(T, std::max(Mmax, 1)) * sizeof(uint16_t);
+    Wh.alloc(pool, w);
+    Wl.alloc(pool, w);
   }
   if (want_var) Kt.alloc(pool, std::max<size_t>(1, (size_t)T * kld * sizeof(double)));
   double sig2 = m->sigma * m->sigma;
@@ -445,15 +464,8 @@ static void predict_tiled(fm_model m, fm_structure s, int flags, int form, doubl
           gemm_f64(st, EP_STORE, cnt, nd, Ms, Wt.as<double>(), Ms, m->XT[t].as<double>(), Ms, 0,
                    eg);
         } else {
-          long long lm = split_ld(Ms);
-          SplitOperand A, Bx;
-          A.piece[0] = Wh.as<uint16_t>();
-          A.piece[1] = Wl.as<uint16_t>();
-          A.ld = lm;
-          Bx.piece[0] = m->XTs0[t].as<uint16_t>();
-          Bx.piece[1] = m->XTs1[t].as<uint16_t>();
-          Bx.ld = lm;
-          gemm_split(st, EP_STORE, 2, cnt, nd, (int)lm, A, Bx, eg);
+          gemm_split_groups(st, {gradient_contraction(m, t, Wh.as<uint16_t>(),
+                                                      Wl.as<uint16_t>(), cnt, nd, eg)});
         }
       }
       hipLaunchKernelGGL(k_species_final, dim3((cnt + 255) / 256), dim3(256), 0, st, cnt, r0, ep,
@@ -506,7 +518,7 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
   size_t n_out = (size_t)s->mean_off[s->n_struct];
   // Per-species slices of the atom-major w and k matrices (n_s x M_s each)
   // and of the energy / variance partials.
-  // The chosen form keeps w as BF16 pairs with padded rows (ws = split_ld).
+  // The chosen form keeps w as BF16 pairs in the tiled split layout.
   // k is FP64 in both forms, rows padded to 16 values (whole 128-byte lines).
   std::vector<size_t> wo(nos + 1, 0), eo(nos + 1, 0), qo(nos + 1, 0), so(nos + 1, 0),
       ko(nos + 1, 0), kld(nos, 0);
@@ -515,7 +527,7 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
     kld[t] = (Ms + 15) / 16 * 16;  // rows of whole 128-byte lines (w and k)
     wo[t + 1] = wo[t] + ns * kld[t];
     ko[t + 1] = ko[t] + ns * kld[t];
-    so[t + 1] = so[t] + ns * (size_t)split_ld((long long)Ms);
+    so[t + 1] = so[t] + split_elems((long long)ns, (long long)Ms);
     eo[t + 1] = eo[t] + ns * (size_t)std::max(1, gemm_col_tiles(form, (int)Ms));
     int Lr = want_var ? m->L_rows[t] : 0;
     qo[t + 1] = qo[t] + ns * (size_t)gemm_row_tiles(Lr);
@@ -556,6 +568,7 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
   ctx->mark_begin(ST_SGEMM);
   std::vector<F64Gemm> f64_k, f64_g, f64_q;
   std::vector<I8Gemm> i8_k;
+  std::vector<SplitGemm> split_g;
   for (int t = 0; t < nos; t++) {
     int ns = s->n_by_type[t], Ms = m->M_by_type[t], ro = s->type_off[t];
     if (ns == 0) continue;
@@ -616,22 +629,15 @@ void predict(fm_model m, fm_structure s, int flags, int form, double *mean_efs,
       f64_g.push_back({W.as<double>() + wo[t], m->XT[t].as<double>(), (long long)kld[t], Ms, ns,
                        nd, Ms, 0, eg});
     } else {
-      KScope timer(ctx, KT_GGEMM);
-      long long ldm = split_ld(Ms);
-      SplitOperand A, Bx;
-      A.piece[0] = Wh.as<uint16_t>() + so[t];
-      A.piece[1] = Wl.as<uint16_t>() + so[t];
-      A.ld = ldm;
-      Bx.piece[0] = m->XTs0[t].as<uint16_t>();
-      Bx.piece[1] = m->XTs1[t].as<uint16_t>();
-      Bx.ld = ldm;
-      gemm_split(st, EP_STORE, 2, ns, nd, (int)ldm, A, Bx, eg);
+      split_g.push_back(gradient_contraction(m, t, Wh.as<uint16_t>() + so[t],
+                                             Wl.as<uint16_t>() + so[t], ns, nd, eg));
     }
     ctx->launches[ST_GGEMM]++;
   }
-  if (!f64_g.empty()) {
+  if (!f64_g.empty() || !split_g.empty()) {
     KScope timer(ctx, KT_GGEMM);
     gemm_f64_groups(st, EP_STORE, f64_g);
+    gemm_split_groups(st, split_g);
   }
   ctx->mark_end(ST_GGEMM);
 

@@ -1,5 +1,5 @@
-"""The integer contraction at both of its tile widths: few tiles and many, an
-odd and an even number of 64-column tiles, column counts at and past a tile's
+"""The chosen form's contractions at both of their tile sizes: few tiles and
+many, an odd and an even number of 64-column tiles, column counts at and past a tile's
 edge, one to six steps of the reduction, a last row tile with one row, several
 species in one launch. The chosen form against the FP64 form."""
 import numpy as np
@@ -20,6 +20,10 @@ SIGMA = 1.5
     ((1, 8, 3), (13, 13, 13), (320,)),   # 8788 atoms
     ((2, 6, 3), (4, 11, 1), (64, 65)),   # 176 atoms
     ((2, 4, 9), (16, 16, 16), (129, 190)),
+    # d = 1088: 576 tiles of 128 x 128 of the gradient contraction or 160 of
+    # 256 x 256, one and three steps of 32.
+    ((1, 16, 7), (13, 13, 12), (30,)),
+    ((1, 16, 7), (13, 13, 12), (70,)),
 ])
 def test_integer_contraction(settings, reps, n_sparse):
     from flare_amd import _C_flare as C
