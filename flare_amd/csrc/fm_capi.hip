@@ -223,6 +223,7 @@ int fm_context_create(int device, fm_context *out) {
     FM_HIP(hipSetDevice(device));
     fm::scratch_setup(device);
     fm::descriptor_setup();
+    fm::dense_setup();
     auto *c = new fm_context_s();
     c->device = device;
     FM_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));

@@ -188,9 +188,7 @@ __device__ __forceinline__ void atom_sync() {
   if constexpr (W > 1) {
     __syncthreads();
   } else {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_sync();
   }
 }
 

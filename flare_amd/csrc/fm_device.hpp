@@ -167,4 +167,11 @@ __device__ __forceinline__ void sph_harm_lane(int l, int m, T knorm, T ux, T uy,
   }
 }
 
+// Orders this wave's LDS accesses before and after it.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 }  // namespace fm

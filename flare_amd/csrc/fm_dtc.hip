@@ -24,26 +24,49 @@ constexpr int kMaxHCd = 2;
 
 __constant__ double c_knorm_d[kMaxH];
 
+// Species-sorted bonds: rows in species order, the bonds of a row contiguous
+// (b2.cpp:150-154). One wavefront per row.
+__global__ __launch_bounds__(256) void k_row_bonds(int n, const int *atom_of_row,
+                                                   const int *bond_off, int *cnt) {
+  int r = blockIdx.x * 256 + threadIdx.x;
+  if (r < n) cnt[r] = bond_off[atom_of_row[r] + 1] - bond_off[atom_of_row[r]];
+}
+__global__ __launch_bounds__(256) void k_sorted_bonds(int n, const int *atom_of_row,
+                                                      const int *bond_off, const int *sb_off,
+                                                      int *sb_pos, int *sb_row, int *sb_bond) {
+  int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (r >= n) return;
+  int i = atom_of_row[r], b0 = bond_off[i], b1 = bond_off[i + 1], f0 = sb_off[r];
+  for (int b = b0 + lane; b < b1; b += 64) {
+    int f = f0 + b - b0;
+    sb_pos[b] = f;
+    sb_row[f] = r;
+    sb_bond[f] = b;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Dense dB/dr per bond and component (b2.cpp:219-228), written at the
 // bond's species-sorted position f (rows 3 f + m: the layout of
 // DescriptorValues::descriptor_force_dervs), and the force dots dB . B
-// (b2.cpp:236-240). One wavefront per atom.
+// (b2.cpp:236-240). A wavefront per bond at a time: the blocks of atom
+// blockIdx.x (gridDim.y of them) deal its bonds to their waves. c comes from the
+// descriptor pass. What bounds it: the LDS reads of the pair loop; 14,000 bonds
+// of d = 544 take 80 us (640 with one wave per atom, which summed c first, at
+// 256 waves on the whole GPU).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void k_b2_dervs(
-    int n, int nos, int N, int lmax, int H, int nrad, int nd, int cutkind, double r1,
-    const int *species, const int *bond_off, const int *bond_q, const int *nspec,
-    const double *rel, const double *cutoffs, const int *row_of_atom, const int *sb_off,
-    const int2 *pairs, const double *B, double *DB, double *fdots) {
+__global__ __launch_bounds__(256) void k_b2_dervs(
+    int nos, int N, int H, int nrad, int nd, int L1, int cutkind, double r1, const int *species,
+    const int *bond_off, const int *bond_q, const int *nspec, const double *rel,
+    const double *cutoffs, const int *row_of_atom, const int *sb_off, const double *C,
+    const double *B, double *DB, double *fdots) {
   extern __shared__ __align__(16) unsigned char smem[];
-  int i = blockIdx.x, lane = threadIdx.x;
-  if (i >= n) return;
-  double *c = reinterpret_cast<double *>(smem);  // nrad x H
-  double *dc = c + (size_t)nrad * H;              // N x H x 3 (current bond)
-  int si = species[i];
-  int b0 = bond_off[i], b1 = bond_off[i + 1];
-  int row = row_of_atom[i];
-  int f0 = sb_off[row];
+  int i = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6, W = blockDim.x >> 6;
+  double *c = reinterpret_cast<double *>(smem);                          // nrad x H
+  double *dc = c + (size_t)nrad * H + (size_t)w * N * H * 3;  // N x H x 3 (this wave's bond)
+  int si = species[i], b0 = bond_off[i], b1 = bond_off[i + 1], row = row_of_atom[i];
+  for (int q = threadIdx.x; q < nrad * H; q += blockDim.x) c[q] = C[(size_t)i * nrad * H + q];
+  __syncthreads();
   int ls[kMaxHCd], ms[kMaxHCd];
   double kn[kMaxHCd];
   for (int ch = 0; ch < kMaxHCd; ch++) {
@@ -55,30 +78,8 @@ __global__ __launch_bounds__(64) void k_b2_dervs(
     ms[ch] = lmc - l * l - l;
     kn[ch] = c_knorm_d[lmc];
   }
-  // Single-bond coefficients c (b2.cpp:367-395), every neighbour species.
-  for (int q = lane; q < nrad * H; q += 64) c[q] = 0;
-  __syncthreads();
-  for (int b = b0; b < b1; b++) {
-    int qn = bond_q[b];
-    int sj = nspec[qn];
-    const double *rp = rel + 4 * (size_t)qn;
-    double rc = cutoffs[si * nos + sj];
-    double g[kMaxN], dg[kMaxN];
-    radial_basis<double>(rp[0], rc, r1, N, cutkind, g, dg);
-    double rinv = 1.0 / rp[0];
-    double ux = rp[1] * rinv, uy = rp[2] * rinv, uz = rp[3] * rinv;
-    for (int ch = 0; ch < kMaxHCd; ch++) {
-      int lm = lane + 64 * ch;
-      if (lm >= H) continue;
-      double Y, d0, d1, d2;
-      sph_harm_lane<double, false>(ls[ch], ms[ch], kn[ch], ux, uy, uz, rinv, Y, d0, d1, d2);
-      for (int nn = 0; nn < N; nn++) c[(sj * N + nn) * H + lm] += g[nn] * Y;
-    }
-  }
-  __syncthreads();
   const double *Brow = B + (size_t)row * nd;
-  int L1 = lmax + 1;
-  for (int b = b0; b < b1; b++) {
+  for (int b = b0 + blockIdx.y * W + w; b < b1; b += gridDim.y * W) {
     int qn = bond_q[b];
     int sj = nspec[qn];
     const double *rp = rel + 4 * (size_t)qn;
@@ -87,6 +88,7 @@ __global__ __launch_bounds__(64) void k_b2_dervs(
     radial_basis<double>(rp[0], rc, r1, N, cutkind, g, dg);
     double r = rp[0], rinv = 1.0 / r;
     double ux = rp[1] * rinv, uy = rp[2] * rinv, uz = rp[3] * rinv;
+    wave_lds_sync();  // the last bond's dc has been read
     for (int ch = 0; ch < kMaxHCd; ch++) {
       int lm = lane + 64 * ch;
       if (lm >= H) continue;
@@ -99,22 +101,29 @@ __global__ __launch_bounds__(64) void k_b2_dervs(
         o[2] = dg[nn] * uz * Y + g[nn] * Yz;
       }
     }
-    __syncthreads();
-    int f = f0 + (b - b0);
+    wave_lds_sync();
+    int f = sb_off[row] + (b - b0);
     double fd[3] = {0, 0, 0};
     for (int k = lane; k < nd; k += 64) {
       int p = k / L1, l = k - p * L1;
-      int2 pr = pairs[p];
-      int n1 = pr.x, n2 = pr.y;
-      bool in1 = n1 / N == sj, in2 = n2 / N == sj;
+      // Pair p is (n1, n2 >= n1), those of n1 from first(n1) on.
+      auto first = [&](int a) { return a * nrad - a * (a - 1) / 2; };
+      float t = 2 * nrad + 1;
+      int n1 = (int)((t - sqrtf(t * t - 8 * p)) * 0.5f);
+      n1 += first(n1 + 1) <= p;
+      n1 -= first(n1) > p;
+      int n2 = n1 + p - first(n1);
       double acc[3] = {0, 0, 0};
-      for (int mm = 0; mm < 2 * l + 1; mm++) {
-        int lm = l * l + mm;
-        double c1v = c[n1 * H + lm], c2v = c[n2 * H + lm];
-        for (int comp = 0; comp < 3; comp++) {
-          double d1 = in1 ? dc[((size_t)(n1 - sj * N) * H + lm) * 3 + comp] : 0.0;
-          double d2 = in2 ? dc[((size_t)(n2 - sj * N) * H + lm) * 3 + comp] : 0.0;
-          acc[comp] += c1v * d2 + d1 * c2v;
+      // dB = c1 dc2 + dc1 c2; dc is zero but for the neighbour's species.
+      if (n2 / N == sj || n1 / N == sj) {
+        bool in1 = n1 / N == sj, in2 = n2 / N == sj;
+        const double *d1 = dc + ((size_t)(in1 ? n1 - sj * N : 0) * H + l * l) * 3;
+        const double *d2 = dc + ((size_t)(in2 ? n2 - sj * N : 0) * H + l * l) * 3;
+        const double *c1 = c + n1 * H + l * l, *c2 = c + n2 * H + l * l;
+        for (int mm = 0; mm < 2 * l + 1; mm++) {
+          double c1v = in2 ? c1[mm] : 0.0, c2v = in1 ? c2[mm] : 0.0;
+          for (int comp = 0; comp < 3; comp++)
+            acc[comp] += c1v * d2[3 * mm + comp] + d1[3 * mm + comp] * c2v;
         }
       }
       for (int comp = 0; comp < 3; comp++) {
@@ -126,14 +135,7 @@ __global__ __launch_bounds__(64) void k_b2_dervs(
       double v = wave_sum(fd[comp]);
       if (lane == 0) fdots[3 * (size_t)f + comp] = v;
     }
-    __syncthreads();
   }
-}
-
-__global__ void k_bond_owner(int n, const int *bond_off, int *owner) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  for (int b = bond_off[i]; b < bond_off[i + 1]; b++) owner[b] = i;
 }
 
 __device__ __forceinline__ double dpow(double x, double p) {
@@ -147,87 +149,106 @@ __device__ __forceinline__ double dpow(double x, double p) {
 // transposed (Kt: n_out x M, column cs + j).
 // ---------------------------------------------------------------------------
 struct EnvsArgs {
-  int n, nd, M, cs, Ms, t, ro, nt, sbo, nbt;
+  int n, M, cs, Ms, t, ro, nt, sbo, nbt;
   double sig2, power, vol_inv;
-  const int *species, *row_of_atom, *bond_off, *in_off, *in_bond, *sb_pos, *sb_row, *sb_bond,
-      *bond_q;
+  const int *species, *row_of_atom, *bond_off, *in_off, *in_bond, *sb_pos, *sb_row, *bond_q;
   const double *norm, *xnorm, *rel;
-  const double *S;   // Ms x nt: x_hat_j . B_r (raw B)
-  const double *FD;  // Ms x 3 nbt: x_hat_j . dB_f,m
+  const double *S;   // nt x Ms: x_hat_j . B_r (raw B)
+  const double *FD;  // 3 nbt x Ms: x_hat_j . dB_f,m
   const double *fdots;
+  double *P;   // nt x 7 x Ms: energy and sums of fk(m) coord(n), n >= m, per row
   double *Kt;
 };
 
-// fk(j, f, m) = sigma^2 p S^(p-1) (x_hat . dB / |B| - S fdot / |B|^2), the
-// force kernel of normalized_dot_product.cpp:187-195 with S = x.B/(|x||B|).
-__device__ __forceinline__ double fk_of(const EnvsArgs &e, int j, int f, int m) {
-  int r = e.sb_row[f];
-  double nb = e.norm[r];
-  if (nb < kEmptyThresh) return 0.0;
-  double s = e.S[(size_t)j * e.nt + (r - e.ro)] / nb;
-  double dval = e.power * dpow(s, e.power - 1);
-  double f1 = e.FD[(size_t)j * 3 * e.nbt + 3 * (size_t)(f - e.sbo) + m] / nb;
-  double f2 = s * e.fdots[3 * (size_t)f + m] / (nb * nb);
-  return e.sig2 * dval * (f1 - f2);
-}
-
-// Force columns: + bonds owned by a, - bonds pointing at a
-// (normalized_dot_product.cpp:197-199), owners of species t only.
-__global__ void k_envs_forces(EnvsArgs e) {
-  int j = blockIdx.y;
-  int a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= e.Ms || a >= e.n) return;
-  size_t col = (size_t)e.cs + j;
-  double acc[3] = {0, 0, 0};
-  if (e.xnorm[j] >= kEmptyThresh) {
-    if (e.species[a] == e.t)
-      for (int b = e.bond_off[a]; b < e.bond_off[a + 1]; b++)
-        for (int m = 0; m < 3; m++) acc[m] += fk_of(e, j, e.sb_pos[b], m);
-    for (int q = e.in_off[a]; q < e.in_off[a + 1]; q++) {
-      int f = e.sb_pos[e.in_bond[q]];
-      if (f < e.sbo || f >= e.sbo + e.nbt) continue;  // owner of another species
-      for (int m = 0; m < 3; m++) acc[m] -= fk_of(e, j, f, m);
-    }
-  }
-  for (int m = 0; m < 3; m++) e.Kt[(size_t)(1 + 3 * a + m) * e.M + col] = acc[m];
-}
-
-// Energy and stress columns of sparse env j (one block of 256 per j):
-// E = sum_r sigma^2 S^p; S_mn = -1/V sum_f fk(m) coord_f(n), n >= m
-// (normalized_dot_product.cpp:175-177, 201-206).
-__global__ __launch_bounds__(256) void k_envs_energy_stress(EnvsArgs e) {
-  __shared__ double sh[7][256];
-  int j = blockIdx.x;
-  double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-  if (e.xnorm[j] >= kEmptyThresh) {
-    for (int r = threadIdx.x; r < e.nt; r += blockDim.x) {
-      double nb = e.norm[e.ro + r];
-      if (nb < kEmptyThresh) continue;
-      double s = e.S[(size_t)j * e.nt + r] / nb;
-      acc[0] += e.sig2 * dpow(s, e.power);
-    }
-    for (int fl = threadIdx.x; fl < e.nbt; fl += blockDim.x) {
-      int f = e.sbo + fl;
-      const double *co = e.rel + 4 * (size_t)e.bond_q[e.sb_bond[f]] + 1;
-      int sc = 0;
+// Forces on atom blockIdx.x: + its own bonds, - bonds pointing at it
+// (normalized_dot_product.cpp:197-199), owners of species t only, and the row's
+// part of the energy and stress, with fk(j, f, m) = sigma^2 p S^(p-1)
+// (x_hat . dB / |B| - S fdot / |B|^2), the force kernel of
+// normalized_dot_product.cpp:187-195 with S = x.B/(|x||B|). Lanes are sparse
+// environments (S, FD and Kt are read and written in whole lines), the block's
+// four waves split the bonds. 256 atoms, 150 environments: 25 us (165 with
+// threads on atoms, whose loads and stores of one environment were a row apart).
+__global__ __launch_bounds__(256) void k_envs_rows(EnvsArgs e) {
+  __shared__ double sh[4][10][64];
+  int a = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int j = blockIdx.y * 64 + lane, jc = min(j, e.Ms - 1);
+  double acc[10] = {};  // force, energy, stress
+  auto fk = [&](int r, int f, double *out) {
+    double inv = 1.0 / e.norm[r], s = e.S[(size_t)(r - e.ro) * e.Ms + jc] * inv;
+    double dval = e.sig2 * e.power * dpow(s, e.power - 1) * inv;
+    const double *FD = e.FD + (size_t)3 * (f - e.sbo) * e.Ms + jc;
+#pragma unroll
+    for (int m = 0; m < 3; m++)
+      out[m] = dval * (FD[(size_t)m * e.Ms] - s * e.fdots[3 * (size_t)f + m] * inv);
+  };
+  int row = e.row_of_atom[a];
+  bool own = e.species[a] == e.t;
+  if (own && e.norm[row] >= kEmptyThresh) {
+    if (w == 0)
+      acc[3] = e.sig2 * dpow(e.S[(size_t)(row - e.ro) * e.Ms + jc] / e.norm[row], e.power);
+    for (int b = e.bond_off[a] + w; b < e.bond_off[a + 1]; b += 4) {
+      double v[3];
+      fk(row, e.sb_pos[b], v);
+      const double *co = e.rel + 4 * (size_t)e.bond_q[b] + 1;
+      int sc = 4;
+#pragma unroll
       for (int m = 0; m < 3; m++) {
-        double fk = fk_of(e, j, f, m);
-        for (int nn = m; nn < 3; nn++) acc[1 + sc++] -= fk * co[nn] * e.vol_inv;
+        acc[m] += v[m];
+#pragma unroll
+        for (int nn = m; nn < 3; nn++) acc[sc++] += v[m] * co[nn];
       }
     }
   }
-  for (int q = 0; q < 7; q++) sh[q][threadIdx.x] = acc[q];
+  for (int q = e.in_off[a] + w; q < e.in_off[a + 1]; q += 4) {
+    int f = e.sb_pos[e.in_bond[q]];
+    if (f < e.sbo || f >= e.sbo + e.nbt) continue;  // owner of another species
+    int r = e.sb_row[f];
+    if (e.norm[r] < kEmptyThresh) continue;
+    double v[3];
+    fk(r, f, v);
+#pragma unroll
+    for (int m = 0; m < 3; m++) acc[m] -= v[m];
+  }
+#pragma unroll
+  for (int q = 0; q < 10; q++) sh[w][q][lane] = acc[q];
   __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (threadIdx.x < st)
-      for (int q = 0; q < 7; q++) sh[q][threadIdx.x] += sh[q][threadIdx.x + st];
-    __syncthreads();
+  if (j >= e.Ms) return;
+  bool empty = e.xnorm[j] < kEmptyThresh;
+  for (int q = w; q < (own ? 10 : 3); q += 4) {
+    double v = (sh[0][q][lane] + sh[1][q][lane]) + (sh[2][q][lane] + sh[3][q][lane]);
+    if (empty) v = 0;
+    if (q < 3) e.Kt[(size_t)(1 + 3 * a + q) * e.M + e.cs + j] = v;
+    else e.P[((size_t)(row - e.ro) * 7 + (q - 3)) * e.Ms + j] = v;
   }
-  if (threadIdx.x < 7) {
-    size_t col = (size_t)e.cs + j;
-    int c = threadIdx.x == 0 ? 0 : 1 + 3 * e.n + (threadIdx.x - 1);
-    e.Kt[(size_t)c * e.M + col] = sh[threadIdx.x][0];
-  }
+}
+
+// Energy and stress of the sparse environments: E = sum_r sigma^2 S^p;
+// S_mn = -1/V sum_f fk(m) coord_f(n), n >= m (normalized_dot_product.cpp:175-177,
+// 201-206) from the rows' parts, quantity blockIdx.y, 16 waves over the rows.
+__global__ __launch_bounds__(1024) void k_envs_sums(EnvsArgs e) {
+  __shared__ double sh[16][64];
+  int lane = threadIdx.x & 63, w = threadIdx.x >> 6, q = blockIdx.y;
+  int j = blockIdx.x * 64 + lane, jc = min(j, e.Ms - 1);
+  double v = 0;
+  for (int r = w; r < e.nt; r += 16) v += e.P[((size_t)r * 7 + q) * e.Ms + jc];
+  sh[w][lane] = v;
+  __syncthreads();
+  if (w > 0 || j >= e.Ms) return;
+  for (int u = 1; u < 16; u++) v += sh[u][lane];
+  int c = q == 0 ? 0 : 1 + 3 * e.n + (q - 1);
+  e.Kt[(size_t)c * e.M + e.cs + j] = q == 0 ? v : -v * e.vol_inv;
+}
+
+// out (cols x rows) = in (rows x cols)^T.
+__global__ __launch_bounds__(256) void k_transpose(int rows, int cols, const double *in,
+                                                   double *out) {
+  __shared__ double t[32][33];
+  int c0 = blockIdx.x * 32, r0 = blockIdx.y * 32, x = threadIdx.x & 31, y = threadIdx.x >> 5;
+  for (int k = y; k < 32; k += 8)
+    if (r0 + k < rows && c0 + x < cols) t[k][x] = in[(size_t)(r0 + k) * cols + c0 + x];
+  __syncthreads();
+  for (int k = y; k < 32; k += 8)
+    if (c0 + k < cols && r0 + x < rows) out[(size_t)(c0 + k) * rows + r0 + x] = t[x][k];
 }
 
 // ---------------------------------------------------------------------------
@@ -380,11 +401,10 @@ __global__ void k_var_efs(int n_out, int dtc, const double *kself, const double 
 // ---------------------------------------------------------------------------
 // Host orchestration
 // ---------------------------------------------------------------------------
-static void upload_knorm_d(hipStream_t st, int) {
-  static thread_local double host[kMaxH];
-  knorm_values(kMaxL, host);
-  FM_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_knorm_d), host, sizeof(host), 0,
-                                hipMemcpyHostToDevice, st));
+void dense_setup() {
+  double kn[kMaxH];
+  knorm_values(kMaxL, kn);
+  FM_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_knorm_d), kn, sizeof(kn), 0, hipMemcpyHostToDevice));
 }
 
 void compute_dervs(fm_structure s) {
@@ -400,135 +420,124 @@ void compute_dervs(fm_structure s) {
   size_t nb = (size_t)s->n_bonds;
   FM_CHECK((double)nb * 3 * nd * 8 < 64e9, FM_ERR_CAPACITY,
            "dense descriptor derivatives exceed 64 GB; the adjoint path needs none");
-  // Species-sorted bond layout: rows in species order, bonds of a row
-  // contiguous (b2.cpp:150-154).
-  std::vector<int> bo(n + 1), aor(n), sp(n);
-  FM_HIP(hipMemcpyAsync(bo.data(), s->bond_off.as<int>(), (n + 1) * sizeof(int),
-                        hipMemcpyDeviceToHost, st));
-  FM_HIP(hipMemcpyAsync(aor.data(), s->atom_of_row.as<int>(), n * sizeof(int),
-                        hipMemcpyDeviceToHost, st));
-  FM_HIP(hipMemcpyAsync(sp.data(), s->species.as<int>(), n * sizeof(int), hipMemcpyDeviceToHost,
-                        st));
-  FM_HIP(hipStreamSynchronize(st));
-  std::vector<int> sb_off(n + 1, 0), sb_pos(nb), sb_row(nb), sb_bond(nb);
   s->nbt_off.assign(s->nos + 1, 0);
-  for (int r = 0; r < n; r++) {
-    int i = aor[r];
-    int cnt = bo[i + 1] - bo[i];
-    sb_off[r + 1] = sb_off[r] + cnt;
-    for (int k = 0; k < cnt; k++) {
-      int f = sb_off[r] + k, b = bo[i] + k;
-      sb_pos[b] = f;
-      sb_row[f] = r;
-      sb_bond[f] = b;
-    }
-    s->nbt_off[sp[i] + 1] += cnt;
-  }
-  for (int t = 0; t < s->nos; t++) s->nbt_off[t + 1] += s->nbt_off[t];
-  auto up = [&](DevBuf &buf, const void *src, size_t bytes) {
-    buf.alloc(pool, std::max<size_t>(1, bytes));
-    if (bytes) FM_HIP(hipMemcpyAsync(buf.as<void>(), src, bytes, hipMemcpyHostToDevice, st));
-  };
-  up(s->sb_off, sb_off.data(), sb_off.size() * sizeof(int));
-  up(s->sb_pos, sb_pos.data(), sb_pos.size() * sizeof(int));
-  up(s->sb_row, sb_row.data(), sb_row.size() * sizeof(int));
-  up(s->sb_bond, sb_bond.data(), sb_bond.size() * sizeof(int));
+  for (int t = 0; t < s->nos; t++) s->nbt_off[t + 1] = s->nbt_off[t] + s->nb_by_type[t];
+  for (DevBuf *b : {&s->sb_pos, &s->sb_row, &s->sb_bond})
+    b->alloc(pool, std::max<size_t>(1, nb * sizeof(int)));
+  s->sb_off.alloc(pool, (size_t)(n + 1) * sizeof(int));
   s->DB.alloc(pool, std::max<size_t>(1, nb * 3 * nd * sizeof(double)));
   s->fdots.alloc(pool, std::max<size_t>(1, nb * 3 * sizeof(double)));
-  upload_knorm_d(st, s->lmax);
-  // n1, n2 of each radial pair in B2 order.
-  std::vector<int> pairs;
-  for (int a = 0; a < nrad; a++)
-    for (int b = a; b < nrad; b++) {
-      pairs.push_back(a);
-      pairs.push_back(b);
-    }
-  DevBuf pair_table;
-  up(pair_table, pairs.data(), pairs.size() * sizeof(int));
-  size_t lds = ((size_t)nrad * H + (size_t)s->N * H * 3) * sizeof(double);
+  DevBuf cnt(pool, std::max<size_t>(1, (size_t)n * sizeof(int)));
+  if (n > 0) {
+    hipLaunchKernelGGL(k_row_bonds, dim3((n + 255) / 256), dim3(256), 0, st, n,
+                       s->atom_of_row.as<int>(), s->bond_off.as<int>(), cnt.as<int>());
+    scan_exclusive(ctx, cnt.as<int>(), s->sb_off.as<int>(), n);
+    hipLaunchKernelGGL(k_sorted_bonds, dim3((n + 3) / 4), dim3(256), 0, st, n,
+                       s->atom_of_row.as<int>(), s->bond_off.as<int>(), s->sb_off.as<int>(),
+                       s->sb_pos.as<int>(), s->sb_row.as<int>(), s->sb_bond.as<int>());
+  }
+  // Four waves per block where their workspaces keep two blocks on a CU, and
+  // blocks per atom for some 8192 waves in all, no more than the bonds need.
+  auto lds_of = [&](int W) {
+    return ((size_t)nrad * H + (size_t)W * s->N * H * 3) * sizeof(double);
+  };
+  int W = lds_of(4) <= 80 * 1024 ? 4 : 1;
+  size_t lds = lds_of(W);
   FM_CHECK(lds <= 160 * 1024, FM_ERR_CAPACITY, "derivative workspace exceeds LDS");
-  if (n > 0)
-    hipLaunchKernelGGL(k_b2_dervs, dim3(n), dim3(64), lds, st, n, s->nos, s->N, s->lmax, H, nrad,
-                       nd, s->cutkind, s->r1, s->species.as<int>(), s->bond_off.as<int>(),
-                       s->bond_q.as<int>(), s->nspecies.as<int>(), s->rel.as<double>(),
-                       s->d_cutoffs.as<double>(), s->row_of_atom.as<int>(), s->sb_off.as<int>(),
-                       pair_table.as<int2>(), s->B.as<double>(), s->DB.as<double>(),
-                       s->fdots.as<double>());
+  if (n > 0) {
+    int need = (int)std::min<size_t>((nb / n + W) / W, 1024);
+    int y = std::max(1, std::min(need, 8192 / (n * W)));
+    hipLaunchKernelGGL(k_b2_dervs, dim3(n, y), dim3(64 * W), lds, st, s->nos, s->N, H, nrad, nd,
+                       s->lmax + 1, s->cutkind, s->r1, s->species.as<int>(),
+                       s->bond_off.as<int>(), s->bond_q.as<int>(), s->nspecies.as<int>(),
+                       s->rel.as<double>(), s->d_cutoffs.as<double>(), s->row_of_atom.as<int>(),
+                       s->sb_off.as<int>(), s->C.as<double>(),
+                       s->B.as<double>(), s->DB.as<double>(), s->fdots.as<double>());
+  }
   FM_HIP(hipGetLastError());
-  FM_HIP(hipStreamSynchronize(st));
   s->has_dervs = true;
 }
 
-// Kt (n_out x M) = envs_struc(sparse, structure)^T.
-static void envs_struc_t(fm_model m, fm_structure s, DevBuf &Kt, DevBuf &owner) {
+// Kt (n_out x M) = envs_struc(sparse, structure)^T. The products of all species
+// in one launch, up to 4 GB of them at a time.
+static void envs_struc_t(fm_model m, fm_structure s, DevBuf &Kt) {
   fm_context ctx = s->ctx;
   hipStream_t st = ctx->stream;
   Pool *pool = &ctx->pool;
   int n = s->n, nd = s->nd, M = m->M;
   size_t n_out = 1 + 3 * (size_t)n + 6;
   Kt.alloc(pool, std::max<size_t>(1, n_out * M * sizeof(double)));
-  FM_HIP(hipMemsetAsync(Kt.as<double>(), 0, n_out * M * sizeof(double), st));
-  owner.alloc(pool, std::max<size_t>(1, (size_t)s->n_bonds * sizeof(int)));
-  if (n > 0)
-    hipLaunchKernelGGL(k_bond_owner, dim3((n + 255) / 256), dim3(256), 0, st, n,
-                       s->bond_off.as<int>(), owner.as<int>());
-  for (int t = 0; t < s->nos; t++) {
-    int Ms = m->M_by_type[t], nt = s->n_by_type[t], ro = s->type_off[t];
-    int sbo = s->nbt_off[t], nbt = s->nbt_off[t + 1] - s->nbt_off[t];
-    if (Ms == 0) continue;
-    FM_CHECK(Ms < 65536, FM_ERR_CAPACITY, "more than 65535 sparse environments of one species");
-    DevBuf S(pool, std::max<size_t>(1, (size_t)Ms * std::max(nt, 1) * sizeof(double)));
-    DevBuf FD(pool, std::max<size_t>(1, (size_t)Ms * 3 * std::max(nbt, 1) * sizeof(double)));
-    DevBuf xn(pool, (size_t)Ms * sizeof(double));
-    FM_HIP(hipMemcpyAsync(xn.as<double>(), m->xnorm[t].data(), Ms * sizeof(double),
+  std::vector<double> xn(M);
+  for (int t = 0; t < s->nos; t++)
+    std::copy(m->xnorm[t].begin(), m->xnorm[t].end(), xn.begin() + m->off[t]);
+  DevBuf xnorm(pool, std::max<size_t>(1, (size_t)M * sizeof(double)));
+  if (M > 0)
+    FM_HIP(hipMemcpyAsync(xnorm.as<double>(), xn.data(), M * sizeof(double),
                           hipMemcpyHostToDevice, st));
-    if (nt > 0) {
-      EpArgs e1;
-      e1.W = S.as<void>();
-      e1.ldw = nt;
-      gemm_f64(st, EP_STORE, Ms, nt, nd, m->X[t].as<double>(), nd,
-               s->B.as<double>() + (size_t)ro * nd, nd, 0, e1);
+  auto doubles = [&](int t) {  // S, FD and P of species t
+    return (size_t)m->M_by_type[t] * (8 * (size_t)s->n_by_type[t] + 3 * (size_t)s->nb_by_type[t]);
+  };
+  for (int t0 = 0, t1; t0 < s->nos; t0 = t1) {
+    size_t total = doubles(t0);
+    for (t1 = t0 + 1; t1 < s->nos && total + doubles(t1) <= (4ull << 30) / 8; t1++)
+      total += doubles(t1);
+    DevBuf work(pool, std::max<size_t>(1, total * sizeof(double)));
+    double *at = work.as<double>();
+    std::vector<F64Gemm> products;
+    std::vector<EnvsArgs> envs;
+    for (int t = t0; t < t1; t++) {
+      int Ms = m->M_by_type[t], nt = s->n_by_type[t], ro = s->type_off[t];
+      int sbo = s->nbt_off[t], nbt = s->nbt_off[t + 1] - s->nbt_off[t];
+      if (Ms == 0) continue;
+      FM_CHECK(Ms < 65536, FM_ERR_CAPACITY,
+               "more than 65535 sparse environments of one species");
+      EnvsArgs e;
+      e.S = at;
+      e.FD = at + (size_t)nt * Ms;
+      e.P = at + ((size_t)nt + 3 * (size_t)nbt) * Ms;
+      at += doubles(t);
+      auto product = [&](const double *rows, int count, const double *out) {
+        EpArgs ep;
+        ep.W = const_cast<double *>(out);
+        ep.ldw = Ms;
+        products.push_back(
+            {rows, m->X[t].as<double>(), nd, nd, count, Ms, nd, 0, ep});
+      };
+      product(s->B.as<double>() + (size_t)ro * nd, nt, e.S);
+      product(s->DB.as<double>() + (size_t)3 * sbo * nd, 3 * nbt, e.FD);
+      e.n = n;
+      e.M = M;
+      e.cs = m->off[t];
+      e.Ms = Ms;
+      e.t = t;
+      e.ro = ro;
+      e.nt = nt;
+      e.sbo = sbo;
+      e.nbt = nbt;
+      e.sig2 = m->sigma * m->sigma;
+      e.power = m->power;
+      e.vol_inv = 1.0 / s->volume;
+      e.species = s->species.as<int>();
+      e.row_of_atom = s->row_of_atom.as<int>();
+      e.bond_off = s->bond_off.as<int>();
+      e.in_off = s->in_off.as<int>();
+      e.in_bond = s->in_bond.as<int>();
+      e.sb_pos = s->sb_pos.as<int>();
+      e.sb_row = s->sb_row.as<int>();
+      e.bond_q = s->bond_q.as<int>();
+      e.norm = s->norm.as<double>();
+      e.xnorm = xnorm.as<double>() + m->off[t];
+      e.rel = s->rel.as<double>();
+      e.fdots = s->fdots.as<double>();
+      e.Kt = Kt.as<double>();
+      envs.push_back(e);
     }
-    if (nbt > 0) {
-      EpArgs e2;
-      e2.W = FD.as<void>();
-      e2.ldw = 3 * (long long)nbt;
-      gemm_f64(st, EP_STORE, Ms, 3 * nbt, nd, m->X[t].as<double>(), nd,
-               s->DB.as<double>() + (size_t)3 * sbo * nd, nd, 0, e2);
+    gemm_f64_groups(st, EP_STORE, products);
+    for (const EnvsArgs &e : envs) {
+      unsigned by = (e.Ms + 63) / 64;
+      if (n > 0) hipLaunchKernelGGL(k_envs_rows, dim3(n, by), dim3(256), 0, st, e);
+      hipLaunchKernelGGL(k_envs_sums, dim3(by, 7), dim3(1024), 0, st, e);
     }
-    EnvsArgs e;
-    e.n = n;
-    e.nd = nd;
-    e.M = M;
-    e.cs = m->off[t];
-    e.Ms = Ms;
-    e.t = t;
-    e.ro = ro;
-    e.nt = nt;
-    e.sbo = sbo;
-    e.nbt = nbt;
-    e.sig2 = m->sigma * m->sigma;
-    e.power = m->power;
-    e.vol_inv = 1.0 / s->volume;
-    e.species = s->species.as<int>();
-    e.row_of_atom = s->row_of_atom.as<int>();
-    e.bond_off = s->bond_off.as<int>();
-    e.in_off = s->in_off.as<int>();
-    e.in_bond = s->in_bond.as<int>();
-    e.sb_pos = s->sb_pos.as<int>();
-    e.sb_row = s->sb_row.as<int>();
-    e.sb_bond = s->sb_bond.as<int>();
-    e.bond_q = s->bond_q.as<int>();
-    e.norm = s->norm.as<double>();
-    e.xnorm = xn.as<double>();
-    e.rel = s->rel.as<double>();
-    e.S = S.as<double>();
-    e.FD = FD.as<double>();
-    e.fdots = s->fdots.as<double>();
-    e.Kt = Kt.as<double>();
-    if (n > 0)
-      hipLaunchKernelGGL(k_envs_forces, dim3((n + 127) / 128, Ms), dim3(128), 0, st, e);
-    hipLaunchKernelGGL(k_envs_energy_stress, dim3(Ms), dim3(256), 0, st, e);
     FM_HIP(hipGetLastError());
     FM_HIP(hipStreamSynchronize(st));
   }
@@ -638,15 +647,18 @@ static void self_kernel(fm_model m, fm_structure s, DevBuf &kself) {
 void envs_struc(fm_model m, fm_structure s, double *K_out) {
   FM_CHECK(s->n_struct == 1, FM_ERR_INVALID, "kernel matrices are per single structure");
   compute_dervs(s);
-  DevBuf Kt, owner;
-  envs_struc_t(m, s, Kt, owner);
-  size_t n_out = 1 + 3 * (size_t)s->n + 6;
-  std::vector<double> kt(n_out * m->M);
-  FM_HIP(hipMemcpyAsync(kt.data(), Kt.as<double>(), kt.size() * sizeof(double),
-                        hipMemcpyDeviceToHost, s->ctx->stream));
-  FM_HIP(hipStreamSynchronize(s->ctx->stream));
-  for (int j = 0; j < m->M; j++)
-    for (size_t c = 0; c < n_out; c++) K_out[(size_t)j * n_out + c] = kt[c * m->M + j];
+  DevBuf Kt;
+  envs_struc_t(m, s, Kt);
+  hipStream_t st = s->ctx->stream;
+  int n_out = 1 + 3 * s->n + 6, M = m->M;
+  if (M == 0) return;
+  size_t bytes = (size_t)n_out * M * sizeof(double);
+  DevBuf K(&s->ctx->pool, bytes);
+  hipLaunchKernelGGL(k_transpose, dim3((M + 31) / 32, (n_out + 31) / 32), dim3(256), 0, st, n_out,
+                     M, Kt.as<double>(), K.as<double>());
+  FM_HIP(hipGetLastError());
+  FM_HIP(hipMemcpyAsync(K_out, K.as<double>(), bytes, hipMemcpyDeviceToHost, st));
+  FM_HIP(hipStreamSynchronize(st));
 }
 
 void self_kernel_struc(fm_model m, fm_structure s, double *kself_out) {
@@ -672,8 +684,8 @@ void predict_dense(fm_model m, fm_structure s, int kind, double *mean_efs, doubl
   compute_dervs(s);
   int M = m->M;
   size_t n_out = 1 + 3 * (size_t)s->n + 6;
-  DevBuf Kt, owner, ks;
-  envs_struc_t(m, s, Kt, owner);
+  DevBuf Kt, ks;
+  envs_struc_t(m, s, Kt);
   // mean = K^T alpha
   DevBuf mean(pool, n_out * sizeof(double));
   {

@@ -373,6 +373,7 @@ void predict_dense(fm_model m, fm_structure s, int kind, double *mean_efs, doubl
 void knorm_values(int lmax, double *out);
 // Constant tables of the current device (called when a context is created).
 void descriptor_setup();
+void dense_setup();
 // out[0..n] = exclusive scan of in[0..n), out[n] the total (fm_neighbors.hip);
 // with `host` (device address of pinned words) the total goes to host[0] too and
 // the device word `extra`, if given, to host[1].
