@@ -708,24 +708,24 @@ int fm_model_create(fm_context ctx, const fm_model_desc *d, fm_model *out) {
     m->M = M;
     FM_CHECK(M == 0 || (d->sparse_descriptors && d->sparse_norms), FM_ERR_INVALID,
              "null sparse descriptors");
-    m->host_alpha.assign(d->alpha, d->alpha + M);
     m->has_L = d->L_inv != nullptr;
     fm::Pool *pool = &ctx->pool;
+    // Norms, alpha and alpha without the empty sparse environments, which
+    // contribute nothing (normalized_dot_product.cpp:158-162).
+    std::vector<double> vec(3 * (size_t)M);
+    for (int j = 0; j < M; j++) {
+      vec[j] = d->sparse_norms[j];
+      vec[M + j] = d->alpha[j];
+      vec[2 * (size_t)M + j] = vec[j] < 1e-8 ? 0.0 : d->alpha[j];
+    }
+    m->vectors.alloc(pool, std::max<size_t>(1, vec.size() * sizeof(double)));
+    if (M)
+      FM_HIP(hipMemcpyAsync(m->vectors.as<double>(), vec.data(), vec.size() * sizeof(double),
+                            hipMemcpyHostToDevice, st));
+    m->xnorm.view(m->vectors, 0, M * sizeof(double));
+    m->alpha_full.view(m->vectors, M * sizeof(double), M * sizeof(double));
     for (int t = 0; t < m->nos; t++) {
       int Ms = m->M_by_type[t], c0 = m->off[t];
-      std::vector<double> X((size_t)Ms * nd, 0.0), XT((size_t)nd * Ms, 0.0), a(Ms, 0.0);
-      for (int j = 0; j < Ms; j++) {
-        double nrm = d->sparse_norms[c0 + j];
-        // Empty sparse environments contribute nothing
-        // (normalized_dot_product.cpp:158-162).
-        if (nrm < 1e-8) continue;
-        for (int k = 0; k < nd; k++) {
-          double v = d->sparse_descriptors[(size_t)(c0 + j) * nd + k] / nrm;
-          X[(size_t)j * nd + k] = v;
-          XT[(size_t)k * Ms + j] = v;
-        }
-        a[j] = d->alpha[c0 + j];
-      }
       auto up = [&](fm::DevBuf &buf, const void *src, size_t bytes) {
         buf.alloc(pool, std::max<size_t>(1, bytes));
         if (bytes) FM_HIP(hipMemcpyAsync(buf.as<void>(), src, bytes, hipMemcpyHostToDevice, st));
@@ -734,9 +734,12 @@ int fm_model_create(fm_context ctx, const fm_model_desc *d, fm_model *out) {
       m->XT.emplace_back();
       m->alpha.emplace_back();
       m->L.emplace_back();
-      up(m->X.back(), X.data(), X.size() * sizeof(double));
-      up(m->XT.back(), XT.data(), XT.size() * sizeof(double));
-      up(m->alpha.back(), a.data(), a.size() * sizeof(double));
+      size_t bytes = (size_t)Ms * nd * sizeof(double);
+      up(m->X.back(), d->sparse_descriptors + (size_t)c0 * nd, bytes);
+      m->XT.back().alloc(pool, std::max<size_t>(1, bytes));
+      m->alpha.back().view(m->vectors, (2 * (size_t)M + c0) * sizeof(double), Ms * sizeof(double));
+      fm::normalize_rows(st, Ms, nd, m->xnorm.as<double>() + c0, m->X.back().as<double>(),
+                         m->XT.back().as<double>());
       int rows = 0, lower = 1;
       if (m->has_L && Ms > 0) {
         // Rows [c0, r_end) of the L_inv column block; the reference takes
@@ -764,14 +767,7 @@ int fm_model_create(fm_context ctx, const fm_model_desc *d, fm_model *out) {
       m->L_rows.push_back(rows);
       m->L_lower.push_back(lower);
       if (rows != Ms) m->L_block_diag = false;
-      m->xnorm.emplace_back(d->sparse_norms ? d->sparse_norms + c0 : nullptr,
-                            d->sparse_norms ? d->sparse_norms + c0 + Ms : nullptr);
-      FM_HIP(hipStreamSynchronize(st));
     }
-    m->alpha_full.alloc(pool, std::max<size_t>(1, (size_t)M * sizeof(double)));
-    if (M)
-      FM_HIP(hipMemcpyAsync(m->alpha_full.as<double>(), m->host_alpha.data(), M * sizeof(double),
-                            hipMemcpyHostToDevice, st));
     m->has_R = d->R_inv != nullptr && M > 0;
     if (m->has_R) {
       // R_inv^T, the left operand of |R_inv^T k|^2; lower triangular when

@@ -243,7 +243,7 @@ __global__ __launch_bounds__(1024) void k_envs_sums(EnvsArgs e) {
 __global__ __launch_bounds__(256) void k_transpose(int rows, int cols, const double *in,
                                                    double *out) {
   __shared__ double t[32][33];
-  int c0 = blockIdx.x * 32, r0 = blockIdx.y * 32, x = threadIdx.x & 31, y = threadIdx.x >> 5;
+  int c0 = blockIdx.y * 32, r0 = blockIdx.x * 32, x = threadIdx.x & 31, y = threadIdx.x >> 5;
   for (int k = y; k < 32; k += 8)
     if (r0 + k < rows && c0 + x < cols) t[k][x] = in[(size_t)(r0 + k) * cols + c0 + x];
   __syncthreads();
@@ -467,13 +467,6 @@ static void envs_struc_t(fm_model m, fm_structure s, DevBuf &Kt) {
   int n = s->n, nd = s->nd, M = m->M;
   size_t n_out = 1 + 3 * (size_t)n + 6;
   Kt.alloc(pool, std::max<size_t>(1, n_out * M * sizeof(double)));
-  std::vector<double> xn(M);
-  for (int t = 0; t < s->nos; t++)
-    std::copy(m->xnorm[t].begin(), m->xnorm[t].end(), xn.begin() + m->off[t]);
-  DevBuf xnorm(pool, std::max<size_t>(1, (size_t)M * sizeof(double)));
-  if (M > 0)
-    FM_HIP(hipMemcpyAsync(xnorm.as<double>(), xn.data(), M * sizeof(double),
-                          hipMemcpyHostToDevice, st));
   auto doubles = [&](int t) {  // S, FD and P of species t
     return (size_t)m->M_by_type[t] * (8 * (size_t)s->n_by_type[t] + 3 * (size_t)s->nb_by_type[t]);
   };
@@ -526,7 +519,7 @@ static void envs_struc_t(fm_model m, fm_structure s, DevBuf &Kt) {
       e.sb_row = s->sb_row.as<int>();
       e.bond_q = s->bond_q.as<int>();
       e.norm = s->norm.as<double>();
-      e.xnorm = xnorm.as<double>() + m->off[t];
+      e.xnorm = m->xnorm.as<double>() + m->off[t];
       e.rel = s->rel.as<double>();
       e.fdots = s->fdots.as<double>();
       e.Kt = Kt.as<double>();
@@ -541,6 +534,34 @@ static void envs_struc_t(fm_model m, fm_structure s, DevBuf &Kt) {
     FM_HIP(hipGetLastError());
     FM_HIP(hipStreamSynchronize(st));
   }
+}
+
+// One 32 x 32 tile per block, both results in whole lines.
+__global__ __launch_bounds__(256) void k_normalize_rows(int rows, int cols, const double *norm,
+                                                        double *X, double *XT) {
+  __shared__ double t[32][33];
+  int r0 = blockIdx.x * 32, c0 = blockIdx.y * 32, x = threadIdx.x & 31, y = threadIdx.x >> 5;
+  for (; c0 < cols; c0 += 32 * gridDim.y) {
+    for (int k = y; k < 32; k += 8) {
+      int r = r0 + k, c = c0 + x;
+      if (r >= rows || c >= cols) continue;
+      double v = norm[r] < kEmptyThresh ? 0.0 : X[(size_t)r * cols + c] / norm[r];
+      X[(size_t)r * cols + c] = t[k][x] = v;
+    }
+    __syncthreads();
+    for (int k = y; k < 32; k += 8)
+      if (c0 + k < cols && r0 + x < rows) XT[(size_t)(c0 + k) * rows + r0 + x] = t[x][k];
+    __syncthreads();
+  }
+}
+
+void normalize_rows(hipStream_t st, int rows, int cols, const double *norm, double *X,
+                    double *XT) {
+  if (rows == 0) return;
+  int ty = std::min((cols + 31) / 32, 65535);
+  hipLaunchKernelGGL(k_normalize_rows, dim3((rows + 31) / 32, ty), dim3(256), 0, st, rows, cols,
+                     norm, X, XT);
+  FM_HIP(hipGetLastError());
 }
 
 static void self_kernel(fm_model m, fm_structure s, DevBuf &kself) {
@@ -654,7 +675,7 @@ void envs_struc(fm_model m, fm_structure s, double *K_out) {
   if (M == 0) return;
   size_t bytes = (size_t)n_out * M * sizeof(double);
   DevBuf K(&s->ctx->pool, bytes);
-  hipLaunchKernelGGL(k_transpose, dim3((M + 31) / 32, (n_out + 31) / 32), dim3(256), 0, st, n_out,
+  hipLaunchKernelGGL(k_transpose, dim3((n_out + 31) / 32, (M + 31) / 32), dim3(256), 0, st, n_out,
                      M, Kt.as<double>(), K.as<double>());
   FM_HIP(hipGetLastError());
   FM_HIP(hipMemcpyAsync(K_out, K.as<double>(), bytes, hipMemcpyDeviceToHost, st));

@@ -280,15 +280,13 @@ struct fm_model_s {
   // the B3 reordering.
   std::vector<fm::DevBuf> Xq, Xq_scale, XTs0, XTs1;
   bool xq_ready = false;
-  std::vector<double> host_alpha;
   // Non-zero once the sparse set has been permuted to the device order of
   // B3 descriptors (l-set major) for (n_tri, n_ls) = (b3_ntri, b3_nls).
   int b3_ntri = 0, b3_nls = 0;
-  // Dense (DTC / SOR) predictions: sparse norms per species, alpha in one
-  // vector, R_inv^T (M x M) and whether it is lower triangular, and whether
-  // L_inv is block diagonal over species.
-  std::vector<std::vector<double>> xnorm;
-  fm::DevBuf alpha_full, RinvT;
+  // Dense (DTC / SOR) predictions: sparse norms, alpha in one vector (both, as
+  // alpha, views of `vectors`), R_inv^T (M x M) and whether it is lower
+  // triangular, and whether L_inv is block diagonal over species.
+  fm::DevBuf vectors, xnorm, alpha_full, RinvT;
   bool has_R = false;
   int R_lower = 0;
   bool L_block_diag = true;
@@ -374,6 +372,9 @@ void knorm_values(int lmax, double *out);
 // Constant tables of the current device (called when a context is created).
 void descriptor_setup();
 void dense_setup();
+// X (rows x cols) with every row divided by its norm (zero below the empty
+// threshold), and its transpose.
+void normalize_rows(hipStream_t st, int rows, int cols, const double *norm, double *X, double *XT);
 // out[0..n] = exclusive scan of in[0..n), out[n] the total (fm_neighbors.hip);
 // with `host` (device address of pinned words) the total goes to host[0] too and
 // the device word `extra`, if given, to host[1].
