@@ -73,7 +73,8 @@ __device__ __forceinline__ void ylm_m_begin(YlmState<T, kGrad> &y, int mm, T ux,
 }
 
 template <typename T, bool kGrad, typename F>
-__device__ __forceinline__ void ylm_step(YlmState<T, kGrad> &y, int mm, int l, T uz, F &f) {
+__device__ __forceinline__ void ylm_step(YlmState<T, kGrad> &y, int mm, int l, T uz, F &f,
+                                         const double *knorm = c_knorm) {
   T ql, pl = 0;
   if (l == mm) {
     ql = y.dfact;
@@ -95,7 +96,7 @@ __device__ __forceinline__ void ylm_step(YlmState<T, kGrad> &y, int mm, int l, T
   for (int sgn = 0; sgn < 2; sgn++) {
     if (sgn == 1 && mm == 0) break;
     int lm = sgn ? base - mm : base + mm;
-    T K = (T)c_knorm[lm];
+    T K = (T)knorm[lm];
     T trig, dtx = 0, dty = 0;
     if (mm == 0) {
       trig = 1;
@@ -121,7 +122,8 @@ struct AllM {
   __device__ __forceinline__ bool operator()(int) const { return true; }
 };
 template <typename T, bool kGrad, int LC = -1, typename F, typename Mine = AllM>
-__device__ __forceinline__ void ylm_sweep(int L, T ux, T uy, T uz, F &&f, Mine mine = Mine()) {
+__device__ __forceinline__ void ylm_sweep(int L, T ux, T uy, T uz, F &&f, Mine mine = Mine(),
+                                          const double *knorm = c_knorm) {
   YlmState<T, kGrad> y;
   if constexpr (LC >= 0) {
 #pragma unroll
@@ -129,13 +131,13 @@ __device__ __forceinline__ void ylm_sweep(int L, T ux, T uy, T uz, F &&f, Mine m
       ylm_m_begin<T, kGrad>(y, mm, ux, uy);
       if (!mine(mm)) continue;
 #pragma unroll
-      for (int l = mm; l <= LC; l++) ylm_step<T, kGrad>(y, mm, l, uz, f);
+      for (int l = mm; l <= LC; l++) ylm_step<T, kGrad>(y, mm, l, uz, f, knorm);
     }
   } else {
     for (int mm = 0; mm <= L; mm++) {
       ylm_m_begin<T, kGrad>(y, mm, ux, uy);
       if (!mine(mm)) continue;
-      for (int l = mm; l <= L; l++) ylm_step<T, kGrad>(y, mm, l, uz, f);
+      for (int l = mm; l <= L; l++) ylm_step<T, kGrad>(y, mm, l, uz, f, knorm);
     }
   }
 }
@@ -162,6 +164,13 @@ __device__ __forceinline__ MfmaAcc<double>::type mfma_4(double a, double b,
                                                         MfmaAcc<double>::type c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
+// Keeps an accumulator in its registers across a loop's iterations (the
+// compiler otherwise moves it to vector registers and back in each, after
+// waiting for the product).
+template <typename A>
+__device__ __forceinline__ void keep_acc(A &acc) {
+  asm volatile("" : "+a"(acc));
+}
 template <typename T>
 __device__ __forceinline__ int mfma_row(int lane, int q) {
   return sizeof(T) == 8 ? (lane >> 4) + 4 * q : 4 * (lane >> 4) + q;
@@ -182,6 +191,12 @@ __host__ __device__ inline size_t b2_work(int nc, int H, int N, int ch, int nd) 
   return (size_t)pad2(nc) + ((tab > row ? tab : row) + 1) / 2 * 2;
 }
 
+// Products of sizes and indices below 2^24 (a full 32-bit product takes four
+// times as long).
+__device__ __forceinline__ int mul24(int a, int b) {
+  return (int)__umul24((unsigned)a, (unsigned)b);
+}
+
 // Ordering of LDS accesses among the W waves of an atom.
 template <int W>
 __device__ __forceinline__ void atom_sync() {
@@ -199,15 +214,16 @@ __device__ __forceinline__ void atom_sync() {
 // per species t and 16 harmonics, c_t += G_t^T Y_t on the matrix cores over
 // that species' rows only (A = g_n of the bonds, B = their Y_lm). Of W waves
 // per atom, wave w takes the harmonics with m mod 2 W in {w, 2 W - 1 - w}
-// (wave 0 the radial basis too) and every W-th (t, 16 harmonics) tile; each value is the
-// same whoever computes it.
+// (wave 0 the radial basis too) and every W-th tile of 16 harmonics; each value
+// is the same whoever computes it.
 template <typename T, int LC, int W>
 __device__ void accumulate_c(const B2Args &a, int i, int lane, int w, int ch, T *c, T *tab) {
   int si = a.species[i];
   int b0 = a.bond_off[i], b1 = a.bond_off[i + 1];
   int nc = a.nrad * a.H, H = a.H, N = a.N;
   T *Yt = tab, *gt = tab + ch * (size_t)H;
-  for (int k = 64 * w + lane; k < nc; k += 64 * W) c[k] = 0;
+  if (b0 == b1)
+    for (int k = 64 * w + lane; k < nc; k += 64 * W) c[k] = 0;
   int r16 = lane & 15, k4 = lane >> 4;
   unsigned long long below = (1ull << lane) - 1ull;
   for (int bb = b0; bb < b1; bb += ch) {
@@ -237,50 +253,70 @@ __device__ void accumulate_c(const B2Args &a, int i, int lane, int w, int ch, T 
       }
       T rinv = T(1) / (T)rp[0];
       T *yrow = Yt + (size_t)pos * H;
+      // Read in here, not before the loop: all of them exceed the scalar
+      // registers.
+      const double *knorm = c_knorm;
+      if (LC < 0 || LC > 4) asm volatile("" : "+s"(knorm));
       ylm_sweep<T, false, LC>(
           a.lmax, (T)rp[1] * rinv, (T)rp[2] * rinv, (T)rp[3] * rinv,
           [&](int lm, T Y, T, T, T) { yrow[lm] = Y; },
-          [&](int m) { m &= 2 * W - 1; return W == 1 || m == w || m == 2 * W - 1 - w; });
+          [&](int m) { m &= 2 * W - 1; return W == 1 || m == w || m == 2 * W - 1 - w; },
+          knorm);
     }
     atom_sync<W>();
-    int r0 = 0, tile = 0;
+    // Wave w takes the tiles of 16 harmonics w, w + W, ..: g_n is read once for
+    // all of them.
+    constexpr int HT = LC >= 0 ? ((LC + 1) * (LC + 1) + 15) / 16 : (kMaxH + 15) / 16;
+    constexpr int NT = (HT + W - 1) / W, n_step = sizeof(T) == 8 ? 4 : 1;
+    int n0 = mfma_row<T>(lane, 0), lm0 = 16 * w + r16;
+    int rc = min(r16, N - 1), r0 = 0;
     for (int t = 0; t < a.nos; t++) {
       int r1 = r0 + __popcll(__ballot(sj == t));  // rows [r0, r1) are species t
-      if (r1 > r0) {
-        for (int ct = 0; ct < H; ct += 16) {
-          if (W > 1 && tile++ % W != w) continue;
-          int lm = ct + r16;
-          typename MfmaAcc<T>::type acc;
+      if (r1 > r0 || bb == b0) {  // the first chunk sets all of c
+        typename MfmaAcc<T>::type acc[NT];
+        // c of this lane's first value; the others are n_step H apart.
+        int at = mul24(t * N + n0, H) + lm0;
 #pragma unroll
-          for (int qq = 0; qq < 4; qq++) {
-            int n = mfma_row<T>(lane, qq);
-            acc[qq] = (n < N && lm < H) ? c[(t * N + n) * H + lm] : T(0);
+        for (int j = 0; j < NT; j++) {
+          acc[j] = {};
+          if (bb > b0 && lm0 + 16 * W * j < H) {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+              if (n0 + q * n_step < N) acc[j][q] = c[at + 16 * W * j + q * n_step * H];
           }
-          // Four k-steps per iteration: the loads (clamped in bounds, then
-          // zeroed outside the species' rows) all issue before the MFMAs.
-          int rc = r16 < N ? r16 : N - 1, lc = lm < H ? lm : H - 1;
-          int rn = r16 < N ? r1 : 0, rh = lm < H ? r1 : 0;
-          for (int k0 = r0; k0 < r1; k0 += 16) {
-            T av[4], bv[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-              int b = k0 + 4 * u + k4;
-              int bc = min(b, ch - 1);
-              T x = gt[bc * N + rc];
-              T y = Yt[bc * H + lc];
-              av[u] = b < rn ? x : T(0);
-              bv[u] = b < rh ? y : T(0);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-              if (k0 + 4 * u < r1) acc = mfma_4(av[u], bv[u], acc);
-          }
-#pragma unroll
-          for (int qq = 0; qq < 4; qq++) {
-            int n = mfma_row<T>(lane, qq);
-            if (n < N && lm < H) c[(t * N + n) * H + lm] = acc[qq];
-          }
+          keep_acc(acc[j]);
         }
+        // Loads are clamped in bounds, then zeroed outside the species' rows.
+        int rn = r16 < N ? r1 : 0;
+#pragma unroll 1
+        for (int k0 = r0; k0 < r1; k0 += 8) {
+          T av[2], bv[NT][2];
+#pragma unroll
+          for (int u = 0; u < 2; u++) {
+            int b = k0 + 4 * u + k4, bc = min(b, ch - 1);
+            T x = gt[mul24(bc, N) + rc];
+            av[u] = b < rn ? x : T(0);
+            int yb = mul24(bc, H);
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+              T y = Yt[yb + min(lm0 + 16 * W * j, H - 1)];
+              bv[j][u] = b < r1 ? y : T(0);
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) acc[j] = mfma_4(av[u], bv[j][u], acc[j]);
+#pragma unroll
+          for (int j = 0; j < NT; j++) keep_acc(acc[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+          if (lm0 + 16 * W * j < H) {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+              if (n0 + q * n_step < N) c[at + 16 * W * j + q * n_step * H] = acc[j][q];
+          }
       }
       r0 = r1;
     }
@@ -325,11 +361,13 @@ __device__ __forceinline__ void slice4(double (&r)[4], unsigned (&packed)[kI8Sli
 // the atom's species-sorted row, with |B| and B.B; the coefficients c go to
 // HBM (Cg) for the adjoint. T = float is the bond pass of B3: c alone.
 //
-// What bounds it: vector instructions (five wave instructions in six cycles on
-// the 512-structure batch, where slicing each value on its own where the MFMA
-// tile leaves it was more than half of them). So the FP64 row is staged in LDS
-// (over the bond tables, no longer needed) and sliced four consecutive values
-// at a time, and the indices of a tile's values are formed once for all l. The
+// What bounds it: each wave's chain of vector instructions (they take half of
+// the cycles, the products an eighth; slicing each value on its own where the
+// MFMA tile leaves it was more than half of them). So the FP64 row is staged in
+// LDS (over the bond tables, no longer needed) and sliced four consecutive
+// values at a time, the three tiles of an l share two operands, and the tiles of
+// a species share g. 262144 atoms of three species, l_max 6, 42 bonds: 6.5 ms
+// (10.4 before, 2.4 at the rates of copies and FP64 products). The
 // row is the largest part of an atom's LDS; where that leaves a CU few atoms,
 // W = 2 or 4 waves share one and split every phase. B.B keeps its order of
 // sums (the variances depend on its last bit): wave 0 takes it from the staged
@@ -371,28 +409,27 @@ __global__ __launch_bounds__(256) void k_b2(B2Args a, T *B, double *norm, double
       typename MfmaAcc<T>::type acc = {};
       const T *ca = c + min(rt + r16, nr - 1) * H + lm0 + k4;
       const T *cb = c + min(cc + r16, nr - 1) * H + lm0 + k4;
-#pragma unroll 2
+#pragma unroll 1
       for (int k0 = 0; k0 < nm; k0 += 4) {
         T x = ca[k0], y = cb[k0];
         bool in = k0 + k4 < nm;
         acc = mfma_4(in ? x : T(0), in ? y : T(0), acc);
+        keep_acc(acc);
       }
       return acc;
     };
     // Place of this lane's value q of tile (rt, cc) for l = 0, or -1.
     auto place = [&](int rt, int cc, int q) {
       int n1 = rt + mfma_row<T>(lane, q), n2 = cc + r16;
-      return n1 < nr && n2 < nr && n2 >= n1 ? (n1 * nr - (n1 * (n1 - 1)) / 2 + (n2 - n1)) * L1
-                                            : -1;
+      int at = mul24(mul24(n1, nr) - (mul24(n1, n1 - 1) >> 1) + (n2 - n1), L1);
+      return n1 < nr && n2 < nr && n2 >= n1 ? at : -1;
     };
     // The row's power-of-two scale 2^E from its largest element, which is a
     // diagonal one (Cauchy-Schwarz within each l); every wave finds it.
     auto exponent = [&](auto diagonal) {
       double mx = 0;
-      for (int q = lane; q < nr * L1; q += 64) {
-        int n = q / L1;
-        mx = fmax(mx, diagonal(n, q - n * L1));
-      }
+      for (int n = lane; n < nr; n += 64)
+        for (int l = 0; l < L1; l++) mx = fmax(mx, diagonal(n, l));
 #pragma unroll
       for (int off = 32; off >= 1; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
       int E = 0;
@@ -400,23 +437,52 @@ __global__ __launch_bounds__(256) void k_b2(B2Args a, T *B, double *norm, double
       return E;
     };
     if (nr <= 32) {
-      // Up to three tiles: (0, 0), (0, 16), (16, 16), their places kept.
+      // Up to three tiles, (0, 0), (0, 16) and (16, 16), of two operands; their
+      // places kept. Wave of an l: the long ones first, each paired with a short
+      // one.
       int at[3][4];
 #pragma unroll
       for (int u = 0; u < 3; u++)
 #pragma unroll
         for (int q = 0; q < 4; q++) at[u][q] = place(u == 2 ? 16 : 0, u ? 16 : 0, q);
-      int nt = nr > 16 ? 3 : 1, tile = 0;
+      int nt = nr > 16 ? 3 : 1;
+      const T *c0 = c + mul24(min(r16, nr - 1), H) + k4;
+      const T *c1 = c + mul24(min(16 + r16, nr - 1), H) + k4;
       for (int l = 0; l <= a.lmax; l++) {
+        if (W > 1 && (2 * l > a.lmax ? a.lmax - l : l + 1) % W != w) continue;
+        int nm = 2 * l + 1, lm0 = l * l;
+        typename MfmaAcc<T>::type acc[3] = {};
+#pragma unroll
+        for (int u = 0; u < 3; u++) keep_acc(acc[u]);
+        if (nt == 3) {
+#pragma unroll 1
+          for (int k0 = 0; k0 < nm; k0 += 4) {
+            bool in = k0 + k4 < nm;
+            T x = c0[lm0 + k0], y = c1[lm0 + k0];
+            x = in ? x : T(0);
+            y = in ? y : T(0);
+            acc[0] = mfma_4(x, x, acc[0]);
+            acc[1] = mfma_4(x, y, acc[1]);
+            acc[2] = mfma_4(y, y, acc[2]);
+#pragma unroll
+            for (int u = 0; u < 3; u++) keep_acc(acc[u]);
+          }
+        } else {
+#pragma unroll 1
+          for (int k0 = 0; k0 < nm; k0 += 4) {
+            T x = c0[lm0 + k0];
+            x = k0 + k4 < nm ? x : T(0);
+            acc[0] = mfma_4(x, x, acc[0]);
+            keep_acc(acc[0]);
+          }
+        }
 #pragma unroll
         for (int u = 0; u < 3; u++) {
           if (u >= nt) continue;
-          if (W > 1 && tile++ % W != w) continue;
-          auto acc = tile_of(l, u == 2 ? 16 : 0, u ? 16 : 0);
 #pragma unroll
           for (int q = 0; q < 4; q++)
             if (at[u][q] >= 0) {
-              T v = acc[q];
+              T v = acc[u][q];
               bst[at[u][q] + l] = v;
               if (W == 1) s2 += v * v;
             }
@@ -515,7 +581,7 @@ __global__ __launch_bounds__(256) void k_b2(B2Args a, T *B, double *norm, double
     if (!stage) {
     } else if constexpr (MIXED) {
       int E = exponent([&](int n, int l) {
-        return (double)bst[(n * nr - (n * (n - 1)) / 2) * L1 + l];
+        return (double)bst[mul24(mul24(n, nr) - (mul24(n, n - 1) >> 1), L1) + l];
       });
       double inv = ldexp(1.0, -E);
       if (tid == 0) mo.scale[row] = ldexp(1.0, E);
@@ -544,10 +610,13 @@ __global__ __launch_bounds__(256) void k_b2(B2Args a, T *B, double *norm, double
         slice4(r, packed);
         // k0's step of the row tile (kI8Slices blocks of kI8TileA rows), then
         // its place in the row.
-        int8_t *dst = qp + (size_t)(k0 >> 6) * (kI8Slices * kI8TileA * kI8Pad) + (k0 & (kI8Pad - 1));
+        unsigned at = mul24(k0 >> 6, kI8Slices * kI8TileA * kI8Pad) + (k0 & (kI8Pad - 1));
 #pragma unroll
-        for (int p = 0; p < kI8Slices; p++)
-          *reinterpret_cast<unsigned *>(dst + p * (kI8TileA * kI8Pad)) = packed[p];
+        for (int p = 0; p < kI8Slices; p++) {
+          int8_t *dst = qp + p * (kI8TileA * kI8Pad);
+          asm volatile("" : "+s"(dst));  // scalar base, one vector offset
+          *reinterpret_cast<unsigned *>(dst + at) = packed[p];
+        }
       }
     } else {
       T *Brow = B + (size_t)row * a.nd;
@@ -1070,13 +1139,12 @@ void launch_b2(fm_structure s, bool want_b2) {
   // 64-bond chunks fill all lanes of the bond basis and take half the passes;
   // they cost LDS only where the row is shorter than their tables, and are
   // used where four atoms still fit a CU (times with 64 and with 32 are within
-  // 5 %: 6.75 and 6.77 ms for 262144 atoms of three species, 0.62 and 0.60 ms
-  // for 32000 of two).
+  // 5 %).
   // Waves per atom: the fewest that give the CU 12 waves (its registers hold
-  // 16). One, two and four waves: 8.7, 8.0 and 6.8 ms (262144 atoms, three
-  // species, l_max 6, four atoms per CU), 0.78, 0.74 and 0.61 ms (32000 atoms, two
-  // species, four per CU), 2.43, 2.35 and 3.19 ms (512 structures, l_max 4,
-  // seven per CU: four waves only add instructions).
+  // 16). One, two and four waves: 8.5, 7.7 and 6.5 ms (262144 atoms, three
+  // species, l_max 6, four atoms per CU), 0.71, 0.70 and 0.57 ms (32000 atoms, two
+  // species, four per CU), 2.31, 2.24 and 3.22 ms (512 structures, l_max 4,
+  // seven per CU).
   int row = a.nd;
   auto work_of = [&](int ch) {
     return b2_work(a.nrad * a.H, a.H, a.N, ch, want_b2 ? row : 0);
