@@ -25,28 +25,29 @@ namespace fm {
 // ---------------------------------------------------------------------------
 constexpr int kScanBlock = 1024;
 
-__device__ __forceinline__ int block_excl_scan(int v, int *sh, int &total) {
+template <typename V>
+__device__ __forceinline__ V block_excl_scan(V v, V *sh, V &total) {
   // 1024 threads = 16 waves.
   int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  int x = v;
+  V x = v;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
-    int y = __shfl_up(x, off, 64);
+    V y = __shfl_up(x, off, 64);
     if (lane >= off) x += y;
   }
   if (lane == 63) sh[wid] = x;
   __syncthreads();
   if (wid == 0) {
-    int w = lane < 16 ? sh[lane] : 0;
+    V w = lane < 16 ? sh[lane] : 0;
 #pragma unroll
     for (int off = 1; off < 16; off <<= 1) {
-      int y = __shfl_up(w, off, 64);
+      V y = __shfl_up(w, off, 64);
       if (lane >= off) w += y;
     }
     if (lane < 16) sh[lane] = w;
   }
   __syncthreads();
-  int base = wid ? sh[wid - 1] : 0;
+  V base = wid ? sh[wid - 1] : 0;
   total = sh[15];
   __syncthreads();
   return base + x - v;
@@ -137,66 +138,126 @@ struct SetupWords {
   int flags, max_species, max_count;
 };
 
-// Per atom: the structure it belongs to, its own copy of the caller's species
-// and position (where those are in device memory), their checks (flags: bit 1
+struct SetupArgs {
+  int n, n_struct, n_bins;
+  const double *src_pos;
+  const int *src_species;
+  double *pos;
+  int *species;
+  const CellArgs *cas;
+  const int *atom_off, *bin_off;
+  int *atom_struct;
+  double *wrapped;
+  int *bin, *bstart, *order;
+  SetupWords *words;
+};
+
+// Atom i: the structure it belongs to, its own copy of the caller's species
+// and position (where those are in device memory), their checks (bad: bit 1
 // non-finite position, bit 2 negative species), the wrapped position
-// (structure.cpp:120-133), its bin and the bin's count.
-__global__ __launch_bounds__(256) void k_setup(int n, int n_struct, const double *src_pos,
-                                               const int *src_species, double *pos, int *species,
-                                               const CellArgs *cas, const int *atom_off,
-                                               const int *bin_off, int *atom_struct,
-                                               double *wrapped, int *bin, int *bcount,
-                                               SetupWords *words) {
+// (structure.cpp:120-133) and its bin, which is returned.
+__device__ __forceinline__ int setup_atom(const SetupArgs &a, int i, int &sp, int &bad) {
+  sp = a.src_species[i];
+  int k = 0;  // the structure with atom_off[k] <= i < atom_off[k + 1]
+  if (a.n_struct > 1) {
+    int lo = 0, hi = a.n_struct;
+    while (hi - lo > 1) {
+      int mid = (lo + hi) >> 1;
+      if (a.atom_off[mid] <= i) lo = mid;
+      else hi = mid;
+    }
+    k = lo;
+  }
+  a.atom_struct[i] = k;
+  const CellArgs &ca = a.cas[k];
+  double p[3] = {a.src_pos[3 * i], a.src_pos[3 * i + 1], a.src_pos[3 * i + 2]};
+  if (a.pos != a.src_pos) {
+    for (int q = 0; q < 3; q++) a.pos[3 * i + q] = p[q];
+    a.species[i] = sp;
+  }
+  for (int q = 0; q < 3; q++)
+    if (!isfinite(p[q])) bad |= 1;
+  if (sp < 0) bad |= 2;
+  double r1[3], fr[3], w1[3], w[3];
+  row3(p, ca.ct, r1);
+  row3(r1, ca.cdi, fr);
+  for (int q = 0; q < 3; q++) fr[q] = fr[q] - floor(fr[q]);
+  row3(fr, ca.cd, w1);
+  row3(w1, ca.cti, w);
+  for (int q = 0; q < 3; q++) a.wrapped[3 * i + q] = w[q];
+  // Bin from the fractional coordinates of the wrapped position.
+  row3(w, ca.ct, r1);
+  row3(r1, ca.cdi, fr);
+  int q3[3];
+  for (int q = 0; q < 3; q++) {
+    int b = (int)floor(fr[q] * ca.nb[q]);
+    q3[q] = min(max(b, 0), ca.nb[q] - 1);
+  }
+  return a.bin_off[k] + (q3[0] * ca.nb[1] + q3[1]) * ca.nb[2] + q3[2];
+}
+
+// One atom per thread; bcount is zero on entry.
+__global__ __launch_bounds__(256) void k_setup(SetupArgs a, int *bcount) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
-  bool live = i < n;
-  int sp = live ? src_species[i] : -1;
-  int bad = 0;
-  if (live) {
-    int k = 0;  // the structure with atom_off[k] <= i < atom_off[k + 1]
-    if (n_struct > 1) {
-      int lo = 0, hi = n_struct;
-      while (hi - lo > 1) {
-        int mid = (lo + hi) >> 1;
-        if (atom_off[mid] <= i) lo = mid;
-        else hi = mid;
-      }
-      k = lo;
-    }
-    atom_struct[i] = k;
-    const CellArgs &ca = cas[k];
-    double p[3] = {src_pos[3 * i], src_pos[3 * i + 1], src_pos[3 * i + 2]};
-    if (pos != src_pos) {
-      for (int q = 0; q < 3; q++) pos[3 * i + q] = p[q];
-      species[i] = sp;
-    }
-    for (int q = 0; q < 3; q++)
-      if (!isfinite(p[q])) bad |= 1;
-    if (sp < 0) bad |= 2;
-    double r1[3], fr[3], w1[3], w[3];
-    row3(p, ca.ct, r1);
-    row3(r1, ca.cdi, fr);
-    for (int q = 0; q < 3; q++) fr[q] = fr[q] - floor(fr[q]);
-    row3(fr, ca.cd, w1);
-    row3(w1, ca.cti, w);
-    for (int q = 0; q < 3; q++) wrapped[3 * i + q] = w[q];
-    // Bin from the fractional coordinates of the wrapped position.
-    row3(w, ca.ct, r1);
-    row3(r1, ca.cdi, fr);
-    int q3[3];
-    for (int q = 0; q < 3; q++) {
-      int b = (int)floor(fr[q] * ca.nb[q]);
-      q3[q] = min(max(b, 0), ca.nb[q] - 1);
-    }
-    int b = bin_off[k] + (q3[0] * ca.nb[1] + q3[1]) * ca.nb[2] + q3[2];
-    bin[i] = b;
+  int sp = -1, bad = 0;
+  if (i < a.n) {
+    int b = setup_atom(a, i, sp, bad);
+    a.bin[i] = b;
     atomicAdd(&bcount[b], 1);
   }
   // One atomic per wave for the largest species.
   int mx = sp;
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) mx = max(mx, __shfl_xor(mx, off, 64));
-  if ((threadIdx.x & 63) == 0 && mx > 0) atomicMax(&words->max_species, mx);
-  if (bad) atomicOr(&words->flags, bad);
+  if ((threadIdx.x & 63) == 0 && mx > 0) atomicMax(&a.words->max_species, mx);
+  if (bad) atomicOr(&a.words->flags, bad);
+}
+
+// The whole of it (zeros, k_setup, the scan of the bins and k_bin_fill) in one
+// workgroup, for up to kSmallAtoms atoms and as many bins as one scan takes:
+// 5 us for 108 atoms and 13 us for 1,024 of them, where the four launches took
+// 12 and 15 and the gaps between them.
+constexpr int kSmallAtoms = 2048;
+__global__ __launch_bounds__(kScanBlock) void k_setup_small(SetupArgs a, int *host_words) {
+  __shared__ int cnt[kScanBlock * kScanItems], sh[16], flags, mx;
+  for (int k = threadIdx.x; k < a.n_bins; k += kScanBlock) cnt[k] = 0;
+  if (threadIdx.x == 0) flags = mx = 0;
+  __syncthreads();
+  int bin[kSmallAtoms / kScanBlock];
+#pragma unroll
+  for (int e = 0; e < kSmallAtoms / kScanBlock; e++) {
+    int i = threadIdx.x + e * kScanBlock, sp = -1, bad = 0;
+    if (i >= a.n) continue;
+    bin[e] = a.bin[i] = setup_atom(a, i, sp, bad);
+    atomicAdd(&cnt[bin[e]], 1);
+    if (sp > 0) atomicMax(&mx, sp);
+    if (bad) atomicOr(&flags, bad);
+  }
+  __syncthreads();
+  int i0 = threadIdx.x * kScanItems, v[kScanItems], sum = 0, tot;
+#pragma unroll
+  for (int e = 0; e < kScanItems; e++) {
+    v[e] = i0 + e < a.n_bins ? cnt[i0 + e] : 0;
+    sum += v[e];
+  }
+  int x = block_excl_scan(sum, sh, tot);
+#pragma unroll
+  for (int e = 0; e < kScanItems; e++) {
+    if (i0 + e < a.n_bins) a.bstart[i0 + e] = cnt[i0 + e] = x;
+    x += v[e];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < kSmallAtoms / kScanBlock; e++) {
+    int i = threadIdx.x + e * kScanBlock;
+    if (i < a.n) a.order[atomicAdd(&cnt[bin[e]], 1)] = i;
+  }
+  if (threadIdx.x == 0) {
+    a.bstart[a.n_bins] = tot;
+    a.words->max_count = 0;
+    host_words[0] = flags;
+    host_words[1] = mx;
+  }
 }
 
 // Places each atom in its bin (any order within a bin: neighbours are sorted
@@ -533,16 +594,32 @@ void build_neighbors(fm_structure s, const int *species_dev, const double *posit
   int *bcount = reinterpret_cast<int *>(words + 1), *maxc = &words->max_count;
   int *hw = ctx->pinned_dev;
   int tpb = 256, nblk = (n + tpb - 1) / tpb;
-  FM_HIP(hipMemsetAsync(zeros.as<void>(), 0, sizeof(SetupWords) + (size_t)ncell * sizeof(int), st));
-  hipLaunchKernelGGL(k_setup, dim3(nblk), dim3(tpb), 0, st, n, s->n_struct,
-                     positions_dev ? positions_dev : s->positions.as<double>(),
-                     species_dev ? species_dev : s->species.as<int>(), s->positions.as<double>(),
-                     s->species.as<int>(), cas, s->d_atom_off.as<int>(), boffp,
-                     s->atom_struct.as<int>(), s->wrapped.as<double>(), bin.as<int>(), bcount,
-                     words);
-  scan_exclusive(ctx, bcount, bstart.as<int>(), ncell);
-  hipLaunchKernelGGL(k_bin_fill, dim3(nblk), dim3(tpb), 0, st, n, bin.as<int>(), bstart.as<int>(),
-                     bcount, order.as<int>(), words, hw);
+  SetupArgs sa{n,
+               s->n_struct,
+               ncell,
+               positions_dev ? positions_dev : s->positions.as<double>(),
+               species_dev ? species_dev : s->species.as<int>(),
+               s->positions.as<double>(),
+               s->species.as<int>(),
+               cas,
+               s->d_atom_off.as<int>(),
+               boffp,
+               s->atom_struct.as<int>(),
+               s->wrapped.as<double>(),
+               bin.as<int>(),
+               bstart.as<int>(),
+               order.as<int>(),
+               words};
+  if (n <= kSmallAtoms && ncell <= kScanBlock * kScanItems) {
+    hipLaunchKernelGGL(k_setup_small, dim3(1), dim3(kScanBlock), 0, st, sa, hw);
+  } else {
+    FM_HIP(hipMemsetAsync(zeros.as<void>(), 0, sizeof(SetupWords) + (size_t)ncell * sizeof(int),
+                          st));
+    hipLaunchKernelGGL(k_setup, dim3(nblk), dim3(tpb), 0, st, sa, bcount);
+    scan_exclusive(ctx, bcount, bstart.as<int>(), ncell);
+    hipLaunchKernelGGL(k_bin_fill, dim3(nblk), dim3(tpb), 0, st, n, bin.as<int>(),
+                       bstart.as<int>(), bcount, order.as<int>(), words, hw);
+  }
   int wblk = (n + kNbrWaves - 1) / kNbrWaves;
   // One pass over the candidates that also parks each atom's sorted keys
   // (kNbrCapSmall per atom, while that area stays within 16 GB); else a
@@ -607,17 +684,26 @@ void build_neighbors(fm_structure s, const int *species_dev, const double *posit
 // Bonds are the neighbours within the species-pair cutoff, kept in neighbour
 // order. One wave per atom walks its neighbour list 64 entries at a time; a
 // ballot gives each kept entry its place.
+// Cutoffs passed by value for up to four species, written to memory by the
+// first kernel that has them.
+struct CutoffArgs {
+  double c[16];
+  int n;  // 0: in memory already
+};
+
 __global__ __launch_bounds__(256) void k_bond_count(int n, const int *species, const int *cum,
                                                     const int *nspec, const double *rel,
-                                                    const double *cutoffs, int nos, int *bcount,
-                                                    int *in_count) {
+                                                    CutoffArgs cut, double *cutoffs, int nos,
+                                                    int *bcount, int *in_count) {
   int lane = threadIdx.x & 63;
   int i = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (blockIdx.x == 0 && threadIdx.x < cut.n) cutoffs[threadIdx.x] = cut.c[threadIdx.x];
+  const double *rc = cut.n ? cut.c : cutoffs;
   if (i >= n) return;
   int si = species[i], c = 0;
   for (int q0 = cum[i]; q0 < cum[i + 1]; q0 += 64) {
     int q = q0 + lane;
-    bool keep = q < cum[i + 1] && rel[4 * (size_t)q] <= cutoffs[si * nos + nspec[q]];
+    bool keep = q < cum[i + 1] && rel[4 * (size_t)q] <= rc[si * nos + nspec[q]];
     c += __popcll(__ballot(keep));
   }
   if (lane == 0) {
@@ -630,11 +716,12 @@ __global__ __launch_bounds__(256) void k_bond_fill(int n, const int *species, co
                                                    const int *nspec, const double *rel,
                                                    const double *cutoffs, int nos,
                                                    const int *boff, const int *sidx, int *bond_q,
-                                                   int *in_count, const int *bonds_by_type,
-                                                   int *host_by_type) {
+                                                   int *in_count, int *in_slot,
+                                                   const int *bonds_by_type, int *host_by_type) {
   int lane = threadIdx.x & 63;
   int i = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (blockIdx.x == 0 && threadIdx.x < nos) host_by_type[threadIdx.x] = bonds_by_type[threadIdx.x];
+  if (bonds_by_type && blockIdx.x == 0 && threadIdx.x < nos)
+    host_by_type[threadIdx.x] = bonds_by_type[threadIdx.x];
   if (i >= n) return;
   int si = species[i], o = boff[i];
   unsigned long long below = (1ull << lane) - 1ull;
@@ -643,22 +730,44 @@ __global__ __launch_bounds__(256) void k_bond_fill(int n, const int *species, co
     bool keep = q < cum[i + 1] && rel[4 * (size_t)q] <= cutoffs[si * nos + nspec[q]];
     unsigned long long m = __ballot(keep);
     if (keep) {
-      bond_q[o + __popcll(m & below)] = q;
-      atomicAdd(&in_count[sidx[q]], 1);
+      int b = o + __popcll(m & below);
+      bond_q[b] = q;
+      in_slot[b] = atomicAdd(&in_count[sidx[q]], 1);
     }
     o += __popcll(m);
   }
 }
 
-// Incoming bonds of each atom in any order, counting in_count down (the launch
-// covers all neighbours; the bonds are the first bond_off[n] of them).
-__global__ __launch_bounds__(256) void k_in_fill(int n, const int *bond_off, const int *bond_q,
-                                                 const int *sidx, const int *in_off,
-                                                 int *in_count, int *in_bond) {
-  int b = blockIdx.x * blockDim.x + threadIdx.x;
+// Incoming bonds of each atom in the order in which the fill counted them (the
+// launch covers all neighbours; the bonds are the first bond_off[n] of them).
+// With in_count (up to one scan of atoms) every workgroup scans the counts itself
+// and the first one writes in_off, for a launch less.
+__global__ __launch_bounds__(kScanBlock) void k_in_fill(int n, const int *bond_off,
+                                                        const int *bond_q, const int *sidx,
+                                                        const int *in_count, int *in_off,
+                                                        const int *in_slot, int *in_bond) {
+  __shared__ int off[kScanBlock * kScanItems], sh[16];
+  if (in_count) {
+    int i0 = threadIdx.x * kScanItems, v[kScanItems], sum = 0, tot;
+#pragma unroll
+    for (int e = 0; e < kScanItems; e++) {
+      v[e] = i0 + e < n ? in_count[i0 + e] : 0;
+      sum += v[e];
+    }
+    int x = block_excl_scan(sum, sh, tot);
+#pragma unroll
+    for (int e = 0; e < kScanItems; e++) {
+      off[i0 + e] = x;
+      if (blockIdx.x == 0 && i0 + e < n) in_off[i0 + e] = x;
+      x += v[e];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) in_off[n] = tot;
+    __syncthreads();
+  }
+  int b = blockIdx.x * kScanBlock + threadIdx.x;
   if (b >= bond_off[n]) return;
   int j = sidx[bond_q[b]];
-  in_bond[in_off[j] + atomicAdd(&in_count[j], -1) - 1] = b;
+  in_bond[(in_count ? off[j] : in_off[j]) + in_slot[b]] = b;
 }
 
 // Incoming bonds of atom j in ascending bond order (so the force gather sums
@@ -698,23 +807,16 @@ __global__ __launch_bounds__(kRowBlock) void k_species_count(int n, const int *s
   for (int t = threadIdx.x; t < nos; t += kRowBlock) hist[(size_t)t * gridDim.x + blockIdx.x] = cnt[t];
 }
 
-// Cutoffs passed by value for up to four species.
-struct CutoffArgs {
-  double c[16];
-};
-
 // Row of each atom: the rows of the lower species and of the blocks before
 // (`off`, the scan of the counts above; with one block from the block itself),
 // then the atom's rank in its block. Block 0 also writes the species' atom
 // counts to the host, the slice-row shift of each species (its rows start a
-// tile of `tile` slice rows), zeros for the bond counts by species, and the
-// cutoffs when they come by value.
+// tile of `tile` slice rows) and zeros for the bond counts by species.
 __global__ __launch_bounds__(kRowBlock) void k_species_rows(int n, const int *species, int nos,
                                                             const int *off, int *row_of_atom,
                                                             int *atom_of_row, int *host_by_type,
                                                             int tile, int *shift,
-                                                            int *bonds_by_type, CutoffArgs cut,
-                                                            int n_cut, double *cutoffs) {
+                                                            int *bonds_by_type) {
   extern __shared__ int wc[];  // [16 waves][nos], then the species' first rows [nos + 1]
   int *first = wc + 16 * nos;
   int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nb = gridDim.x;
@@ -747,7 +849,6 @@ __global__ __launch_bounds__(kRowBlock) void k_species_rows(int n, const int *sp
       host_by_type[t] = first[t + 1] - first[t];
       bonds_by_type[t] = 0;
     }
-    if (threadIdx.x < n_cut) cutoffs[threadIdx.x] = cut.c[threadIdx.x];
     if (threadIdx.x == 0) {
       int rows = 0;
       for (int t = 0; t < nos; t++) {
@@ -772,6 +873,61 @@ __global__ __launch_bounds__(256) void k_bonds_by_type(int n, const int *species
     if (cnt[t]) atomicAdd(&bonds_by_type[t], cnt[t]);
 }
 
+// Species rows, bonds by species and bond offsets in one workgroup, for as many
+// atoms as one scan takes (eight consecutive ones per thread): a scan of (atoms,
+// bonds) per species, then one of the bonds. 5 us for 108 atoms, 7 us for 1,024
+// and 20 us for 8,190, where three to five launches took 10 to 20 and the gaps
+// between them.
+__global__ __launch_bounds__(kScanBlock) void k_rows_bonds(int n, const int *species, int nos,
+                                                           const int *bcount, int *row_of_atom,
+                                                           int *atom_of_row, int *bond_off,
+                                                           int tile, int *shift,
+                                                           int *host_by_type, int *host_bonds,
+                                                           int *host_total) {
+  __shared__ long long sh[16];
+  __shared__ int sh1[16];
+  int i0 = threadIdx.x * kScanItems, sp[kScanItems], bc[kScanItems], sum = 0, tot;
+#pragma unroll
+  for (int e = 0; e < kScanItems; e++) {
+    bool in = i0 + e < n;
+    sp[e] = in ? species[i0 + e] : -1;
+    bc[e] = in ? bcount[i0 + e] : 0;
+    sum += bc[e];
+  }
+  int first = 0, slice_rows = 0;
+  for (int t = 0; t < nos; t++) {
+    long long v = 0, all;
+#pragma unroll
+    for (int e = 0; e < kScanItems; e++)
+      if (sp[e] == t) v += (1ll << 32) + bc[e];
+    int r = first + (int)(block_excl_scan(v, sh, all) >> 32);
+#pragma unroll
+    for (int e = 0; e < kScanItems; e++)
+      if (sp[e] == t) {
+        row_of_atom[i0 + e] = r;
+        atom_of_row[r++] = i0 + e;
+      }
+    int atoms = (int)(all >> 32);
+    if (threadIdx.x == 0) {
+      host_by_type[t] = atoms;
+      host_bonds[t] = (int)all;
+      shift[t] = slice_rows - first;
+    }
+    first += atoms;
+    slice_rows += (atoms + tile - 1) / tile * tile;
+  }
+  int x = block_excl_scan(sum, sh1, tot);
+#pragma unroll
+  for (int e = 0; e < kScanItems; e++) {
+    if (i0 + e < n) bond_off[i0 + e] = x;
+    x += bc[e];
+  }
+  if (threadIdx.x == 0) {
+    bond_off[n] = tot;
+    host_total[0] = tot;
+  }
+}
+
 // Pinned words of a bond build: the bond total, then atoms and bonds by species.
 constexpr int kWordBonds = 4, kWordTypes = 8;
 
@@ -786,55 +942,66 @@ void build_bonds(fm_structure s) {
   int nc = nos * nos;
   s->d_cutoffs.alloc(pool, nc * sizeof(double));
   CutoffArgs cut{};
-  bool by_value = nc <= 16;
-  if (by_value)
+  if (nc <= 16) {
     std::copy(s->cutoffs.begin(), s->cutoffs.end(), cut.c);
-  else
+    cut.n = nc;
+  } else {
     FM_HIP(hipMemcpyAsync(s->d_cutoffs.as<double>(), s->cutoffs.data(), nc * sizeof(double),
                           hipMemcpyHostToDevice, st));
-  // Species-sorted rows: one launch up to 1,024 atoms, else three.
+  }
   s->row_of_atom.alloc(pool, (size_t)n * sizeof(int));
   s->atom_of_row.alloc(pool, (size_t)n * sizeof(int));
   s->q_shift.alloc(pool, nos * sizeof(int));
+  s->bond_off.alloc(pool, ((size_t)n + 1) * sizeof(int));
   DevBuf by_type(pool, nos * sizeof(int));
-  int nb = (n + kRowBlock - 1) / kRowBlock;
+  DevBuf bcount(pool, (size_t)n * sizeof(int)), in_count(pool, (size_t)n * sizeof(int));
+  hipLaunchKernelGGL(k_bond_count, dim3((n + 3) / 4), dim3(256), 0, st, n, s->species.as<int>(),
+                     s->cumulative.as<int>(), s->nspecies.as<int>(), s->rel.as<double>(), cut,
+                     s->d_cutoffs.as<double>(), nos, bcount.as<int>(), in_count.as<int>());
+  bool one_block = n <= kScanBlock * kScanItems;
   DevBuf hist, off;
-  if (nb > 1) {
+  if (one_block) {
+    hipLaunchKernelGGL(k_rows_bonds, dim3(1), dim3(kScanBlock), 0, st, n, s->species.as<int>(),
+                       nos, bcount.as<int>(), s->row_of_atom.as<int>(),
+                       s->atom_of_row.as<int>(), s->bond_off.as<int>(), kI8TileA,
+                       s->q_shift.as<int>(), host_types, host_bonds, hw + kWordBonds);
+  } else {
+    int nb = (n + kRowBlock - 1) / kRowBlock;
     hist.alloc(pool, (size_t)nos * nb * sizeof(int));
     off.alloc(pool, ((size_t)nos * nb + 1) * sizeof(int));
     hipLaunchKernelGGL(k_species_count, dim3(nb), dim3(kRowBlock), nos * sizeof(int), st, n,
                        s->species.as<int>(), nos, hist.as<int>());
     scan_exclusive(ctx, hist.as<int>(), off.as<int>(), nos * nb);
+    hipLaunchKernelGGL(k_species_rows, dim3(nb), dim3(kRowBlock), (17 * nos + 1) * sizeof(int),
+                       st, n, s->species.as<int>(), nos, off.as<int>(), s->row_of_atom.as<int>(),
+                       s->atom_of_row.as<int>(), host_types, kI8TileA, s->q_shift.as<int>(),
+                       by_type.as<int>());
+    hipLaunchKernelGGL(k_bonds_by_type, dim3(std::min(64, (n + 255) / 256)), dim3(256),
+                       nos * sizeof(int), st, n, s->species.as<int>(), bcount.as<int>(), nos,
+                       by_type.as<int>());
+    scan_exclusive(ctx, bcount.as<int>(), s->bond_off.as<int>(), n, hw + kWordBonds);
   }
-  hipLaunchKernelGGL(k_species_rows, dim3(nb), dim3(kRowBlock), (17 * nos + 1) * sizeof(int), st,
-                     n, s->species.as<int>(), nos, off.as<int>(), s->row_of_atom.as<int>(),
-                     s->atom_of_row.as<int>(), host_types, kI8TileA, s->q_shift.as<int>(),
-                     by_type.as<int>(), cut, by_value ? nc : 0, s->d_cutoffs.as<double>());
-  DevBuf bcount(pool, (size_t)n * sizeof(int)), in_count(pool, (size_t)n * sizeof(int));
-  s->bond_off.alloc(pool, ((size_t)n + 1) * sizeof(int));
-  hipLaunchKernelGGL(k_bond_count, dim3((n + 3) / 4), dim3(256), 0, st, n, s->species.as<int>(),
-                     s->cumulative.as<int>(), s->nspecies.as<int>(), s->rel.as<double>(),
-                     s->d_cutoffs.as<double>(), nos, bcount.as<int>(), in_count.as<int>());
-  hipLaunchKernelGGL(k_bonds_by_type, dim3(std::min(64, (n + 255) / 256)), dim3(256),
-                     nos * sizeof(int), st, n, s->species.as<int>(), bcount.as<int>(), nos,
-                     by_type.as<int>());
-  scan_exclusive(ctx, bcount.as<int>(), s->bond_off.as<int>(), n, hw + kWordBonds);
   // Bond arrays hold every neighbour, so nothing waits for the bond total.
   size_t cap = std::max<size_t>(1, (size_t)s->n_nb);
   s->bond_q.alloc(pool, cap * sizeof(int));
+  DevBuf in_slot(pool, cap * sizeof(int));
+  if (one_block) FM_HIP(hipEventRecord(ctx->ev_sizes, st));
   hipLaunchKernelGGL(k_bond_fill, dim3((n + 3) / 4), dim3(256), 0, st, n, s->species.as<int>(),
                      s->cumulative.as<int>(), s->nspecies.as<int>(), s->rel.as<double>(),
                      s->d_cutoffs.as<double>(), nos, s->bond_off.as<int>(), s->sidx.as<int>(),
-                     s->bond_q.as<int>(), in_count.as<int>(), by_type.as<int>(), host_bonds);
-  FM_HIP(hipEventRecord(ctx->ev_sizes, st));
+                     s->bond_q.as<int>(), in_count.as<int>(), in_slot.as<int>(),
+                     one_block ? nullptr : by_type.as<int>(), host_bonds);
+  if (!one_block) FM_HIP(hipEventRecord(ctx->ev_sizes, st));
   s->in_off.alloc(pool, ((size_t)n + 1) * sizeof(int));
-  scan_exclusive(ctx, in_count.as<int>(), s->in_off.as<int>(), n);
+  bool own_scan = one_block && s->n_nb > 0;
+  if (!own_scan) scan_exclusive(ctx, in_count.as<int>(), s->in_off.as<int>(), n);
   s->in_bond.alloc(pool, cap * sizeof(int));
   DevBuf unordered(pool, cap * sizeof(int));
   if (s->n_nb > 0) {
-    hipLaunchKernelGGL(k_in_fill, dim3((unsigned)((s->n_nb + tpb - 1) / tpb)), dim3(tpb), 0, st, n,
-                       s->bond_off.as<int>(), s->bond_q.as<int>(), s->sidx.as<int>(),
-                       s->in_off.as<int>(), in_count.as<int>(), unordered.as<int>());
+    hipLaunchKernelGGL(k_in_fill, dim3((unsigned)((s->n_nb + kScanBlock - 1) / kScanBlock)),
+                       dim3(kScanBlock), 0, st, n, s->bond_off.as<int>(), s->bond_q.as<int>(),
+                       s->sidx.as<int>(), own_scan ? in_count.as<int>() : nullptr,
+                       s->in_off.as<int>(), in_slot.as<int>(), unordered.as<int>());
     hipLaunchKernelGGL(k_in_rank, dim3((n + 3) / 4), dim3(256), 0, st, n, s->in_off.as<int>(),
                        unordered.as<int>(), s->in_bond.as<int>());
   }

@@ -108,17 +108,33 @@ static void for_final_types(fm_structure s, Part &&part, Launch &&launch) {
 
 // Per structure (one wave each): energy and stress -1/V sum_b f (x) r
 // (normalized_dot_product.cpp:201-206).
-__global__ __launch_bounds__(64) void k_final_sum(const int *struct_chunk_off, const double *part,
-                                                  const double *vol_inv, const long long *mean_off,
-                                                  const int *atom_off, double *out) {
-  int k = blockIdx.x;
-  double acc[7];
-  structure_sums<7>(struct_chunk_off, part, k, acc);
+__device__ __forceinline__ void write_sums(const double (&acc)[7], int k, const double *vol_inv,
+                                           const long long *mean_off, const int *atom_off,
+                                           double *out) {
   if (threadIdx.x != 0) return;
   double *o = out + mean_off[k];
   int nk = atom_off[k + 1] - atom_off[k];
   o[0] = acc[0];
   for (int q = 0; q < 6; q++) o[1 + 3 * nk + q] = acc[1 + q] * vol_inv[k];
+}
+__global__ __launch_bounds__(64) void k_final_sum(const int *struct_chunk_off, const double *part,
+                                                  const double *vol_inv, const long long *mean_off,
+                                                  const int *atom_off, double *out) {
+  double acc[7];
+  structure_sums<7>(struct_chunk_off, part, blockIdx.x, acc);
+  write_sums(acc, blockIdx.x, vol_inv, mean_off, atom_off, out);
+}
+// The same from the atoms, for structures of up to kDirectChunks chunks.
+__global__ __launch_bounds__(1024) void k_direct_sum(const int *struct_chunk_off,
+                                                     const int *chunk_begin, const int *chunk_end,
+                                                     const int *row_of_atom, const double *E_row,
+                                                     const double *vir, const double *vol_inv,
+                                                     const long long *mean_off,
+                                                     const int *atom_off, double *out) {
+  double acc[7];
+  direct_sums<7>(struct_chunk_off, chunk_begin, chunk_end, row_of_atom, E_row, vir, blockIdx.x,
+                 acc);
+  write_sums(acc, blockIdx.x, vol_inv, mean_off, atom_off, out);
 }
 
 __global__ void k_fill(double *p, long long n, double v) {
@@ -132,7 +148,6 @@ static void gather_forces(fm_structure s, bool f64, DevBuf &fbond, DevBuf &vir, 
                           double *o) {
   hipStream_t st = s->ctx->stream;
   Pool *pool = &s->ctx->pool;
-  DevBuf blk(pool, (size_t)s->n_chunks * 7 * sizeof(double));
   KScope timer(s->ctx, KT_GATHER);
   auto forces = [&](auto *f) {
     using TF = std::remove_const_t<std::remove_pointer_t<decltype(f)>>;
@@ -144,6 +159,15 @@ static void gather_forces(fm_structure s, bool f64, DevBuf &fbond, DevBuf &vir, 
   };
   if (f64) forces(fbond.as<double>());
   else forces(fbond.as<float>());
+  if (s->max_chunks <= kDirectChunks) {
+    hipLaunchKernelGGL(k_direct_sum, dim3(s->n_struct), dim3(1024), 0, st,
+                       s->d_struct_chunk_off.as<int>(), s->d_chunk_begin.as<int>(),
+                       s->d_chunk_end.as<int>(), s->row_of_atom.as<int>(), E_row.as<double>(),
+                       vir.as<double>(), s->d_vol_inv.as<double>(),
+                       s->d_mean_off.as<long long>(), s->d_atom_off.as<int>(), o);
+    return;
+  }
+  DevBuf blk(pool, (size_t)s->n_chunks * 7 * sizeof(double));
   hipLaunchKernelGGL(k_chunk_sums<7>, dim3(s->n_chunks), dim3(256), 0, st,
                      s->d_chunk_begin.as<int>(), s->d_chunk_end.as<int>(),
                      s->row_of_atom.as<int>(), E_row.as<double>(), vir.as<double>(),
@@ -222,6 +246,23 @@ void build_var_pos(fm_structure s) {
 // each).
 constexpr size_t kStageOut = 256 << 10;
 
+struct StageOut {
+  const double *src[3];
+  size_t count[3];
+};
+// Up to three arrays to pinned host memory, one after the other: one launch (4 us
+// for 108 atoms) where a copy each took 4 us and 9 of the caller's time.
+__global__ __launch_bounds__(256) void k_stage_out(StageOut a, double *dst) {
+  size_t i = blockIdx.x * (size_t)256 + threadIdx.x, at = i;
+  for (int k = 0; k < 3; k++) {
+    if (at < a.count[k]) {
+      dst[i] = a.src[k][at];
+      return;
+    }
+    at -= a.count[k];
+  }
+}
+
 static void read_outputs(fm_structure s, const double *o, size_t n_out, const double *var_row,
                          const double *E_row, double *mean_efs, double *local_var,
                          double *local_energy) {
@@ -258,15 +299,22 @@ static void read_outputs(fm_structure s, const double *o, size_t n_out, const do
   for (const Part &p : parts)
     if (p.dst) total += p.count * sizeof(double);
   char *stage = total <= kStageOut ? s->ctx->stage(total) : nullptr;
-  char *at = stage;
-  for (const Part &p : parts) {
-    if (!p.dst) continue;
-    FM_HIP(hipMemcpyAsync(stage ? (void *)at : (void *)p.dst, p.src, p.count * sizeof(double),
-                          hipMemcpyDeviceToHost, st));
-    if (stage) at += p.count * sizeof(double);
+  if (stage && total > 0) {
+    StageOut so{};
+    for (int k = 0; k < 3; k++)
+      if (parts[k].dst) so.src[k] = parts[k].src, so.count[k] = parts[k].count;
+    size_t count = total / sizeof(double);
+    void *dev = nullptr;
+    FM_HIP(hipHostGetDevicePointer(&dev, stage, 0));
+    hipLaunchKernelGGL(k_stage_out, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st, so,
+                       (double *)dev);
+    FM_HIP(hipGetLastError());
   }
+  for (const Part &p : parts)
+    if (p.dst && !stage)
+      FM_HIP(hipMemcpyAsync(p.dst, p.src, p.count * sizeof(double), hipMemcpyDeviceToHost, st));
   FM_HIP(hipStreamSynchronize(st));
-  at = stage;
+  char *at = stage;
   for (const Part &p : parts) {
     if (!p.dst || !stage) continue;
     std::memcpy(p.dst, at, p.count * sizeof(double));

@@ -36,3 +36,9 @@ def test_lists_and_rows(oracle, n, nos):
     assert d.n_neighbors_by_type == [int(keep[centre == t].sum()) for t in range(nos)]
     per_atom = np.add.reduceat(np.r_[keep, 0], np.r_[0, np.cumsum(ref.neighbor_count)[:-1]]) * (ref.neighbor_count > 0)
     assert np.array_equal(np.concatenate(d.neighbor_counts), per_atom[order])
+
+
+@pytest.mark.parametrize("n", [2, 2047, 2048, 2049, 8191])
+def test_lists_and_rows_small(oracle, n):
+    """At the edges of the builds in one workgroup (2,048 atoms; 8,192)."""
+    test_lists_and_rows(oracle, n, 3)

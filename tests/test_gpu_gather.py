@@ -43,3 +43,16 @@ def test_forces_and_sums(oracle, model):
         alone = C.Structure(*st, 4.2, [calc])
         sgp.predict_mean(alone)
         assert np.array_equal(alone.mean_efs, mean), n
+
+
+def test_sums_of_large_and_small(model):
+    """Structures of up to 2,048 atoms are summed in one launch, a batch with a
+    larger one in two: the same bits either way."""
+    from flare_amd.batch import Batch
+    C, calc, cut, sgp = model
+    structs = [structure(n) for n in (2048, 2049, 1025, 3)]
+    means, _ = Batch(structs, 4.2, calc).predict(sgp)
+    for st, mean in zip(structs, means):
+        alone = C.Structure(*st, 4.2, [calc])
+        sgp.predict_mean(alone)
+        assert np.array_equal(alone.mean_efs, mean)
