@@ -300,6 +300,14 @@ struct fm_mapped_s {
 };
 
 namespace fm {
+// fm_predict.hip
+struct HostOut {
+  double *dst = nullptr;  // host memory, or null
+  const double *src = nullptr;
+  size_t count = 0;
+};
+void read_back(fm_context ctx, const HostOut (&parts)[3]);
+
 // fm_mapped.hip
 void mapping_coefficients(fm_model m, std::vector<double> &beta, int64_t &beta_size);
 void mapped_compute(fm_mapped mp, fm_structure s, double *atom_energy, double *forces,

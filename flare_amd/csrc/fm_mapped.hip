@@ -86,20 +86,27 @@ void mapping_coefficients(fm_model m, std::vector<double> &beta, int64_t &beta_s
   }
 }
 
-// Per atom: energy and G (the input of the adjoint) from P = B beta.
+// Per atom: energy and G (the input of the adjoint) from P = B beta, which the
+// rows of G hold on entry (p=2).
 //   normalized p=2: E = B.P/|B|^2, G = 2P/|B| (projected in the adjoint)
 //   normalized p=1: E = B.beta/|B|, G = beta
 //   unnormalised p=2: E = B.P, w = 2P;  p=1: E = B.beta, w = beta
 // (lammps_descriptor.cpp:259-282). Atoms with |B|^2 < 1e-8 get E = 0
-// (pair_flare.cpp:134-136).
-__global__ void k_mapped_energy(int ns, int ro, int d, const double *B, const double *P,
-                                const double *beta, int power, int normalized,
-                                const double *norm, const double *nn, double *E_row,
-                                double *G) {
+// (pair_flare.cpp:134-136). One wave per row, the species' rows ro[u] .. ro[u + 1].
+constexpr int kMappedTypes = 8;
+struct MappedTypes {
+  int types, ro[kMappedTypes + 1];
+  const double *beta[kMappedTypes];
+};
+__global__ __launch_bounds__(256) void k_mapped_energy(MappedTypes a, int d, const double *B,
+                                                       int power, int normalized,
+                                                       const double *norm, const double *nn,
+                                                       double *E_row, double *G) {
   int lane = threadIdx.x & 63;
-  int r = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (r >= ns) return;
-  int row = ro + r;
+  int row = a.ro[0] + blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  if (row >= a.ro[a.types]) return;
+  int u = 0;
+  while (row >= a.ro[u + 1]) u++;
   const double *b = B + (size_t)row * d;
   double *g = G + (size_t)row * d;
   double n2 = nn[row], nrm = norm[row];
@@ -108,7 +115,7 @@ __global__ void k_mapped_energy(int ns, int ro, int d, const double *B, const do
     if (lane == 0) E_row[row] = 0;
     return;
   }
-  const double *v = power == 2 ? P + (size_t)r * d : beta;
+  const double *v = power == 2 ? g : a.beta[u];
   double acc = 0;
   for (int k = lane; k < d; k += 64) acc += b[k] * v[k];
   acc = wave_sum(acc);
@@ -138,7 +145,7 @@ __global__ void k_zero(double *x, long long n) {
 // Working buffers of one evaluation (device memory, at least the sizes
 // mapped_layout gives).
 struct MappedBufs {
-  double *G, *E_row, *P, *fbond, *vir, *F, *Ea, *vsum, *blk;
+  double *G, *E_row, *fbond, *vir, *F, *Ea, *vsum, *blk;
   void *U;
 };
 
@@ -155,47 +162,66 @@ static void mapped_checks(fm_mapped mp, fm_structure s) {
 }
 
 // Byte sizes of the buffers, in MappedBufs order.
-static void mapped_layout(fm_mapped mp, fm_structure s, size_t sz[10]) {
-  size_t n = s->n, d = s->nd, maxns = 0;
-  for (int t = 0; t < s->nos; t++) maxns = std::max(maxns, (size_t)s->n_by_type[t]);
-  size_t w = sizeof(double);
+constexpr int kMappedBufs = 9;
+static void mapped_layout(fm_structure s, size_t sz[kMappedBufs]) {
+  size_t n = s->n, d = s->nd, w = sizeof(double);
   sz[0] = n * d * w;                                // G
   sz[1] = n * w;                                    // E_row
-  sz[2] = mp->power == 2 ? maxns * d * w : 0;       // P
-  sz[3] = 3 * (size_t)s->n_bonds * w;               // fbond
-  sz[4] = 6 * n * w;                                // vir
-  sz[5] = 3 * n * w;                                // F
-  sz[6] = n * w;                                    // Ea
-  sz[7] = 6 * (size_t)s->n_struct * w;              // vsum
-  sz[8] = 6 * (size_t)s->n_chunks * w;              // blk
-  sz[9] = adjoint_u_bytes(s);                       // U
-  for (int k = 0; k < 10; k++) sz[k] = std::max<size_t>(sz[k], 1);
+  sz[2] = 3 * (size_t)s->n_bonds * w;               // fbond
+  sz[3] = 6 * n * w;                                // vir
+  sz[4] = 3 * n * w;                                // F
+  sz[5] = n * w;                                    // Ea
+  sz[6] = 6 * (size_t)s->n_struct * w;              // vsum
+  sz[7] = 6 * (size_t)s->n_chunks * w;              // blk
+  sz[8] = adjoint_u_bytes(s);                       // U
+  for (int k = 0; k < kMappedBufs; k++) sz[k] = std::max<size_t>(sz[k], 1);
+}
+
+// Host memory that the runtime does not know.
+static bool pageable_host(const void *p) {
+  hipPointerAttribute_t a{};
+  hipError_t rc = hipPointerGetAttributes(&a, p);
+  if (rc != hipSuccess) (void)hipGetLastError();
+  return rc != hipSuccess || a.type == hipMemoryTypeUnregistered;
 }
 
 // pair_flare.cpp:68-184 on the given buffers; outputs (host or device
-// memory, any may be null) are copied on the context stream, then the
-// stream is synchronised.
-static void mapped_run(fm_mapped mp, fm_structure s, const MappedBufs &b, double *atom_energy,
-                       double *forces, double *virial) {
+// memory, any may be null) are copied on the context stream (with may_stage
+// through its pinned memory where all are pageable), then the stream is
+// synchronised.
+static void mapped_run(fm_mapped mp, fm_structure s, const MappedBufs &b, bool may_stage,
+                       double *atom_energy, double *forces, double *virial) {
   hipStream_t st = s->ctx->stream;
   int n = s->n, d = s->nd;
-  for (int t = 0; t < s->nos; t++) {
-    int ns = s->n_by_type[t], ro = s->type_off[t];
-    if (ns == 0) continue;
-    const double *Bs = s->B.as<double>() + (size_t)ro * d;
-    if (mp->power == 2) {
-      EpArgs e;
-      e.W = b.P;
-      e.ldw = d;
-      gemm_f64(st, EP_STORE, ns, d, d, Bs, d, mp->beta[t].as<double>(), d, 0, e);
-    }
-    hipLaunchKernelGGL(k_mapped_energy, dim3((ns + 3) / 4), dim3(256), 0, st, ns, ro, d,
-                       s->B.as<double>(), mp->power == 2 ? b.P : nullptr,
-                       mp->beta[t].as<double>(), mp->power, mp->normalized,
-                       s->norm.as<double>(), s->nn.as<double>(), b.E_row, b.G);
+  // P = B beta of all species in one launch, into the rows of G.
+  std::vector<F64Gemm> products;
+  for (int t = 0; t < s->nos && mp->power == 2; t++) {
+    size_t at = (size_t)s->type_off[t] * d;
+    EpArgs e;
+    e.W = b.G + at;
+    e.ldw = d;
+    products.push_back({s->B.as<double>() + at, mp->beta[t].as<double>(), d, d, s->n_by_type[t],
+                        d, d, 0, e});
   }
-  long long nv = 6 * (long long)s->n_struct;
-  hipLaunchKernelGGL(k_zero, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, st, b.vsum, nv);
+  gemm_f64_groups(st, EP_STORE, products);
+  for (int t0 = 0; t0 < s->nos; t0 += kMappedTypes) {
+    MappedTypes a{};
+    a.types = std::min(kMappedTypes, s->nos - t0);
+    for (int u = 0; u < a.types; u++) {
+      a.ro[u] = s->type_off[t0 + u];
+      a.beta[u] = mp->beta[t0 + u].as<double>();
+    }
+    a.ro[a.types] = s->type_off[t0 + a.types];
+    int rows = a.ro[a.types] - a.ro[0];
+    if (rows > 0)
+      hipLaunchKernelGGL(k_mapped_energy, dim3((rows + 3) / 4), dim3(256), 0, st, a, d,
+                         s->B.as<double>(), mp->power, mp->normalized, s->norm.as<double>(),
+                         s->nn.as<double>(), b.E_row, b.G);
+  }
+  if (n == 0) {
+    long long nv = 6 * (long long)s->n_struct;
+    hipLaunchKernelGGL(k_zero, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, st, b.vsum, nv);
+  }
   if (n > 0) {
     launch_adjoint(s, b.G, d, b.fbond, b.vir, mp->normalized ? 1 : 0, -1.0, 1e-8, nullptr, 0,
                    b.U);
@@ -210,13 +236,18 @@ static void mapped_run(fm_mapped mp, fm_structure s, const MappedBufs &b, double
                        s->d_struct_chunk_off.as<int>(), b.blk, b.vsum);
   }
   FM_HIP(hipGetLastError());
-  if (n > 0 && atom_energy)
-    FM_HIP(hipMemcpyAsync(atom_energy, b.Ea, n * sizeof(double), hipMemcpyDefault, st));
-  if (n > 0 && forces)
-    FM_HIP(hipMemcpyAsync(forces, b.F, 3 * (size_t)n * sizeof(double), hipMemcpyDefault, st));
-  if (virial)
-    FM_HIP(hipMemcpyAsync(virial, b.vsum, 6 * (size_t)s->n_struct * sizeof(double),
-                          hipMemcpyDefault, st));
+  HostOut parts[3] = {{n > 0 ? atom_energy : nullptr, b.Ea, (size_t)n},
+                      {n > 0 ? forces : nullptr, b.F, 3 * (size_t)n},
+                      {virial, b.vsum, 6 * (size_t)s->n_struct}};
+  bool pageable = may_stage;
+  for (const HostOut &p : parts) pageable = pageable && (!p.dst || pageable_host(p.dst));
+  if (pageable) {
+    read_back(s->ctx, parts);
+    return;
+  }
+  for (const HostOut &p : parts)
+    if (p.dst)
+      FM_HIP(hipMemcpyAsync(p.dst, p.src, p.count * sizeof(double), hipMemcpyDefault, st));
   FM_HIP(hipStreamSynchronize(st));
 }
 
@@ -224,15 +255,14 @@ void mapped_compute(fm_mapped mp, fm_structure s, double *atom_energy, double *f
                     double *virial) {
   mapped_checks(mp, s);
   Pool *pool = &s->ctx->pool;
-  size_t sz[10];
-  mapped_layout(mp, s, sz);
-  DevBuf buf[10];
-  for (int k = 0; k < 10; k++) buf[k].alloc(pool, sz[k]);
+  size_t sz[kMappedBufs];
+  mapped_layout(s, sz);
+  DevBuf buf[kMappedBufs];
+  for (int k = 0; k < kMappedBufs; k++) buf[k].alloc(pool, sz[k]);
   MappedBufs b{buf[0].as<double>(), buf[1].as<double>(), buf[2].as<double>(),
                buf[3].as<double>(), buf[4].as<double>(), buf[5].as<double>(),
-               buf[6].as<double>(), buf[7].as<double>(), buf[8].as<double>(),
-               buf[9].as<void>()};
-  mapped_run(mp, s, b, atom_energy, forces, virial);
+               buf[6].as<double>(), buf[7].as<double>(), buf[8].as<void>()};
+  mapped_run(mp, s, b, true, atom_energy, forces, virial);
 }
 
 // ---------------------------------------------------------------------------
@@ -270,12 +300,18 @@ static unsigned char *scratch_ptr(int device) {
 void mapped_compute_noalloc(fm_mapped mp, fm_structure s, double *atom_energy, double *forces,
                             double *virial) {
   mapped_checks(mp, s);
-  size_t sz[10], off[10], total = 0;
-  mapped_layout(mp, s, sz);
-  for (int k = 0; k < 10; k++) {
+  size_t sz[kMappedBufs], off[kMappedBufs], total = 0;
+  mapped_layout(s, sz);
+  for (int k = 0; k < kMappedBufs; k++) {
     off[k] = total;
     total += (sz[k] + 255) / 256 * 256;
   }
+  // The largest species' rows once more: the sizes that this entry point takes
+  // are those with a buffer of their own for B beta.
+  size_t ns = 0;
+  for (int t = 0; t < s->nos; t++) ns = std::max(ns, (size_t)s->n_by_type[t]);
+  size_t p = mp->power == 2 ? ns * s->nd * sizeof(double) : 0;
+  total += (std::max<size_t>(p, 1) + 255) / 256 * 256;
   FM_CHECK(total <= kNoAllocScratchBytes, FM_ERR_CAPACITY,
            "the structure needs " + std::to_string(total) +
                " bytes of working memory; the allocation-free entry point holds " +
@@ -283,12 +319,11 @@ void mapped_compute_noalloc(fm_mapped mp, fm_structure s, double *atom_energy, d
   unsigned char *base = scratch_ptr(s->ctx->device);
   auto at = [&](int k) { return static_cast<void *>(base + off[k]); };
   MappedBufs b{(double *)at(0), (double *)at(1), (double *)at(2), (double *)at(3),
-               (double *)at(4), (double *)at(5), (double *)at(6), (double *)at(7),
-               (double *)at(8), at(9)};
+               (double *)at(4), (double *)at(5), (double *)at(6), (double *)at(7), at(8)};
   fm_context ctx = s->ctx;
   ctx->kt_on = false;  // the timers would create events
   try {
-    mapped_run(mp, s, b, atom_energy, forces, virial);
+    mapped_run(mp, s, b, false, atom_energy, forces, virial);
   } catch (...) {
     ctx->kt_on = true;
     throw;

@@ -240,12 +240,6 @@ void build_var_pos(fm_structure s) {
   FM_HIP(hipGetLastError());
 }
 
-// Results to the caller's host buffers (any may be null); returns after the
-// copies have finished. Results of up to kStageOut bytes go through the
-// context's pinned memory (a copy to pageable memory waits for itself, 15 us
-// each).
-constexpr size_t kStageOut = 256 << 10;
-
 struct StageOut {
   const double *src[3];
   size_t count[3];
@@ -263,6 +257,41 @@ __global__ __launch_bounds__(256) void k_stage_out(StageOut a, double *dst) {
   }
 }
 
+// Arrays to the caller's host memory; returns after the copies have finished.
+// Up to kStageOut bytes in all go through the context's pinned memory (a copy to
+// pageable memory waits for itself, 15 us each).
+constexpr size_t kStageOut = 256 << 10;
+
+void read_back(fm_context ctx, const HostOut (&parts)[3]) {
+  hipStream_t st = ctx->stream;
+  size_t total = 0;
+  StageOut so{};
+  for (int k = 0; k < 3; k++)
+    if (parts[k].dst) {
+      so.src[k] = parts[k].src;
+      so.count[k] = parts[k].count;
+      total += parts[k].count;
+    }
+  char *stage = total * sizeof(double) <= kStageOut ? ctx->stage(total * sizeof(double)) : nullptr;
+  if (stage && total > 0) {
+    void *dev = nullptr;
+    FM_HIP(hipHostGetDevicePointer(&dev, stage, 0));
+    hipLaunchKernelGGL(k_stage_out, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, so,
+                       (double *)dev);
+    FM_HIP(hipGetLastError());
+  }
+  for (const HostOut &p : parts)
+    if (p.dst && !stage)
+      FM_HIP(hipMemcpyAsync(p.dst, p.src, p.count * sizeof(double), hipMemcpyDeviceToHost, st));
+  FM_HIP(hipStreamSynchronize(st));
+  for (const HostOut &p : parts) {
+    if (!p.dst || !stage) continue;
+    std::memcpy(p.dst, stage, p.count * sizeof(double));
+    stage += p.count * sizeof(double);
+  }
+}
+
+// Results to the caller's host buffers (any may be null).
 static void read_outputs(fm_structure s, const double *o, size_t n_out, const double *var_row,
                          const double *E_row, double *mean_efs, double *local_var,
                          double *local_energy) {
@@ -270,11 +299,7 @@ static void read_outputs(fm_structure s, const double *o, size_t n_out, const do
   Pool *pool = &s->ctx->pool;
   size_t n = s->n;
   DevBuf vperm, eperm;
-  struct Part {
-    double *dst;
-    const double *src;
-    size_t count;
-  } parts[3] = {{mean_efs, o, n_out}, {nullptr, nullptr, 0}, {nullptr, nullptr, 0}};
+  HostOut parts[3] = {{mean_efs, o, n_out}, {}, {}};
   if (local_var && var_row && n > 0) {
     // Species-sorted rows of the batch to each structure's species-sorted
     // order (compute_cluster_uncertainties order).
@@ -295,31 +320,7 @@ static void read_outputs(fm_structure s, const double *o, size_t n_out, const do
     parts[2] = {local_energy, eperm.as<double>(), n};
   }
   FM_HIP(hipGetLastError());
-  size_t total = 0;
-  for (const Part &p : parts)
-    if (p.dst) total += p.count * sizeof(double);
-  char *stage = total <= kStageOut ? s->ctx->stage(total) : nullptr;
-  if (stage && total > 0) {
-    StageOut so{};
-    for (int k = 0; k < 3; k++)
-      if (parts[k].dst) so.src[k] = parts[k].src, so.count[k] = parts[k].count;
-    size_t count = total / sizeof(double);
-    void *dev = nullptr;
-    FM_HIP(hipHostGetDevicePointer(&dev, stage, 0));
-    hipLaunchKernelGGL(k_stage_out, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st, so,
-                       (double *)dev);
-    FM_HIP(hipGetLastError());
-  }
-  for (const Part &p : parts)
-    if (p.dst && !stage)
-      FM_HIP(hipMemcpyAsync(p.dst, p.src, p.count * sizeof(double), hipMemcpyDeviceToHost, st));
-  FM_HIP(hipStreamSynchronize(st));
-  char *at = stage;
-  for (const Part &p : parts) {
-    if (!p.dst || !stage) continue;
-    std::memcpy(p.dst, at, p.count * sizeof(double));
-    at += p.count * sizeof(double);
-  }
+  read_back(s->ctx, parts);
 }
 
 // Rows per tile of one species in the chosen form: at most T and, when T
