@@ -454,7 +454,15 @@ __global__ __launch_bounds__(256) void k_dEdc_b3(int n, B3Dev t, const T *Cg,
 // arrays (uniform indices, so no scratch); the sums over pairs that end on
 // one target (n, mu) run with one thread per target after a barrier.
 // Summation orders are fixed, so results are deterministic.
+//
+// Up to 64 pairs are one wave, whose chain of an l-set after the other is all
+// that an atom has: with SPLIT (FP64) the block's waves take every fourth l-set
+// each, with a workspace and an adjoint of their own, summed at the end. |B|^2 is
+// then taken from the stored row in the order of one wave. 1,024 atoms of 36
+// pairs: 110 us and 290 us (124 and 340 with one wave per atom; two waves of 204
+// registers fit a SIMD).
 // ---------------------------------------------------------------------------
+constexpr int kB3Waves = 4;
 
 // Sum over the block in a fixed order (red: one slot per wave).
 template <typename T>
@@ -476,7 +484,7 @@ __device__ __forceinline__ void load_block(const T *r, int nm, T *v) {
   for (int k = 0; k < kLM; k++) v[k] = k < nm ? r[k] : T(0);
 }
 
-template <typename T>
+template <typename T, bool SPLIT>
 __global__ __launch_bounds__(512) void k_b3p(int n, B3Dev t, const int *__restrict__ rt_off,
                                               const int *__restrict__ rt_pk,
                                               const T *__restrict__ rt_w, const T *Cg,
@@ -485,14 +493,20 @@ __global__ __launch_bounds__(512) void k_b3p(int n, B3Dev t, const int *__restri
   extern __shared__ __align__(16) unsigned char smem[];
   int k = blockIdx.x;
   if (k >= n) return;
-  int tid = threadIdx.x, nt = blockDim.x;
+  // The threads of an l-set: a wave (SPLIT) or the block.
+  int tid = SPLIT ? threadIdx.x & 63 : threadIdx.x, nt = SPLIT ? 64 : blockDim.x;
+  int w = SPLIT ? threadIdx.x >> 6 : 0;
   int i, row, brow;
   rr.map(k, row_of_atom, i, row, brow);
   int nr = t.nr, H = t.H, nc = nr * H, n_tri = t.n_tri;
   T *rc = reinterpret_cast<T *>(smem);  // r of the atom
-  T *bl = rc + nc;                        // one l-set's slice of the row
-  T *red = bl + n_tri;                    // 16 wave slots
-  for (int g = tid; g < nc; g += nt) rc[g] = Cg[(size_t)i * nc + g];
+  T *red = rc + nc;                       // 16 wave slots
+  T *bl = red + 16 + (size_t)w * n_tri;   // one l-set's slice of the row
+  auto sync = [] {
+    if constexpr (SPLIT) wave_lds_sync();
+    else __syncthreads();
+  };
+  for (int g = threadIdx.x; g < nc; g += blockDim.x) rc[g] = Cg[(size_t)i * nc + g];
   bool act = tid < t.npair;
   int n1 = 0, n2 = 0, tb = 0;
   if (act) {
@@ -504,7 +518,7 @@ __global__ __launch_bounds__(512) void k_b3p(int n, B3Dev t, const int *__restri
   __syncthreads();
   T s2 = 0;
   T *Brow = B + (size_t)brow * t.nd;
-  for (int ls = 0; ls < t.n_ls; ls++) {
+  for (int ls = w; ls < t.n_ls; ls += SPLIT ? kB3Waves : 1) {
     int l1 = t.ls_l[3 * ls], l2 = t.ls_l[3 * ls + 1], l3 = t.ls_l[3 * ls + 2];
     if (act) {
       T x[kLM], y[kLM], p[kLM];
@@ -536,23 +550,35 @@ __global__ __launch_bounds__(512) void k_b3p(int n, B3Dev t, const int *__restri
         bl[tb + n3 - n2] = acc;
       }
     }
-    __syncthreads();
+    sync();
     for (int kk = tid; kk < n_tri; kk += nt) {
       T v = bl[kk];
       size_t kd = (size_t)ls * n_tri + kk;
       Brow[kd] = v;
-      s2 += v * v;
+      if (!SPLIT) s2 += v * v;
     }
-    __syncthreads();
+    sync();
   }
-  s2 = block_sum(s2, red);
+  if constexpr (SPLIT) {
+    __syncthreads();
+    if (w > 0) return;
+#pragma unroll 2
+    for (int ls = 0; ls < t.n_ls; ls++)
+      for (int kk = tid; kk < n_tri; kk += 64) {
+        T v = Brow[(size_t)ls * n_tri + kk];
+        s2 += v * v;
+      }
+    s2 = wave_sum(s2);
+  } else {
+    s2 = block_sum(s2, red);
+  }
   if (tid == 0) {
     norm[row] = (double)sqrt(s2);
     nnv[row] = (double)s2;
   }
 }
 
-template <typename T>
+template <typename T, bool SPLIT>
 __global__ __launch_bounds__(512) void k_dEdc_b3p(int n, B3Dev t, const int *__restrict__ rt_off,
                                                    const int *__restrict__ rt_pk,
                                                    const T *__restrict__ rt_w, const T *Cg,
@@ -564,33 +590,37 @@ __global__ __launch_bounds__(512) void k_dEdc_b3p(int n, B3Dev t, const int *__r
   extern __shared__ __align__(16) unsigned char smem[];
   int k = blockIdx.x;
   if (k >= n) return;
-  int tid = threadIdx.x, nt = blockDim.x;
+  int tid = SPLIT ? threadIdx.x & 63 : threadIdx.x, nt = SPLIT ? 64 : blockDim.x;
+  int w = SPLIT ? threadIdx.x >> 6 : 0, bt = threadIdx.x, bn = blockDim.x;
   int i, row, brow;
   rr.map(k, row_of_atom, i, row, brow);
   int nr = t.nr, H = t.H, nc = nr * H, n_tri = t.n_tri, npair = t.npair;
   T *urow = Ug + (size_t)i * nc;
   double nrm = norm[row];
   if (nrm < empty_norm || nnv[row] < empty_nn) {
-    for (int g = tid; g < nc; g += nt) urow[g] = 0;
+    for (int g = bt; g < nc; g += bn) urow[g] = 0;
     return;
   }
   T *rc = reinterpret_cast<T *>(smem);  // r of the atom
-  T *gc = rc + nc;                        // dE/dr
+  T *red = rc + nc;                       // 16 wave slots
+  size_t per = (size_t)nc + n_tri + 2 * (size_t)kLM * npair;  // workspace of a wave or block
+  T *gc = red + 16 + w * per;             // dE/dr
   T *wl = gc + nc;                        // w of one l-set
   T *Pl = wl + n_tri;                     // P, then Q: [mu][pair]
   T *El = Pl + (size_t)kLM * npair;       // factor-1, then factor-2 partials
-  T *red = El + (size_t)kLM * npair;      // 16 wave slots
-  for (int g = tid; g < nc; g += nt) {
-    rc[g] = Cg[(size_t)i * nc + g];
-    gc[g] = 0;
-  }
+  auto sync = [] {
+    if constexpr (SPLIT) wave_lds_sync();
+    else __syncthreads();
+  };
+  for (int g = bt; g < nc; g += bn) rc[g] = Cg[(size_t)i * nc + g];
+  for (int g = tid; g < nc; g += nt) gc[g] = 0;
   const T *Brow = B + (size_t)brow * t.nd;
   const T *Grow = G + (size_t)brow * g_ld;
   T ninv = T(1) / (T)nrm, gb = 0;
   if (project) {
     T part = 0;
 #pragma unroll 16
-    for (int kk = tid; kk < t.nd; kk += nt) part += Grow[kk] * Brow[kk];
+    for (int kk = bt; kk < t.nd; kk += bn) part += Grow[kk] * Brow[kk];
     gb = block_sum(part, red) * ninv;
   }
   // FP32: the next l-set's slices of dE/dB and B are loaded into registers
@@ -609,6 +639,7 @@ __global__ __launch_bounds__(512) void k_dEdc_b3p(int n, B3Dev t, const int *__r
       }
     }
   };
+  if constexpr (SPLIT) __syncthreads();
   fetch(0);
   bool act = tid < npair;
   int n1 = 0, n2 = 0, tb = 0;
@@ -618,7 +649,7 @@ __global__ __launch_bounds__(512) void k_dEdc_b3p(int n, B3Dev t, const int *__r
     n2 = pk >> 8;
     tb = t.pair_tb[tid];
   }
-  for (int ls = 0; ls < t.n_ls; ls++) {
+  for (int ls = w; ls < t.n_ls; ls += SPLIT ? kB3Waves : 1) {
     int l1 = t.ls_l[3 * ls], l2 = t.ls_l[3 * ls + 1], l3 = t.ls_l[3 * ls + 2];
     int n1m = 2 * l1 + 1, n2m = 2 * l2 + 1, n3m = 2 * l3 + 1;
     if constexpr (sizeof(T) == 4) {
@@ -633,7 +664,7 @@ __global__ __launch_bounds__(512) void k_dEdc_b3p(int n, B3Dev t, const int *__r
       for (int kk = tid; kk < n_tri; kk += nt)
         wl[kk] = project ? (gs[kk] - gb * bs[kk] * ninv) * ninv : gs[kk];
     }
-    __syncthreads();
+    sync();
     if (ls + 1 < t.n_ls) fetch(ls + 1);
     T e2[kLM];
     if (act) {
@@ -676,7 +707,7 @@ __global__ __launch_bounds__(512) void k_dEdc_b3p(int n, B3Dev t, const int *__r
         if (m < n1m) El[m * npair + tid] = e1[m];
       }
     }
-    __syncthreads();
+    sync();
     // Factor 1 targets (n, l1 mu1): pairs (n, n2 >= n).
     for (int tg = tid; tg < nr * n1m; tg += nt) {
       int nn = tg / n1m, m1 = tg - nn * n1m;
@@ -703,7 +734,7 @@ __global__ __launch_bounds__(512) void k_dEdc_b3p(int n, B3Dev t, const int *__r
         pp += 1;
       }
     }
-    __syncthreads();
+    sync();
     if (act) {
 #pragma unroll
       for (int m = 0; m < kLM; m++) {
@@ -711,7 +742,7 @@ __global__ __launch_bounds__(512) void k_dEdc_b3p(int n, B3Dev t, const int *__r
         if (m < n2m) El[m * npair + tid] = e2[m];
       }
     }
-    __syncthreads();
+    sync();
     // Factor 3 targets (n, l3 mu3): Q over the pairs (n2 <= n, n), and factor
     // 2 targets (n, l2 mu2): E2 over the pairs (n1 <= n, n); both contiguous.
     // With l2 == l3 the targets coincide and one thread adds both.
@@ -734,9 +765,19 @@ __global__ __launch_bounds__(512) void k_dEdc_b3p(int n, B3Dev t, const int *__r
         for (int a = 0; a <= nn; a++) acc += e[a];
         gc[nn * H + l2 * l2 + m2] += acc;
       }
-    __syncthreads();
+    sync();
   }
-  for (int g = tid; g < nc; g += nt) urow[g] = gc[g];
+  if constexpr (SPLIT) {
+    __syncthreads();
+    const T *g0 = red + 16;
+    for (int g = bt; g < nc; g += bn) {
+      T v = g0[g];
+      for (int u = 1; u < kB3Waves; u++) v += g0[u * per + g];
+      urow[g] = v;
+    }
+  } else {
+    for (int g = tid; g < nc; g += nt) urow[g] = gc[g];
+  }
 }
 
 // Column / row permutations between the reference's B3 order and the
@@ -909,15 +950,21 @@ static int waves_per_block(size_t lds_per_atom) {
 
 // Workgroup size and LDS bytes of the pair kernels, or 0 when the pairs do
 // not fit one workgroup of 512 threads or the workspace does not fit LDS
-// (then the wave-per-atom kernels run).
-static size_t b3_pair_lds(const B3Dev &d, size_t esz, bool adjoint, int &nt) {
+// (then the wave-per-atom kernels run). split: kB3Waves waves per atom.
+static size_t b3_pair_lds(const B3Dev &d, size_t esz, bool adjoint, int &nt, bool &split) {
+  split = false;
   if (d.npair > 512) return 0;
   nt = std::max(64, (d.npair + 63) / 64 * 64);
   if (d.n_tri > kPre * nt) return 0;
   size_t nc = (size_t)d.nr * d.H;
-  size_t el = nc + d.n_tri + 16;
-  if (adjoint) el += nc + 2 * (size_t)kLM * d.npair;
-  size_t bytes = el * esz;
+  size_t per = d.n_tri;
+  if (adjoint) per += nc + 2 * (size_t)kLM * d.npair;
+  size_t all = nc + 16;
+  // FP64 with one wave of pairs: up to 40 KB keep four blocks of four waves on a
+  // CU.
+  split = esz == 8 && nt == 64 && (all + kB3Waves * per) * esz <= 40 * 1024;
+  if (split) nt *= kB3Waves;
+  size_t bytes = (all + (split ? kB3Waves : 1) * per) * esz;
   return bytes <= 160 * 1024 ? bytes : 0;
 }
 
@@ -934,15 +981,16 @@ void launch_b3_rows(fm_structure s, int r0, int n, bool tile, void *Bout) {
   bool f64 = s->form == FM_FORM_FP64;
   size_t esz = f64 ? 8 : 4;
   int nt = 0;
-  size_t lds = b3_pair_lds(d, esz, false, nt);
+  bool split = false;
+  size_t lds = b3_pair_lds(d, esz, false, nt, split);
   if (lds) {
     if (f64)
-      hipLaunchKernelGGL(k_b3p<double>, dim3(n), dim3(nt), lds, st, n, d, b->rt_off.as<int>(),
+      hipLaunchKernelGGL((split ? k_b3p<double, true> : k_b3p<double, false>), dim3(n), dim3(nt), lds, st, n, d, b->rt_off.as<int>(),
                          b->rt_pk.as<int>(), b->rt_w<double>(), s->C.as<double>(),
                          s->row_of_atom.as<int>(), rr, (double *)Bout, s->norm.as<double>(),
                          s->nn.as<double>());
     else
-      hipLaunchKernelGGL(k_b3p<float>, dim3(n), dim3(nt), lds, st, n, d, b->rt_off.as<int>(),
+      hipLaunchKernelGGL((k_b3p<float, false>), dim3(n), dim3(nt), lds, st, n, d, b->rt_off.as<int>(),
                          b->rt_pk.as<int>(), b->rt_w<float>(), s->C.as<float>(),
                          s->row_of_atom.as<int>(), rr, (float *)Bout, s->norm.as<double>(),
                          s->nn.as<double>());
@@ -980,17 +1028,18 @@ void launch_dEdc_b3_rows(fm_structure s, int r0, int n, bool tile, const void *B
   bool f64 = s->form == FM_FORM_FP64;
   size_t esz = f64 ? 8 : 4;
   int nt = 0;
-  size_t plds = b3_pair_lds(d, esz, true, nt);
+  bool split = false;
+  size_t plds = b3_pair_lds(d, esz, true, nt, split);
   if (plds) {
     if (f64)
-      hipLaunchKernelGGL(k_dEdc_b3p<double>, dim3(n), dim3(nt), plds, st, n, d,
+      hipLaunchKernelGGL((split ? k_dEdc_b3p<double, true> : k_dEdc_b3p<double, false>), dim3(n), dim3(nt), plds, st, n, d,
                          b->rt_off.as<int>(), b->rt_pk.as<int>(), b->rt_w<double>(),
                          s->C.as<double>(),
                          s->row_of_atom.as<int>(), rr, (const double *)B, s->norm.as<double>(),
                          s->nn.as<double>(), (const double *)G, (long long)g_ld, project,
                          empty_norm, empty_nn, (double *)U);
     else
-      hipLaunchKernelGGL(k_dEdc_b3p<float>, dim3(n), dim3(nt), plds, st, n, d,
+      hipLaunchKernelGGL((k_dEdc_b3p<float, false>), dim3(n), dim3(nt), plds, st, n, d,
                          b->rt_off.as<int>(), b->rt_pk.as<int>(), b->rt_w<float>(),
                          s->C.as<float>(), s->row_of_atom.as<int>(), rr,
                          (const float *)B, s->norm.as<double>(), s->nn.as<double>(),
