@@ -61,9 +61,41 @@ __device__ __forceinline__ double fpow(double x, double p, int pi) {
 }
 
 // ---------------------------------------------------------------------------
+// Shared by the two contractions of the chosen form, whose operands are laid
+// out in pieces that a wave copies straight to LDS (1 KB: 16 rows of 64 bytes).
+// ---------------------------------------------------------------------------
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) const void gvoid;
+typedef __attribute__((address_space(3))) void lvoid;
+
+// 16-byte chunk position of k chunk c (0..3) in row r of an LDS slice block
+// (rows of 64 bytes, no padding): an XOR swizzle that keeps the fragment
+// reads (16 rows at four chunks) free of bank conflicts (a third of the LDS
+// cycles were conflicts with r / 2 xor r / 8 in its place).
+__device__ __forceinline__ int i8_chunk(int r, int c) { return c ^ (-(r >> 2) & 3); }
+
+// This lane's 16 bytes of a piece: they land at 16 lane, so it fetches the chunk
+// that belongs there.
+__device__ __forceinline__ unsigned piece_lane(int lane) {
+  return (lane >> 2) * 64 + 16 * i8_chunk(lane >> 2, lane & 3);
+}
+// Wave-uniform base `src`, kept in scalar registers so that one vector register
+// addresses every piece.
+__device__ __forceinline__ void copy_piece(const void *src, unsigned vsrc, void *dst) {
+  asm volatile("" : "+s"(src));
+  __builtin_amdgcn_global_load_lds((gvoid *)((const char *)src + vsrc), (lvoid *)dst, 16, 0, 0);
+}
+// Waits for this wave's copies, then for the other waves.
+__device__ __forceinline__ void copies_landed() {
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+  __syncthreads();
+}
+
+// ---------------------------------------------------------------------------
 // FP64 contraction C = A B^T (rows of both K-contiguous) on
-// v_mfma_f64_16x16x4: k_gemm_f64 with fragments straight from global memory
-// and k_gemm_f64_lds with 128 x 128 tiles staged in LDS; f64_tile chooses.
+// v_mfma_f64_16x16x4: k_gemm_f64 with fragments straight from global memory,
+// k_gemm_f64_dma with 32 x 32 and 64 x 64 tiles copied straight to LDS and
+// k_gemm_f64_lds with 128 x 128 tiles staged there; f64_tile chooses.
 //
 // What bounds them: an FP64 16x16x4 MFMA holds its SIMD's vector ALU for 64
 // cycles, so a wave with 64 x 64 outputs needs 16 KB per 4096 cycles; smaller
@@ -444,6 +476,147 @@ __global__ __launch_bounds__(256) void k_gemm_f64(F64Groups gs) {
   }
 }
 
+// The same 16T x 16T outputs per wave, T = 1 and 2, from operands that the
+// workgroup's four waves copy straight to LDS once: four stages of 16 k, three
+// of them on their way. k_gemm_f64 is bound by what a CU gets from L2 (20 bytes
+// a cycle), where its waves fetch every row twice. Needs 16-byte aligned rows.
+// LDS rows are 128 bytes, their 16-byte chunks swizzled by row / 2, so that the
+// 8-byte fragment reads (16 rows at two k) are free of bank conflicts.
+template <int EP, int T>
+__global__ __launch_bounds__(256, 2) void k_gemm_f64_dma(F64Groups gs) {
+  constexpr int R = 32 * T, ST = 2 * R * 128;
+  __shared__ double red[EP == EP_SUMSQ && T == 1 ? 128 : 1];
+  __shared__ __align__(16) int8_t s0[ST], s1[ST], s2[ST], s3[ST];
+  int tx, ty;
+  const F64Gemm &g = gs.g[f64_workgroup(gs, tx, ty)];
+  const int M = g.M, N = g.N;
+  int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int r16 = lane & 15, q4 = lane >> 4;
+  int rowb = ty * R, colb = tx * R, row0 = rowb + (wid >> 1) * 16 * T, col0 = colb + (wid & 1) * 16 * T;
+  // Past the diagonal of a lower triangular A every term is zero.
+  constexpr bool ORD = EP != EP_STORE;
+  int K = g.lower_tri ? min(g.K, rowb + R) : g.K, steps = K / 16;
+  int head = ORD ? 0 : K & 15;  // k before the first step (even); in plain order the rest follows
+  // Wave w copies the pieces (8 rows of 128 bytes) w T .. of either operand; rows
+  // past the end repeat the last one.
+  int ra0 = min(rowb, M - 1), rb0 = min(colb, N - 1);
+  const char *pa = reinterpret_cast<const char *>(g.A) + ((size_t)ra0 * g.lda + head) * 8;
+  const char *pb = reinterpret_cast<const char *>(g.B) + ((size_t)rb0 * g.ldb + head) * 8;
+  unsigned va[T], vb[T];
+#pragma unroll
+  for (int p = 0; p < T; p++) {
+    int r = 8 * (wid * T + p) + (lane >> 3), chunk = 16 * ((lane & 7) ^ ((r >> 1) & 7));
+    va[p] = (unsigned)((min(rowb + r, M - 1) - ra0) * g.lda * 8) + chunk;
+    vb[p] = (unsigned)((min(colb + r, N - 1) - rb0) * g.ldb * 8) + chunk;
+  }
+  auto copy = [&](int8_t *dst, int s) {
+#pragma unroll
+    for (int p = 0; p < T; p++) {
+      copy_piece(pa + (size_t)s * 128, va[p], dst + (wid * T + p) * 1024);
+      copy_piece(pb + (size_t)s * 128, vb[p], dst + R * 128 + (wid * T + p) * 1024);
+    }
+  };
+  v4d acc[T][T];
+#pragma unroll
+  for (int a = 0; a < T; a++)
+#pragma unroll
+    for (int b = 0; b < T; b++) acc[a][b] = v4d{0, 0, 0, 0};
+  auto pin = [&] {
+#pragma unroll
+    for (int a = 0; a < T; a++)
+#pragma unroll
+      for (int b = 0; b < T; b++) asm volatile("" : "+a"(acc[a][b]));
+  };
+  // MFMA j of 16 k takes k = 4 j + l / 16, or the k of k_gemm_f64 for EP_STORE.
+  auto k_of = [&](int j) { return ORD ? 4 * j + q4 : 8 * (j >> 1) + 2 * q4 + (j & 1); };
+  int ra = ((wid >> 1) * 16 * T + r16) * 128, swz = (r16 >> 1) & 7;
+  int rb = R * 128 + ((wid & 1) * 16 * T + r16) * 128;
+  int at[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) at[j] = 16 * ((k_of(j) >> 1) ^ swz) + 8 * (k_of(j) & 1);
+  auto step = [&](const int8_t *__restrict__ rd, int8_t *__restrict__ wr, int s) {
+    pin();
+    // This wave's copies but those of the newest two stages have landed, and with
+    // the barrier the other waves'; a __syncthreads would wait for all of them.
+    // The stage that `wr` held was multiplied in the step before.
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (4 * T));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    copy(wr, min(s + 3, steps - 1));
+    double fa[T][4], fb[T][4];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int t = 0; t < T; t++) {
+        fa[t][j] = *reinterpret_cast<const double *>(rd + ra + t * 2048 + at[j]);
+        fb[t][j] = *reinterpret_cast<const double *>(rd + rb + t * 2048 + at[j]);
+      }
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int a = 0; a < T; a++)
+#pragma unroll
+        for (int b = 0; b < T; b++)
+          acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[a][j], fb[b][j], acc[a][b], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // The K % 16 of k outside the steps, zeros around them.
+  double ta[T][4], tb[T][4];
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+#pragma unroll
+    for (int t = 0; t < T; t++) {
+      int k = (ORD ? 16 * steps : head - 16) + k_of(j);
+      bool in = k >= 0 && k < K;
+      ta[t][j] = in ? g.A[min(row0 + 16 * t + r16, M - 1) * (size_t)g.lda + k] : 0.0;
+      tb[t][j] = in ? g.B[min(col0 + 16 * t + r16, N - 1) * (size_t)g.ldb + k] : 0.0;
+    }
+  auto rest = [&] {
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (ORD ? 16 * steps + 4 * j < K : head > 0) {
+#pragma unroll
+        for (int a = 0; a < T; a++)
+#pragma unroll
+          for (int b = 0; b < T; b++)
+            acc[a][b] =
+                __builtin_amdgcn_mfma_f64_16x16x4f64(ta[a][j], tb[b][j], acc[a][b], 0, 0, 0);
+      }
+    pin();
+  };
+  if constexpr (!ORD) rest();
+  pin();
+  if (steps > 0) {
+    copy(s0, 0);
+    copy(s1, min(1, steps - 1));
+    copy(s2, min(2, steps - 1));
+    int s = 0;
+#pragma unroll 1
+    for (; s + 4 <= steps; s += 4) {
+      step(s0, s3, s);
+      step(s1, s0, s + 1);
+      step(s2, s1, s + 2);
+      step(s3, s2, s + 3);
+    }
+    if (s < steps) step(s0, s3, s);
+    if (s + 1 < steps) step(s1, s0, s + 1);
+    if (s + 2 < steps) step(s2, s1, s + 2);
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // no copy outlives the workgroup
+  }
+  pin();
+  if constexpr (ORD) rest();
+  if constexpr (EP == EP_SUMSQ && T == 1) {
+    if (!(wid >> 1)) f64_epilogue<EP, T>(g, acc, row0, col0, wid, red);
+    __syncthreads();
+    if (wid >> 1) f64_epilogue<EP, T>(g, acc, row0, col0, wid, red);
+  } else if (EP == EP_SUMSQ || (row0 < M && col0 < N)) {
+    f64_epilogue<EP, T>(g, acc, row0, col0, wid, red);
+  }
+}
+
 // 128 x 128 tiles in plain k order, four waves of 64 x 64: the next 16 k of
 // both operands are in flight to registers while the current ones, in LDS,
 // feed the MFMAs; two LDS buffers, one barrier per 16 k (4096 MFMA cycles), two
@@ -573,37 +746,6 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f64_lds(F64Groups gs) {
   }
   pin();
   f64_epilogue<EP, T>(g, acc, row0, col0, wid, nullptr);
-}
-
-// ---------------------------------------------------------------------------
-// Shared by the two contractions of the chosen form, whose operands are laid
-// out in pieces that a wave copies straight to LDS (1 KB: 16 rows of 64 bytes).
-// ---------------------------------------------------------------------------
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(1))) const void gvoid;
-typedef __attribute__((address_space(3))) void lvoid;
-
-// 16-byte chunk position of k chunk c (0..3) in row r of an LDS slice block
-// (rows of 64 bytes, no padding): an XOR swizzle that keeps the fragment
-// reads (16 rows at four chunks) free of bank conflicts (a third of the LDS
-// cycles were conflicts with r / 2 xor r / 8 in its place).
-__device__ __forceinline__ int i8_chunk(int r, int c) { return c ^ (-(r >> 2) & 3); }
-
-// This lane's 16 bytes of a piece: they land at 16 lane, so it fetches the chunk
-// that belongs there.
-__device__ __forceinline__ unsigned piece_lane(int lane) {
-  return (lane >> 2) * 64 + 16 * i8_chunk(lane >> 2, lane & 3);
-}
-// Wave-uniform base `src`, kept in scalar registers so that one vector register
-// addresses every piece.
-__device__ __forceinline__ void copy_piece(const void *src, unsigned vsrc, void *dst) {
-  asm volatile("" : "+s"(src));
-  __builtin_amdgcn_global_load_lds((gvoid *)((const char *)src + vsrc), (lvoid *)dst, 16, 0, 0);
-}
-// Waits for this wave's copies, then for the other waves.
-__device__ __forceinline__ void copies_landed() {
-  __builtin_amdgcn_s_waitcnt(0x0f70);
-  __syncthreads();
 }
 
 // This workgroup's tile of a launch over several contractions (first tiles
@@ -1133,9 +1275,12 @@ int pinned_shape(int n_shapes) {
 }
 
 template <int EP>
-void f64_launch(hipStream_t st, int T, int blocks, const F64Groups &gs) {
+void f64_launch(hipStream_t st, int T, bool dma, int blocks, const F64Groups &gs) {
   dim3 grid(blocks), block(256);
-  if (T == 1) {
+  if (T <= 2 && dma) {
+    if (T == 1) hipLaunchKernelGGL((k_gemm_f64_dma<EP, 1>), grid, block, 0, st, gs);
+    else hipLaunchKernelGGL((k_gemm_f64_dma<EP, 2>), grid, block, 0, st, gs);
+  } else if (T == 1) {
     hipLaunchKernelGGL((k_gemm_f64<EP, 1, 2>), grid, block, 0, st, gs);
   } else if (T == 2) {
     hipLaunchKernelGGL((k_gemm_f64<EP, 2, 1>), grid, block, 0, st, gs);
@@ -1218,15 +1363,15 @@ void gemm_i8_groups(hipStream_t st, const std::vector<I8Gemm> &all) {
 //                  through LDS; the matrix cores' limit, where the kernel
 //                  before had 48)
 //   T = 3  1.25   (63, EP_STORE only)
-//   T = 2  0.72   (50, 47; bound by its loads)
-//   T = 1  0.35   (27, the same)
-// EP_KERNEL in us at T = 4, 2, 1: 2 x 2,000 x 500 x 2,100 takes 309, 193, 332;
-// 3 x 8,000 x 200 x 1,500 405, 411, 613; 2 x 512 x 200 x 4,080 574, 228, 117;
-// 3 x 170 x 167 x 1,500 218, 78, 35 (one species after the other on 64 x 64
-// workgroup tiles it had taken 309). EP_SUMSQ, 2 x 1,000 x 16,000, triangular:
-// 592, 677, 1229 (941 before).
-static int f64_tile(int ep, const std::vector<F64Gemm> &gs) {
-  constexpr double kTime[5] = {0, 0.35, 0.72, 1.25, 2.1};
+//   T = 2  0.58   (63, 61; k_gemm_f64 without aligned rows 0.72: 50, 47)
+//   T = 1  0.18   (54, 53; without 0.35: 27)
+// EP_KERNEL in us at T = 4, 2, 1 (and 2, 1 without aligned rows): 2 x 2,000 x
+// 500 x 2,100 takes 309, 159, 174 (207, 359); 3 x 8,000 x 200 x 1,500 402, 312, 344
+// (421, 615); 2 x 512 x 200 x 4,080 572, 158, 51 (228, 120); 3 x 170 x 167 x
+// 1,500 219, 62, 21 (73, 34); 108 x 32 x 144 31, 11, 5 (13, 9). EP_SUMSQ, 3 x 200 x
+// 8,000, triangular: 64, 42, 43 (50, 66).
+static int f64_tile(int ep, const std::vector<F64Gemm> &gs, bool dma) {
+  const double kTime[5] = {0, dma ? 0.18 : 0.35, dma ? 0.58 : 0.72, 1.25, 2.1};
   int pin = pinned_shape(4);
   if (pin >= 0 && !(pin == 1 && ep != EP_STORE)) return 4 - pin;
   constexpr int kSimds = 1024;  // 256 CUs
@@ -1254,7 +1399,13 @@ void gemm_f64_groups(hipStream_t st, int ep, const std::vector<F64Gemm> &all) {
   for (const F64Gemm &g : all)
     if (g.M > 0 && g.N > 0) live.push_back(g);
   if (live.empty()) return;
-  int T = f64_tile(ep, live);
+  // Operands whose rows start at 16 bytes (and 64 rows within 2 GB); for EP_STORE
+  // the steps end at the last k, so K is even, too.
+  bool dma = true;
+  for (const F64Gemm &g : live)
+    dma = dma && ((uintptr_t)g.A | (uintptr_t)g.B) % 16 == 0 && g.lda % 2 == 0 &&
+          g.ldb % 2 == 0 && std::max(g.lda, g.ldb) < (1ll << 22) && (ep != EP_STORE || g.K % 2 == 0);
+  int T = f64_tile(ep, live, dma);
   for (size_t g0 = 0; g0 < live.size(); g0 += kF64Groups) {
     F64Groups gs{};
     gs.n = (int)std::min<size_t>(kF64Groups, live.size() - g0);
@@ -1272,10 +1423,10 @@ void gemm_f64_groups(hipStream_t st, int ep, const std::vector<F64Gemm> &all) {
     }
     gs.first[gs.n] = (int)blocks;
     bool p12 = live[g0].e.power == 2.0 || live[g0].e.power == 1.0;  // one model, one power
-    if (ep == EP_KERNEL && p12) f64_launch<EP_KERNEL>(st, T, (int)blocks, gs);
-    else if (ep == EP_KERNEL) f64_launch<EP_KERNEL_POW>(st, T, (int)blocks, gs);
-    else if (ep == EP_STORE) f64_launch<EP_STORE>(st, T, (int)blocks, gs);
-    else f64_launch<EP_SUMSQ>(st, T, (int)blocks, gs);
+    if (ep == EP_KERNEL && p12) f64_launch<EP_KERNEL>(st, T, dma, (int)blocks, gs);
+    else if (ep == EP_KERNEL) f64_launch<EP_KERNEL_POW>(st, T, dma, (int)blocks, gs);
+    else if (ep == EP_STORE) f64_launch<EP_STORE>(st, T, dma, (int)blocks, gs);
+    else f64_launch<EP_SUMSQ>(st, T, dma, (int)blocks, gs);
     FM_HIP(hipGetLastError());
   }
 }
