@@ -758,53 +758,60 @@ __device__ __forceinline__ void stage_w(const T *G, const T *B, T sg, T sb, T *w
     w[k] = withb ? w_elem(sg, G[k], sb, B[k]) : sg * G[k];
 }
 
-// FP32 rows: G . B and w = sg G - sb B (sb = (G . B) s3) in one pass over
-// both rows. Each of the atom's 128 threads stores its V-vectors of G to LDS
-// as they arrive and keeps those of B (at most R, rows of at most 128 R E
-// elements) in registers until sb is known; the partition and summation
-// order of the dot are those of row_dot. red holds the two wavefronts'
-// partial dots; the barrier inside is reached by every thread of the block
-// (dead atoms load nothing).
-template <typename V, int R>
+// FP32 rows: G . B and w = sg G - sb B in one pass over both rows. Each of the
+// atom's 128 threads loads all of its V-vectors of G and B (at most R of each,
+// rows of at most 128 R E elements) before it uses the first; waiting for each
+// in turn kept 80 % of the wave cycles idle (262144 atoms of 3,255 elements: the
+// call 44.1 ms, now 42.7; 512 structures of 1,500 in two passes 11.6, now 11.4,
+// beside the variance on the other stream). The partition and the order of the dot
+// are those of row_dot for vectors of four, and single elements 128 apart for V =
+// float. sb_of(a, b) makes sb of the two wavefronts' dots; red holds them; the
+// barrier inside is reached by every thread of the block (dead atoms load the
+// first row).
+template <typename V, int R, typename F>
 __device__ __forceinline__ void stage_w_onepass(const float *G, const float *B, float sg,
-                                                float s3, float *wl, int n, bool live, int t2,
+                                                F &&sb_of, float *wl, int n, bool live, int t2,
                                                 int lane, int w, int slot, float *red) {
   constexpr int E = sizeof(V) / sizeof(float);
   const V *gv = reinterpret_cast<const V *>(G), *bv = reinterpret_cast<const V *>(B);
-  V *wv = reinterpret_cast<V *>(wl);
-  int nv = live ? n / E : 0;
-  V b[R];
+  int nv = n / E;
+  V g[R], b[R];
+#pragma unroll
+  for (int j = 0; j < R; j++) {
+    int v = max(min(t2 + 128 * j, nv - 1), 0);
+    g[j] = nv > 0 ? gv[v] : V{};
+    b[j] = nv > 0 ? bv[v] : V{};
+  }
+  int kt = nv * E + t2;
+  bool tail = kt < n;
+  float gt = tail ? G[kt] : 0.f, bt = tail ? B[kt] : 0.f;
   float acc = 0;
 #pragma unroll
   for (int j = 0; j < R; j++) {
-    int v = t2 + 128 * j;
-    if (v < nv) {
-      V g = gv[v];
-      b[j] = bv[v];
-      const float *xs = reinterpret_cast<const float *>(&g);
-      const float *ys = reinterpret_cast<const float *>(&b[j]);
+    const float *xs = reinterpret_cast<const float *>(&g[j]);
+    const float *ys = reinterpret_cast<const float *>(&b[j]);
+    float sum = acc;
 #pragma unroll
-      for (int e = 0; e < E; e++) acc = fma(xs[e], ys[e], acc);
-      wv[v] = g;
-    }
+    for (int e = 0; e < E; e++) sum = fma(xs[e], ys[e], sum);
+    acc = t2 + 128 * j < nv ? sum : acc;
   }
-  int kt = nv * E + t2;
-  bool tail = live && kt < n;
-  float gt = tail ? G[kt] : 0.f, bt = tail ? B[kt] : 0.f;
   acc = fma(gt, bt, acc);
   acc = wave_sum(acc);
   if (lane == 0) red[w] = acc;
   __syncthreads();
-  float sb = (red[2 * slot] + red[2 * slot + 1]) * s3;
+  if (!live) return;
+  float sb = sb_of(red[2 * slot], red[2 * slot + 1]);
+  V *wv = reinterpret_cast<V *>(wl);
 #pragma unroll
   for (int j = 0; j < R; j++) {
     int v = t2 + 128 * j;
     if (v < nv) {
-      V r = wv[v];
+      V r;
       float *rs = reinterpret_cast<float *>(&r);
+      const float *xs = reinterpret_cast<const float *>(&g[j]);
       const float *ys = reinterpret_cast<const float *>(&b[j]);
 #pragma unroll
-      for (int e = 0; e < E; e++) rs[e] = w_elem(sg, rs[e], sb, ys[e]);
+      for (int e = 0; e < E; e++) rs[e] = w_elem(sg, xs[e], sb, ys[e]);
       wv[v] = r;
     }
   }
@@ -815,17 +822,19 @@ __device__ __forceinline__ void stage_w_onepass(const float *G, const float *B, 
 constexpr int kOnePassRow = 128 * 32;
 
 // LC >= 0: l_max known at compile time (one accumulator per l up to it, in
-// place of kMaxL + 1); LC = -1 for any l_max. OP (FP32 only):
-// projection from the rows with one pass over G and B (more registers;
-// chosen where LDS, not registers, bounds the atoms per CU). Two wavefronts per atom share
+// place of kMaxL + 1); LC = -1 for any l_max. OP > 0 (FP32 only):
+// projection from the rows with one pass over G and B, of at most 512 OP elements
+// (`single`: by single elements where rows are not 16-byte aligned). Two
+// wavefronts per atom share
 // its LDS rows: both stage (twice the loads in flight per atom for the same
 // LDS) and each takes half of the 16-row output tiles.
-template <typename T, int LC, bool OP = false>
+template <typename T, int LC, int OP = 0>
 __global__ __launch_bounds__(128 * kAtomsPerBlock) void k_dEdc(B2Args a, const T *B,
                                                                  const double *norm,
                                                                  const double *nnv, const T *G,
                                                                  long long g_ld, AdjArgs aa,
-                                                                 const T *Cg, T *Ug) {
+                                                                 const T *Cg, T *Ug,
+                                                                 int single) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ T red[2 * kAtomsPerBlock];
   int lane = threadIdx.x & 63, w = threadIdx.x >> 6, slot = w >> 1, sub = w & 1;
@@ -844,19 +853,26 @@ __global__ __launch_bounds__(128 * kAtomsPerBlock) void k_dEdc(B2Args a, const T
   // w = dE/dB = (G - (G . B_hat) B_hat) / |B| = sg G - sb B.
   T ninv = T(1) / (T)nrm;
   T sg = aa.project ? ninv : T(1), sb = 0;
-  if constexpr (OP && sizeof(T) == 4) {
-    // The launch guarantees project, no energies and nd <= kOnePassRow.
+  if constexpr (OP > 0 && sizeof(T) == 4) {
+    // The launch guarantees project, no energies and nd <= 512 OP.
     if (live) stage_row(Cg + (size_t)i * nc, c, nc, t2, 128);
     // Every row 16-byte aligned: the same for all atoms of the grid, so the
     // whole block takes one branch and one barrier.
     bool al = ((reinterpret_cast<uintptr_t>(G) | reinterpret_cast<uintptr_t>(B)) & 15) == 0 &&
               (g_ld & 3) == 0 && (a.nd & 3) == 0;
-    if (al)
-      stage_w_onepass<float4, kOnePassRow / 512>(Grow, Brow, sg, ninv * ninv * ninv, wl, a.nd,
-                                                 live, t2, lane, w, slot, red);
+    float s3 = ninv * ninv * ninv;
+    if (!single)
+      stage_w_onepass<f4u, OP>(
+          Grow, Brow, sg, [&](float x, float y) { return (x + y) * ninv * ninv * ninv; }, wl,
+          a.nd, live, t2, lane, w, slot, red);
+    else if (al)
+      stage_w_onepass<f4u, OP>(
+          Grow, Brow, sg, [&](float x, float y) { return (x + y) * s3; }, wl, a.nd, live, t2,
+          lane, w, slot, red);
     else
-      stage_w_onepass<float, kOnePassRow / 128>(Grow, Brow, sg, ninv * ninv * ninv, wl, a.nd,
-                                                live, t2, lane, w, slot, red);
+      stage_w_onepass<float, 4 * OP>(
+          Grow, Brow, sg, [&](float x, float y) { return (x + y) * s3; }, wl, a.nd, live, t2,
+          lane, w, slot, red);
   } else {
     if (aa.project) {
       if (aa.energy) {
@@ -1236,11 +1252,11 @@ void launch_adjoint(fm_structure s, const void *G, int64_t g_ld, void *fbond,
   if (s->n == 0) return;
   if (s->desc_kind == 3)
     launch_dEdc_b3(s, G, g_ld, project, empty_norm, empty_nn, u_buf);
-  // FP32 projection from the rows in one pass over G and B where LDS
-  // already holds the CU to two blocks (the one-pass registers cost no
-  // occupancy there; with three or more blocks they would).
-  bool one_pass = !f64 && project && !energy && a.nd <= kOnePassRow &&
-                  3 * (size_t)apb1 * per1 > (size_t)160 * 1024;
+  // FP32 projection from the rows in one pass over G and B. Rows whose LDS holds
+  // a CU to two workgroups take single elements where they are not aligned and
+  // the cube of 1 / |B| in one factor; the others have the order of row_dot.
+  bool one_pass = !f64 && project && !energy && a.nd <= kOnePassRow;
+  int single = 3 * (size_t)apb1 * per1 > (size_t)160 * 1024;
   if (s->desc_kind == 2) {
     KScope timer(ctx, KT_DEDC);
     with_lmax(a.lmax, [&](auto lc) {
@@ -1249,17 +1265,18 @@ void launch_adjoint(fm_structure s, const void *G, int64_t g_ld, void *fbond,
         hipLaunchKernelGGL((k_dEdc<double, LC>), dim3(nblk1), dim3(128 * apb1), apb1 * per1, st,
                            a, s->B.as<double>(), s->norm.as<double>(), s->nn.as<double>(),
                            (const double *)G, (long long)g_ld, aa, s->C.as<double>(),
-                           (double *)u_buf);
+                           (double *)u_buf, 0);
       else if (one_pass)
-        hipLaunchKernelGGL((k_dEdc<float, LC, true>), dim3(nblk1), dim3(128 * apb1),
-                           apb1 * per1, st, a, s->B.as<float>(), s->norm.as<double>(),
-                           s->nn.as<double>(), (const float *)G, (long long)g_ld, aa,
-                           s->C.as<float>(), (float *)u_buf);
+        hipLaunchKernelGGL((a.nd <= kOnePassRow / 2 ? k_dEdc<float, LC, kOnePassRow / 1024>
+                                                    : k_dEdc<float, LC, kOnePassRow / 512>),
+                           dim3(nblk1), dim3(128 * apb1), apb1 * per1, st, a, s->B.as<float>(),
+                           s->norm.as<double>(), s->nn.as<double>(), (const float *)G,
+                           (long long)g_ld, aa, s->C.as<float>(), (float *)u_buf, single);
       else
         hipLaunchKernelGGL((k_dEdc<float, LC>), dim3(nblk1), dim3(128 * apb1), apb1 * per1, st,
                            a, s->B.as<float>(), s->norm.as<double>(), s->nn.as<double>(),
                            (const float *)G, (long long)g_ld, aa, s->C.as<float>(),
-                           (float *)u_buf);
+                           (float *)u_buf, 0);
     });
   }
   FM_HIP(hipGetLastError());

@@ -47,3 +47,10 @@ def test_descriptor_rows(oracle, settings, n, rc):
     scale = max(np.max(np.abs(mean[1:])), 1e-3 * abs(mean[0]))
     assert np.max(np.abs(m[1:] - mean[1:])) < 1e-3 * scale
     assert np.max(np.abs(p.local_uncertainties[0] - var)) < 1e-3 * 1.5 ** 2
+
+
+@pytest.mark.parametrize("settings", [(3, 10, 6), (2, 9, 4), (1, 5, 0), (3, 10, 5), (2, 14, 4)])
+def test_projection_rows(oracle, settings):
+    """The adjoint's rows in one pass: 3255 values (single elements), 855 and 15
+    (unaligned vectors), 2790 and 2030 (odd counts of vectors)."""
+    test_descriptor_rows(oracle, settings, 37, 4.5)
