@@ -456,9 +456,8 @@ def serving_leg(sgp, calc, batched, n_requests=2000, n_fp64=200):
                  max_batch_atoms=32768)
     try:
         # Untimed warm-up stream of the same length and distribution (other
-        # structures): the contraction tiles of each batch shape are
-        # autotuned on first use, and the batch shapes that only form under
-        # load would otherwise stall the timed run.
+        # structures): the workers' buffer pools grow to the batch shapes that
+        # only form under load, which would otherwise stall the timed run.
         poisson_run(srv, batch_structures(n_requests, seed=43, n_min=32, n_max=8192),
                     rate=rate, seed=4)
         srv.batches.clear()
