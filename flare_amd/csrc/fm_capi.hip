@@ -525,6 +525,9 @@ static void compute_descriptor(fm_structure s, const fm_b2_settings *st_in, int 
     FM_HIP(hipSetDevice(ctx->device));
     hipStream_t stream = ctx->stream;
     fm::Pool *pool = &ctx->pool;
+    // From here to the end the structure has no descriptors: a failure leaves it
+    // without any, not with sizes of these settings beside lists of earlier ones.
+    s->has_b2 = s->has_q = s->has_dervs = false;
     s->nos = st_in->n_species;
     s->N = st_in->n_max;
     s->lmax = st_in->l_max;
@@ -547,6 +550,7 @@ static void compute_descriptor(fm_structure s, const fm_b2_settings *st_in, int 
     if (s->n > 0) {
       // Species must lie in [0, n_species) for this descriptor.
       FM_CHECK(s->max_species < s->nos, FM_ERR_INVALID, "species outside [0, n_species)");
+      fm::check_b2_limits(s);
     }
     ctx->mark_begin(fm::ST_DESC);
     ctx->kt_clear(fm::KT_DESC, fm::KT_DESC);
@@ -582,8 +586,7 @@ static void compute_descriptor(fm_structure s, const fm_b2_settings *st_in, int 
     ctx->mark_end(fm::ST_DESC);
     // Per-structure species-sorted position of every row (batches only).
     fm::build_var_pos(s);
-    s->has_dervs = false;    // dense derivatives are rebuilt on demand
-    s->DB.release();
+    s->DB.release();  // dense derivatives are rebuilt on demand
     s->has_b2 = true;
   }
 }

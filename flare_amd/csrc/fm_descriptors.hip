@@ -1173,11 +1173,14 @@ void descriptor_setup() {
   FM_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_rcp), rcp, sizeof(rcp), 0, hipMemcpyHostToDevice));
 }
 
+void check_b2_limits(fm_structure s) {
+  FM_CHECK(s->N <= kMaxN, FM_ERR_INVALID, "n_max above 16 is not supported");
+  FM_CHECK(s->lmax <= kMaxL, FM_ERR_INVALID, "l_max above 10 is not supported");
+}
+
 void launch_b2(fm_structure s, bool want_b2) {
   fm_context ctx = s->ctx;
   hipStream_t st = ctx->stream;
-  FM_CHECK(s->N <= kMaxN, FM_ERR_INVALID, "n_max above 16 is not supported");
-  FM_CHECK(s->lmax <= kMaxL, FM_ERR_INVALID, "l_max above 10 is not supported");
   B2Args a = make_args(s);
   // The chosen form's B2 rows are computed in FP64 (mixed: FP32 row and c
   // for the adjoint, int8 slices of the FP64 row for the kernel

@@ -332,7 +332,9 @@ void build_neighbors(fm_structure s, const int *species_dev, const double *posit
 // in between.
 void build_bonds(fm_structure s);
 void bonds_ready(fm_structure s);
-// fm_descriptors.hip (want_b2 = false computes and keeps only c)
+// fm_descriptors.hip: the largest n_max and l_max of the bond kernels (checked
+// before any launch), and the descriptors (want_b2 = false: only c)
+void check_b2_limits(fm_structure s);
 void launch_b2(fm_structure s, bool want_b2 = true);
 // Device var_pos of a batch (after build_bonds); releases it for one structure.
 void build_var_pos(fm_structure s);
