@@ -156,6 +156,7 @@ void *Pool::get(size_t bytes, size_t *cls) {
   void *p = nullptr;
   hipError_t e = hipMalloc(&p, c);
   if (e != hipSuccess) {
+    (void)hipGetLastError();  // or the next launch's check would report it
     // Drop the cache and retry once before giving up.
     for (auto &kv : free_)
       for (void *q : kv.second) (void)hipFree(q);
@@ -427,6 +428,9 @@ static int structure_create(fm_context ctx, int n_struct, const double *cells,
       }
       ctx->mark_end(fm::ST_NEIGH);
     } catch (...) {
+      // The upload from the staging buffer and the kernels that follow it may
+      // still be queued, and the next structure fills that buffer again.
+      (void)hipStreamSynchronize(ctx->stream);
       delete s;
       throw;
     }
@@ -696,7 +700,14 @@ int fm_model_create(fm_context ctx, const fm_model_desc *d, fm_model *out) {
     FM_HIP(hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
     auto *m = new fm_model_s();
-    std::unique_ptr<fm_model_s> owner(m);  // deleted if a check below throws
+    // Deleted if a check below throws, after the uploads from the caller's arrays
+    // and the local ones.
+    std::vector<double> vec, RT;
+    auto undo = [st](fm_model_s *p) {
+      (void)hipStreamSynchronize(st);
+      delete p;
+    };
+    std::unique_ptr<fm_model_s, decltype(undo)> owner(m, undo);
     m->ctx = ctx;
     m->sigma = d->sigma;
     m->power = d->power;
@@ -716,7 +727,7 @@ int fm_model_create(fm_context ctx, const fm_model_desc *d, fm_model *out) {
     fm::Pool *pool = &ctx->pool;
     // Norms, alpha and alpha without the empty sparse environments, which
     // contribute nothing (normalized_dot_product.cpp:158-162).
-    std::vector<double> vec(3 * (size_t)M);
+    vec.resize(3 * (size_t)M);
     for (int j = 0; j < M; j++) {
       vec[j] = d->sparse_norms[j];
       vec[M + j] = d->alpha[j];
@@ -776,7 +787,7 @@ int fm_model_create(fm_context ctx, const fm_model_desc *d, fm_model *out) {
     if (m->has_R) {
       // R_inv^T, the left operand of |R_inv^T k|^2; lower triangular when
       // R_inv is upper triangular (the QR factor's inverse).
-      std::vector<double> RT((size_t)M * M);
+      RT.resize((size_t)M * M);
       int upper = 1;
       for (int r = 0; r < M; r++)
         for (int c = 0; c < M; c++) {

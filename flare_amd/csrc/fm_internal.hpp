@@ -22,12 +22,16 @@ struct Error : std::runtime_error {
   Error(int c, const std::string &m) : std::runtime_error(m), code(c) {}
 };
 
+// A failed call leaves its error behind for hipGetLastError; it is taken here, or
+// the check of the next call's launches would report it again.
 #define FM_HIP(call)                                                          \
   do {                                                                        \
     hipError_t e_ = (call);                                                   \
-    if (e_ != hipSuccess)                                                     \
+    if (e_ != hipSuccess) {                                                   \
+      (void)hipGetLastError();                                                \
       throw ::fm::Error(FM_ERR_HIP, std::string(#call) + ": " +              \
                                         hipGetErrorString(e_));               \
+    }                                                                         \
   } while (0)
 
 // Sets the calling thread's fm_last_error() message (entry points that do

@@ -39,3 +39,38 @@ def test_failed_recompute(settings):
     _lib.check(L.fm_structure_compute_b2(s._h, ctypes.byref(good), 0))
     _lib.check(L.fm_predict(model.h, s._h, _lib.PREDICT_MEAN, 0, _lib.ptr(mean), None, None))
     assert np.array_equal(mean, before)
+
+
+def test_failed_creation():
+    """Structures and models that are refused while their uploads are queued do
+    not disturb the ones made next from the same buffers."""
+    from flare_amd import _C_flare as C
+    calc = C.B2("chebyshev", "quadratic", [0.0, 4.0], [], [2, 4, 3])
+    cell, species, pos = random_cell(300, 5, nos=2, scale=16.0, skew=0.2)
+    want = C.Structure(cell, species, pos, 4.0, [calc])
+    sgp = C.SparseGP([C.NormalizedDotProduct(1.5, 2.0)], 0.1, 0.1, 0.1)
+    sgp.add_specific_environments(want, [int(a) for t in range(2)
+                                         for a in np.flatnonzero(species == t)[:2]])
+    sgp.update_L_inverse()
+    sgp.set_alpha(np.linspace(-0.2, 0.3, sgp.n_sparse))
+    sgp.predict_local_uncertainties(want)
+    L_inv = sgp.L_inv.copy()
+    for _ in range(20):
+        bad = pos.copy()
+        bad[17, 1] = np.nan
+        with pytest.raises(ValueError):
+            C.Structure(cell * 1.1, species, bad, 4.0, [calc])
+        with pytest.raises(ValueError):
+            C.Structure(cell * 1.1, -species - 1, pos, 4.0, [calc])
+        s = C.Structure(cell, species, pos, 4.0, [calc])
+        wrong = L_inv.copy()
+        wrong[0, -1] = 1.0  # above the diagonal block of the second species
+        sgp.L_inv = wrong
+        sgp._invalidate()
+        with pytest.raises(ValueError):
+            sgp.predict_local_uncertainties(s)
+        sgp.L_inv = L_inv
+        sgp._invalidate()
+        sgp.predict_local_uncertainties(s)
+        assert np.array_equal(s.mean_efs, want.mean_efs)
+        assert np.array_equal(s.local_uncertainties[0], want.local_uncertainties[0])
