@@ -299,6 +299,22 @@ int fm_context_stream(fm_context ctx, void **stream) {
   return guarded([&] { *stream = (void *)ctx->stream; });
 }
 
+// An array that the setup kernel may read where it is: memory of the context's
+// own GPU, allocated over all of [p, p + bytes) and aligned. Everything else
+// (another GPU's memory, host memory, an array that is too short) goes through a
+// copy, which the runtime checks.
+static bool readable_in_place(fm_context ctx, const void *p, size_t bytes, size_t align) {
+  hipPointerAttribute_t a{};
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  bool known = hipPointerGetAttributes(&a, p) == hipSuccess && a.type == hipMemoryTypeDevice &&
+               a.device == ctx->device &&
+               hipMemGetAddressRange(&base, &size, const_cast<void *>(p)) == hipSuccess;
+  if (!known) (void)hipGetLastError();
+  size_t at = known ? (uintptr_t)p - (uintptr_t)base : 0;
+  return known && (uintptr_t)p % align == 0 && at <= size && bytes <= size - at;
+}
+
 // Host species and positions up to this many bytes join the pinned upload.
 constexpr size_t kStageAtoms = 256 << 10;
 
@@ -371,6 +387,9 @@ static int structure_create(fm_context ctx, int n_struct, const double *cells,
       // species and positions among them.
       size_t n_pos = 3 * (size_t)n * sizeof(double), n_sp = (size_t)n * sizeof(int);
       bool staged = !device_ptrs && n_pos + n_sp <= kStageAtoms;
+      bool in_place = device_ptrs && n > 0 &&
+                      readable_in_place(ctx, species, n_sp, sizeof(int)) &&
+                      readable_in_place(ctx, positions, n_pos, sizeof(double));
       struct Part {
         fm::DevBuf *buf;
         const void *src;
@@ -404,10 +423,10 @@ static int structure_create(fm_context ctx, int n_struct, const double *cells,
       if (!staged) {
         s->species.alloc(pool, std::max<size_t>(1, n_sp));
         s->positions.alloc(pool, std::max<size_t>(1, n_pos));
-        if (n > 0 && !device_ptrs) {
-          FM_HIP(hipMemcpyAsync(s->species.as<int>(), species, n_sp, hipMemcpyHostToDevice, st));
-          FM_HIP(hipMemcpyAsync(s->positions.as<double>(), positions, n_pos,
-                                hipMemcpyHostToDevice, st));
+        if (n > 0 && !in_place) {
+          hipMemcpyKind kind = device_ptrs ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+          FM_HIP(hipMemcpyAsync(s->species.as<int>(), species, n_sp, kind, st));
+          FM_HIP(hipMemcpyAsync(s->positions.as<double>(), positions, n_pos, kind, st));
         }
       }
       ctx->mark_begin(fm::ST_NEIGH);
@@ -416,7 +435,7 @@ static int structure_create(fm_context ctx, int n_struct, const double *cells,
         // synchronisation); the neighbour kernels only bin (clamped) and copy
         // species, so bad input cannot take them out of bounds before it is
         // reported.
-        fm::build_neighbors(s, device_ptrs ? species : nullptr, device_ptrs ? positions : nullptr);
+        fm::build_neighbors(s, in_place ? species : nullptr, in_place ? positions : nullptr);
         int hf0 = ctx->pinned[0], hf1 = ctx->pinned[1];
         FM_CHECK(!(hf0 & 1), FM_ERR_INVALID, "positions contain NaN or Inf");
         FM_CHECK(!(hf0 & 2), FM_ERR_INVALID, "species must be non-negative");

@@ -70,7 +70,9 @@ int fm_context_stream(fm_context ctx, void **stream);
 int fm_structure_create(fm_context ctx, const double *cell, int n_atoms,
                         const int32_t *species, const double *positions,
                         double cutoff, fm_structure *out);
-/* As above with species and positions already in device memory. */
+/* As above with species and positions already in device memory (of the
+ * context's GPU: read in place; anything else is copied first, and an array
+ * shorter than n_atoms is an error). They are not needed after the call. */
 int fm_structure_create_device(fm_context ctx, const double *cell, int n_atoms,
                                const int32_t *species_dev,
                                const double *positions_dev, double cutoff,

@@ -1,0 +1,92 @@
+"""Caller memory of every kind at the entry points that take device pointers."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from helpers import random_cell
+
+pytestmark = pytest.mark.gpu
+
+RC = 4.0
+
+
+@pytest.fixture(scope="module")
+def system():
+    return random_cell(50, 5, nos=2, scale=8.8, skew=0.2)
+
+
+def neighbors(h):
+    from flare_amd import _lib
+    L = _lib.load()
+    sweep, nnb, vol, ssc = ctypes.c_int(), ctypes.c_int64(), ctypes.c_double(), ctypes.c_double()
+    _lib.check(L.fm_structure_info(h, ctypes.byref(sweep), ctypes.byref(nnb), ctypes.byref(vol),
+                                   ctypes.byref(ssc)))
+    sp, rel = np.zeros(nnb.value, np.int32), np.zeros((nnb.value, 4))
+    _lib.check(L.fm_structure_get_neighbors(h, None, None, None, None, _lib.ptr(sp),
+                                            _lib.ptr(rel)))
+    _lib.check(L.fm_structure_destroy(h))
+    return sp, rel
+
+
+def create(fn, system, species, positions):
+    from flare_amd import _lib
+    h = ctypes.c_void_p()
+    cell = _lib.f64(system[0].reshape(-1))
+    rc = getattr(_lib.load(), fn)(_lib.default_context().h, _lib.ptr(cell), len(system[1]),
+                                  species, positions, RC, ctypes.byref(h))
+    return rc, h
+
+
+@pytest.mark.parametrize("kind", ["device", "slice", "misaligned", "pinned"])
+def test_structure_sources(system, kind):
+    """Species and positions in the GPU's memory, inside a larger array, at an
+    address that is no multiple of the element's size, and in pinned memory."""
+    import torch
+    from flare_amd import _lib
+    sp, pos = _lib.i32(system[1]), _lib.f64(system[2]).reshape(-1)
+    rc, h = create("fm_structure_create", system, _lib.ptr(sp), _lib.ptr(pos))
+    _lib.check(rc)
+    want = neighbors(h)
+    lead = {"device": 0, "slice": 16, "misaligned": 2, "pinned": 0}[kind]
+    held = []
+    for a in (sp, pos):
+        raw = torch.zeros(lead + a.nbytes, dtype=torch.uint8)
+        raw[lead:] = torch.from_numpy(a.view(np.uint8))
+        held.append(raw.pin_memory() if kind == "pinned" else raw.cuda())
+    torch.cuda.synchronize()
+    rc, h = create("fm_structure_create_device", system, *(t.data_ptr() + lead for t in held))
+    _lib.check(rc)
+    got = neighbors(h)
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("short", [0, 1])
+def test_short_array(system, short):
+    """An array shorter than the atom count is an error, as for a copy, and the
+    next structure is built as if it had not been."""
+    from flare_amd import _lib
+    hip = ctypes.CDLL("libamdhip64.so")
+    hip.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
+    hip.hipMemcpy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
+    hip.hipFree.argtypes = [ctypes.c_void_p]
+    arrays = [_lib.i32(system[1]), _lib.f64(system[2]).reshape(-1)]
+    rc, h = create("fm_structure_create", system, *map(_lib.ptr, arrays))
+    _lib.check(rc)
+    want = neighbors(h)
+    ptrs = []
+    for k, a in enumerate(arrays):
+        p = ctypes.c_void_p()
+        size = a.nbytes - (16 if k == short else 0)
+        assert hip.hipMalloc(ctypes.byref(p), size) == 0
+        assert hip.hipMemcpy(p, a.ctypes.data, size, 1) == 0
+        ptrs.append(p)
+    for _ in range(5):
+        rc, h = create("fm_structure_create_device", system, *ptrs)
+        assert rc == _lib.FM_ERR_HIP
+        rc, h = create("fm_structure_create", system, *map(_lib.ptr, arrays))
+        _lib.check(rc)
+        got = neighbors(h)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    for p in ptrs:
+        assert hip.hipFree(p) == 0
