@@ -304,13 +304,15 @@ struct fm_mapped_s {
 };
 
 namespace fm {
-// fm_predict.hip
-struct HostOut {
-  double *dst = nullptr;  // host memory, or null
+// fm_predict.hip: arrays to the caller's memory (host or device, any may be
+// null); returns after the copies have finished. may_stage: through the
+// context's pinned memory, which may grow for it.
+struct Output {
+  double *dst = nullptr;
   const double *src = nullptr;
   size_t count = 0;
 };
-void read_back(fm_context ctx, const HostOut (&parts)[3]);
+void read_back(fm_context ctx, const Output (&parts)[3], bool may_stage = true);
 
 // fm_mapped.hip
 void mapping_coefficients(fm_model m, std::vector<double> &beta, int64_t &beta_size);

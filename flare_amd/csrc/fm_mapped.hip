@@ -177,18 +177,7 @@ static void mapped_layout(fm_structure s, size_t sz[kMappedBufs]) {
   for (int k = 0; k < kMappedBufs; k++) sz[k] = std::max<size_t>(sz[k], 1);
 }
 
-// Host memory that the runtime does not know.
-static bool pageable_host(const void *p) {
-  hipPointerAttribute_t a{};
-  hipError_t rc = hipPointerGetAttributes(&a, p);
-  if (rc != hipSuccess) (void)hipGetLastError();
-  return rc != hipSuccess || a.type == hipMemoryTypeUnregistered;
-}
-
-// pair_flare.cpp:68-184 on the given buffers; outputs (host or device
-// memory, any may be null) are copied on the context stream (with may_stage
-// through its pinned memory where all are pageable), then the stream is
-// synchronised.
+// pair_flare.cpp:68-184 on the given buffers; outputs as read_back.
 static void mapped_run(fm_mapped mp, fm_structure s, const MappedBufs &b, bool may_stage,
                        double *atom_energy, double *forces, double *virial) {
   hipStream_t st = s->ctx->stream;
@@ -236,19 +225,10 @@ static void mapped_run(fm_mapped mp, fm_structure s, const MappedBufs &b, bool m
                        s->d_struct_chunk_off.as<int>(), b.blk, b.vsum);
   }
   FM_HIP(hipGetLastError());
-  HostOut parts[3] = {{n > 0 ? atom_energy : nullptr, b.Ea, (size_t)n},
+  Output parts[3] = {{n > 0 ? atom_energy : nullptr, b.Ea, (size_t)n},
                       {n > 0 ? forces : nullptr, b.F, 3 * (size_t)n},
                       {virial, b.vsum, 6 * (size_t)s->n_struct}};
-  bool pageable = may_stage;
-  for (const HostOut &p : parts) pageable = pageable && (!p.dst || pageable_host(p.dst));
-  if (pageable) {
-    read_back(s->ctx, parts);
-    return;
-  }
-  for (const HostOut &p : parts)
-    if (p.dst)
-      FM_HIP(hipMemcpyAsync(p.dst, p.src, p.count * sizeof(double), hipMemcpyDefault, st));
-  FM_HIP(hipStreamSynchronize(st));
+  read_back(s->ctx, parts, may_stage);
 }
 
 void mapped_compute(fm_mapped mp, fm_structure s, double *atom_energy, double *forces,

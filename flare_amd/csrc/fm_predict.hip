@@ -257,12 +257,20 @@ __global__ __launch_bounds__(256) void k_stage_out(StageOut a, double *dst) {
   }
 }
 
-// Arrays to the caller's host memory; returns after the copies have finished.
-// Up to kStageOut bytes in all go through the context's pinned memory (a copy to
-// pageable memory waits for itself, 15 us each).
+// Memory that the runtime does not know: pageable host memory.
+static bool pageable_host(const void *p) {
+  hipPointerAttribute_t a{};
+  hipError_t rc = hipPointerGetAttributes(&a, p);
+  if (rc != hipSuccess) (void)hipGetLastError();
+  return rc != hipSuccess || a.type == hipMemoryTypeUnregistered;
+}
+
+// Up to kStageOut bytes in all go through the context's pinned memory if every
+// destination is pageable (a copy to pageable memory waits for itself, 15 us
+// each).
 constexpr size_t kStageOut = 256 << 10;
 
-void read_back(fm_context ctx, const HostOut (&parts)[3]) {
+void read_back(fm_context ctx, const Output (&parts)[3], bool may_stage) {
   hipStream_t st = ctx->stream;
   size_t total = 0;
   StageOut so{};
@@ -272,26 +280,30 @@ void read_back(fm_context ctx, const HostOut (&parts)[3]) {
       so.count[k] = parts[k].count;
       total += parts[k].count;
     }
-  char *stage = total * sizeof(double) <= kStageOut ? ctx->stage(total * sizeof(double)) : nullptr;
-  if (stage && total > 0) {
-    void *dev = nullptr;
-    FM_HIP(hipHostGetDevicePointer(&dev, stage, 0));
-    hipLaunchKernelGGL(k_stage_out, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, so,
-                       (double *)dev);
-    FM_HIP(hipGetLastError());
+  bool staged = may_stage && total > 0 && total * sizeof(double) <= kStageOut;
+  for (const Output &p : parts) staged = staged && (!p.dst || pageable_host(p.dst));
+  if (!staged) {
+    for (const Output &p : parts)
+      if (p.dst && p.count)
+        FM_HIP(hipMemcpyAsync(p.dst, p.src, p.count * sizeof(double), hipMemcpyDefault, st));
+    FM_HIP(hipStreamSynchronize(st));
+    return;
   }
-  for (const HostOut &p : parts)
-    if (p.dst && !stage)
-      FM_HIP(hipMemcpyAsync(p.dst, p.src, p.count * sizeof(double), hipMemcpyDeviceToHost, st));
+  char *stage = ctx->stage(total * sizeof(double));
+  void *dev = nullptr;
+  FM_HIP(hipHostGetDevicePointer(&dev, stage, 0));
+  hipLaunchKernelGGL(k_stage_out, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, so,
+                     (double *)dev);
+  FM_HIP(hipGetLastError());
   FM_HIP(hipStreamSynchronize(st));
-  for (const HostOut &p : parts) {
-    if (!p.dst || !stage) continue;
+  for (const Output &p : parts) {
+    if (!p.dst) continue;
     std::memcpy(p.dst, stage, p.count * sizeof(double));
     stage += p.count * sizeof(double);
   }
 }
 
-// Results to the caller's host buffers (any may be null).
+// Results to the caller's buffers (any may be null).
 static void read_outputs(fm_structure s, const double *o, size_t n_out, const double *var_row,
                          const double *E_row, double *mean_efs, double *local_var,
                          double *local_energy) {
@@ -299,7 +311,7 @@ static void read_outputs(fm_structure s, const double *o, size_t n_out, const do
   Pool *pool = &s->ctx->pool;
   size_t n = s->n;
   DevBuf vperm, eperm;
-  HostOut parts[3] = {{mean_efs, o, n_out}, {}, {}};
+  Output parts[3] = {{mean_efs, o, n_out}, {}, {}};
   if (local_var && var_row && n > 0) {
     // Species-sorted rows of the batch to each structure's species-sorted
     // order (compute_cluster_uncertainties order).

@@ -166,7 +166,8 @@ int fm_model_destroy(fm_model m);
 /* SparseGP::predict_mean / predict_local_uncertainties for one kernel
  * (sparse_gp.cpp:643-665, 731-757; kernel columns of
  * normalized_dot_product.cpp:117-214 contracted with alpha by the adjoint,
- * so dB/dr is never formed). Outputs, any may be NULL:
+ * so dB/dr is never formed). Outputs, in host or device memory, any may be
+ * NULL; the call returns when they are written:
  *   mean_efs     1 + 3N + 6: [E, F (atom-major xyz), S (xx,xy,xz,yy,yz,zz)]
  *                (for a batch, one such block per structure, concatenated)
  *   local_var    N, species-sorted order (compute_cluster_uncertainties),
@@ -238,7 +239,7 @@ int fm_mapped_destroy(fm_mapped mp);
  * FP64 B2 descriptors were computed with the potential's settings
  * (radial_r1 = 0): per-atom energies (atom order), forces N x 3, and for
  * each structure the virial sum_bonds -f (x) r (xx, xy, xz, yy, yz, zz).
- * Any output may be NULL. */
+ * Outputs may be host or device memory, any may be NULL. */
 int fm_mapped_compute(fm_mapped mp, fm_structure s, double *atom_energy,
                       double *forces, double *virial);
 /* fm_mapped_compute without any allocation: no reference counterpart; it is

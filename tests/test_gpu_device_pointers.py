@@ -90,3 +90,42 @@ def test_short_array(system, short):
         assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
     for p in ptrs:
         assert hip.hipFree(p) == 0
+
+
+@pytest.mark.parametrize("reps", [2, 15])
+@pytest.mark.parametrize("where", ["device", "pinned", "mixed"])
+def test_prediction_outputs(reps, where):
+    """Results in device and in pinned memory, small ones (which reach pageable
+    memory through a staging buffer) and large ones."""
+    import torch
+    from flare_amd import _C_flare as C
+    from flare_amd import _lib
+    from helpers import fcc
+    calc = C.B2("chebyshev", "quadratic", [0.0, RC], [], [1, 4, 2])
+    train = C.Structure(*fcc(4.0, (3, 3, 3), 0.1, 3), RC, [calc])
+    sgp = C.SparseGP([C.NormalizedDotProduct(1.5, 2.0)], 0.1, 0.1, 0.1)
+    sgp.add_specific_environments(train, [0, 9, 40])
+    sgp.update_L_inverse()
+    sgp.set_alpha(np.linspace(0.2, 0.5, sgp.n_sparse))
+    s = C.Structure(*fcc(4.0, (reps,) * 3, 0.1, 4), RC, [calc])
+    sizes = (1 + 3 * s.noa + 6, s.noa, s.noa)
+    model = sgp._model(0, s._ctx)
+
+    def predict(ptrs):
+        _lib.check(_lib.load().fm_predict(model.h, s._h, _lib.PREDICT_MEAN | _lib.PREDICT_LOCAL,
+                                          0, *ptrs))
+
+    want = [np.zeros(k) for k in sizes]
+    predict([_lib.ptr(w) for w in want])
+    assert (sum(sizes) * 8 > 256 << 10) == (reps == 15)
+    out = [torch.zeros(k, dtype=torch.float64) for k in sizes]
+    if where == "device":
+        out = [t.cuda() for t in out]
+    elif where == "pinned":
+        out = [t.pin_memory() for t in out]
+    else:
+        out[1] = out[1].cuda()
+    torch.cuda.synchronize()
+    predict([t.data_ptr() for t in out])
+    for t, w in zip(out, want):
+        assert np.array_equal(t.cpu().numpy(), w)
