@@ -145,7 +145,7 @@ struct fm_context_s {
   // Pinned host words that kernels write sizes and flags to directly (pinned_dev
   // is their device address), read after the stream synchronisation of the
   // call. Calls on one context are sequential (they share its stream).
-  static constexpr int kPinnedWords = 256;
+  static constexpr int kPinnedWords = 1024;
   int *pinned = nullptr, *pinned_dev = nullptr;
   // Pinned staging for a structure's small host arrays (one upload per
   // structure). Reused by the next structure: each build waits for its stream

@@ -930,13 +930,15 @@ __global__ __launch_bounds__(kScanBlock) void k_rows_bonds(int n, const int *spe
 
 // Pinned words of a bond build: the bond total, then atoms and bonds by species.
 constexpr int kWordBonds = 4, kWordTypes = 8;
+constexpr int kMaxSpecies = 255;
+static_assert(kWordTypes + 2 * kMaxSpecies <= fm_context_s::kPinnedWords, "pinned words");
 
 void build_bonds(fm_structure s) {
   fm_context ctx = s->ctx;
   hipStream_t st = ctx->stream;
   Pool *pool = &ctx->pool;
   int n = s->n, nos = s->nos, tpb = 256;
-  FM_CHECK(nos < 64, FM_ERR_INVALID, "too many species");
+  FM_CHECK(nos <= kMaxSpecies, FM_ERR_INVALID, "too many species");
   int *hw = ctx->pinned_dev;
   int *host_types = hw + kWordTypes, *host_bonds = hw + kWordTypes + nos;
   int nc = nos * nos;
