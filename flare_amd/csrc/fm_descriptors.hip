@@ -266,13 +266,14 @@ __device__ void accumulate_c(const B2Args &a, int i, int lane, int w, int ch, T 
     atom_sync<W>();
     // Wave w takes the tiles of 16 harmonics w, w + W, ..: g_n is read once for
     // all of them.
-    constexpr int HT = LC >= 0 ? ((LC + 1) * (LC + 1) + 15) / 16 : (kMaxH + 15) / 16;
+    constexpr int HT = LC >= 0 ? ((LC + 1) * (LC + 1) + 15) / 16 : -LC;
     constexpr int NT = (HT + W - 1) / W, n_step = sizeof(T) == 8 ? 4 : 1;
     int n0 = mfma_row<T>(lane, 0), lm0 = 16 * w + r16;
     int rc = min(r16, N - 1), r0 = 0;
     for (int t = 0; t < a.nos; t++) {
       int r1 = r0 + __popcll(__ballot(sj == t));  // rows [r0, r1) are species t
-      if (r1 > r0 || bb == b0) {  // the first chunk sets all of c
+      // The first chunk sets all of c; a wave past the last harmonic has no tile.
+      if ((r1 > r0 || bb == b0) && (W == 1 || 16 * w < H)) {
         typename MfmaAcc<T>::type acc[NT];
         // c of this lane's first value; the others are n_step H apart.
         int at = mul24(t * N + n0, H) + lm0;
@@ -1131,6 +1132,27 @@ static void with_lmax(int lmax, F &&f) {
   }
 }
 
+// The same for the descriptor kernel, whose instances for other l_max values are
+// by their tiles of 16 harmonics, L = -tiles: every tile of an instance is
+// multiplied, whatever l_max (l_max 8 and 9 have 6 and 7 of the 8). 4,000 atoms of
+// two species, 8 functions, FP64: l_max 2 18 us and 5 57 us (37 and 67 with one
+// instance of eight tiles, 22 and 66 with a loop over the tiles).
+template <typename F>
+static void with_tiles(int lmax, F &&f) {
+  switch (lmax) {
+    case 0:
+    case 1:
+    case 2: f(std::integral_constant<int, -1>{}); break;
+    case 5: f(std::integral_constant<int, -3>{}); break;
+    case 7: f(std::integral_constant<int, -4>{}); break;
+    case 8:
+    case 9:
+    case 10: f(std::integral_constant<int, -8>{}); break;
+    default: with_lmax(lmax, f); break;
+  }
+}
+static_assert(kMaxL == 10, "tiles of harmonics of the descriptor kernel");
+
 static B2Args make_args(fm_structure s) {
   B2Args a;
   a.n = s->n;
@@ -1188,15 +1210,19 @@ void launch_b2(fm_structure s, bool want_b2) {
   bool mixed = want_b2 && s->form != FM_FORM_FP64;
   size_t esz = s->form == FM_FORM_FP64 ? sizeof(double) : sizeof(float);
   size_t csz = s->form == FM_FORM_FP64 || mixed ? sizeof(double) : sizeof(float);
-  // 64-bond chunks fill all lanes of the bond basis and take half the passes;
-  // they cost LDS only where the row is shorter than their tables, and are
-  // used where four atoms still fit a CU (times with 64 and with 32 are within
-  // 5 %).
   // Waves per atom: the fewest that give the CU 12 waves (its registers hold
   // 16). One, two and four waves: 8.5, 7.7 and 6.5 ms (262144 atoms, three
   // species, l_max 6, four atoms per CU), 0.71, 0.70 and 0.57 ms (32000 atoms, two
   // species, four per CU), 2.31, 2.24 and 3.22 ms (512 structures, l_max 4,
   // seven per CU).
+  // 64-bond chunks fill all lanes of the bond basis and take half the passes;
+  // they cost LDS only where the row is shorter than their tables, and are
+  // used where four atoms still fit a CU. Where they leave fewer than twelve and
+  // chunks of 32 leave sixteen, one wave with the latter is faster than two with
+  // the former: 32,000 atoms in FP64, 132 and 156 us (two species of 8 functions,
+  // l_max 3, 20 and 10 atoms per CU), 140 and 168 (one species of 8, l_max 4, 16
+  // and 8); with fewer it is not: 192 and 181 (two species of 8, l_max 4, 14 and
+  // 8), 371 and 290 (one of 8, l_max 5, 12 and 6).
   int row = a.nd;
   auto work_of = [&](int ch) {
     return b2_work(a.nrad * a.H, a.H, a.N, ch, want_b2 ? row : 0);
@@ -1204,8 +1230,9 @@ void launch_b2(fm_structure s, bool want_b2) {
   bool stage = work_of(32) * csz <= (size_t)160 * 1024;
   if (!stage && a.nrad > 32) row = 0;
   size_t res = resident_atoms(work_of(64) * csz);
-  int chunk = res >= 4 ? 64 : 32;
-  if (chunk == 32) res = resident_atoms(work_of(32) * csz);
+  size_t res32 = resident_atoms(work_of(32) * csz);
+  int chunk = res >= 12 ? 64 : res32 >= 16 ? 32 : res >= 4 ? 64 : 32;
+  if (chunk == 32) res = res32;
   size_t work = work_of(chunk);
   size_t per = work * csz;
   int W = csz == 4 || !stage ? 1 : res >= 12 ? 1 : res >= 6 ? 2 : 4;
@@ -1238,7 +1265,7 @@ void launch_b2(fm_structure s, bool want_b2) {
   auto go = [&](auto waves) {
     constexpr int NW = decltype(waves)::value;
     dim3 grid(nblk), block(64 * NW * apb);
-    with_lmax(a.lmax, [&](auto lc) {
+    with_tiles(a.lmax, [&](auto lc) {
       constexpr int LC = decltype(lc)::value;
       if (mixed)
         hipLaunchKernelGGL((k_b2<double, LC, true, NW>), grid, block, lds, st, a,
@@ -1253,7 +1280,7 @@ void launch_b2(fm_structure s, bool want_b2) {
   {
     KScope timer(ctx, KT_DESC);
     if (csz == 4)
-      with_lmax(a.lmax <= 4 ? a.lmax : -1, [&](auto lc) {
+      with_tiles(a.lmax, [&](auto lc) {
         hipLaunchKernelGGL((k_b2<float, decltype(lc)::value, false, 1>), dim3(nblk),
                            dim3(64 * apb), lds, st, a, (float *)nullptr, s->norm.as<double>(),
                            s->nn.as<double>(), s->C.as<float>(), 0, (int)work, chunk, 1, mo);

@@ -54,3 +54,12 @@ def test_projection_rows(oracle, settings):
     """The adjoint's rows in one pass: 3255 values (single elements), 855 and 15
     (unaligned vectors), 2790 and 2030 (odd counts of vectors)."""
     test_descriptor_rows(oracle, settings, 37, 4.5)
+
+
+# One (l_max 2), three (5), four (7) and eight tiles of harmonics (8 to 10) on
+# one, two and four waves; one wave with chunks of 32 bonds.
+@pytest.mark.parametrize("settings", [(1, 5, 2), (1, 1, 5), (1, 4, 5), (2, 9, 5), (2, 6, 7), (1, 3, 8),
+                                      (1, 4, 9), (2, 5, 10), (2, 8, 3), (1, 8, 4)])
+@pytest.mark.parametrize("n,rc", [(1, 4.0), (50, 6.5)])
+def test_tiles_of_harmonics(oracle, settings, n, rc):
+    test_descriptor_rows(oracle, settings, n, rc)
