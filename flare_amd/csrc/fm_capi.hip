@@ -378,7 +378,6 @@ static int structure_create(fm_context ctx, int n_struct, const double *cells,
           ce.push_back(std::min(a + 256, s->atom_off[k + 1]));
         }
         sco[k + 1] = (int)cb.size();
-        s->max_chunks = std::max(s->max_chunks, sco[k + 1] - sco[k]);
       }
       s->n_chunks = (int)cb.size();
       std::vector<long long> mo(s->mean_off.begin(), s->mean_off.end());

@@ -47,34 +47,25 @@ __global__ __launch_bounds__(256) void k_forces(int n, const int *atom_struct, c
   }
 }
 
-// Sums over a chunk of <= 256 atoms [i0, i1) of one structure by 256 threads
-// (t: the thread among them): its atoms' energies (first, when NQ is 7) and six
-// virial components, wave sums to sh.
-template <int NQ>
-__device__ __forceinline__ void chunk_sums(int i0, int i1, int t, const int *row_of_atom,
-                                           const double *E_row, const double *vir,
-                                           double (*sh)[NQ]) {
-  double v[NQ];
-  int i = i0 + t;
-  bool in = i < i1;
-  if (NQ == 7) v[0] = in ? E_row[row_of_atom[i]] : 0.0;
-#pragma unroll
-  for (int q = 0; q < 6; q++) v[NQ - 6 + q] = in ? vir[6 * (size_t)i + q] : 0.0;
-#pragma unroll
-  for (int q = 0; q < NQ; q++) v[q] = wave_sum(v[q]);
-  if ((t & 63) == 0)
-#pragma unroll
-    for (int q = 0; q < NQ; q++) sh[t >> 6][q] = v[q];
-}
-
-// The sums of every chunk, NQ values each.
+// Sums of every chunk of <= 256 atoms of one structure: its atoms' energies
+// (first, when NQ is 7) and six virial components.
 template <int NQ>
 __global__ __launch_bounds__(256) void k_chunk_sums(const int *chunk_begin, const int *chunk_end,
                                                     const int *row_of_atom, const double *E_row,
                                                     const double *vir, double *part) {
   __shared__ double sh[4][NQ];
   int c = blockIdx.x;
-  chunk_sums<NQ>(chunk_begin[c], chunk_end[c], threadIdx.x, row_of_atom, E_row, vir, sh);
+  int i = chunk_begin[c] + threadIdx.x;
+  bool in = i < chunk_end[c];
+  double v[NQ];
+  if (NQ == 7) v[0] = in ? E_row[row_of_atom[i]] : 0.0;
+#pragma unroll
+  for (int q = 0; q < 6; q++) v[NQ - 6 + q] = in ? vir[6 * (size_t)i + q] : 0.0;
+#pragma unroll
+  for (int q = 0; q < NQ; q++) v[q] = wave_sum(v[q]);
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int q = 0; q < NQ; q++) sh[threadIdx.x >> 6][q] = v[q];
   __syncthreads();
   if (threadIdx.x < NQ) {
     int q = threadIdx.x;
@@ -82,35 +73,13 @@ __global__ __launch_bounds__(256) void k_chunk_sums(const int *chunk_begin, cons
   }
 }
 
-// Chunks that one workgroup of 1,024 takes by itself, four at a time, to save the
-// launch of k_chunk_sums: structures of up to 2,048 atoms (9 us for 108 atoms,
-// the two launches 8 and the gap between them). The order of the sums is the same.
-constexpr int kDirectChunks = 8;
-template <int NQ>
-__device__ __forceinline__ void direct_sums(const int *struct_chunk_off, const int *chunk_begin,
-                                            const int *chunk_end, const int *row_of_atom,
-                                            const double *E_row, const double *vir, int k,
-                                            double (&acc)[NQ]) {
-  __shared__ double sh[4][4][NQ], part[kDirectChunks][NQ];
-  int c0 = struct_chunk_off[k], nc = struct_chunk_off[k + 1] - c0, g = threadIdx.x >> 8;
-  for (int u = 0; u < nc; u += 4) {
-    int c = c0 + u + g;
-    bool in = u + g < nc;
-    chunk_sums<NQ>(in ? chunk_begin[c] : 0, in ? chunk_end[c] : 0, threadIdx.x & 255, row_of_atom,
-                   E_row, vir, sh[g]);
-    __syncthreads();
-    int q = threadIdx.x & 255;
-    if (in && q < NQ) part[u + g][q] = (sh[g][0][q] + sh[g][1][q]) + (sh[g][2][q] + sh[g][3][q]);
-    __syncthreads();
-  }
-  int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int q = 0; q < NQ; q++) acc[q] = wave_sum(lane < nc ? 0 + part[lane][q] : 0.0);
-}
-
 // Sum of one structure's chunk values, by one wave: lanes take chunks 64
 // apart, then sum over the lanes (one thread over all 1,024 chunks of a
-// 262,144-atom structure took 164 us, now 8).
+// 262,144-atom structure took 164 us, now 8). With the chunks in a launch before
+// at every size: one workgroup that went through a structure's chunks itself was
+// slower for one structure (gather and sums of 108 atoms 15 us, in three launches
+// 11; of 2,048 atoms 21 and 12) and more so for many (2,000 of 40 atoms 78 and
+// 32).
 template <int NQ>
 __device__ __forceinline__ void structure_sums(const int *struct_chunk_off, const double *part,
                                                int k, double (&acc)[NQ]) {

@@ -219,7 +219,7 @@ struct fm_structure_s {
   // Output offsets of each structure in mean_efs (1 + 3 N_k + 6 per structure)
   // and the reduction chunks (<= 256 atoms, never crossing a structure).
   std::vector<int64_t> mean_off;
-  int n_chunks = 0, max_chunks = 0;  // of all structures, of the largest
+  int n_chunks = 0;
   fm::DevBuf d_chunk_begin, d_chunk_end, d_struct_chunk_off;
   // Position of each species-sorted row in the per-structure species-sorted
   // order of the local variances (device ints; empty for a single

@@ -108,33 +108,17 @@ static void for_final_types(fm_structure s, Part &&part, Launch &&launch) {
 
 // Per structure (one wave each): energy and stress -1/V sum_b f (x) r
 // (normalized_dot_product.cpp:201-206).
-__device__ __forceinline__ void write_sums(const double (&acc)[7], int k, const double *vol_inv,
-                                           const long long *mean_off, const int *atom_off,
-                                           double *out) {
+__global__ __launch_bounds__(64) void k_final_sum(const int *struct_chunk_off, const double *part,
+                                                  const double *vol_inv, const long long *mean_off,
+                                                  const int *atom_off, double *out) {
+  int k = blockIdx.x;
+  double acc[7];
+  structure_sums<7>(struct_chunk_off, part, k, acc);
   if (threadIdx.x != 0) return;
   double *o = out + mean_off[k];
   int nk = atom_off[k + 1] - atom_off[k];
   o[0] = acc[0];
   for (int q = 0; q < 6; q++) o[1 + 3 * nk + q] = acc[1 + q] * vol_inv[k];
-}
-__global__ __launch_bounds__(64) void k_final_sum(const int *struct_chunk_off, const double *part,
-                                                  const double *vol_inv, const long long *mean_off,
-                                                  const int *atom_off, double *out) {
-  double acc[7];
-  structure_sums<7>(struct_chunk_off, part, blockIdx.x, acc);
-  write_sums(acc, blockIdx.x, vol_inv, mean_off, atom_off, out);
-}
-// The same from the atoms, for structures of up to kDirectChunks chunks.
-__global__ __launch_bounds__(1024) void k_direct_sum(const int *struct_chunk_off,
-                                                     const int *chunk_begin, const int *chunk_end,
-                                                     const int *row_of_atom, const double *E_row,
-                                                     const double *vir, const double *vol_inv,
-                                                     const long long *mean_off,
-                                                     const int *atom_off, double *out) {
-  double acc[7];
-  direct_sums<7>(struct_chunk_off, chunk_begin, chunk_end, row_of_atom, E_row, vir, blockIdx.x,
-                 acc);
-  write_sums(acc, blockIdx.x, vol_inv, mean_off, atom_off, out);
 }
 
 __global__ void k_fill(double *p, long long n, double v) {
@@ -159,14 +143,6 @@ static void gather_forces(fm_structure s, bool f64, DevBuf &fbond, DevBuf &vir, 
   };
   if (f64) forces(fbond.as<double>());
   else forces(fbond.as<float>());
-  if (s->max_chunks <= kDirectChunks) {
-    hipLaunchKernelGGL(k_direct_sum, dim3(s->n_struct), dim3(1024), 0, st,
-                       s->d_struct_chunk_off.as<int>(), s->d_chunk_begin.as<int>(),
-                       s->d_chunk_end.as<int>(), s->row_of_atom.as<int>(), E_row.as<double>(),
-                       vir.as<double>(), s->d_vol_inv.as<double>(),
-                       s->d_mean_off.as<long long>(), s->d_atom_off.as<int>(), o);
-    return;
-  }
   DevBuf blk(pool, (size_t)s->n_chunks * 7 * sizeof(double));
   hipLaunchKernelGGL(k_chunk_sums<7>, dim3(s->n_chunks), dim3(256), 0, st,
                      s->d_chunk_begin.as<int>(), s->d_chunk_end.as<int>(),
