@@ -84,14 +84,19 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_block_sums(const int *in, i
   if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
 }
 
-// Every block sums the totals of the blocks before it, then scans its own.
+// Every block takes the sum of the blocks before it (bsum holds these sums if
+// `scanned`, else the blocks' totals, which it sums), then scans its own values.
 __global__ __launch_bounds__(kScanBlock) void k_scan_apply(const int *in, int n, const int *bsum,
-                                                           int *out, int *host,
+                                                           int scanned, int *out, int *host,
                                                            const int *extra) {
   __shared__ int sh[16];
   int before = 0, base, tot;
-  for (int b = threadIdx.x; b < blockIdx.x; b += kScanBlock) before += bsum[b];
-  block_excl_scan(before, sh, base);  // base: the sum over all threads
+  if (scanned) {
+    base = bsum[blockIdx.x];
+  } else {
+    for (int b = threadIdx.x; b < blockIdx.x; b += kScanBlock) before += bsum[b];
+    block_excl_scan(before, sh, base);  // base: the sum over all threads
+  }
   int i = blockIdx.x * kScanBlock + threadIdx.x;
   int v = i < n ? in[i] : 0;
   int e = block_excl_scan(v, sh, tot);
@@ -103,9 +108,14 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_apply(const int *in, int n,
   }
 }
 
-// One launch up to 8,192 values (a block of 1,024 threads, 4 us), else two (the
-// launch that scanned the block totals in between is gone: every block of the
-// second sums those before it, at most a few loads per thread).
+// One launch up to 8,192 values (a block of 1,024 threads, 4 us). Then two, in
+// which every block of the second sums the totals before it, a load per thread
+// and 1,024 blocks. That grows with the square of the blocks, so from kScanSums
+// blocks on the totals are scanned first, for two more launches. A structure of
+// 3,000 atoms in an ever larger cell, without and with them: 65 and 67 us (a
+// million bins), 88 and 89 (4), 193 and 156 (16), 925 and 472 (64), 28 and 3.6 ms
+// (512).
+constexpr int kScanSums = 4096;
 void scan_exclusive(fm_context ctx, const int *in, int *out, int n, int *host,
                     const int *extra) {
   hipStream_t st = ctx->stream;
@@ -113,12 +123,17 @@ void scan_exclusive(fm_context ctx, const int *in, int *out, int n, int *host,
     hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(kScanBlock), 0, st, in, n, out, host,
                        extra);
   } else {
-    int nb = (n + kScanBlock - 1) / kScanBlock;
-    DevBuf bsum(&ctx->pool, nb * sizeof(int));
+    int nb = (n - 1) / kScanBlock + 1;
+    DevBuf bsum(&ctx->pool, nb * sizeof(int)), boff;
     hipLaunchKernelGGL(k_scan_block_sums, dim3(nb), dim3(kScanBlock), 0, st, in, n,
                        bsum.as<int>());
-    hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(kScanBlock), 0, st, in, n, bsum.as<int>(),
-                       out, host, extra);
+    bool scanned = nb >= kScanSums;
+    if (scanned) {
+      boff.alloc(&ctx->pool, ((size_t)nb + 1) * sizeof(int));
+      scan_exclusive(ctx, bsum.as<int>(), boff.as<int>(), nb);
+    }
+    hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(kScanBlock), 0, st, in, n,
+                       scanned ? boff.as<int>() : bsum.as<int>(), (int)scanned, out, host, extra);
   }
   FM_HIP(hipGetLastError());
 }

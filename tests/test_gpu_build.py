@@ -42,3 +42,22 @@ def test_lists_and_rows(oracle, n, nos):
 def test_lists_and_rows_small(oracle, n):
     """At the edges of the builds in one workgroup (2,048 atoms; 8,192)."""
     test_lists_and_rows(oracle, n, 3)
+
+
+@pytest.mark.parametrize("side", [161, 162, 211])
+def test_lists_in_a_large_cell(oracle, side):
+    """Pairs of atoms in cells of 4.17, 4.25 and 9.4 million bins: from 4,096 blocks
+    of 1,024 on the scan of the bins scans the blocks' totals first."""
+    from flare_amd import _C_flare as C
+    rng = np.random.default_rng(side)
+    cell = np.eye(3) * (side * (1 + 1e-6))
+    one = rng.uniform(0, side, (150, 3))
+    one[0], one[1] = 0.1, side - 0.05  # the first and the last bin
+    pos = np.concatenate([one, one + rng.uniform(-0.6, 0.6, one.shape)])
+    species = np.zeros(len(pos), np.int32)
+    s = C.Structure(cell, species, pos, 0.999, [])
+    ref = oracle.Neighbors(cell, species, pos, 0.999, "literal")
+    assert s.n_neighbors == ref.n_neighbors > 100
+    assert np.array_equal(s.neighbor_count, ref.neighbor_count)
+    assert np.array_equal(s.structure_indices, ref.structure_indices)
+    assert np.array_equal(s.relative_positions, ref.relative_positions)
