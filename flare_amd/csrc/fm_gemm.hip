@@ -12,7 +12,7 @@
 //             variance term |L_inv k|^2 (sparse_gp.cpp:121-131); A is lower
 //             triangular so each row tile stops at its last nonzero column.
 //
-// FP64 form: k_gemm_f64 for all three. Chosen form: EP_KERNEL is exact on
+// FP64 form: k_gemm_f64, k_gemm_f64_dma or k_gemm_f64_lds for all three. Chosen form: EP_KERNEL is exact on
 // int8 MFMA (v_mfma_i32_16x16x64_i8) over five power-of-two-scaled slices of
 // each operand row, int32 accumulation per slice-pair diagonal and an FP64
 // epilogue (k_gemm_i8); EP_STORE is split-BF16 x3 on
@@ -1266,8 +1266,10 @@ int gemm_row_tiles(int M) { return (M + 63) / 64 * 2; }
 
 namespace {
 
-// FLARE_MI_TILE_SHAPE=i pins shape i of each contraction's table (tests check
-// that every shape gives the same results); -1 without it or past the table.
+// FLARE_MI_TILE_SHAPE=i pins shape i of every contraction that has as many (tests
+// check that every shape gives the same results); -1 without it or past the last.
+// Largest first: wave tiles of 64, 48, 32 and 16 (FP64; 48 for EP_STORE only),
+// tiles of 128 and 64 columns (int8), of 256 and 128 (split BF16).
 int pinned_shape(int n_shapes) {
   const char *f = std::getenv("FLARE_MI_TILE_SHAPE");
   int i = f ? std::atoi(f) : -1;
@@ -1342,7 +1344,9 @@ void gemm_i8_groups(hipStream_t st, const std::vector<I8Gemm> &all) {
       FM_CHECK(b2 < (1LL << 31), FM_ERR_CAPACITY, "contraction too large for one launch");
     }
     bool is_long = nk * kI8Pad > kI8Flush;
-    int RA = !is_long && 7 * ((b4 + 255) / 256) <= 4 * ((b2 + 255) / 256) ? 4 : 2;
+    int pin = pinned_shape(2);
+    bool wide = pin < 0 ? 7 * ((b4 + 255) / 256) <= 4 * ((b2 + 255) / 256) : pin == 0;
+    int RA = wide && !is_long ? 4 : 2;
     for (int k = 0, first = 0; k < gs.n; k++) {
       gs.first[k] = first;
       first += (gs.g[k].M + kI8TileA - 1) / kI8TileA * ((gs.g[k].N + 32 * RA - 1) / (32 * RA));
@@ -1469,7 +1473,8 @@ void gemm_split_groups(hipStream_t st, const std::vector<SplitGemm> &all) {
       large += tiles(k, 256, 256);
       FM_CHECK(small < (1LL << 31), FM_ERR_CAPACITY, "contraction too large for one launch");
     }
-    bool big = 25 * ((large + 255) / 256) <= 13 * ((small + 511) / 512);
+    int pin = pinned_shape(2);
+    bool big = pin < 0 ? 25 * ((large + 255) / 256) <= 13 * ((small + 511) / 512) : pin == 0;
     int t = big ? 256 : 128;
     for (int k = 0, first = 0; k < gs.n; k++) {
       gs.first[k] = first;

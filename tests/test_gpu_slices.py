@@ -52,3 +52,37 @@ def test_integer_contraction(settings, reps, n_sparse):
     assert abs(m[0] - m64[0]) < 1e-7 * abs(m64[0])
     assert np.max(np.abs(m[1:-6] - m64[1:-6])) < 1e-3 * np.max(np.abs(m64[1:-6]))
     assert np.max(np.abs(v - v64)) < 1e-5 * SIGMA ** 2
+
+
+# 8112 and 8788 atoms: the library takes the 128-column tiles of the integer
+# contraction (144 functions, 320 environments) or the 256-wide ones of the
+# gradient contraction (1088 functions); 176 atoms: the smaller ones of both.
+@pytest.mark.parametrize("settings,reps,n_sparse", [
+    ((1, 8, 3), (13, 13, 13), (320,)),
+    ((1, 16, 7), (13, 13, 12), (70,)),
+    ((2, 6, 3), (4, 11, 1), (64, 65)),
+])
+def test_tile_sizes_bitwise(settings, reps, n_sparse, monkeypatch):
+    """Both tile sizes of either contraction give the results of the one that
+    the library picks, bit for bit."""
+    from flare_amd import _C_flare as C
+    nos = settings[0]
+    calc = C.B2("chebyshev", "quadratic", [0.0, 4.2], [], list(settings), np.full((nos, nos), 4.2))
+    system = fcc(4.0, reps, 0.1, 11, nos=nos)
+    train = C.Structure(*system, 4.2, [calc])
+    d = train.descriptors[0]
+    sgp = C.SparseGP([C.NormalizedDotProduct(SIGMA, 2.0)], 0.01, 0.05, 0.005)
+    sgp.Kuu_jitter = 1e-4
+    sgp.add_specific_environments(train, [int(a) for t, m in enumerate(n_sparse)
+                                          for a in d.atom_indices[t][:m]])
+    sgp.update_L_inverse()
+    sgp.set_alpha(np.random.default_rng(5).uniform(0.1, 1.0, size=sgp.n_sparse))
+    out = []
+    for shape in (None, "0", "1"):
+        if shape:
+            monkeypatch.setenv("FLARE_MI_TILE_SHAPE", shape)
+        s = C.Structure(*system, 4.2, [calc], form=C.FORM_CHOSEN)
+        sgp.predict_local_uncertainties(s)
+        out.append((s.mean_efs, s.local_uncertainties[0]))
+    for mean, var in out[1:]:
+        assert np.array_equal(mean, out[0][0]) and np.array_equal(var, out[0][1])
