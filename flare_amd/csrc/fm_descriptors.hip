@@ -1210,19 +1210,22 @@ void launch_b2(fm_structure s, bool want_b2) {
   bool mixed = want_b2 && s->form != FM_FORM_FP64;
   size_t esz = s->form == FM_FORM_FP64 ? sizeof(double) : sizeof(float);
   size_t csz = s->form == FM_FORM_FP64 || mixed ? sizeof(double) : sizeof(float);
-  // Waves per atom: the fewest that give the CU 12 waves (its registers hold
-  // 16). One, two and four waves: 8.5, 7.7 and 6.5 ms (262144 atoms, three
-  // species, l_max 6, four atoms per CU), 0.71, 0.70 and 0.57 ms (32000 atoms, two
-  // species, four per CU), 2.31, 2.24 and 3.22 ms (512 structures, l_max 4,
-  // seven per CU).
   // 64-bond chunks fill all lanes of the bond basis and take half the passes;
   // they cost LDS only where the row is shorter than their tables, and are
-  // used where four atoms still fit a CU. Where they leave fewer than twelve and
-  // chunks of 32 leave sixteen, one wave with the latter is faster than two with
-  // the former: 32,000 atoms in FP64, 132 and 156 us (two species of 8 functions,
-  // l_max 3, 20 and 10 atoms per CU), 140 and 168 (one species of 8, l_max 4, 16
-  // and 8); with fewer it is not: 192 and 181 (two species of 8, l_max 4, 14 and
-  // 8), 371 and 290 (one of 8, l_max 5, 12 and 6).
+  // used where four atoms still fit a CU. The size of a chunk is part of the order
+  // of the sums, so it must not depend on the number of atoms (a batch equals its
+  // structures); waves per atom may. In FP64, one wave with chunks of 32 is faster
+  // than this on many atoms of a short row and slower on few (8 functions of one
+  // species, l_max 4: 32,000 atoms 140 us, here 161; 108 atoms 14.7, here 12.2).
+  // Waves per atom: one where it leaves the CU eight atoms, two where six, else
+  // four (a CU's registers hold 16 waves). One, two and four waves: 8.5, 7.7 and
+  // 6.5 ms (262144 atoms, three species, l_max 6, four atoms per CU), 0.71, 0.70 and
+  // 0.57 ms (32000 atoms, two species, four per CU), 2.31, 2.24 and 3.22 ms (512
+  // structures, l_max 4, seven per CU). 32,000 atoms in FP64, one and two waves:
+  // 138 and 156 us (two species of 8 functions, l_max 3, ten per CU), 178 and 182
+  // (the same, l_max 4, eight), 194 and 192 (one of 12, l_max 4, seven), 340 and
+  // 291 (one of 8, l_max 5, six); 1,372 atoms of the first 14.1 and 15.6, 256 10.8
+  // and 11.0.
   int row = a.nd;
   auto work_of = [&](int ch) {
     return b2_work(a.nrad * a.H, a.H, a.N, ch, want_b2 ? row : 0);
@@ -1230,12 +1233,11 @@ void launch_b2(fm_structure s, bool want_b2) {
   bool stage = work_of(32) * csz <= (size_t)160 * 1024;
   if (!stage && a.nrad > 32) row = 0;
   size_t res = resident_atoms(work_of(64) * csz);
-  size_t res32 = resident_atoms(work_of(32) * csz);
-  int chunk = res >= 12 ? 64 : res32 >= 16 ? 32 : res >= 4 ? 64 : 32;
-  if (chunk == 32) res = res32;
+  int chunk = res >= 4 ? 64 : 32;
+  if (chunk == 32) res = resident_atoms(work_of(32) * csz);
   size_t work = work_of(chunk);
   size_t per = work * csz;
-  int W = csz == 4 || !stage ? 1 : res >= 12 ? 1 : res >= 6 ? 2 : 4;
+  int W = csz == 4 || !stage ? 1 : res >= 8 ? 1 : res >= 6 ? 2 : 4;
   int apb = W > 1 ? 1 : atoms_per_block(per);
   FM_CHECK(per <= (size_t)160 * 1024, FM_ERR_CAPACITY,
            "per-atom descriptor workspace exceeds LDS");

@@ -57,7 +57,7 @@ def test_projection_rows(oracle, settings):
 
 
 # One (l_max 2), three (5), four (7) and eight tiles of harmonics (8 to 10) on
-# one, two and four waves; one wave with chunks of 32 bonds.
+# one, two and four waves; one wave with eight and ten atoms on a CU.
 @pytest.mark.parametrize("settings", [(1, 5, 2), (1, 1, 5), (1, 4, 5), (2, 9, 5), (2, 6, 7), (1, 3, 8),
                                       (1, 4, 9), (2, 5, 10), (2, 8, 3), (1, 8, 4)])
 @pytest.mark.parametrize("n,rc", [(1, 4.0), (50, 6.5)])
