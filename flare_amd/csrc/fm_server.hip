@@ -67,15 +67,17 @@ struct fm_server_s {
   bool stop = false;
   std::vector<std::thread> workers;
 
-  // Device bytes of a batch: neighbour list, bond list and bond forces per
+  // Device bytes of a batch: neighbour list, bond lists and bond forces per
   // neighbour; descriptors, gradient rows, density coefficients and their
-  // adjoint, int8 slices, w and k per atom, for every kernel.
+  // adjoint, int8 slices, w, k and the partial sums per atom, for every kernel
+  // (as footprint_bytes of serving.py).
   int64_t bytes(int64_t n_atoms, int64_t n_neighbors) const {
-    int64_t esz = form == FM_FORM_FP64 ? 8 : 4, total = 0;
+    bool f64 = form == FM_FORM_FP64;
+    int64_t esz = f64 ? 8 : 4, total = 0;
     for (const Kernel &k : kernels)
       total += n_neighbors * (56 + 3 * esz) +
-               n_atoms * (2 * esz * k.nd + 2 * esz * k.nrad_h + 5 * k.nd + 12 * k.max_sparse +
-                          256);
+               n_atoms * (2 * esz * k.nd + 2 * esz * k.nrad_h + 5 * k.nd +
+                          (f64 ? 17 : 13) * k.max_sparse + 256);
     return total;
   }
 

@@ -24,14 +24,17 @@ from .batch import Batch
 
 
 def footprint_bytes(n_atoms, n_neighbors, n_descriptors, n_rad_h, max_sparse, esz=4):
-    """Device bytes a batch needs: neighbour list (40 B per entry), bond list
-    and bond forces, and per atom the descriptors and the gradient rows, the
-    density coefficients and their adjoint, the int8 slices of the
-    descriptors, w (BF16 pairs) and k (FP64) against the largest species
-    block of the sparse set, and small per-atom partials."""
-    per_nb = 40 + 8 + 3 * esz + 8
+    """Device bytes a batch needs: neighbour list (40 B per entry), bond lists
+    (as long as the neighbour list) and bond forces, and per atom the
+    descriptors and the gradient rows, the density coefficients and their
+    adjoint, the int8 slices of the descriptors (in FP64, which has none, slack
+    for the pool's size classes), w (BF16 pairs or FP64) and k (FP64) against the
+    largest species block of the sparse set, the partial sums of energy and
+    variance (a value per 16 environments and per 32 in FP64, per 64 and per 32
+    in the chosen form), and small per-atom values."""
+    per_nb = 40 + 16 + 3 * esz
     per_atom = (2 * esz * n_descriptors + 2 * esz * n_rad_h + 5 * n_descriptors
-                + (4 + 8) * max_sparse + 256)
+                + (17 if esz == 8 else 13) * max_sparse + 256)
     return int(n_neighbors * per_nb + n_atoms * per_atom)
 
 
