@@ -317,6 +317,9 @@ static bool readable_in_place(fm_context ctx, const void *p, size_t bytes, size_
 
 // Host species and positions up to this many bytes join the pinned upload.
 constexpr size_t kStageAtoms = 256 << 10;
+// All of a structure's host arrays (some 450 bytes per structure of a batch) up to
+// this many bytes go through the context's pinned buffer, which it keeps.
+constexpr size_t kStageMeta = 4 << 20;
 
 static int structure_create(fm_context ctx, int n_struct, const double *cells,
                             const int32_t *n_atoms, const int32_t *species,
@@ -338,6 +341,7 @@ static int structure_create(fm_context ctx, int n_struct, const double *cells,
     s->ctx = ctx;
     s->n = n;
     s->n_struct = n_struct;
+    std::vector<char> unstaged;  // outlives the wait for its upload
     try {
       fm::Pool *pool = &ctx->pool;
       hipStream_t st = ctx->stream;
@@ -409,7 +413,13 @@ static int structure_create(fm_context ctx, int n_struct, const double *cells,
       }
       size_t total = 0;
       for (const Part &p : parts) total += (p.bytes + 15) / 16 * 16;
-      char *stage = ctx->stage(total);
+      char *stage;
+      if (total <= kStageMeta) {
+        stage = ctx->stage(total);
+      } else {
+        unstaged.resize(total);
+        stage = unstaged.data();
+      }
       s->meta.alloc(pool, std::max<size_t>(1, total));
       size_t at = 0;
       for (const Part &p : parts) {

@@ -147,9 +147,9 @@ struct fm_context_s {
   // call. Calls on one context are sequential (they share its stream).
   static constexpr int kPinnedWords = 1024;
   int *pinned = nullptr, *pinned_dev = nullptr;
-  // Pinned staging for a structure's small host arrays (one upload per
-  // structure). Reused by the next structure: each build waits for its stream
-  // after the upload.
+  // Pinned staging, a few MB at most, for a structure's small host arrays (one
+  // upload per structure) and for small results. Reused by the next call: each
+  // waits for its stream after the copy.
   char *staging = nullptr;
   size_t staging_bytes = 0;
   char *stage(size_t bytes);

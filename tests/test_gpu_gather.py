@@ -56,3 +56,14 @@ def test_sums_of_large_and_small(model):
         alone = C.Structure(*st, 4.2, [calc])
         sgp.predict_mean(alone)
         assert np.array_equal(alone.mean_efs, mean)
+
+
+def test_batch_of_very_many(model):
+    """12,000 structures, whose cells and offsets exceed the staging buffer."""
+    from flare_amd.batch import Batch
+    C, calc, cut, sgp = model
+    structs = [structure(n) for n in (1, 2, 15, 3)]
+    few, _ = Batch(structs, 4.2, calc).predict(sgp)
+    many, _ = Batch(structs * 3000, 4.2, calc).predict(sgp)
+    for k, mean in enumerate(many):
+        assert np.array_equal(mean, few[k % 4]), k
