@@ -973,7 +973,7 @@ __device__ __forceinline__ void load4_lds(const double *p, double (&o)[4]) {
 // radial functions, l_max 6, 42 bonds), and 204 us, now 143 (FP64, 64
 // structures, 8 functions, l_max 4). fma is written out where the product that
 // the compiler chooses to fuse depends on NG.
-template <typename T, int LC, int NG>
+template <typename T, int NG>
 __global__ __launch_bounds__(64 * kAtomsPerBlock) void k_bond_forces(B2Args a,
                                                                        const double *norm,
                                                                        const double *nnv,
@@ -1056,7 +1056,7 @@ __global__ __launch_bounds__(64 * kAtomsPerBlock) void k_bond_forces(B2Args a,
       T ux = x * rinv, uy = y * rinv, uz = z * rinv;
       const T *ub = u + (size_t)sj * H * Np;
       T acc_a = 0, Px = 0, Py = 0, Pz = 0;
-      ylm_sweep<T, true, LC>(L, ux, uy, uz, [&](int lm, T Y, T px, T py, T pz) {
+      ylm_sweep<T, true>(L, ux, uy, uz, [&](int lm, T Y, T px, T py, T pz) {
         T s0 = 0, s1 = 0, uu[NG][4];
         const T *ul = ub + lm * Np;
 #pragma unroll
@@ -1261,9 +1261,13 @@ void launch_b2(fm_structure s, bool want_b2) {
   }
   s->has_q = mixed;
   if (nblk == 0) return;
-  // The unrolled sweep (compile-time l_max) is faster for the FP64 kernel;
-  // for FP32 its extra registers cost more occupancy than it saves at
-  // l_max 6.
+  // FP32: the bond pass of B3 only, l_max <= 4.
+  FM_CHECK(csz == 8 || a.lmax <= 4, FM_ERR_INVALID, "l_max above 4 of the FP32 bond pass");
+  auto bond_pass = [&](auto &&f) {
+    if (a.lmax == 3) f(std::integral_constant<int, 3>{});
+    else if (a.lmax == 4) f(std::integral_constant<int, 4>{});
+    else f(std::integral_constant<int, -1>{});
+  };
   auto go = [&](auto waves) {
     constexpr int NW = decltype(waves)::value;
     dim3 grid(nblk), block(64 * NW * apb);
@@ -1282,7 +1286,7 @@ void launch_b2(fm_structure s, bool want_b2) {
   {
     KScope timer(ctx, KT_DESC);
     if (csz == 4)
-      with_tiles(a.lmax, [&](auto lc) {
+      bond_pass([&](auto lc) {
         hipLaunchKernelGGL((k_b2<float, decltype(lc)::value, false, 1>), dim3(nblk),
                            dim3(64 * apb), lds, st, a, (float *)nullptr, s->norm.as<double>(),
                            s->nn.as<double>(), s->C.as<float>(), 0, (int)work, chunk, 1, mo);
@@ -1367,27 +1371,24 @@ void launch_bond_forces(fm_structure s, const void *U, void *fbond, double *viri
   int apb2 = atoms_per_block(per2);
   int nblk2 = (n_list + apb2 - 1) / apb2;
   KScope timer(s->ctx, KT_BOND);
-  auto launch = [&](auto lc, auto ng) {
-    constexpr int LC = decltype(lc)::value, NG = decltype(ng)::value;
+  auto launch = [&](auto ng) {
+    constexpr int NG = decltype(ng)::value;
     if (f64)
-      hipLaunchKernelGGL((k_bond_forces<double, LC, NG>), dim3(nblk2), dim3(64 * apb2),
+      hipLaunchKernelGGL((k_bond_forces<double, NG>), dim3(nblk2), dim3(64 * apb2),
                          apb2 * per2, st, a, s->norm.as<double>(), s->nn.as<double>(), aa,
                          (const double *)U, (double *)fbond, virial_atom, atom_list, n_list);
     else
-      hipLaunchKernelGGL((k_bond_forces<float, LC, NG>), dim3(nblk2), dim3(64 * apb2),
+      hipLaunchKernelGGL((k_bond_forces<float, NG>), dim3(nblk2), dim3(64 * apb2),
                          apb2 * per2, st, a, s->norm.as<double>(), s->nn.as<double>(), aa,
                          (const float *)U, (float *)fbond, virial_atom, atom_list, n_list);
   };
-  auto groups = [&](auto lc) {
-    switch (pad4(a.N) / 4) {
-      case 1: launch(lc, std::integral_constant<int, 1>{}); break;
-      case 2: launch(lc, std::integral_constant<int, 2>{}); break;
-      case 3: launch(lc, std::integral_constant<int, 3>{}); break;
-      default: launch(lc, std::integral_constant<int, 4>{}); break;
-    }
-  };
+  switch (pad4(a.N) / 4) {
+    case 1: launch(std::integral_constant<int, 1>{}); break;
+    case 2: launch(std::integral_constant<int, 2>{}); break;
+    case 3: launch(std::integral_constant<int, 3>{}); break;
+    default: launch(std::integral_constant<int, 4>{}); break;
+  }
   static_assert(kMaxN == 16, "radial groups of k_bond_forces");
-  groups(std::integral_constant<int, -1>{});
   FM_HIP(hipGetLastError());
 }
 

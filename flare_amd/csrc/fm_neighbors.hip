@@ -823,17 +823,16 @@ __global__ __launch_bounds__(kRowBlock) void k_species_count(int n, const int *s
 }
 
 // Row of each atom: the rows of the lower species and of the blocks before
-// (`off`, the scan of the counts above; with one block from the block itself),
-// then the atom's rank in its block. Block 0 also writes the species' atom
-// counts to the host, the slice-row shift of each species (its rows start a
-// tile of `tile` slice rows) and zeros for the bond counts by species.
+// (`off`, the scan of the counts above), then the atom's rank in its block. Block 0
+// also writes the species' atom counts to the host, the slice-row shift of each
+// species (its rows start a tile of `tile` slice rows) and zeros for the bond
+// counts by species.
 __global__ __launch_bounds__(kRowBlock) void k_species_rows(int n, const int *species, int nos,
                                                             const int *off, int *row_of_atom,
                                                             int *atom_of_row, int *host_by_type,
                                                             int tile, int *shift,
                                                             int *bonds_by_type) {
-  extern __shared__ int wc[];  // [16 waves][nos], then the species' first rows [nos + 1]
-  int *first = wc + 16 * nos;
+  extern __shared__ int wc[];  // [16 waves][nos]
   int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nb = gridDim.x;
   int i = blockIdx.x * kRowBlock + threadIdx.x;
   int sp = i < n ? species[i] : -1;
@@ -844,31 +843,23 @@ __global__ __launch_bounds__(kRowBlock) void k_species_rows(int n, const int *sp
     if (lane == 0) wc[w * nos + t] = __popcll(m);
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int o = 0;
-    for (int t = 0; t <= nos; t++) {
-      first[t] = nb > 1 ? off[(size_t)t * nb] : o;  // off[nos nb] = n
-      if (nb == 1 && t < nos)
-        for (int v = 0; v < 16; v++) o += wc[v * nos + t];
-    }
-  }
-  __syncthreads();
   if (sp >= 0) {
-    int r = (nb > 1 ? off[(size_t)sp * nb + blockIdx.x] : first[sp]) + rank;
+    int r = off[(size_t)sp * nb + blockIdx.x] + rank;
     for (int v = 0; v < w; v++) r += wc[v * nos + sp];
     row_of_atom[i] = r;
     atom_of_row[r] = i;
   }
   if (blockIdx.x == 0) {
+    auto first = [&](int t) { return off[(size_t)t * nb]; };  // first(nos) = n
     for (int t = threadIdx.x; t < nos; t += kRowBlock) {
-      host_by_type[t] = first[t + 1] - first[t];
+      host_by_type[t] = first(t + 1) - first(t);
       bonds_by_type[t] = 0;
     }
     if (threadIdx.x == 0) {
       int rows = 0;
       for (int t = 0; t < nos; t++) {
-        shift[t] = rows - first[t];
-        rows += (first[t + 1] - first[t] + tile - 1) / tile * tile;
+        shift[t] = rows - first(t);
+        rows += (first(t + 1) - first(t) + tile - 1) / tile * tile;
       }
     }
   }
@@ -989,7 +980,7 @@ void build_bonds(fm_structure s) {
     hipLaunchKernelGGL(k_species_count, dim3(nb), dim3(kRowBlock), nos * sizeof(int), st, n,
                        s->species.as<int>(), nos, hist.as<int>());
     scan_exclusive(ctx, hist.as<int>(), off.as<int>(), nos * nb);
-    hipLaunchKernelGGL(k_species_rows, dim3(nb), dim3(kRowBlock), (17 * nos + 1) * sizeof(int),
+    hipLaunchKernelGGL(k_species_rows, dim3(nb), dim3(kRowBlock), 16 * nos * sizeof(int),
                        st, n, s->species.as<int>(), nos, off.as<int>(), s->row_of_atom.as<int>(),
                        s->atom_of_row.as<int>(), host_types, kI8TileA, s->q_shift.as<int>(),
                        by_type.as<int>());
