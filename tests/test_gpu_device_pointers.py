@@ -11,6 +11,46 @@ pytestmark = pytest.mark.gpu
 RC = 4.0
 
 
+class Memory:
+    """Arrays in device or pinned host memory, by the HIP runtime itself."""
+
+    def __init__(self):
+        self.hip = ctypes.CDLL("libamdhip64.so")
+        p, n = ctypes.c_void_p, ctypes.c_size_t
+        for fn, args in (("hipMalloc", [ctypes.POINTER(p), n]), ("hipFree", [p]),
+                         ("hipHostMalloc", [ctypes.POINTER(p), n, ctypes.c_uint]),
+                         ("hipHostFree", [p]), ("hipMemcpy", [p, p, n, ctypes.c_int])):
+            getattr(self.hip, fn).argtypes = args
+        self.held = []
+
+    def get(self, size, pinned=False):
+        p = ctypes.c_void_p()
+        if pinned:
+            assert self.hip.hipHostMalloc(ctypes.byref(p), size, 0) == 0
+        else:
+            assert self.hip.hipMalloc(ctypes.byref(p), size) == 0
+        self.held.append((p, pinned))
+        return p.value
+
+    def put(self, p, a, size=None):
+        assert self.hip.hipMemcpy(p, a.ctypes.data, size or a.nbytes, 4) == 0
+
+    def read(self, p, a):
+        assert self.hip.hipMemcpy(a.ctypes.data, p, a.nbytes, 4) == 0
+        return a
+
+    def free(self):
+        for p, pinned in self.held:
+            assert (self.hip.hipHostFree if pinned else self.hip.hipFree)(p) == 0
+
+
+@pytest.fixture
+def memory():
+    m = Memory()
+    yield m
+    m.free()
+
+
 @pytest.fixture(scope="module")
 def system():
     return random_cell(50, 5, nos=2, scale=8.8, skew=0.2)
@@ -39,48 +79,37 @@ def create(fn, system, species, positions):
 
 
 @pytest.mark.parametrize("kind", ["device", "slice", "misaligned", "pinned"])
-def test_structure_sources(system, kind):
+def test_structure_sources(system, memory, kind):
     """Species and positions in the GPU's memory, inside a larger array, at an
     address that is no multiple of the element's size, and in pinned memory."""
-    import torch
     from flare_amd import _lib
-    sp, pos = _lib.i32(system[1]), _lib.f64(system[2]).reshape(-1)
-    rc, h = create("fm_structure_create", system, _lib.ptr(sp), _lib.ptr(pos))
+    arrays = [_lib.i32(system[1]), _lib.f64(system[2]).reshape(-1)]
+    rc, h = create("fm_structure_create", system, *map(_lib.ptr, arrays))
     _lib.check(rc)
     want = neighbors(h)
     lead = {"device": 0, "slice": 16, "misaligned": 2, "pinned": 0}[kind]
-    held = []
-    for a in (sp, pos):
-        raw = torch.zeros(lead + a.nbytes, dtype=torch.uint8)
-        raw[lead:] = torch.from_numpy(a.view(np.uint8))
-        held.append(raw.pin_memory() if kind == "pinned" else raw.cuda())
-    torch.cuda.synchronize()
-    rc, h = create("fm_structure_create_device", system, *(t.data_ptr() + lead for t in held))
+    ptrs = [memory.get(lead + a.nbytes, kind == "pinned") + lead for a in arrays]
+    for p, a in zip(ptrs, arrays):
+        memory.put(p, a)
+    rc, h = create("fm_structure_create_device", system, *ptrs)
     _lib.check(rc)
     got = neighbors(h)
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
 
 
 @pytest.mark.parametrize("short", [0, 1])
-def test_short_array(system, short):
+def test_short_array(system, memory, short):
     """An array shorter than the atom count is an error, as for a copy, and the
     next structure is built as if it had not been."""
     from flare_amd import _lib
-    hip = ctypes.CDLL("libamdhip64.so")
-    hip.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
-    hip.hipMemcpy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
-    hip.hipFree.argtypes = [ctypes.c_void_p]
     arrays = [_lib.i32(system[1]), _lib.f64(system[2]).reshape(-1)]
     rc, h = create("fm_structure_create", system, *map(_lib.ptr, arrays))
     _lib.check(rc)
     want = neighbors(h)
-    ptrs = []
-    for k, a in enumerate(arrays):
-        p = ctypes.c_void_p()
-        size = a.nbytes - (16 if k == short else 0)
-        assert hip.hipMalloc(ctypes.byref(p), size) == 0
-        assert hip.hipMemcpy(p, a.ctypes.data, size, 1) == 0
-        ptrs.append(p)
+    sizes = [a.nbytes - (16 if k == short else 0) for k, a in enumerate(arrays)]
+    ptrs = [memory.get(size) for size in sizes]
+    for p, a, size in zip(ptrs, arrays, sizes):
+        memory.put(p, a, size)
     for _ in range(5):
         rc, h = create("fm_structure_create_device", system, *ptrs)
         assert rc == _lib.FM_ERR_HIP
@@ -88,16 +117,13 @@ def test_short_array(system, short):
         _lib.check(rc)
         got = neighbors(h)
         assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
-    for p in ptrs:
-        assert hip.hipFree(p) == 0
 
 
 @pytest.mark.parametrize("reps", [2, 15])
 @pytest.mark.parametrize("where", ["device", "pinned", "mixed"])
-def test_prediction_outputs(reps, where):
+def test_prediction_outputs(memory, reps, where):
     """Results in device and in pinned memory, small ones (which reach pageable
     memory through a staging buffer) and large ones."""
-    import torch
     from flare_amd import _C_flare as C
     from flare_amd import _lib
     from helpers import fcc
@@ -118,14 +144,11 @@ def test_prediction_outputs(reps, where):
     want = [np.zeros(k) for k in sizes]
     predict([_lib.ptr(w) for w in want])
     assert (sum(sizes) * 8 > 256 << 10) == (reps == 15)
-    out = [torch.zeros(k, dtype=torch.float64) for k in sizes]
-    if where == "device":
-        out = [t.cuda() for t in out]
-    elif where == "pinned":
-        out = [t.pin_memory() for t in out]
-    else:
-        out[1] = out[1].cuda()
-    torch.cuda.synchronize()
-    predict([t.data_ptr() for t in out])
-    for t, w in zip(out, want):
-        assert np.array_equal(t.cpu().numpy(), w)
+    out = [np.zeros(k) for k in sizes]
+    ptrs = [_lib.ptr(o).value if where == "mixed" and k != 1
+            else memory.get(8 * sizes[k], where == "pinned") for k, o in enumerate(out)]
+    predict(ptrs)
+    for k, (p, o) in enumerate(zip(ptrs, out)):
+        if p != o.ctypes.data:
+            memory.read(p, o)
+        assert np.array_equal(o, want[k])
