@@ -315,7 +315,10 @@ static bool readable_in_place(fm_context ctx, const void *p, size_t bytes, size_
   return known && (uintptr_t)p % align == 0 && at <= size && bytes <= size - at;
 }
 
-// Host species and positions up to this many bytes join the pinned upload.
+// Host species and positions up to this many bytes join the pinned upload. It is
+// the faster way at every size measured (creating a structure of 1,024, 8,192,
+// 24,000 and 65,536 atoms: 59, 102, 164 and 334 us, with copies from pageable
+// memory 77, 119, 175 and 337); the limit bounds the pinned memory.
 constexpr size_t kStageAtoms = 256 << 10;
 // All of a structure's host arrays (some 450 bytes per structure of a batch) up to
 // this many bytes go through the context's pinned buffer, which it keeps.

@@ -819,7 +819,8 @@ __device__ __forceinline__ void stage_w_onepass(const float *G, const float *B, 
   if (tail) wl[kt] = w_elem(sg, gt, sb, bt);
 }
 
-// Longest row for the one-pass staging of k_dEdc<float, LC, true>.
+// Longest row whose G and B k_dEdc<float, LC, OP> holds in registers, OP = 4 up to
+// half of it and 8 above.
 constexpr int kOnePassRow = 128 * 32;
 
 // LC >= 0: l_max known at compile time (one accumulator per l up to it, in
